@@ -13,6 +13,8 @@
 //   small slices (short rows, or R x inner of a few KiB)  a workgroup stages a
 //               run of whole slices in LDS, a thread per column scans in
 //               place, the run goes back out as aligned packs;
+//   long rows   cut into chunks that scan side by side in one read, what lies
+//               before a chunk coming from the totals the others publish;
 //   long scans with few columns  chunk totals, their scan (this code again on
 //               the accumulator type), then every chunk scans from its carry.
 // Accumulation is fp32 for float and half (rounded per output element), double
@@ -371,6 +373,212 @@ __global__ __launch_bounds__(kBlock) void scan_cols_totals_kernel(typename ScanA
   }
 }
 
+// Accumulator of the one-read scan: the results of the integer types up to 4 bytes are their sums (products)
+// modulo 2^8, 2^16 or 2^32, which 32-bit arithmetic gives bit for bit as the wrapping 64-bit one does.
+template <typename T>
+struct OnePassAcc {
+  using type = typename std::conditional<std::is_integral<T>::value && sizeof(T) <= 4, uint32_t, typename ScanAcc<T>::type>::type;
+};
+template <typename Op, typename A>
+struct WithAcc;
+template <template <typename> class Op, typename Old, typename A>
+struct WithAcc<Op<Old>, A> {
+  using type = Op<A>;
+};
+constexpr int kOnePassPacks = 8;  // packs a lane holds
+
+// Wave-wide inclusive scan on the data-parallel-primitive lanes (row_shr 1, 2, 4, 8 inside the rows of 16
+// lanes, then lane 15 / 31 broadcast into the rows behind them): six VALU steps and no LDS traffic, where
+// a shuffle per step goes through the LDS pipe. Lanes without a source combine with the identity.
+template <typename A, int CTRL, int ROWS>
+__device__ __forceinline__ A dpp_or(A id, A v) {
+  constexpr int W = sizeof(A) / 4;
+  uint32_t a[W], b[W];
+  __builtin_memcpy(a, &id, sizeof(A));
+  __builtin_memcpy(b, &v, sizeof(A));
+#pragma unroll
+  for (int i = 0; i < W; ++i) b[i] = __builtin_amdgcn_update_dpp(a[i], b[i], CTRL, ROWS, 0xf, false);
+  __builtin_memcpy(&v, b, sizeof(A));
+  return v;
+}
+template <typename Op, typename A>
+__device__ __forceinline__ A wave_scan(A t) {
+  const A id = Op::id();
+  t = Op::op(dpp_or<A, 0x111, 0xf>(id, t), t);
+  t = Op::op(dpp_or<A, 0x112, 0xf>(id, t), t);
+  t = Op::op(dpp_or<A, 0x114, 0xf>(id, t), t);
+  t = Op::op(dpp_or<A, 0x118, 0xf>(id, t), t);
+  t = Op::op(dpp_or<A, 0x142, 0xa>(id, t), t);
+  t = Op::op(dpp_or<A, 0x143, 0xc>(id, t), t);
+  return t;
+}
+template <typename A>
+__device__ __forceinline__ A read_lane(A v, int lane) {
+  return lane_exchange(v, [lane](uint32_t w) { return (uint32_t)__builtin_amdgcn_readlane((int)w, lane); });
+}
+
+// Accumulator values published between workgroups: every 32-bit half of the value is a 64-bit word
+// (1 << 32) | half, stored and loaded with relaxed device-scope atomics. Word 0 is "not there yet", so
+// value and flag arrive together and no fence (which would write back an XCD's L2) is needed.
+template <typename A>
+__device__ __forceinline__ void publish_word(uint64_t* words, A v) {
+  constexpr int W = sizeof(A) / 4;
+  uint32_t h[W];
+  __builtin_memcpy(h, &v, sizeof(A));
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+    __hip_atomic_store(words + i, (uint64_t(1) << 32) | h[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename A>
+__device__ __forceinline__ bool poll_word(const uint64_t* words, A& v) {
+  constexpr int W = sizeof(A) / 4;
+  uint32_t h[W];
+  uint64_t there = uint64_t(1) << 32;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const uint64_t w = __hip_atomic_load(words + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    there &= w;
+    h[i] = (uint32_t)w;
+  }
+  __builtin_memcpy(&v, h, sizeof(A));
+  return there != 0;
+}
+
+__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) words[i] = 0;
+}
+
+// Long rows in ONE read of the input. A row is cut into chunks of BT * 8 packs; a workgroup of BT threads draws a
+// chunk by ticket, keeps its packs in registers, publishes the chunk's total, adds up what lies before
+// the chunk and stores. What lies before is a sum over a tree that the position alone fixes, so every run
+// gives the same bits: the totals of the chunks before it in its group of 64, of the groups before that one
+// in their group of 64 (a group's total is published by its last chunk), and of those of 64 x 64. Nothing
+// waits for a chain of carries: a total waits for no other total, a group's for the 63 totals before it.
+// Every wait ends: tickets are drawn in order, so all chunks before this one belong to workgroups that
+// are running or done, and each of them publishes its total before it waits for anything.
+// Bound by reads and writes of HBM at the large sizes, by ticket, look-back and chunk latency below 2^22 elements.
+// fp32, before (totals of pieces, their scan, then every piece from its carry: two reads, 3 to 5 launches) and
+// now: 2^26 elements 178 -> 110 us (4.9 TB/s on 8 bytes an element), 2^24 56 -> 31, 2^22 40 -> 14, 2^17 22 -> 6.5,
+// 1000 x 65536 145 -> 99, 1000 x 16384 44 -> 24; the error against float64 sums halves (1.2e-7 -> 6.5e-8).
+// A chunk costs about 13 ns at its row's ticket and look-back words wherever it runs, so chunks have to be large:
+// 16 KiB chunks took 525 us on 2^26 elements, 64 KiB 116, 128 KiB 110, 256 KiB 115 (too few in flight).
+// words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, all zeroed, W words per value.
+// In place (out == in) is fine: a chunk is read only by the workgroup that then writes it.
+// words == nullptr: every row is one chunk (S == 1), nothing to look back for.
+template <typename T, typename Op, int BT>
+__global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, uint64_t* words, uint32_t* ticket,
+                                                              uint32_t outer, uint64_t R, uint32_t S, uint32_t S1,
+                                                              uint32_t S2, int nts) {
+  using A = typename OnePassAcc<T>::type;
+  constexpr int VEC = 16 / sizeof(T), W = sizeof(A) / 4, kWaves = BT / 64, K = kOnePassPacks;
+  constexpr uint32_t kSeg = 64 * VEC;  // elements of one pack per lane of a wave
+  constexpr uint32_t kChunk = kSeg * K * kWaves;
+  using P = Pack<T, VEC>;
+  __shared__ uint32_t drawn;
+  __shared__ A waveTotal[kWaves];
+  __shared__ A carryS;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t t = blockIdx.x;
+  if (words) {
+    if (threadIdx.x == 0) drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    t = __builtin_amdgcn_readfirstlane(drawn);
+  }
+  const uint32_t row = t / S, c = t - row * S;
+  const uint64_t first = (uint64_t)c * kChunk + wave * (kSeg * K);  // the wave's first element in its row
+  const T* src = in + (uint64_t)row * R + first;
+  T* dst = out + (uint64_t)row * R + first;
+  const uint64_t left = R > first ? R - first : 0;
+  const bool full = left >= kSeg * K;
+  const T idT = scan_down<T>(Op::id());
+  P v[K];
+  if (full) {
+#pragma unroll
+    for (int u = 0; u < K; ++u) v[u] = load_pack_unaligned<true, P>(src + u * kSeg + lane * VEC);
+  } else {
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      const uint32_t i0 = u * kSeg + lane * VEC;
+      if (i0 + VEC <= left) {
+        v[u] = load_pack_unaligned<true, P>(src + i0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[u].v[e] = i0 + e < left ? src[i0 + e] : idT;
+      }
+    }
+  }
+  // what lies before each pack inside the wave's part
+  A off[K], run = Op::id();
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    A tot = scan_up<A>(v[u].v[0]);
+#pragma unroll
+    for (int e = 1; e < VEC; ++e) tot = Op::op(tot, scan_up<A>(v[u].v[e]));
+    tot = wave_scan<Op>(tot);
+    off[u] = Op::op(run, dpp_or<A, 0x138, 0xf>(Op::id(), tot));
+    run = Op::op(run, read_lane(tot, 63));
+  }
+  if (lane == 0) waveTotal[wave] = run;
+  lds_barrier();
+  A before = Op::id(), total = Op::id();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if ((uint32_t)w == wave) before = total;
+    total = Op::op(total, waveTotal[w]);
+  }
+  if (words) {
+    if (wave == 0) {
+      uint64_t* w0 = words + (uint64_t)row * S * W;
+      uint64_t* w1 = words + ((uint64_t)outer * S + (uint64_t)row * S1) * W;
+      uint64_t* w2 = words + ((uint64_t)outer * (S + S1) + (uint64_t)row * S2) * W;
+      if (lane == 0) publish_word(w0 + (uint64_t)c * W, total);
+      const uint32_t g = c / 64, j = c % 64, sg = g / 64, gj = g % 64;
+      // lanes below `n` wait for words[lane]; their sum, in the order of wave_scan
+      auto sum_of = [&](const uint64_t* w, uint32_t n) -> A {
+        A x = Op::id();
+        bool have = lane >= n;
+        while (!__all(have)) {
+          if (!have) have = poll_word(w + (uint64_t)lane * W, x);
+        }
+        if (lane >= n) x = Op::id();
+        return read_lane(wave_scan<Op>(x), 63);
+      };
+      A carry = j ? sum_of(w0 + (uint64_t)(c - j) * W, j) : Op::id();
+      if (j == 63 && lane == 0) publish_word(w1 + (uint64_t)g * W, Op::op(carry, total));
+      if (gj) carry = Op::op(sum_of(w1 + (uint64_t)(g - gj) * W, gj), carry);
+      if (j == 63 && gj == 63 && lane == 0) publish_word(w2 + (uint64_t)sg * W, Op::op(carry, total));
+      if (sg) {
+        A far = Op::id();
+        for (uint32_t b = 0; b < sg; b += 64) far = Op::op(far, sum_of(w2 + (uint64_t)b * W, min(64u, sg - b)));
+        carry = Op::op(far, carry);
+      }
+      if (lane == 0) carryS = carry;
+    }
+    lds_barrier();
+    before = Op::op(carryS, before);
+  }
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    const uint32_t i0 = u * kSeg + lane * VEC;
+    const A base = Op::op(before, off[u]);
+    P r;
+    A sum = Op::id();
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      sum = e ? Op::op(sum, scan_up<A>(v[u].v[e])) : scan_up<A>(v[u].v[0]);
+      r.v[e] = scan_down<T>(Op::op(base, sum));
+    }
+    if (full || i0 + VEC <= left) {
+      if (nts) store_pack_unaligned<true>(dst + i0, r);
+      else store_pack_unaligned<false>(dst + i0, r);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        if (i0 + e < left) dst[i0 + e] = r.v[e];
+    }
+  }
+}
+
 // Small slices of the dense [outer][R][inner] block (short rows when
 // inner == 1): a wave per row, or a workgroup per slice and column tile,
 // leaves most lanes idle (10-element rows scanned at 0.24 TB/s, 8 x 16 slices
@@ -562,10 +770,6 @@ __global__ __launch_bounds__(kBlock) void scan_chunk_totals_kernel(
 // that chunk's column total itself from the input, in the owner's order of operations. A grid that
 // is not resident all at once (the GPU shared with other work) therefore still ends.
 constexpr uint32_t kKindTotal = 1, kKindPrefix = 2;
-
-__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) words[i] = 0;
-}
 
 template <typename T, typename Op>
 __global__ __launch_bounds__(kBlock) void scan_lookback_kernel(T* __restrict__ out, const T* __restrict__ in,
@@ -759,13 +963,52 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // totals of 32 KiB chunks of rows, their scan (this function again, on the
   // accumulator type), then every chunk scans from its carry. The input is
   // read twice, which still is 500x faster.
-  // Few long rows (a 1-D cumsum above all): a wave per row leaves the chip idle, and the chunks of rows
-  // below hand every thread a contiguous band of its chunk in LDS, 32 elements apart from its
-  // neighbour's, i.e. all lanes in one bank (2^26 elements: 0.12 of peak). Instead every row is cut
-  // into pieces that scan side by side, a wave per piece: totals of the pieces, their scan by this
-  // function on the accumulator type, then every piece from its carry (0.12 -> 0.44 with 8 workgroups of
-  // pieces per CU; 0.39 with 2, 0.42 with 4). The input is read twice.
-  if (inner == 1 && tuning("scan.rows.split", 1)) {
+  // Long rows, up to 16 per CU (a 1-D cumsum above all): a wave per row leaves the chip idle, and a wave
+  // walks its row at a microsecond per KiB or two. They are cut into chunks that scan side by side in one
+  // read; from 4096 elements (one row of 4097: 18 us with a wave, 4.4 this way; 1000 rows of 5001: 28 and
+  // 11; 4000 rows of 5001: 57 and 35, 4000 of 16384: 133 and 97). A row that fits 1024 threads x 8 packs is
+  // one chunk and looks back for nothing (15571 elements: 4.4 us, 7.2 as two chunks). Longer rows: chunks of
+  // 1024 threads where that still gives two workgroups per CU (2^24 fp32: 32 us against 38 with 512 threads
+  // and 50 with 256; 2^20: 9.6 against 8.5), else of 512; 1-byte elements always 512, since their 128 elements
+  // a lane take more registers than 1024 threads have (2^27 bytes: 74 us against 236).
+  // Products of floating elements keep the two reads of scan_rows_kernel's pieces below: the product of a chunk
+  // that overflows turns a zero before it into NaN, and these chunks are longer than those pieces.
+  constexpr bool kFloatProduct =
+      std::is_same<Op, ScanMul<typename ScanAcc<T>::type>>::value && !std::is_integral<T>::value;
+  if constexpr (!kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1) && outer > 0 && R >= 4096) {
+    using A = typename OnePassAcc<T>::type;
+    using OpA = typename WithAcc<Op, A>::type;
+    const int64_t cus = num_compute_units(s), unit = (int64_t)kFull * kOnePassPacks;  // elements per thread
+    const auto chunks = [&](int64_t threads) { return outer * ((R + threads * unit - 1) / (threads * unit)); };
+    const int64_t most = sizeof(T) == 1 ? 512 : 1024;
+    int64_t threads = chunks(most) >= 2 * cus ? most : 512;
+    for (int64_t one = most; one >= 256; one /= 2)
+      if (R <= one * unit) threads = one;
+    const int64_t S = chunks(threads) / outer, S1 = S / 64, S2 = S1 / 64;
+    if (!scratch) scratch = (char*)scratch_space(s, &scratchBytes);
+    const uint64_t nwords = (uint64_t)(outer * (S + S1 + S2)) * (sizeof(A) / 4) + 1;  // the last one is the ticket
+    if (outer <= 16 * cus && outer * S < (int64_t(1) << 31) && nwords * sizeof(uint64_t) <= scratchBytes) {
+      uint64_t* words = S > 1 ? (uint64_t*)scratch : nullptr;
+      uint32_t* ticket = (uint32_t*)((uint64_t*)scratch + (nwords - 1));
+      if (words)
+        hipLaunchKernelGGL(scan_clear_words_kernel, dim3((unsigned)std::min<uint64_t>((nwords + kBlock - 1) / kBlock, 1024)),
+                           dim3(kBlock), 0, st, words, nwords);
+      const auto go = [&](auto tag) {
+        constexpr int BT = decltype(tag)::value;
+        hipLaunchKernelGGL((scan_onepass_kernel<T, OpA, BT>), dim3((unsigned)(outer * S)), dim3(BT), 0, st, out, in, words,
+                           ticket, (uint32_t)outer, (uint64_t)R, (uint32_t)S, (uint32_t)S1, (uint32_t)S2, streaming);
+      };
+      if (threads == 256) go(std::integral_constant<int, 256>{});
+      else if (threads == 512 || sizeof(T) == 1) go(std::integral_constant<int, 512>{});
+      else go(std::integral_constant<int, sizeof(T) == 1 ? 512 : 1024>{});
+      note_kernel("scan-rows-split");
+      return;
+    }
+  }
+  // Few long rows of floating products: every row is cut into pieces that scan side by side, a wave per piece:
+  // totals of the pieces, their scan by this function on the accumulator type, then every piece from its carry.
+  // The input is read twice (2^26 fp32: 175 us).
+  if constexpr (kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1)) {
     using A = typename ScanAcc<T>::type;
     const bool vec = aligned && R % VEC == 0;
     const int64_t perIter = 64 * (vec ? VEC : 1) * 4;  // elements a wave takes per iteration

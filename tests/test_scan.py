@@ -308,3 +308,44 @@ def test_gpu_scan_over_a_strided_dim_in_every_strip_width(thc, oracle, kind):
         thc.set_tuning("scan.cols.prefetch", -1)
         thc.set_tuning("scan.cols.min_tx", 8)
         thc.set_tuning("scan.cols.max_tx", 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "int", "double", "byte", "long"])
+def test_gpu_one_read_scans_at_the_edges_of_their_chunks(thc, kind):
+    """Rows of 4096 elements and more are cut into chunks of 256, 512 or 1024 threads x 8 packs: lengths one
+    below, at and one above every chunk and every group of 64 chunks, rows and offsets off the 16-byte
+    grid. Exact on small integers; a NaN reaches everything behind it and nothing before."""
+    dtype = {"float": np.float32, "half": np.float16, "int": np.int32, "double": np.float64, "byte": np.uint8,
+             "long": np.int64}[kind]
+    unit = 16 // np.dtype(dtype).itemsize * 8
+    rng = np.random.default_rng(31)
+    sizes = [4096, 4097] + [n + d for n in (256 * unit, 512 * unit, 1024 * unit, 64 * 512 * unit) for d in (-1, 0, 1) if n + d >= 4096]
+    for n in sizes:
+        for rows, off in ((1, 0), (3, 1)):
+            every = 6000 if kind == "byte" else 600
+            x = ((rng.integers(0, every, rows * n + off) == 0) * rng.integers(0 if kind == "byte" else -2, 3, rows * n + off)).astype(dtype)
+            dev = thc.Tensor.from_storage(x, off, (rows, n), (n, 1), kind=kind)
+            got = thc.Tensor(kind).cumsum(dev, 1)
+            assert thc.last_kernel() == "scan-rows-split", (n, thc.last_kernel())
+            want = np.cumsum(x[off:].reshape(rows, n).astype(np.int64), axis=1)
+            assert kind not in ("half", "float") or np.abs(want).max() < 2048
+            assert_bit_equal(got.numpy(), want.astype(dtype), "%s %d x %d" % (kind, rows, n))
+    if kind in ("float", "half", "double"):
+        n = 64 * 512 * unit + 5
+        for at in (0, 4097, 512 * unit, n - 1):
+            x = np.zeros(n, dtype)
+            x[::5000] = 1
+            want = np.cumsum(x.astype(np.float64)).astype(dtype)
+            x[at] = want[at:] = np.nan
+            assert_bit_equal(thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 0).numpy(), want, "%s NaN at %d" % (kind, at))
+
+
+@pytest.mark.gpu
+def test_gpu_one_read_scan_beyond_4096_chunks(thc):
+    """More than 64 x 64 chunks in a row: the third level of published totals."""
+    n = 4097 * 1024 * 32 + 3
+    x = (np.arange(n, dtype=np.int32) % 7) - 2
+    got = thc.Tensor("int").cumsum(thc.Tensor.from_numpy(x), 0)
+    assert thc.last_kernel() == "scan-rows-split"
+    assert_bit_equal(got.numpy(), np.cumsum(x, dtype=np.int32))
