@@ -9,6 +9,7 @@ not been built (`python -m cutorch_amd.build`): there is no fallback path.
 """
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -33,6 +34,7 @@ class _Tensor(C.Structure):
 _lib = None
 _state = None
 _err_cb = None
+_pending = None     # the library's count of threads that hold an error message
 
 
 class THCError(RuntimeError):
@@ -41,12 +43,13 @@ class THCError(RuntimeError):
 
 def lib():
     """The loaded libTHC.so (loads on first use)."""
-    global _lib, _err_cb
+    global _lib, _err_cb, _pending
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise ImportError("%s is missing: run `python -m cutorch_amd.build`" % LIB_PATH)
         _lib = C.CDLL(LIB_PATH)
         _declare(_lib)
+        _pending = C.c_long.in_dll(_lib, "THCAmd_pendingErrors")
         # Handlers that return: the failed entry point returns to us and the
         # message is picked up from THCAmd_lastError by _check().
         _err_cb = (C.CFUNCTYPE(None, C.c_char_p, C.c_void_p)(lambda m, d: None),
@@ -57,6 +60,10 @@ def lib():
 
 
 def _check():
+    # A plain read: the question for this thread's own message is a foreign call (0.25 us of every method)
+    # and is put only while some thread holds one.
+    if not _pending.value:
+        return
     msg = _lib.THCAmd_lastError()
     if msg:
         text = msg.decode()
@@ -92,6 +99,7 @@ _TYPES = {
 _COPY_SUFFIX = {"byte": "Byte", "char": "Char", "short": "Short", "int": "Int", "long": "Long",
                 "float": "Float", "double": "Double", "half": "Half"}
 _FLOAT_KINDS = ("float", "half")
+_FUNCTIONS = {kind: {} for kind in _TYPES}      # method name -> foreign function, filled as they are used
 
 
 def _declare(l):
@@ -220,8 +228,20 @@ def _longs(seq):
 
 
 def _half_bits(v):
+    if type(v) in (int, float):     # numpy's conversion of one number takes a microsecond
+        try:
+            return _HALF_BITS.unpack(_HALF.pack(v))[0]
+        except (OverflowError, struct.error):      # beyond half's range
+            pass
+    return _half_bits_numpy(v)
+
+
+def _half_bits_numpy(v):
     with np.errstate(over="ignore"):          # a scalar beyond half's range is +-inf, as in C
         return int(np.array(v, dtype=np.float16).view(np.uint16))
+
+
+_HALF, _HALF_BITS = struct.Struct("<e"), struct.Struct("<H")
 
 
 class Tensor(object):
@@ -230,11 +250,15 @@ class Tensor(object):
     def __init__(self, kind="float", handle=None):
         self.kind = kind
         self.T, self.S, self.creal, self.np_dtype = _TYPES[kind]
+        self._fns = _FUNCTIONS[kind]
         self._st = state()
         self.h = handle if handle is not None else self._fn("new")(self._st)
 
     def _fn(self, name):
-        return getattr(lib(), self.T + "_" + name)
+        f = self._fns.get(name)
+        if f is None:
+            f = self._fns[name] = getattr(lib(), self.T + "_" + name)
+        return f
 
     def _sfn(self, name):
         return getattr(lib(), self.S + "_" + name)

@@ -26,6 +26,11 @@ struct THCState {
   size_t scratchBytes = 0;
 };
 
+// Threads whose THCAmd_lastError holds a message; a binding reads it instead of asking after every call.
+extern "C" {
+__attribute__((visibility("default"))) long THCAmd_pendingErrors = 0;
+}
+
 namespace thc {
 
 namespace {
@@ -79,7 +84,9 @@ void raise_arg_error(int arg, const char* fmt, ...) {
 }
 
 void deliver_error(const Error& e) noexcept {
+  const bool pending = !t_last_error.empty();
   t_last_error = e.arg > 0 ? "invalid argument " + std::to_string(e.arg) + ": " + e.msg : e.msg;
+  if (!pending && !t_last_error.empty()) __atomic_fetch_add(&THCAmd_pendingErrors, 1, __ATOMIC_RELAXED);
   if (e.arg > 0 && g_arg_handler) {
     g_arg_handler(e.arg, e.msg.c_str(), g_arg_data);
     return;
@@ -181,7 +188,10 @@ THC_API void THSetArgErrorHandler(THArgErrorHandlerFunction h, void* data) {
 THC_API const char* THCAmd_lastError(void) {
   return t_last_error.empty() ? nullptr : t_last_error.c_str();
 }
-THC_API void THCAmd_clearLastError(void) { t_last_error.clear(); }
+THC_API void THCAmd_clearLastError(void) {
+  if (!t_last_error.empty()) __atomic_fetch_sub(&THCAmd_pendingErrors, 1, __ATOMIC_RELAXED);
+  t_last_error.clear();
+}
 
 THC_API THCState* THCState_alloc(void) {
   THCState* state = new THCState();
