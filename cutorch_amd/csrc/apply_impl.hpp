@@ -750,6 +750,19 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_kernel(TOut* out, const T*
   }
 }
 
+// Offset of column q of operand k: q runs over the args.nq fused dims, innermost first.
+template <typename I>
+__device__ __forceinline__ I column_offset(const TiledArgs<I>& args, int k, uint32_t q) {
+  if (args.nq == 1) return (I)q * args.strideQ[k];
+  I off = 0;
+  for (int j = 0; j < args.nq - 1; ++j) {
+    uint32_t c;
+    args.qsub[j].divmod(q, q, c);
+    off += (I)c * args.qstride[k][j];
+  }
+  return off + (I)q * args.qstride[k][args.nq - 1];
+}
+
 // The tiled kernel for rows that do not start on 16-byte boundaries (odd
 // sizes, views at odd offsets). Every global access is still an aligned
 // 16-byte pack: a lane row covers a window of LX*VEC elements that starts at
@@ -797,8 +810,8 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
 #pragma unroll
   for (int k = 0; k < NOPS; ++k) {
     if (staged[k]) {
-      vo[k] = lyp * (uint32_t)args.strideQ[k];
-      rowStep[k] = (size_t)ROWS_P * (size_t)args.strideQ[k];
+      vo[k] = 0;   // (column_offset places every row)
+      rowStep[k] = 0;
     } else {
       vo[k] = lyq * (uint32_t)args.strideP[k];
       rowStep[k] = (size_t)ROWS_Q * (size_t)args.strideP[k];
@@ -836,7 +849,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
     const T* tbase[kMaxOps];
 #pragma unroll
     for (int k = 0; k < NOPS; ++k)
-      tbase[k] = ptr[k] + (base[k] + (I)p0 * args.strideP[k] + (I)q0 * args.strideQ[k]);
+      tbase[k] = ptr[k] + (base[k] + (I)p0 * args.strideP[k] + (staged[k] ? (I)0 : (I)q0 * args.strideQ[k]));
 
     // phase 1: staged inputs, lanes along p, into lds[slot][q][p]
 #pragma unroll
@@ -848,7 +861,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
 #pragma unroll
       for (int r = 0; r < PASSES_P; ++r) {
         const int qi = (int)lyp + r * ROWS_P;
-        const T* row = tbase[k] + r * rowStep[k] + vo[k];
+        const T* row = tbase[k] + column_offset(args, k, q0 + (uint32_t)min(qi, qn - 1));
         first[r] = (int)(lxp * VEC) - misalignment(row);
         if (qi < qn && first[r] < pn)
           v[r] = args.ntLoad ? load_pack<true>(reinterpret_cast<const P*>(row + first[r]))
@@ -961,6 +974,9 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
   using P = Pack<T, VEC>;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T* lds = reinterpret_cast<T*>(lds_raw);
+  // Fused q: the offsets of the tile's columns, worked out once per column (the divisions in front of every load
+  // broke the batch of loads up and made even the unfused kernel spill: 1266 us on 1001 x 1003 x 129, 390 this way).
+  __shared__ I columnOff[2][SPAN];
 
   const T* ptr[kMaxOps] = {out, in0, in1, in2};
   const uint32_t lxp = threadIdx.x % LXP, lyp = threadIdx.x / LXP;
@@ -1008,6 +1024,15 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
     const int qL = (int)(tq * TQ) - (LINE - 1);  // the first column any row of this tile may hold
     const bool interior = pn == TP && qL >= 0 && qL + SPAN <= sizeQ;
 
+    if (args.nq > 1) {
+#pragma unroll
+      for (int k = 1; k < NOPS; ++k) {
+        if (!staged[k]) continue;
+        for (int cq = (int)threadIdx.x; cq < SPAN; cq += kBlock)
+          columnOff[slot[k] & 1][cq] = column_offset(args, k, (uint32_t)min(max(qL + cq, 0), sizeQ - 1));
+      }
+      lds_barrier();
+    }
     auto body = [&](auto fullTag) {
       constexpr bool FULL = decltype(fullTag)::value;
       // phase 1: staged inputs, lanes along p, LDS row cq holds column qL + cq
@@ -1017,20 +1042,25 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
         T* slab = lds + slot[k] * (SPAN * PITCH);
         const T* origin = ptr[k] + (base[k] + (I)p0 * args.strideP[k]) + lxp * VEC;  // unit stride along p
         P v[PASSES_P];
+        auto request = [&](auto&& offset) {
 #pragma unroll
-        for (int r = 0; r < PASSES_P; ++r) {
-          const int cq = (int)lyp + r * ROWS_P, q = qL + cq;
-          const bool row = cq < SPAN && (FULL || (q >= 0 && q < sizeQ));
-          const int have = FULL ? VEC : pn - (int)(lxp * VEC);
-          if (row && have >= VEC) {
-            const T* at = origin + (I)q * args.strideQ[k];
-            v[r] = args.ntLoad ? load_loose_pack<true, P>(at) : load_loose_pack<false, P>(at);
-          } else if (row) {
+          for (int r = 0; r < PASSES_P; ++r) {
+            const int cq = (int)lyp + r * ROWS_P, q = qL + cq;
+            const bool row = cq < SPAN && (FULL || (q >= 0 && q < sizeQ));
+            const int have = FULL ? VEC : pn - (int)(lxp * VEC);
+            if (row && have >= VEC) {
+              const T* at = origin + offset(cq, q);
+              v[r] = args.ntLoad ? load_loose_pack<true, P>(at) : load_loose_pack<false, P>(at);
+            } else if (row) {
+              const T* at = origin + offset(cq, q);
 #pragma unroll
-            for (int e = 0; e < VEC; ++e)
-              if (e < have) v[r].v[e] = origin[(I)q * args.strideQ[k] + e];
+              for (int e = 0; e < VEC; ++e)
+                if (e < have) v[r].v[e] = at[e];
+            }
           }
-        }
+        };
+        if (args.nq > 1) request([&](int cq, int) { return columnOff[slot[k] & 1][cq]; });
+        else request([&](int, int q) { return (I)q * args.strideQ[k]; });
 #pragma unroll
         for (int r = 0; r < PASSES_P; ++r) {
           const int cq = (int)lyp + r * ROWS_P;
@@ -1369,7 +1399,7 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
     ldsR = (size_t)nstaged * (tqV + kRaggedSlack) * (tpV + 1) * sizeof(T);
     // (48 KiB: one staged operand of 4-byte elements; two of them leave one workgroup per CU, and
     // x:t() * y:t() on 8191 x 8193 then ran at 0.47-0.51 of peak against 0.57 with the shifted windows)
-    ragged = shift && ldsR <= 48 * 1024 && tuning("apply.tiled.ragged", 1);
+    ragged = shift && ldsR <= 48 * 1024 && nstaged <= 2 && tuning("apply.tiled.ragged", 1);
   }
   if (!vec && !shift && ldsS > 64 * 1024) return false;
   const int64_t tileP = vec || ragged ? tpV : (shift ? tpV - VEC : tS);
@@ -1382,14 +1412,17 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
     args.strideQ[k] = (I)pl.lay[k].stride[q];
   }
   // Fuse into q the dims just outside it that continue q's run for every
-  // direct operand (vector variant only: there q has unit stride for them).
+  // direct operand (not the element-wise variant: in the others q has unit stride for them). With odd
+  // sizes as well: on 414 x 646 x 51 floats, all dims of one operand reversed, tiles of 51 of their 128
+  // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390
+  // (halves: 252 and 206); the remap to XCDs stays on for them, their rows sharing lines as unfused ones do.
   bool inQ[kMaxDims] = {};
   inQ[q] = true;
   int64_t sizeQ = pl.lay[0].size[q];
   args.nq = 1;
   args.qsub[0].set((uint64_t)sizeQ);
   for (int k = 0; k < pl.nops; ++k) args.qstride[k][0] = (I)pl.lay[k].stride[q];
-  if (vec && tuning("apply.tiled.fuse_q", 1)) {
+  if ((vec || shift) && tuning("apply.tiled.fuse_q", 1)) {
     for (int d = q - 1; d >= 0 && d != p && args.nq < kMaxFuse; --d) {
       bool ok = sizeQ * pl.lay[0].size[d] < kIndex32Limit;
       for (int k = 0; k < pl.nops && ok; ++k)
@@ -1451,7 +1484,7 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   const int64_t swz = tuning("apply.tiled.xcd_swizzle", 1);
   // (not with fused q: there the direct operands are one long aligned run and
   // the remap cost 2% on a permuted 2048 x 2048 x 520 operand)
-  if ((swz == 2 || (swz == 1 && !lineAligned && args.nq == 1)) && total >= 64 && total < (int64_t(1) << 28))
+  if ((swz == 2 || (swz == 1 && !lineAligned && (args.nq == 1 || !vec))) && total >= 64 && total < (int64_t(1) << 28))
     args.xcdPer = (uint32_t)((total + 7) / 8);
   const int64_t slots = args.xcdPer ? (int64_t)args.xcdPer * 8 : total;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(slots, tuning("apply.tiled.max_grid", 1 << 22)));
