@@ -18,9 +18,11 @@
 //     staging mask), the index type is 64-bit for tile origins only, and the
 //     input and output element types may differ (comparisons, conversions).
 // Rows that are not whole aligned packs (odd sizes, views at odd offsets) take
-// the same kernel with ALIGNED = false: every global access is still an aligned
-// pack covering a window that starts at or below the row piece's first
-// element; the element-wise LDS accesses absorb each operand's own shift.
+// the same kernel with ALIGNED = false: the transposed inputs are read as packs
+// at element-aligned addresses (bytes: word-aligned ones), so that the compute
+// loop reads their slab at constant offsets; the output is written as aligned
+// packs, every row being cut at its own pack boundaries; the other inputs are read
+// as aligned packs over a window that starts at or below the row piece's first element.
 #pragma once
 
 namespace thc {
@@ -59,10 +61,14 @@ struct LdsTileArgs {
 //
 // ALIGNED: the tile is the window, WP x WQ; the transposed slab is [WQ][PITCH_S], the plain slab
 // [WP][WQ].
-// Otherwise a tile advances by TP = WP - VEC and TQ = WQ - VEC, one pack less than the window, and
-//   * along p (transposed inputs) a row's window starts at the aligned pack at or below the tile's
-//     first element of that row, so window element w is tile coordinate w - m, m < VEC the row's
-//     own misalignment;
+// Otherwise a tile is WP wide along p (bytes: a word less) and advances by TQ = WQ - VEC along q, one pack less than the
+// window, and
+//   * along p (transposed inputs) a lane's pack starts at the tile's own coordinate, one 16-byte load at an
+//     element-aligned address. 1-byte elements start at the 32-bit word that holds the tile's first element of the
+//     row, m < GRID elements before it: at byte alignment the loads are slow (a transposed add of 8191 x 8193
+//     bytes: 126 us at byte alignment, 64 at word alignment, 74 with the 16-byte aligned windows and an offset
+//     per element that this replaced; halves: exp 84 at element alignment, 88 at word alignment, 92 before). The
+//     last packs of a tensor row are moved back so that they end with the row (with the word of its last byte);
 //   * along q every OUTPUT row cuts the tensor at its own pack boundaries: with mo < VEC the
 //     misalignment of the output row at column q0, the tile owns of that row the 31 whole packs
 //     [q0 - mo, q0 - mo + TQ). No pack is split between two tiles, so partial (element-wise) stores
@@ -77,7 +83,9 @@ struct LdsTileShape {
   static constexpr int W = sizeof(T) > sizeof(TOut) ? sizeof(T) : sizeof(TOut);
   static constexpr int VEC = 16 / W;
   static constexpr int WP = LXP * VEC, WQ = LXQ * VEC;  // window: lanes x pack
-  static constexpr int TP = ALIGNED ? WP : WP - VEC, TQ = ALIGNED ? WQ : WQ - VEC;
+  static constexpr int EPW = sizeof(T) >= 4 ? 1 : 4 / (int)sizeof(T);   // elements per word
+  static constexpr int GRID = sizeof(T) == 1 ? 4 : 1;   // unaligned windows start at multiples of it
+  static constexpr int TP = ALIGNED ? WP : WP - (GRID - 1), TQ = ALIGNED ? WQ : WQ - VEC;
   static constexpr int ROWS_P = kBlock / LXP, ROWS_Q = kBlock / LXQ;
   static constexpr int NP_S = WQ / ROWS_P;                 // packs per lane, lanes along p
   static constexpr int NP_D = (TP + ROWS_Q - 1) / ROWS_Q;  // packs per lane, lanes along q
@@ -88,23 +96,22 @@ struct LdsTileShape {
   // pack of sub-word elements word-aligned in LDS (16-byte LDS writes at 2-byte alignment stall the
   // LDS pipeline: half and short tiles spent a fifth of their time in such stalls); the odd word
   // count spreads rows over the banks.
-  static constexpr int EPW = sizeof(T) >= 4 ? 1 : 4 / (int)sizeof(T);   // elements per word
-  // Unaligned rows of sub-word elements: the transposed slab keeps every row's WINDOW as loaded
-  // (pack j at column j * VEC, a word-aligned LDS write) instead of shifting it into place, and
-  // the readers add the row's shift, which they derive from the row number.
-  static constexpr bool WIN = !ALIGNED && sizeof(T) < 4;
-  // (shifted into place, a row occupies columns MARG - (VEC - 1) .. MARG + WP - 1)
-  static constexpr int PITCH_S = (((ALIGNED || WIN ? WP : WP + VEC) + EPW - 1) / EPW | 1) * EPW;
-  static constexpr int ROWS_S = ALIGNED ? WQ : WQ + VEC;   // (lane 31 of an unaligned tile reads past row WQ: never stored)
+  static constexpr int PITCH_S = ((WP + EPW - 1) / EPW | 1) * EPW;
+  static constexpr int ROWS_S = WQ;
   // plain slab: row p's window from column MARG on; readers look up to 2 VEC - 2 columns beyond it
   static constexpr int PITCH_D = ALIGNED ? WQ : WQ + 3 * VEC;
   static constexpr int ROWS_D = WP;
   static_assert(NP * ROWS_Q <= ROWS_D && NP * ROWS_P <= ROWS_S, "every lane's row lies inside the slab");
   // Reading the transposed slab, lane lxq takes rows VEC * lxq + e: VEC rows are VEC * odd words, so
   // lanes 32 / VEC apart would meet in one bank. Row r therefore starts skew(r) = (r / 32) words late:
-  // one bank further for every such group of lanes. (Unaligned rows: only the window layout, whose
-  // readers compute an offset per element anyway.)
-  static constexpr int SKEW_UNIT = (ALIGNED || WIN) && sizeof(T) <= 4 ? EPW : 0;
+  // one bank further for every such group of lanes. (Unaligned rows have no skew: see LXC.)
+  static constexpr int SKEW_UNIT = ALIGNED && sizeof(T) <= 4 ? EPW : 0;
+  // Lanes along q while computing; a wave covers 64 / LXC rows. On unaligned rows a lane's slab rows start
+  // anywhere in a group of 32, so a skew would cost an offset per element. Instead as few lanes lie along
+  // q as their distance (VEC rows of an odd word count: 8 words modulo the 32 banks for packs of 8) has
+  // distinct banks for, and the rest along p, where neighbours share words.
+  static constexpr int LXC = ALIGNED ? LXQ : VEC >= 8 ? 4 : 16;
+  static constexpr int ROWS_C = kBlock / LXC;
   static constexpr int skew(int r) { return SKEW_UNIT ? (r / 32) * SKEW_UNIT : 0; }
   static constexpr int SLAB_S = ROWS_S * PITCH_S + skew(ROWS_S);
   static constexpr int SLAB_RAW = SLAB_S > ROWS_D * PITCH_D ? SLAB_S : ROWS_D * PITCH_D;
@@ -120,9 +127,11 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
   using S = LdsTileShape<T, TOut, LXP, LXQ, ALIGNED>;
   constexpr int NIN = Op::NIN;
   constexpr int VEC = S::VEC, TP = S::TP, TQ = S::TQ, ROWS_P = S::ROWS_P, ROWS_Q = S::ROWS_Q;
-  constexpr int NP = S::NP, NP_S = S::NP_S, NP_D = S::NP_D, PITCH_S = S::PITCH_S, PITCH_D = S::PITCH_D, MARG = S::MARG;
-  constexpr bool WIN = S::WIN;
+  constexpr int NP = S::NP, PITCH_S = S::PITCH_S, PITCH_D = S::PITCH_D, MARG = S::MARG, GRID = S::GRID;
   static_assert(NIN >= 1 && NIN <= 3, "one to three inputs");
+  // (the host asks for 8 elements along p: only packs of 16 can be wider than the tensor)
+  constexpr bool kMayBeNarrow = !ALIGNED && VEC > 8 && std::is_integral<T>::value;
+  static_assert(ALIGNED || VEC <= 8 || kMayBeNarrow, "packs of 16 elements are whole bytes");
   using PIN = Pack<T, VEC>;
   using POUT = Pack<TOut, VEC>;
   // Packs travel from global memory to LDS as raw register images: a pack of sub-word elements kept
@@ -141,6 +150,12 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
   auto load = [&](const T* at) -> RAW {
     if constexpr (NTL) return __builtin_nontemporal_load(reinterpret_cast<const RAW*>(at));
     else return *reinterpret_cast<const RAW*>(at);
+  };
+  // the same at an address that is only element aligned
+  auto load_words = [&](const T* at) -> RAW {
+    using U = typename RawBitsU<sizeof(PIN)>::type;
+    if constexpr (NTL) return __builtin_nontemporal_load(reinterpret_cast<const U*>(at));
+    else return *reinterpret_cast<const U*>(at);
   };
 
   struct Tile {       // uniform over the workgroup
@@ -207,6 +222,14 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
     return min(max(-mo, -t.q0), sizeQ - 1 - t.q0);
   };
 
+  // Window column of lane lxp's pack in a row whose window starts m elements before the tile's first one: its own
+  // place, or further back in the last tile along p (below zero where less than a pack of the row is left:
+  // the tensor is at least a pack wide, narrow bytes apart).
+  auto mis_word = [](const T* row) { return (int)((reinterpret_cast<uintptr_t>(row) / sizeof(T)) & (uintptr_t)(GRID - 1)); };
+  auto window_col = [&](const Tile& t, int m) -> int {
+    return min((int)(lxp * VEC), (m + t.pn + GRID - 1) / GRID * GRID - VEC);
+  };
+
   // Requests every pack of the tile's inputs. No load carries a predicate: lanes past the
   // tile's valid extent re-read a pack inside it, so a later wait covers exactly these loads.
   auto issue = [&](const Tile& t, RAW (&v)[NIN][NP]) {
@@ -216,9 +239,31 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
         static_for<0, NP>([&](auto rTag) {
           constexpr int r = decltype(rTag)::value;
           const T* row = staged_row(t, k, (int)lyp + r * ROWS_P);
-          int first = (int)(lxp * VEC) - (ALIGNED ? 0 : mis_in(row));
-          if (first >= t.pn) first = ALIGNED ? 0 : -mis_in(row);
-          v[k][r] = load(row + first);
+          if constexpr (ALIGNED) {
+            int first = (int)(lxp * VEC);
+            if (first >= t.pn) first = 0;
+            v[k][r] = load(row + first);
+          } else {
+            const int m = mis_word(row);
+            const auto whole = [&]() { return load_words(row - m + window_col(t, m)); };
+            if constexpr (kMayBeNarrow) {
+              if (args.sizeP >= (uint32_t)VEC) {
+                v[k][r] = whole();
+              } else {   // byte by byte: the pack is wider than the tensor
+                uint32_t w[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                  w[i] = 0;
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    w[i] |= (uint32_t)(uint8_t)row[min(max((int)(lxp * VEC) + 4 * i + e - m, 0), t.pn - 1)] << (8 * e);
+                }
+                __builtin_memcpy(&v[k][r], w, sizeof(PIN));
+              }
+            } else {
+              v[k][r] = whole();
+            }
+          }
         });
       } else {
         const uint32_t sp = (uint32_t)args.strideP[k + 1];
@@ -250,25 +295,38 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
         static_for<0, NP>([&](auto rTag) {
           constexpr int r = decltype(rTag)::value;
           const int qi = (int)lyp + r * ROWS_P;
-          if constexpr (WIN) {
+          T* row = slab + qi * PITCH_S + S::skew(qi);
+          if constexpr (sizeof(T) < 4 && !ALIGNED) {
             // word by word: the row starts at a multiple of 4 bytes, not of 16, and a 16-byte LDS
             // write there stalls the LDS pipeline (SQ_LDS_UNALIGNED_STALL)
-            T* at = slab + qi * PITCH_S + S::skew(qi) + lxp * VEC;
-            if constexpr (sizeof(RAW) == 16) {
+            int w0 = (int)(lxp * VEC);   // (a full tile's packs end inside its rows' windows)
+            if (t.pn < TP && !(kMayBeNarrow && args.sizeP < (uint32_t)VEC)) w0 = window_col(t, mis_word(staged_row(t, k, qi)));
+            if (sizeof(T) == 2 && t.pn < TP) {   // (packs moved back by any number of elements)
+              PIN pk;
+              __builtin_memcpy(&pk, &v[k][r], sizeof(PIN));
+#pragma unroll
+              for (int e = 0; e < VEC; ++e)
+                if (w0 + e >= 0) row[w0 + e] = pk.v[e];
+            } else if constexpr (sizeof(RAW) >= 4) {
               // (may_alias: the slab is read back as elements of T)
               typedef uint32_t __attribute__((may_alias)) Word;
-              Word* w = reinterpret_cast<Word*>(at);
-              w[0] = v[k][r].x;
-              w[1] = v[k][r].y;
-              w[2] = v[k][r].z;
-              w[3] = v[k][r].w;
+              uint32_t words[sizeof(RAW) / 4];
+              __builtin_memcpy(words, &v[k][r], sizeof(RAW));
+#pragma unroll
+              for (int i = 0; i < (int)(sizeof(RAW) / 4); ++i)
+                if (w0 + i * S::EPW >= 0) *reinterpret_cast<Word*>(row + w0 + i * S::EPW) = words[i];
             } else {
-              *reinterpret_cast<RAW*>(at) = v[k][r];
+              if (w0 >= 0) *reinterpret_cast<RAW*>(row + w0) = v[k][r];
             }
+          } else if (!ALIGNED && t.pn < TP) {   // the last tile along p
+            const int first = window_col(t, 0);
+            PIN pk;
+            __builtin_memcpy(&pk, &v[k][r], sizeof(PIN));
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+              if (first + e >= 0) row[first + e] = pk.v[e];
           } else {
-            int first = (int)(lxp * VEC);
-            if (!ALIGNED) first -= mis_in(staged_row(t, k, qi));
-            T* at = slab + qi * PITCH_S + S::skew(qi) + (first + MARG);
+            T* at = row + lxp * VEC;
             PIN pk;
             __builtin_memcpy(&pk, &v[k][r], sizeof(PIN));
 #pragma unroll
@@ -286,35 +344,42 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
   };
 
   // LDS -> functor -> global, lanes along q. Rolled: the functor's code is fixed outside.
+  constexpr int kParts = LXQ / S::LXC, kPasses = (TP + S::ROWS_C - 1) / S::ROWS_C * kParts;
+  const uint32_t lxc = threadIdx.x % S::LXC;
+  const int cy = (int)(threadIdx.x / S::LXC);
   auto compute = [&](const Tile& t) {
     with_fixed_code(op, [&](auto f) {
 #pragma unroll 2
-      for (int r = 0; r < NP_D; ++r) {
-        const int pi = (int)lyq + r * ROWS_Q;
+      for (int r = 0; r < kPasses; ++r) {
+        const int pi = cy + (r / kParts) * S::ROWS_C;
+        const uint32_t cx = lxc + (r % kParts) * S::LXC;   // the row's pack
         const int pic = ALIGNED ? pi : min(pi, t.pn - 1);
         TOut* orow = t.ob + (uint32_t)pic * (uint32_t)args.strideP[0];
         // tile coordinate of the lane's first element; its slab row is first + MARG
-        const int first = (int)(lxq * VEC) - (ALIGNED ? 0 : mis_out(orow));
+        const int first = (int)(cx * VEC) - (ALIGNED ? 0 : mis_out(orow));
         // (elements are gathered and results kept as scalars: packs of sub-word elements that are
         // filled or read element by element do not stay in registers)
         T x[3][VEC] = {};
 #pragma unroll
         for (int k = 0; k < NIN; ++k) {
           const T* slab = lds + k * S::SLAB;
-          if (args.staged[k + 1] && WIN) {
-            // row j's window starts mis(row j) elements before its first tile element
-            const int sq = (int)((uint32_t)args.strideQ[k + 1] & (uint32_t)(VEC - 1));
-            int m = (mis_in(t.tb[k]) + first * sq) & (VEC - 1);
-            const T* at = slab + (first + MARG) * PITCH_S + pic;
+          if (args.staged[k + 1]) {
+            // (the last pack of an unaligned row's window is not the tile's: its rows may be any)
+            const int r0 = ALIGNED ? first : min(first + MARG, S::WQ - VEC);
+            const T* at = slab + r0 * PITCH_S + S::skew(first) + pic;
+            if constexpr (ALIGNED || GRID == 1) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-              x[k][e] = at[e * PITCH_S + m + S::skew(first + MARG + e)];
-              m = (m + sq) & (VEC - 1);
+              for (int e = 0; e < VEC; ++e) x[k][e] = at[e * PITCH_S];
+            } else {
+              // row e's window starts (m + e * sq) % GRID elements early: GRID addresses, constant offsets from them
+              const int sq = (int)((uint32_t)args.strideQ[k + 1] & (uint32_t)(GRID - 1));
+              const int m = mis_word(t.tb[k]) + first * sq;
+              const T* from[GRID];
+#pragma unroll
+              for (int i = 0; i < GRID; ++i) from[i] = at + ((m + i * sq) & (GRID - 1));
+#pragma unroll
+              for (int e = 0; e < VEC; ++e) x[k][e] = from[e % GRID][e * PITCH_S];
             }
-          } else if (args.staged[k + 1]) {
-            const T* at = slab + (first + MARG) * PITCH_S + S::skew(first) + (pic + MARG);  // (skew: ALIGNED only)
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) x[k][e] = at[e * PITCH_S];
           } else if (ALIGNED) {
             const RAW raw = *reinterpret_cast<const RAW*>(slab + pic * PITCH_D + first);
             PIN pk;
@@ -324,7 +389,7 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
           } else if (args.sameGrid[k + 1]) {
             // every row of this input starts as far from a 16-byte boundary as the output's row does
             // (operands of one shape and pitch): the window's packs are the output row's packs
-            const RAW raw = *reinterpret_cast<const RAW*>(slab + pic * PITCH_D + MARG + lxq * VEC);
+            const RAW raw = *reinterpret_cast<const RAW*>(slab + pic * PITCH_D + MARG + cx * VEC);
             PIN pk;
             __builtin_memcpy(&pk, &raw, sizeof(PIN));
 #pragma unroll
@@ -350,8 +415,8 @@ __global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const 
             else store_pack<false>(reinterpret_cast<POUT*>(orow + first), res);
           }
         } else {
-          const int g = t.q0 + first;   // column of the pack's first element; lanes 0 .. LXQ - 2 own packs
-          if (pi < t.pn && lxq < LXQ - 1 && g + VEC > 0 && g < sizeQ) {
+          const int g = t.q0 + first;   // column of the pack's first element; packs 0 .. LXQ - 2 are the tile's
+          if (pi < t.pn && cx < LXQ - 1 && g + VEC > 0 && g < sizeQ) {
             if (g >= 0 && g + VEC <= sizeQ) {
               if (args.ntStore) store_pack<true>(reinterpret_cast<POUT*>(orow + first), res);
               else store_pack<false>(reinterpret_cast<POUT*>(orow + first), res);
@@ -441,7 +506,12 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
       batch *= pl.lay[0].size[d];
     }
     using SA = LdsTileShape<T, TOut, LXP, LXQ, true>;
-    using SU = LdsTileShape<T, TOut, LXP, LXQ, false>;
+    // Unaligned rows of narrow elements with one input: half as wide along q. 4352 tiles of 64 x 248 halves on
+    // 8191 x 8193 leave the fifth round of 1024 workgroups a quarter full, and twice the workgroups hide the
+    // compute phases (exp 84 -> 79 us). With a second input, whose row pieces would halve as well, it loses (half
+    // cmax 112 -> 124 us).
+    constexpr int LXQU = Op::NIN == 1 && VEC >= 8 ? 16 : LXQ;
+    using SU = LdsTileShape<T, TOut, LXP, LXQU, false>;
     const int64_t tileP = aligned ? SA::TP : SU::TP, tileQ = aligned ? SA::TQ : SU::TQ;
     // (an unaligned row's first run starts up to VEC - 1 columns before the row does)
     const int64_t tp = (args.sizeP + tileP - 1) / tileP, tq = (args.sizeQ + (aligned ? 0 : VEC - 1) + tileQ - 1) / tileQ;
@@ -483,7 +553,8 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
       ntl = knob >= 0 ? knob != 0 : !(sizeof(T) == sizeof(TOut) && sizeof(T) < 4);
     }
     auto go = [&](auto alignedTag, auto ntlTag) {
-      hipLaunchKernelGGL((apply_ldstile_kernel<T, TOut, Op, LXP, LXQ, decltype(alignedTag)::value, decltype(ntlTag)::value>),
+      constexpr bool kAl = decltype(alignedTag)::value;
+      hipLaunchKernelGGL((apply_ldstile_kernel<T, TOut, Op, LXP, kAl ? LXQ : LXQU, kAl, decltype(ntlTag)::value>),
                          dim3(grid), dim3(kBlock), ldsBytes, st, o, i0, i1, i2, args, op);
     };
     if constexpr (Op::NIN == 1) {
