@@ -810,8 +810,8 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
 #pragma unroll
   for (int k = 0; k < NOPS; ++k) {
     if (staged[k]) {
-      vo[k] = 0;   // (column_offset places every row)
-      rowStep[k] = 0;
+      vo[k] = lyp * (uint32_t)args.strideQ[k];
+      rowStep[k] = (size_t)ROWS_P * (size_t)args.strideQ[k];
     } else {
       vo[k] = lyq * (uint32_t)args.strideP[k];
       rowStep[k] = (size_t)ROWS_Q * (size_t)args.strideP[k];
@@ -849,7 +849,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
     const T* tbase[kMaxOps];
 #pragma unroll
     for (int k = 0; k < NOPS; ++k)
-      tbase[k] = ptr[k] + (base[k] + (I)p0 * args.strideP[k] + (staged[k] ? (I)0 : (I)q0 * args.strideQ[k]));
+      tbase[k] = ptr[k] + (base[k] + (I)p0 * args.strideP[k] + (I)q0 * args.strideQ[k]);
 
     // phase 1: staged inputs, lanes along p, into lds[slot][q][p]
 #pragma unroll
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
 #pragma unroll
       for (int r = 0; r < PASSES_P; ++r) {
         const int qi = (int)lyp + r * ROWS_P;
-        const T* row = tbase[k] + column_offset(args, k, q0 + (uint32_t)min(qi, qn - 1));
+        const T* row = tbase[k] + r * rowStep[k] + vo[k];
         first[r] = (int)(lxp * VEC) - misalignment(row);
         if (qi < qn && first[r] < pn)
           v[r] = args.ntLoad ? load_pack<true>(reinterpret_cast<const P*>(row + first[r]))
@@ -1412,17 +1412,19 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
     args.strideQ[k] = (I)pl.lay[k].stride[q];
   }
   // Fuse into q the dims just outside it that continue q's run for every
-  // direct operand (not the element-wise variant: in the others q has unit stride for them). With odd
-  // sizes as well: on 414 x 646 x 51 floats, all dims of one operand reversed, tiles of 51 of their 128
+  // direct operand (q has unit stride for them in these variants). With odd sizes as well, in the line-cut
+  // variant: on 414 x 646 x 51 floats, all dims of one operand reversed, tiles of 51 of their 128
   // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390
-  // (halves: 252 and 206); the remap to XCDs stays on for them, their rows sharing lines as unfused ones do.
+  // The remap to XCDs stays on for it, its rows sharing lines as unfused ones do. Not in the shifted windows:
+  // with the divisions there halves of 1001 x 1003 x 129 took 206 instead of 252 us, but every unfused tile paid for
+  // the choice (a transposed 349 x 256 half division 10.7 -> 11.5 us).
   bool inQ[kMaxDims] = {};
   inQ[q] = true;
   int64_t sizeQ = pl.lay[0].size[q];
   args.nq = 1;
   args.qsub[0].set((uint64_t)sizeQ);
   for (int k = 0; k < pl.nops; ++k) args.qstride[k][0] = (I)pl.lay[k].stride[q];
-  if ((vec || shift) && tuning("apply.tiled.fuse_q", 1)) {
+  if ((vec || ragged) && tuning("apply.tiled.fuse_q", 1)) {
     for (int d = q - 1; d >= 0 && d != p && args.nq < kMaxFuse; --d) {
       bool ok = sizeQ * pl.lay[0].size[d] < kIndex32Limit;
       for (int k = 0; k < pl.nops && ok; ++k)
