@@ -130,6 +130,7 @@ int num_compute_units(THCState* state);
 // kernels can write the scalar result of an *all reduction into.
 constexpr size_t kScratchTailBytes = 64 * 1024;
 constexpr size_t kScratchCounters = (kScratchTailBytes - 256) / sizeof(unsigned);
+constexpr size_t kScanTicket = 2048;  // the counter that deals out the chunks of a one-read scan
 struct StreamScratch {
   void* partials;
   size_t partialBytes;

@@ -2120,7 +2120,7 @@ __device__ __forceinline__ A read_partial(const A* p) {
 // The counters (zero before and after) are 17 words 256 bytes apart: arrivals on ONE word complete about
 // every 13 ns, which 512 workgroups that end together would feel, so they meet in 16 groups first.
 constexpr unsigned kArriveGroups = 16, kArriveStride = 64;
-static_assert((kArriveGroups + 1) * kArriveStride <= kScratchCounters, "room for the arrival counters");
+static_assert((kArriveGroups + 1) * kArriveStride <= kScanTicket, "room for the arrival counters");
 __device__ __forceinline__ bool last_to_arrive(unsigned* arrive) {
   const unsigned g = blockIdx.x % kArriveGroups;
   const unsigned groups = min(kArriveGroups, gridDim.x), members = (gridDim.x - g + kArriveGroups - 1) / kArriveGroups;

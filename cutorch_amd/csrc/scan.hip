@@ -444,7 +444,8 @@ __device__ __forceinline__ bool poll_word(const uint64_t* words, A& v) {
   return there != 0;
 }
 
-__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n) {
+__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n, uint32_t* ticket) {
+  if (ticket && blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) words[i] = 0;
 }
 
@@ -455,14 +456,20 @@ __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* word
 // in their group of 64 (a group's total is published by its last chunk), and of those of 64 x 64. Nothing
 // waits for a chain of carries: a total waits for no other total, a group's for the 63 totals before it.
 // Every wait ends: tickets are drawn in order, so all chunks before this one belong to workgroups that
-// are running or done, and each of them publishes its total before it waits for anything.
+// are running or done, and each of them publishes its total before it waits for anything. The ticket is a
+// counter of its own behind the scratch buffer, zero before and after every scan, and not one of the words:
+// host threads that share a stream may put other launches between the clearing of the words and the scan, and
+// these leave anything in the buffer. Chunks then still are drawn once each, so nothing outside the
+// tensors is touched and nothing waits for a chunk that nobody draws (sums over words that were written over
+// are wrong, as the results of every call in two launches are then: a stream's scratch serves one thread at a time).
 // Bound by reads and writes of HBM at the large sizes, by ticket, look-back and chunk latency below 2^22 elements.
 // fp32, before (totals of pieces, their scan, then every piece from its carry: two reads, 3 to 5 launches) and
 // now: 2^26 elements 178 -> 110 us (4.9 TB/s on 8 bytes an element), 2^24 56 -> 31, 2^22 40 -> 14, 2^17 22 -> 6.5,
 // 1000 x 65536 145 -> 99, 1000 x 16384 44 -> 24; the error against float64 sums halves (1.2e-7 -> 6.5e-8).
 // A chunk costs about 13 ns at its row's ticket and look-back words wherever it runs, so chunks have to be large:
 // 16 KiB chunks took 525 us on 2^26 elements, 64 KiB 116, 128 KiB 110, 256 KiB 115 (too few in flight).
-// words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, all zeroed, W words per value.
+// words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, all zeroed, W words per value;
+// the grid is one workgroup per chunk.
 // In place (out == in) is fine: a chunk is read only by the workgroup that then writes it.
 // words == nullptr: every row is one chunk (S == 1), nothing to look back for.
 template <typename T, typename Op, int BT>
@@ -480,9 +487,13 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t t = blockIdx.x;
   if (words) {
-    if (threadIdx.x == 0) drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) {
+      drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (drawn == gridDim.x - 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (nobody draws after it)
+    }
     __syncthreads();
     t = __builtin_amdgcn_readfirstlane(drawn);
+    if (t >= gridDim.x) return;
   }
   const uint32_t row = t / S, c = t - row * S;
   const uint64_t first = (uint64_t)c * kChunk + wave * (kSeg * K);  // the wave's first element in its row
@@ -986,13 +997,13 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       if (R <= one * unit) threads = one;
     const int64_t S = chunks(threads) / outer, S1 = S / 64, S2 = S1 / 64;
     if (!scratch) scratch = (char*)scratch_space(s, &scratchBytes);
-    const uint64_t nwords = (uint64_t)(outer * (S + S1 + S2)) * (sizeof(A) / 4) + 1;  // the last one is the ticket
+    const uint64_t nwords = (uint64_t)(outer * (S + S1 + S2)) * (sizeof(A) / 4);
     if (outer <= 16 * cus && outer * S < (int64_t(1) << 31) && nwords * sizeof(uint64_t) <= scratchBytes) {
       uint64_t* words = S > 1 ? (uint64_t*)scratch : nullptr;
-      uint32_t* ticket = (uint32_t*)((uint64_t*)scratch + (nwords - 1));
+      uint32_t* ticket = words ? stream_scratch(s).counters + kScanTicket : nullptr;
       if (words)
         hipLaunchKernelGGL(scan_clear_words_kernel, dim3((unsigned)std::min<uint64_t>((nwords + kBlock - 1) / kBlock, 1024)),
-                           dim3(kBlock), 0, st, words, nwords);
+                           dim3(kBlock), 0, st, words, nwords, ticket);
       const auto go = [&](auto tag) {
         constexpr int BT = decltype(tag)::value;
         hipLaunchKernelGGL((scan_onepass_kernel<T, OpA, BT>), dim3((unsigned)(outer * S)), dim3(BT), 0, st, out, in, words,
@@ -1136,7 +1147,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
         const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(outer * S, (int64_t)num_compute_units(s) * perCu));
         const uint64_t nwords = (uint64_t)(outer * S * inner);
         hipLaunchKernelGGL(scan_clear_words_kernel, dim3((unsigned)std::min<uint64_t>((nwords + kBlock - 1) / kBlock, 1024)),
-                           dim3(kBlock), 0, st, words, nwords);
+                           dim3(kBlock), 0, st, words, nwords, (uint32_t*)nullptr);
         hipLaunchKernelGGL((scan_lookback_kernel<T, Op>), dim3(grid), dim3(kBlock), ldsBytes, st, out, in, words,
                            (uint64_t)outer, (uint64_t)R, (uint32_t)inner, (uint64_t)S, (uint32_t)chunkRows,
                            (uint32_t)ldsData, (uint32_t)tuning("scan.lookback_spin", 4096));

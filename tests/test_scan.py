@@ -2,6 +2,8 @@
 pinned against numpy.cumsum/cumprod in float64 (and bit-exactly on
 integer-valued data); HIP path against the oracle: integer-valued data
 bit-exact, random data within 1e-5 of the running mass."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -349,3 +351,38 @@ def test_gpu_one_read_scan_beyond_4096_chunks(thc):
     got = thc.Tensor("int").cumsum(thc.Tensor.from_numpy(x), 0)
     assert thc.last_kernel() == "scan-rows-split"
     assert_bit_equal(got.numpy(), np.cumsum(x, dtype=np.int32))
+
+
+@pytest.mark.gpu
+def test_gpu_one_read_scans_of_two_threads_on_one_stream_stay_in_their_tensors(thc):
+    """Two host threads on the default stream: their launches interleave in the stream's scratch buffer (a scan's
+    words are cleared by one launch and used by the next). Sums are the caller's business then, but every chunk is
+    still drawn once: both threads' calls end, nothing outside the outputs is written, and the next scans are right."""
+    rng = np.random.default_rng(37)
+    guard, jobs = 64, []
+    for kind, dtype, rows, n in (("float", np.float32, 3, 70001), ("long", np.int64, 2, 40003), ("byte", np.uint8, 1, 900001),
+                                 ("double", np.float64, 1, 300007)):
+        x = (rng.integers(0, 600, (rows, n)) == 0).astype(dtype)
+        out = thc.Tensor.from_storage(np.full(rows * n + 2 * guard, 5, dtype), guard, (rows, n), (n, 1), kind=kind)
+        jobs.append((thc.Tensor.from_numpy(x), out, x, dtype))
+    failed = []
+
+    def work(mine):
+        try:
+            for i in range(100):
+                for src, out, _, _ in mine:
+                    out.cumsum(src, 1)
+        except Exception as e:                        # reported by the main thread
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(jobs[i::2],)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for src, out, x, dtype in jobs:
+        out.cumsum(src, 1)
+        got = out.storage_numpy()
+        assert np.all(got[:guard] == 5) and np.all(got[-guard:] == 5)
+        assert_bit_equal(got[guard:-guard].reshape(x.shape), np.cumsum(x, axis=1, dtype=np.int64).astype(dtype))
