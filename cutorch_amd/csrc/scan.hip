@@ -484,7 +484,7 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
   __shared__ uint32_t drawn;
   __shared__ A waveTotal[kWaves];
   __shared__ A carryS;
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t t = blockIdx.x;
   if (words) {
     if (threadIdx.x == 0) {
@@ -501,34 +501,41 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
   T* dst = out + (uint64_t)row * R + first;
   const uint64_t left = R > first ? R - first : 0;
   const bool full = left >= kSeg * K;
+  // Segments (a pack per lane) of the wave that hold elements. Those behind a row's end are not touched: 4000 rows
+  // of 4096 bytes, an eighth of a chunk each, took 78 us with them.
+  const uint32_t segs = full ? K : (uint32_t)((left + kSeg - 1) / kSeg);
   const T idT = scan_down<T>(Op::id());
   P v[K];
-  if (full) {
-#pragma unroll
-    for (int u = 0; u < K; ++u) v[u] = load_pack_unaligned<true, P>(src + u * kSeg + lane * VEC);
-  } else {
+  A off[K], run = Op::id();  // off: what lies before each pack inside the wave's part
+  auto take = [&](auto fullTag) {
+    constexpr bool FULL = decltype(fullTag)::value;
 #pragma unroll
     for (int u = 0; u < K; ++u) {
       const uint32_t i0 = u * kSeg + lane * VEC;
-      if (i0 + VEC <= left) {
+      if (FULL || (u + 1) * kSeg <= left) {
         v[u] = load_pack_unaligned<true, P>(src + i0);
-      } else {
+      } else if ((uint32_t)u < segs) {
+        if (i0 + VEC <= left) {
+          v[u] = load_pack_unaligned<true, P>(src + i0);
+        } else {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) v[u].v[e] = i0 + e < left ? src[i0 + e] : idT;
+          for (int e = 0; e < VEC; ++e) v[u].v[e] = i0 + e < left ? src[i0 + e] : idT;
+        }
       }
     }
-  }
-  // what lies before each pack inside the wave's part
-  A off[K], run = Op::id();
 #pragma unroll
-  for (int u = 0; u < K; ++u) {
-    A tot = scan_up<A>(v[u].v[0]);
+    for (int u = 0; u < K; ++u) {
+      if (!FULL && (uint32_t)u >= segs) break;
+      A tot = scan_up<A>(v[u].v[0]);
 #pragma unroll
-    for (int e = 1; e < VEC; ++e) tot = Op::op(tot, scan_up<A>(v[u].v[e]));
-    tot = wave_scan<Op>(tot);
-    off[u] = Op::op(run, dpp_or<A, 0x138, 0xf>(Op::id(), tot));
-    run = Op::op(run, read_lane(tot, 63));
-  }
+      for (int e = 1; e < VEC; ++e) tot = Op::op(tot, scan_up<A>(v[u].v[e]));
+      tot = wave_scan<Op>(tot);
+      off[u] = Op::op(run, dpp_or<A, 0x138, 0xf>(Op::id(), tot));
+      run = Op::op(run, read_lane(tot, 63));
+    }
+  };
+  if (full) take(std::true_type{});
+  else take(std::false_type{});
   if (lane == 0) waveTotal[wave] = run;
   lds_barrier();
   A before = Op::id(), total = Op::id();
@@ -568,26 +575,32 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
     lds_barrier();
     before = Op::op(carryS, before);
   }
+  auto put = [&](auto fullTag) {
+    constexpr bool FULL = decltype(fullTag)::value;
 #pragma unroll
-  for (int u = 0; u < K; ++u) {
-    const uint32_t i0 = u * kSeg + lane * VEC;
-    const A base = Op::op(before, off[u]);
-    P r;
-    A sum = Op::id();
+    for (int u = 0; u < K; ++u) {
+      if (!FULL && (uint32_t)u >= segs) break;
+      const uint32_t i0 = u * kSeg + lane * VEC;
+      const A base = Op::op(before, off[u]);
+      P r;
+      A sum = Op::id();
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      sum = e ? Op::op(sum, scan_up<A>(v[u].v[e])) : scan_up<A>(v[u].v[0]);
-      r.v[e] = scan_down<T>(Op::op(base, sum));
+      for (int e = 0; e < VEC; ++e) {
+        sum = e ? Op::op(sum, scan_up<A>(v[u].v[e])) : scan_up<A>(v[u].v[0]);
+        r.v[e] = scan_down<T>(Op::op(base, sum));
+      }
+      if (FULL || i0 + VEC <= left) {
+        if (nts) store_pack_unaligned<true>(dst + i0, r);
+        else store_pack_unaligned<false>(dst + i0, r);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (i0 + e < left) dst[i0 + e] = r.v[e];
+      }
     }
-    if (full || i0 + VEC <= left) {
-      if (nts) store_pack_unaligned<true>(dst + i0, r);
-      else store_pack_unaligned<false>(dst + i0, r);
-    } else {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        if (i0 + e < left) dst[i0 + e] = r.v[e];
-    }
-  }
+  };
+  if (full) put(std::true_type{});
+  else put(std::false_type{});
 }
 
 // Small slices of the dense [outer][R][inner] block (short rows when
@@ -982,6 +995,10 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // 1024 threads where that still gives two workgroups per CU (2^24 fp32: 32 us against 38 with 512 threads
   // and 50 with 256; 2^20: 9.6 against 8.5), else of 512; 1-byte elements always 512, since their 128 elements
   // a lane take more registers than 1024 threads have (2^27 bytes: 74 us against 236).
+  // Many short rows of bytes in whole aligned packs stay a wave per row: of a chunk's 256 threads, which their 128
+  // elements a lane leave few of on a CU, they fill an eighth (4000 x 4096 bytes: 9.8 us against 21; 2000 x 6144
+  // 10.7 and 15; 1000 x 6144 9.0 and 8.1; 4000 x 8192 23.1 and 20.1; 2-byte elements win from 4096 on, 4000 x 4096
+  // halves 15.4 and 12.5).
   // Products of floating elements keep the two reads of scan_rows_kernel's pieces below: the product of a chunk
   // that overflows turns a zero before it into NaN, and these chunks are longer than those pieces.
   constexpr bool kFloatProduct =
@@ -998,7 +1015,8 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
     const int64_t S = chunks(threads) / outer, S1 = S / 64, S2 = S1 / 64;
     if (!scratch) scratch = (char*)scratch_space(s, &scratchBytes);
     const uint64_t nwords = (uint64_t)(outer * (S + S1 + S2)) * (sizeof(A) / 4);
-    if (outer <= 16 * cus && outer * S < (int64_t(1) << 31) && nwords * sizeof(uint64_t) <= scratchBytes) {
+    const bool shortBytes = sizeof(T) == 1 && aligned && R % VEC == 0 && R < 8192 && outer > 4 * cus;
+    if (!shortBytes && outer <= 16 * cus && outer * S < (int64_t(1) << 31) && nwords * sizeof(uint64_t) <= scratchBytes) {
       uint64_t* words = S > 1 ? (uint64_t*)scratch : nullptr;
       uint32_t* ticket = words ? stream_scratch(s).counters + kScanTicket : nullptr;
       if (words)

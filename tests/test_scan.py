@@ -354,6 +354,32 @@ def test_gpu_one_read_scan_beyond_4096_chunks(thc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["byte", "char", "half", "short"])
+def test_gpu_rows_that_end_early_in_a_chunk(thc, kind):
+    """Rows of 1- and 2-byte elements that fill a part of a chunk's waves: the segments (64 packs) behind a
+    row's end are left alone. Row ends at, around and between segments, in the first wave and in a later one, rows on
+    and off the 16-byte grid; whole storages are compared. Many short aligned rows of bytes stay a wave per row."""
+    dtype = {"byte": np.uint8, "char": np.int8, "half": np.float16, "short": np.int16}[kind]
+    seg = 64 * 16 // np.dtype(dtype).itemsize
+    rng = np.random.default_rng(43)
+    for n in (4096, 4096 + seg - 1, 4096 + seg, 4096 + seg + 1, 8 * seg - 1, 8 * seg + 1, 13 * seg + 5, 24 * seg, 31 * seg + 3):
+        for rows, off in ((1, 0), (5, 3)):
+            x = ((rng.integers(0, 200, rows * n + off) == 0) * 1).astype(dtype)
+            dev = thc.Tensor.from_storage(x, off, (rows, n), (n, 1), kind=kind)
+            out = thc.Tensor.from_storage(np.full(rows * n + off + 40, 7, dtype), off, (rows, n), (n, 1), kind=kind)
+            out.cumsum(dev, 1)
+            got, want = out.storage_numpy(), np.full(rows * n + off + 40, 7, dtype)
+            want[off:off + rows * n] = np.cumsum(x[off:].reshape(rows, n).astype(np.int64), axis=1).astype(dtype).reshape(-1)
+            assert_bit_equal(got, want, "%s %d x %d" % (kind, rows, n))
+    cus = thc.lib().THCAmd_getNumComputeUnits(thc.state())
+    for rows, n in ((4 * cus + 1, 4096), (4 * cus, 4096), (4 * cus + 1, 4100), (4 * cus + 1, 8192)):
+        x = (rng.integers(0, 400, (rows, n)) == 0).astype(dtype)
+        got = thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 1)
+        assert (thc.last_kernel() == "scan-rows") == (np.dtype(dtype).itemsize == 1 and rows > 4 * cus and n == 4096), (rows, n)
+        assert_bit_equal(got.numpy(), np.cumsum(x, axis=1, dtype=np.int64).astype(dtype))
+
+
+@pytest.mark.gpu
 def test_gpu_one_read_scans_of_two_threads_on_one_stream_stay_in_their_tensors(thc):
     """Two host threads on the default stream: their launches interleave in the stream's scratch buffer (a scan's
     words are cleared by one launch and used by the next). Sums are the caller's business then, but every chunk is
