@@ -1003,7 +1003,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // that overflows turns a zero before it into NaN, and these chunks are longer than those pieces.
   constexpr bool kFloatProduct =
       std::is_same<Op, ScanMul<typename ScanAcc<T>::type>>::value && !std::is_integral<T>::value;
-  if constexpr (!kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1) && outer > 0 && R >= 4096) {
+  if constexpr (!kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1) && tuning("scan.onepass", 1) && outer > 0 && R >= 4096) {
     using A = typename OnePassAcc<T>::type;
     using OpA = typename WithAcc<Op, A>::type;
     const int64_t cus = num_compute_units(s), unit = (int64_t)kFull * kOnePassPacks;  // elements per thread
@@ -1030,14 +1030,15 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       if (threads == 256) go(std::integral_constant<int, 256>{});
       else if (threads == 512 || sizeof(T) == 1) go(std::integral_constant<int, 512>{});
       else go(std::integral_constant<int, sizeof(T) == 1 ? 512 : 1024>{});
-      note_kernel("scan-rows-split");
+      note_kernel("scan-onepass");
       return;
     }
   }
-  // Few long rows of floating products: every row is cut into pieces that scan side by side, a wave per piece:
+  // Few long rows of floating products, or of so many chunks that their words do not fit the scratch buffer (from
+  // 128 GiB of longs, doubles or bytes on): every row is cut into pieces that scan side by side, a wave per piece:
   // totals of the pieces, their scan by this function on the accumulator type, then every piece from its carry.
   // The input is read twice (2^26 fp32: 175 us).
-  if constexpr (kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1)) {
+  if (inner == 1 && tuning("scan.rows.split", 1)) {
     using A = typename ScanAcc<T>::type;
     const bool vec = aligned && R % VEC == 0;
     const int64_t perIter = 64 * (vec ? VEC : 1) * 4;  // elements a wave takes per iteration

@@ -126,9 +126,18 @@ def test_gpu_long_scans_with_few_columns_run_in_chunks(thc, oracle, kind):
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["float", "half", "int", "double", "byte", "long"])
 def test_gpu_few_long_rows_scan_in_pieces(thc, oracle, kind):
-    """A 1-D cumsum (or a few long rows) is cut into pieces that scan side by side, a wave per piece:
-    totals of the pieces, their scan, then every piece from its carry. Exact on small integers; row
-    lengths that are and are not whole packs, storage offsets off the 16-byte grid, in place."""
+    """A 1-D cumprod of floating elements (or a few long rows), and any scan of more chunks than the one-read form has
+    room for (`scan.onepass` = 0 here), is cut into pieces that scan side by side, a wave per piece:
+    totals of the pieces, their scan, then every piece from its carry. Exact on small integers and on products
+    of -1, 2 and 0.5; row lengths that are and are not whole packs, storage offsets off the 16-byte grid, in place."""
+    thc.set_tuning("scan.onepass", 0)
+    try:
+        _few_long_rows_in_pieces(thc, kind)
+    finally:
+        thc.set_tuning("scan.onepass", 1)
+
+
+def _few_long_rows_in_pieces(thc, kind):
     rng = np.random.default_rng(29)
     dtype = {"float": np.float32, "half": np.float16, "int": np.int32, "double": np.float64, "byte": np.uint8,
              "long": np.int64}[kind]
@@ -157,6 +166,29 @@ def test_gpu_few_long_rows_scan_in_pieces(thc, oracle, kind):
         assert_bit_equal(got.numpy(), want.astype(dtype), "%s %s" % (kind, shape))
         assert_bit_equal(dev.numpy(), want.astype(dtype), "%s %s in place" % (kind, shape))
         assert_bit_equal(dev.storage_numpy()[:off], x[:off])       # nothing written before the rows
+        # products: every few hundred elements a factor 2, 0.5, 2, ... (floating types) or -1, so that all are exact
+        at = np.flatnonzero(rng.integers(0, 300, n + off) == 0)
+        f = np.ones(n + off, np.float64)
+        f[at] = -1
+        if kind in ("float", "half", "double"):
+            for r in range(n // shape[dim]):           # (per row: each begins with a 2)
+                mine = at[(at >= off + r * shape[dim]) & (at < off + (r + 1) * shape[dim])]
+                f[mine[0::3]] = np.where(np.arange(len(mine[0::3])) % 2 == 0, 2, 0.5)
+        x = f.astype(np.int64).astype(dtype) if kind not in ("float", "half", "double") else f.astype(dtype)
+        want = np.cumprod(f[off:].reshape(shape), axis=dim)
+        want = want.astype(np.int64).astype(dtype) if kind not in ("float", "half", "double") else want.astype(dtype)
+        thc.set_tuning("scan.rows.split_min_iters", iters)
+        try:
+            dev = thc.Tensor.from_storage(x, off, shape, tuple(strides), kind=kind)
+            got = thc.Tensor(kind).cumprod(dev, dim)
+            assert thc.last_kernel() == "scan-rows-split", (shape, thc.last_kernel())
+            dev.cumprod(dev, dim)
+            assert thc.last_kernel() == "scan-rows-split"
+        finally:
+            thc.set_tuning("scan.rows.split_min_iters", 8)
+        assert_bit_equal(got.numpy(), want, "%s %s product" % (kind, shape))
+        assert_bit_equal(dev.numpy(), want, "%s %s product in place" % (kind, shape))
+        assert_bit_equal(dev.storage_numpy()[:off], x[:off])
     if kind != "byte":
         ones = np.ones((2, 100000), dtype)
         ones[:, ::9000] = 2
@@ -329,7 +361,7 @@ def test_gpu_one_read_scans_at_the_edges_of_their_chunks(thc, kind):
             x = ((rng.integers(0, every, rows * n + off) == 0) * rng.integers(0 if kind == "byte" else -2, 3, rows * n + off)).astype(dtype)
             dev = thc.Tensor.from_storage(x, off, (rows, n), (n, 1), kind=kind)
             got = thc.Tensor(kind).cumsum(dev, 1)
-            assert thc.last_kernel() == "scan-rows-split", (n, thc.last_kernel())
+            assert thc.last_kernel() == "scan-onepass", (n, thc.last_kernel())
             want = np.cumsum(x[off:].reshape(rows, n).astype(np.int64), axis=1)
             assert kind not in ("half", "float") or np.abs(want).max() < 2048
             assert_bit_equal(got.numpy(), want.astype(dtype), "%s %d x %d" % (kind, rows, n))
@@ -341,6 +373,12 @@ def test_gpu_one_read_scans_at_the_edges_of_their_chunks(thc, kind):
             want = np.cumsum(x.astype(np.float64)).astype(dtype)
             x[at] = want[at:] = np.nan
             assert_bit_equal(thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 0).numpy(), want, "%s NaN at %d" % (kind, at))
+    if kind in ("float", "double"):
+        x = rng.standard_normal(3000001).astype(dtype)
+        got = thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 0).numpy().astype(np.float64)
+        assert thc.last_kernel() == "scan-onepass"
+        want, mass = np.cumsum(x.astype(np.float64)), np.cumsum(np.abs(x.astype(np.float64)))
+        assert np.all(np.abs(got - want) <= 1e-5 * np.maximum(np.abs(want), mass / 64))
 
 
 @pytest.mark.gpu
@@ -349,7 +387,7 @@ def test_gpu_one_read_scan_beyond_4096_chunks(thc):
     n = 4097 * 1024 * 32 + 3
     x = (np.arange(n, dtype=np.int32) % 7) - 2
     got = thc.Tensor("int").cumsum(thc.Tensor.from_numpy(x), 0)
-    assert thc.last_kernel() == "scan-rows-split"
+    assert thc.last_kernel() == "scan-onepass"
     assert_bit_equal(got.numpy(), np.cumsum(x, dtype=np.int32))
 
 
