@@ -38,7 +38,18 @@ THErrorHandlerFunction g_err_handler = nullptr;
 void* g_err_data = nullptr;
 THArgErrorHandlerFunction g_arg_handler = nullptr;
 void* g_arg_data = nullptr;
-thread_local std::string t_last_error;
+// The message of the calling thread's last failed call; whoever holds one is in THCAmd_pendingErrors, a thread
+// that ends without having asked for its message no longer.
+struct LastError {
+  std::string text;
+  void set(std::string t) {
+    const long change = long(!t.empty()) - long(!text.empty());
+    text = std::move(t);
+    if (change) __atomic_fetch_add(&THCAmd_pendingErrors, change, __ATOMIC_RELAXED);
+  }
+  ~LastError() { set(std::string()); }
+};
+thread_local LastError t_last_error;
 thread_local const char* t_last_kernel = "";
 thread_local hipStream_t t_stream = nullptr;
 int g_force64 = 0;
@@ -84,18 +95,16 @@ void raise_arg_error(int arg, const char* fmt, ...) {
 }
 
 void deliver_error(const Error& e) noexcept {
-  const bool pending = !t_last_error.empty();
-  t_last_error = e.arg > 0 ? "invalid argument " + std::to_string(e.arg) + ": " + e.msg : e.msg;
-  if (!pending && !t_last_error.empty()) __atomic_fetch_add(&THCAmd_pendingErrors, 1, __ATOMIC_RELAXED);
+  t_last_error.set(e.arg > 0 ? "invalid argument " + std::to_string(e.arg) + ": " + e.msg : e.msg);
   if (e.arg > 0 && g_arg_handler) {
     g_arg_handler(e.arg, e.msg.c_str(), g_arg_data);
     return;
   }
   if (g_err_handler) {
-    g_err_handler(t_last_error.c_str(), g_err_data);
+    g_err_handler(t_last_error.text.c_str(), g_err_data);
     return;
   }
-  fprintf(stderr, "THC error: %s\n", t_last_error.c_str());
+  fprintf(stderr, "THC error: %s\n", t_last_error.text.c_str());
   fflush(stderr);
   abort();
 }
@@ -186,12 +195,9 @@ THC_API void THSetArgErrorHandler(THArgErrorHandlerFunction h, void* data) {
   g_arg_data = data;
 }
 THC_API const char* THCAmd_lastError(void) {
-  return t_last_error.empty() ? nullptr : t_last_error.c_str();
+  return t_last_error.text.empty() ? nullptr : t_last_error.text.c_str();
 }
-THC_API void THCAmd_clearLastError(void) {
-  if (!t_last_error.empty()) __atomic_fetch_sub(&THCAmd_pendingErrors, 1, __ATOMIC_RELAXED);
-  t_last_error.clear();
-}
+THC_API void THCAmd_clearLastError(void) { t_last_error.set(std::string()); }
 
 THC_API THCState* THCState_alloc(void) {
   THCState* state = new THCState();

@@ -3,6 +3,7 @@ import ctypes as C
 import random
 import struct
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -57,4 +58,27 @@ def test_errors_are_seen_by_the_thread_that_made_them():
     with pytest.raises(thc.THCError):
         thc._check()
     thc._check()
+    assert thc._pending.value == before
+
+
+def test_a_thread_that_ends_without_reading_its_error_is_not_counted_on():
+    lib = thc.lib()
+    lib.THCAmd_clearLastError()
+    before = thc._pending.value
+
+    def fail():
+        st = C.c_void_p(lib.THCState_alloc())
+        t = lib.THCudaTensor_new(st)
+        lib.THCudaTensor_size(st, t, 3)
+        lib.THCudaTensor_free(st, t)
+        lib.THCState_free(st)
+
+    workers = [threading.Thread(target=fail) for _ in range(3)]
+    for w in workers:
+        w.start()
+    for w in workers:
+        w.join()
+    deadline = time.time() + 20                         # (join returns a little before the thread's own end)
+    while thc._pending.value != before and time.time() < deadline:
+        time.sleep(0.01)
     assert thc._pending.value == before
