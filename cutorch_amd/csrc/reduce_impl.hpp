@@ -1897,21 +1897,21 @@ __global__ __launch_bounds__(kBlock) void var_tall_kernel(const T* __restrict__ 
 }
 
 // The S partials of every output of var_tall_kernel, merged: a workgroup per slice and tile of CT
-// columns, G = kFoldBlock / CT threads per column take every G-th partial in order, thread 0 of the column
-// merges the G results. 1024 threads, so that every thread
-// takes one batch of partials: the kernel is a chain of memory round trips (6.2 us with 256; var of
-// 6.7M x 10 fp32 53.9 -> 51.1 us, both launches).
-constexpr int kFoldBlock = 1024;
-template <typename T, typename I>
-__global__ __launch_bounds__(kFoldBlock) void var_tall_fold_kernel(const typename Acc<T>::type* __restrict__ partial,
+// columns, G = BT / CT threads per column take every G-th partial in order, eight requested at a time, and the G
+// results meet in a tree. The kernel is a chain of memory round trips, one per 8 * G partials: 1024 threads where 256 would
+// need more than two, or with several column tiles more than one (6.7M x 10 fp32, 768 partials a column, both launches: 53.9 us with 256 threads, 51.1 with
+// 1024; 1M x 10 17.7 and 15.5, 1M x 33 36.3 and 30.4, 40001 x 33 10.8 and 9.8), but their longer tree and start cost
+// 0.6 us and more where 256 do (200003 x 7 10.7 and 13.0, 1M x 3 doubles 14.8 and 16.3, 4M x 5 22.4 and 23.0).
+template <typename T, typename I, int BT>
+__global__ __launch_bounds__(BT) void var_tall_fold_kernel(const typename Acc<T>::type* __restrict__ partial,
                                                                T* __restrict__ out, OuterArgs<I> oa, I outInner,
                                                                uint32_t C, uint32_t S, uint32_t CT, uint32_t colTiles,
                                                                I planeElems, typename Acc<T>::type div, bool wantStd) {
   using A = typename Acc<T>::type;
-  __shared__ A stage[3][kFoldBlock];
+  __shared__ A stage[3][BT];
   const I o = blockIdx.x / colTiles;
   const uint32_t ct = blockIdx.x - (uint32_t)o * colTiles;
-  const uint32_t G = kFoldBlock / CT, t = threadIdx.x;
+  const uint32_t G = BT / CT, t = threadIdx.x;
   const uint32_t g = t / CT, c = ct * CT + (t - g * CT);
   if (g < G) {
     A n = (A)0, mu = (A)0, q = (A)0;
@@ -3216,9 +3216,14 @@ bool reduce_var_cols_type(THCState* s, const ReduceGeom& g, const void* in_, voi
                            (I)(g.R * C), (uint32_t)C, (uint32_t)ST, (I)packsPerWg, (uint32_t)lanes, (uint32_t)pattern,
                            (uint32_t)folds, (I)planeElems);
         const int64_t CT = std::min<int64_t>(C, 16), colTiles = (C + CT - 1) / CT;
-        hipLaunchKernelGGL((var_tall_fold_kernel<T, I>), dim3((unsigned)(O * colTiles)), dim3(kFoldBlock), 0, st,
-                           (const A*)partial, (T*)out_, make_outer<I>(g.in, g.out, nd - 1), (I)g.out.stride[nd - 1],
-                           (uint32_t)C, (uint32_t)ST, (uint32_t)CT, (uint32_t)colTiles, (I)planeElems, (A)div, wantStd);
+        const auto fold = [&](auto tag) {
+          constexpr int BT = decltype(tag)::value;
+          hipLaunchKernelGGL((var_tall_fold_kernel<T, I, BT>), dim3((unsigned)(O * colTiles)), dim3(BT), 0, st,
+                             (const A*)partial, (T*)out_, make_outer<I>(g.in, g.out, nd - 1), (I)g.out.stride[nd - 1],
+                             (uint32_t)C, (uint32_t)ST, (uint32_t)CT, (uint32_t)colTiles, (I)planeElems, (A)div, wantStd);
+        };
+        if (ST > (C > CT ? 8 : 16) * (kBlock / CT)) fold(std::integral_constant<int, 1024>{});
+        else fold(std::integral_constant<int, kBlock>{});
         note_kernel("var-tall");
         return true;
       };
