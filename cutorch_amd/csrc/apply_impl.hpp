@@ -959,7 +959,9 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
 // 128-byte lines (64-byte cut points: less re-fetch of staged rows, 1.07 x, but 4 % more written bytes and 0.60
 // instead of 0.65 of peak)
 constexpr int kRaggedLineBytes = 128;
-template <typename T, typename Op, typename I, int MASK>
+// FUSED: q runs over several joint dims (args.nq > 1). An instantiation of its own: with the choice inside, the
+// kernel of one dim was 5-10 % slower (exp of a transposed 1001 x 1003 fp32 12.5 -> 13.8 us).
+template <typename T, typename Op, typename I, int MASK, bool FUSED>
 __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, const T* in0, const T* in1,
                                                                     const T* in2, TiledArgs<I> args, Op op) {
   static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4- or 8-byte elements");
@@ -975,8 +977,8 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
   extern __shared__ __align__(16) unsigned char lds_raw[];
   T* lds = reinterpret_cast<T*>(lds_raw);
   // Fused q: the offsets of the tile's columns, worked out once per column (the divisions in front of every load
-  // broke the batch of loads up and made even the unfused kernel spill: 1266 us on 1001 x 1003 x 129, 390 this way).
-  __shared__ I columnOff[2][SPAN];
+  // broke the batch of loads up and made the kernel spill: 1266 us on 1001 x 1003 x 129, 390 this way).
+  __shared__ I columnOff[FUSED ? 2 : 1][FUSED ? SPAN : 1];
 
   const T* ptr[kMaxOps] = {out, in0, in1, in2};
   const uint32_t lxp = threadIdx.x % LXP, lyp = threadIdx.x / LXP;
@@ -1024,7 +1026,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
     const int qL = (int)(tq * TQ) - (LINE - 1);  // the first column any row of this tile may hold
     const bool interior = pn == TP && qL >= 0 && qL + SPAN <= sizeQ;
 
-    if (args.nq > 1) {
+    if constexpr (FUSED) {
 #pragma unroll
       for (int k = 1; k < NOPS; ++k) {
         if (!staged[k]) continue;
@@ -1042,25 +1044,24 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
         T* slab = lds + slot[k] * (SPAN * PITCH);
         const T* origin = ptr[k] + (base[k] + (I)p0 * args.strideP[k]) + lxp * VEC;  // unit stride along p
         P v[PASSES_P];
-        auto request = [&](auto&& offset) {
-#pragma unroll
-          for (int r = 0; r < PASSES_P; ++r) {
-            const int cq = (int)lyp + r * ROWS_P, q = qL + cq;
-            const bool row = cq < SPAN && (FULL || (q >= 0 && q < sizeQ));
-            const int have = FULL ? VEC : pn - (int)(lxp * VEC);
-            if (row && have >= VEC) {
-              const T* at = origin + offset(cq, q);
-              v[r] = args.ntLoad ? load_loose_pack<true, P>(at) : load_loose_pack<false, P>(at);
-            } else if (row) {
-              const T* at = origin + offset(cq, q);
-#pragma unroll
-              for (int e = 0; e < VEC; ++e)
-                if (e < have) v[r].v[e] = at[e];
-            }
-          }
+        auto column = [&](int cq, int q) -> I {
+          if constexpr (FUSED) return columnOff[slot[k] & 1][cq];
+          else return (I)q * args.strideQ[k];
         };
-        if (args.nq > 1) request([&](int cq, int) { return columnOff[slot[k] & 1][cq]; });
-        else request([&](int, int q) { return (I)q * args.strideQ[k]; });
+#pragma unroll
+        for (int r = 0; r < PASSES_P; ++r) {
+          const int cq = (int)lyp + r * ROWS_P, q = qL + cq;
+          const bool row = cq < SPAN && (FULL || (q >= 0 && q < sizeQ));
+          const int have = FULL ? VEC : pn - (int)(lxp * VEC);
+          if (row && have >= VEC) {
+            const T* at = origin + column(cq, q);
+            v[r] = args.ntLoad ? load_loose_pack<true, P>(at) : load_loose_pack<false, P>(at);
+          } else if (row) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e)
+              if (e < have) v[r].v[e] = origin[column(cq, q) + e];
+          }
+        }
 #pragma unroll
         for (int r = 0; r < PASSES_P; ++r) {
           const int cq = (int)lyp + r * ROWS_P;
@@ -1504,9 +1505,12 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
     if ((M) < (1 << Op::NIN)) {                                                                   \
       constexpr int MM = (M) < (1 << Op::NIN) ? (M) : 1;                                          \
       if constexpr (kSameType && (sizeof(T) == 4 || sizeof(T) == 8)) {                            \
-        if (ragged)                                                                               \
-          hipLaunchKernelGGL((apply_tiled_ragged_kernel<T, Op, I, MM>), dim3(grid), dim3(kBlock), \
-                             ldsR, st, out, i0, i1, i2, args, op);                                \
+        if (ragged && args.nq > 1)                                                                \
+          hipLaunchKernelGGL((apply_tiled_ragged_kernel<T, Op, I, MM, true>), dim3(grid),         \
+                             dim3(kBlock), ldsR, st, out, i0, i1, i2, args, op);                  \
+        else if (ragged)                                                                          \
+          hipLaunchKernelGGL((apply_tiled_ragged_kernel<T, Op, I, MM, false>), dim3(grid),        \
+                             dim3(kBlock), ldsR, st, out, i0, i1, i2, args, op);                  \
       }                                                                                           \
       if constexpr (kSameType) {                                                                  \
         if (ragged) {                                                                             \
@@ -1532,7 +1536,7 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   }
 #undef THC_TILED_CASE
   note_kernel(vec ? (args.nq > 1 ? "tiled-fused" : "tiled")
-                  : (ragged ? "tiled-ragged" : (shift ? "tiled-shift" : "tiled-scalar")));
+                  : (ragged ? (args.nq > 1 ? "tiled-ragged-fused" : "tiled-ragged") : (shift ? "tiled-shift" : "tiled-scalar")));
   return true;
 }
 
