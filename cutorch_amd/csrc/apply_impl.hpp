@@ -1415,22 +1415,35 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   // Fuse into q the dims just outside it that continue q's run for every
   // direct operand (q has unit stride for them in these variants). With odd sizes as well, in the line-cut
   // variant: on 414 x 646 x 51 floats, all dims of one operand reversed, tiles of 51 of their 128
-  // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390
+  // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390. Long runs of 8-byte
+  // elements, whose tiles are 64 columns wide, only where unfused tiles leave 15 % of their columns empty (c = a + b on
+  // 33 x 355 x 513 28.5 us unfused and 31.6 fused, 33 x 181 x 1001 28 and 32; 129 x 155 x 301 27.5 and 26.5).
   // The remap to XCDs stays on for it, its rows sharing lines as unfused ones do. Not in the shifted windows:
   // with the divisions there halves of 1001 x 1003 x 129 took 206 instead of 252 us, but every unfused tile paid for
   // the choice (a transposed 349 x 256 half division 10.7 -> 11.5 us).
+  constexpr int64_t kFusedRowTiles = 32;
   bool inQ[kMaxDims] = {};
   inQ[q] = true;
   int64_t sizeQ = pl.lay[0].size[q];
+  auto continues = [&](int d, int64_t run) {
+    bool ok = run * pl.lay[0].size[d] < kIndex32Limit;
+    for (int k = 0; k < pl.nops && ok; ++k)
+      if (!staged[k]) ok = pl.lay[k].stride[d] == run;
+    return ok;
+  };
+  const int64_t fuseKnob = tuning("apply.tiled.fuse_q", 1);   // 2: wherever the layout allows it
+  bool fuse = (vec || ragged) && fuseKnob != 0;
+  if (fuse && ragged && sizeof(T) == 8 && fuseKnob == 1) {
+    int64_t run = sizeQ;
+    for (int d = q - 1, n = 1; d >= 0 && d != p && n < kMaxFuse && continues(d, run); --d, ++n) run *= pl.lay[0].size[d];
+    const int64_t columns = (sizeQ + kRaggedSlack + tqV - 1) / tqV * tqV;   // of a row's tiles, unfused
+    fuse = sizeQ * 100 < columns * 85 || run <= kFusedRowTiles * tqV;
+  }
   args.nq = 1;
   args.qsub[0].set((uint64_t)sizeQ);
   for (int k = 0; k < pl.nops; ++k) args.qstride[k][0] = (I)pl.lay[k].stride[q];
-  if ((vec || ragged) && tuning("apply.tiled.fuse_q", 1)) {
-    for (int d = q - 1; d >= 0 && d != p && args.nq < kMaxFuse; --d) {
-      bool ok = sizeQ * pl.lay[0].size[d] < kIndex32Limit;
-      for (int k = 0; k < pl.nops && ok; ++k)
-        if (!staged[k]) ok = pl.lay[k].stride[d] == sizeQ;
-      if (!ok) break;
+  if (fuse) {
+    for (int d = q - 1; d >= 0 && d != p && args.nq < kMaxFuse && continues(d, sizeQ); --d) {
       args.qsub[args.nq].set((uint64_t)pl.lay[0].size[d]);
       for (int k = 0; k < pl.nops; ++k) args.qstride[k][args.nq] = (I)pl.lay[k].stride[d];
       ++args.nq;
@@ -1483,7 +1496,12 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   // 0.66 with 64)
   args.groupP = (uint32_t)std::max<int64_t>(
       1, ragged ? tuning("apply.tiled.group_p_ragged", 32) : (shift ? tuning("apply.tiled.group_p", 8) : bandVec));
-  if ((int64_t)args.groupP * 2 > tp) args.groupP = 1;
+  // Fused columns: once those of one tile row no longer fit an L2 (32 tiles are 2-3 MB), its neighbours along p
+  // run beside it in any case, since their staged row pieces share lines (all dims of one operand reversed, 8-byte
+  // copy of 33 x 181 x 1001 26 us without and 17.5 with, 129 x 47 x 1001 24 and 16.5; below 32 tiles q-fastest order
+  // is up to 9 % faster, c = a + b on 1601 x 3 x 301).
+  if (ragged && args.nq > 1 && tq > kFusedRowTiles) args.groupP = (uint32_t)std::min<int64_t>(tp, tuning("apply.tiled.group_p_fused", 8));
+  else if ((int64_t)args.groupP * 2 > tp) args.groupP = 1;
   const int64_t swz = tuning("apply.tiled.xcd_swizzle", 1);
   // (not with fused q: there the direct operands are one long aligned run and
   // the remap cost 2% on a permuted 2048 x 2048 x 520 operand)
