@@ -1415,9 +1415,10 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   // Fuse into q the dims just outside it that continue q's run for every
   // direct operand (q has unit stride for them in these variants). With odd sizes as well, in the line-cut
   // variant: on 414 x 646 x 51 floats, all dims of one operand reversed, tiles of 51 of their 128
-  // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390. Long runs of 8-byte
-  // elements, whose tiles are 64 columns wide, only where unfused tiles leave 15 % of their columns empty (c = a + b on
-  // 33 x 355 x 513 28.5 us unfused and 31.6 fused, 33 x 181 x 1001 28 and 32; 129 x 155 x 301 27.5 and 26.5).
+  // columns took 83 us and whole ones take 41, 156 x 704 x 41 32 and 19, 1001 x 1003 x 129 659 and 390. Two tiles along p
+  // keep unfused rows that fill 85 % of their tiles' columns, unless a row is short (copy of 33 x 6041 x 301 doubles 223 us
+  // unfused and 268 fused, 33 x 1817 x 1001 211 and 262, 97 x 61 x 1001 fp32 13 and 15; with three and more the two are
+  // within 4 %).
   // The remap to XCDs stays on for it, its rows sharing lines as unfused ones do. Not in the shifted windows:
   // with the divisions there halves of 1001 x 1003 x 129 took 206 instead of 252 us, but every unfused tile paid for
   // the choice (a transposed 349 x 256 half division 10.7 -> 11.5 us).
@@ -1433,7 +1434,7 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   };
   const int64_t fuseKnob = tuning("apply.tiled.fuse_q", 1);   // 2: wherever the layout allows it
   bool fuse = (vec || ragged) && fuseKnob != 0;
-  if (fuse && ragged && sizeof(T) == 8 && fuseKnob == 1) {
+  if (fuse && ragged && fuseKnob == 1 && pl.lay[0].size[p] > tpV && pl.lay[0].size[p] <= 2 * tpV) {
     int64_t run = sizeQ;
     for (int d = q - 1, n = 1; d >= 0 && d != p && n < kMaxFuse && continues(d, run); --d, ++n) run *= pl.lay[0].size[d];
     const int64_t columns = (sizeQ + kRaggedSlack + tqV - 1) / tqV * tqV;   // of a row's tiles, unfused
