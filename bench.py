@@ -417,7 +417,7 @@ def build_configs(thc, hip, which, only=None, stagger=0):
                 "N-cumsum-wide": ("cumsum over dim 0 of 65536x1000 fp32 (rows cut into parts, input read twice, "
                                   "counted once)", 8 * 65536 * 1000, 65536 * 1000,
                                   lambda i: swide.cumsum(vwide, 0)),
-                "N-cumsum-1d": ("cumsum of a 2^26-element fp32 vector (a wave per piece, input read twice, counted once)",
+                "N-cumsum-1d": ("cumsum of a 2^26-element fp32 vector (chunks of one read)",
                                 8 * nr, nr, lambda i: s1d.cumsum(flat, 0)),
                 "N-argmax-tall": ("max+argmax over dim 0 of 6710886x10 fp32", 4 * n10, n10, lambda i: omaxt.max(imaxt, v10, 0)),
                 "N-argmax-1d": ("max+argmax of a 2^26-element fp32 vector", 4 * nr, nr, lambda i: omax1.max(imax1, flat, 0)),
