@@ -70,8 +70,8 @@ struct LdsTileArgs {
 //     per element that this replaced; halves: exp 84 at element alignment, 88 at word alignment, 92 before). The
 //     last packs of a tensor row are moved back so that they end with the row (with the word of its last byte);
 //   * along q every OUTPUT row cuts the tensor at its own pack boundaries: with mo < VEC the
-//     misalignment of the output row at column q0, the tile owns of that row the 31 whole packs
-//     [q0 - mo, q0 - mo + TQ). No pack is split between two tiles, so partial (element-wise) stores
+//     misalignment of the output row at column q0, the tile owns of that row the LXQ - 1 whole
+//     packs [q0 - mo, q0 - mo + TQ). No pack is split between two tiles, so partial (element-wise) stores
 //     only happen at the two ends of a tensor row. (Cutting every row at q0 left two partial packs
 //     per row and tile; stores narrower than 4 bytes make the memory side read, merge and write a
 //     whole sector each: a transposed half / short operand of odd shape moved 2.3 x its bytes.)
@@ -106,10 +106,11 @@ struct LdsTileShape {
   // lanes 32 / VEC apart would meet in one bank. Row r therefore starts skew(r) = (r / 32) words late:
   // one bank further for every such group of lanes. (Unaligned rows have no skew: see LXC.)
   static constexpr int SKEW_UNIT = ALIGNED && sizeof(T) <= 4 ? EPW : 0;
-  // Lanes along q while computing; a wave covers 64 / LXC rows. On unaligned rows a lane's slab rows start
-  // anywhere in a group of 32, so a skew would cost an offset per element. Instead as few lanes lie along
-  // q as their distance (VEC rows of an odd word count: 8 words modulo the 32 banks for packs of 8) has
-  // distinct banks for, and the rest along p, where neighbours share words.
+  // Lanes along q while computing; a wave covers 64 / LXC rows. On unaligned rows a lane's
+  // slab rows start anywhere in a group of 32, so a skew would cost an offset per element. Instead few lanes lie
+  // along q, VEC rows of an odd word count apart, and the rest along p, where neighbours share or follow each other's
+  // words: 16 lanes 4 words apart (packs of 4), 4 lanes 8 words (packs of 8) or 16 words apart (packs of 16), modulo
+  // 64. With all lanes along q 32 of them met in the banks of 8 (half exp on a transposed 8191 x 8193 87.0 -> 84.2 us).
   static constexpr int LXC = ALIGNED ? LXQ : VEC >= 8 ? 4 : 16;
   static constexpr int ROWS_C = kBlock / LXC;
   static constexpr int skew(int r) { return SKEW_UNIT ? (r / 32) * SKEW_UNIT : 0; }
@@ -121,9 +122,15 @@ struct LdsTileShape {
 
 // NTL: inputs are read with the streaming (nontemporal) hint. A compile-time choice: a run-time one
 // makes the compiler merge the two forms of every load into one plain load.
+// Two waves per SIMD at least on unaligned rows of 8-byte elements with one input: the functors' constants brought
+// that kernel to 260 registers, one wave per SIMD (exp of a transposed 8191 x 8193 fp64 314 -> 438 us).
+template <typename T, bool ALIGNED, int NIN>
+constexpr int ldstile_waves() {
+  return !ALIGNED && sizeof(T) == 8 && NIN == 1 ? 2 : 1;
+}
 template <typename T, typename TOut, typename Op, int LXP, int LXQ, bool ALIGNED, bool NTL = true>
-__global__ __launch_bounds__(kBlock) void apply_ldstile_kernel(TOut* out, const T* in0, const T* in1,
-                                                               const T* in2, LdsTileArgs args, Op op) {
+__global__ __launch_bounds__(kBlock, (ldstile_waves<T, ALIGNED, Op::NIN>())) void apply_ldstile_kernel(
+    TOut* out, const T* in0, const T* in1, const T* in2, LdsTileArgs args, Op op) {
   using S = LdsTileShape<T, TOut, LXP, LXQ, ALIGNED>;
   constexpr int NIN = Op::NIN;
   constexpr int VEC = S::VEC, TP = S::TP, TQ = S::TQ, ROWS_P = S::ROWS_P, ROWS_Q = S::ROWS_Q;
@@ -461,8 +468,9 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
     if (!tuning("apply.ldstile.enable", 1) || !tile_plan(pl, p, q, staged)) return false;
     constexpr int W = sizeof(T) > sizeof(TOut) ? sizeof(T) : sizeof(TOut);
     constexpr int VEC = 16 / W;
-    // 512-byte rows (of the wider type) along q; along p 128 bytes of the input type at least
-    // (64 bytes for 1-byte elements, whose 128 x 512 tile would take 66 KiB of LDS per input)
+    // 512-byte rows (of the wider type) along q (256 on unaligned rows with one input of narrow elements, LXQU below);
+    // along p 128 bytes of the input type at least (64 bytes for 1-byte elements, whose 128 x 512 tile would take 66 KiB
+    // of LDS per input)
     constexpr int LXQ = 32;
     constexpr int LXP = (sizeof(T) == 1 && VEC == 16) ? 4 : ((128 / (int)sizeof(T)) / VEC < 8 ? 8 : (128 / (int)sizeof(T)) / VEC);
     const int nd = pl.lay[0].dims;
@@ -506,10 +514,11 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
       batch *= pl.lay[0].size[d];
     }
     using SA = LdsTileShape<T, TOut, LXP, LXQ, true>;
-    // Unaligned rows of narrow elements with one input: half as wide along q. 4352 tiles of 64 x 248 halves on
-    // 8191 x 8193 leave the fifth round of 1024 workgroups a quarter full, and twice the workgroups hide the
-    // compute phases (exp 84 -> 79 us). With a second input, whose row pieces would halve as well, it loses (half
-    // cmax 112 -> 124 us).
+    // Unaligned rows of narrow elements with one input: half as wide along q. Twice the tiles fill the chip where there are few
+    // and hide the compute phases of each other (full and half width: int8 abs on a transposed 349 x 255 8.7 and 6.2 us, 127 x 8193
+    // 8.1 and 6.1, 20001 x 301 10.5 and 8.9, 8191 x 8193 33.6 and 32.6; int16 abs 5.8 and 4.5, 6.2 and 5.1, 9.1 and 7.8, 50.7 and
+    // 50.8; half exp 7.7 and 5.6, 8.0 and 5.8, 13.5 and 11.9, 71.6 and 65.9). With a second input, whose row pieces would halve
+    // as well, it loses (half cmax on 8191 x 8193 112 -> 124 us).
     constexpr int LXQU = Op::NIN == 1 && VEC >= 8 ? 16 : LXQ;
     using SU = LdsTileShape<T, TOut, LXP, LXQU, false>;
     const int64_t tileP = aligned ? SA::TP : SU::TP, tileQ = aligned ? SA::TQ : SU::TQ;
