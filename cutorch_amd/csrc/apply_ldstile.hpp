@@ -256,14 +256,16 @@ __global__ __launch_bounds__(kBlock, (ldstile_waves<T, ALIGNED, Op::NIN>())) voi
             if constexpr (kMayBeNarrow) {
               if (args.sizeP >= (uint32_t)VEC) {
                 v[k][r] = whole();
-              } else {   // byte by byte: the pack is wider than the tensor
+              } else {   // the pack is wider than the tensor: word by word, the row's last word for those behind it
+                typedef uint32_t __attribute__((may_alias)) Word;
+                const Word* words = reinterpret_cast<const Word*>(row - m);
+                const int lastWord = (m + t.pn + GRID - 1) / GRID - 1;
                 uint32_t w[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                  w[i] = 0;
-#pragma unroll
-                  for (int e = 0; e < 4; ++e)
-                    w[i] |= (uint32_t)(uint8_t)row[min(max((int)(lxp * VEC) + 4 * i + e - m, 0), t.pn - 1)] << (8 * e);
+                  const Word* at = words + min((int)lxp * 4 + i, lastWord);
+                  if constexpr (NTL) w[i] = __builtin_nontemporal_load(at);
+                  else w[i] = *at;
                 }
                 __builtin_memcpy(&v[k][r], w, sizeof(PIN));
               }

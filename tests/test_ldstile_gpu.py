@@ -368,3 +368,36 @@ def test_converting_copy_between_different_shapes_and_overlapping_destination(th
             cand[5 * i + j].add(float(10 * i + j))
     for o in range(40):
         assert got[o] in (cand[o] or {0.0}), (o, got[o], cand[o])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["byte", "char", "short", "half"])
+@pytest.mark.parametrize("p", [8, 9, 11, 15, 16, 17, 31, 32, 33, 61, 62, 64, 65, 70, 77])
+def test_tiles_of_few_rows(thc, kind, p):
+    """Transposed operands of odd shapes whose tiles hold few rows: a tensor of p rows, or the last tile of one. The packs that would pass a row's end are moved
+    back, and 1-byte rows narrower than a pack are read word by word. One and two inputs, conversions to wider and narrower
+    types; whole storages are compared, so nothing outside the output is written."""
+    dt = {"byte": np.uint8, "char": np.int8, "short": np.int16, "half": np.float16}[kind]
+    rng = np.random.default_rng(p)
+    for q in (9, 121, 255, 517):
+        for off in (0, 1, 3):
+            n = p * q
+            a = rng.integers(0, 60, n + off + 5).astype(dt)
+            b = rng.integers(0, 60, n + off + 5).astype(dt)
+            ta = thc.Tensor.from_storage(a, off, (p, q), (1, p), kind=kind)
+            tb = thc.Tensor.from_storage(b, off, (p, q), (q, 1), kind=kind)
+            xa, xb = a[off:off + n].reshape(q, p).T, b[off:off + n].reshape(p, q)
+            runs = [(kind, dt, lambda c: c.binary("cmax", ta, tb), np.maximum(xa, xb))]
+            if kind != "half":
+                runs.append((kind, dt, lambda c: c.unary("sign", ta), np.sign(xa)))
+            else:
+                runs.append((kind, dt, lambda c: c.unary("neg", ta), -xa))
+            for to, tdt in (("float", np.float32), ("double", np.float64), ("byte", np.uint8)):
+                if to != kind:
+                    runs.append((to, tdt, lambda c: c.copy_from(ta), xa.astype(tdt)))
+            for to, tdt, run, want in runs:
+                c = np.full(n + off + 9, 77, tdt)
+                tc = thc.Tensor.from_storage(c, off, (p, q), (q, 1), kind=to)
+                run(tc)
+                c[off:off + n] = want.astype(tdt).reshape(-1)
+                assert_bit_equal(tc.storage_numpy(), c, "%s -> %s %d x %d +%d %s" % (kind, to, p, q, off, thc.last_kernel()))
