@@ -465,7 +465,10 @@ __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* word
 // Bound by reads and writes of HBM at the large sizes, by ticket, look-back and chunk latency below 2^22 elements.
 // fp32, before (totals of pieces, their scan, then every piece from its carry: two reads, 3 to 5 launches) and
 // now: 2^26 elements 178 -> 110 us (4.9 TB/s on 8 bytes an element), 2^24 56 -> 31, 2^22 40 -> 14, 2^17 22 -> 6.5,
-// 1000 x 65536 145 -> 99, 1000 x 16384 44 -> 24; the error against float64 sums halves (1.2e-7 -> 6.5e-8).
+// 1000 x 65536 145 -> 99, 1000 x 16384 44 -> 24; the error against float64 sums (2-norm, 2^26
+// uniform values) 1.2e-7 -> 5.3e-8.
+// A chunk's total, those of 64 and of 4096 chunks are formed on their own: where one of them overflows, the row is
+// infinite behind it although its prefixes may be finite (the pieces had this over shorter spans).
 // A chunk costs about 13 ns at its row's ticket and look-back words wherever it runs, so chunks have to be large:
 // 16 KiB chunks took 525 us on 2^26 elements, 64 KiB 116, 128 KiB 110, 256 KiB 115 (too few in flight).
 // words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, all zeroed, W words per value;
