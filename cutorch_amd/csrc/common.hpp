@@ -130,7 +130,8 @@ int num_compute_units(THCState* state);
 // kernels can write the scalar result of an *all reduction into.
 constexpr size_t kScratchTailBytes = 64 * 1024;
 constexpr size_t kScratchCounters = (kScratchTailBytes - 256) / sizeof(unsigned);
-constexpr size_t kScanTicket = 2048;  // the counter that deals out the chunks of a one-read scan
+constexpr size_t kScanTicket = 2048;  // counters kScanTicket and the one behind it: a 64-bit word that deals out the chunks of one-read scans
+constexpr size_t kScanWords = size_t(2) << 20;  // 16 MiB of words behind the tail, which only one-read scans write
 struct StreamScratch {
   void* partials;
   size_t partialBytes;
@@ -138,6 +139,9 @@ struct StreamScratch {
   float* result;        // device slot for a scalar result (last 256 bytes of the tail)
   float* hostResult;    // pinned host memory ...
   float* hostResultDev; // ... and its device-side address
+  uint64_t* scanWord;   // what the workgroups of a one-read scan tell each other (zero at first, tagged values after that)
+  size_t scanWords;     // how many
+  uint64_t* scanTicket;
 };
 const StreamScratch& stream_scratch(THCState* state);
 void* scratch_space(THCState* state, size_t* bytes);

@@ -130,14 +130,17 @@ const StreamScratch& stream_scratch(THCState* s) {
   if (it != s->scratch.end()) return it->second;
   StreamScratch sc{};
   void* p = nullptr;
-  THC_CHECK((hipError_t)s->allocator.malloc(s->allocator.state, &p, s->scratchBytes,
+  THC_CHECK((hipError_t)s->allocator.malloc(s->allocator.state, &p, s->scratchBytes + kScanWords * sizeof(uint64_t),
                                             (hipStream_t_)st));  // scratch stays with hipMalloc
   sc.partials = p;
   sc.partialBytes = s->scratchBytes - kScratchTailBytes;
   sc.counters = reinterpret_cast<unsigned*>(static_cast<char*>(p) + sc.partialBytes);
   sc.result = reinterpret_cast<float*>(static_cast<char*>(p) + s->scratchBytes - 256);
-  // Arrival counters start at zero and every kernel that uses one resets it.
-  THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes, st));
+  sc.scanWord = reinterpret_cast<uint64_t*>(static_cast<char*>(p) + s->scratchBytes);
+  sc.scanWords = kScanWords;
+  sc.scanTicket = reinterpret_cast<uint64_t*>(sc.counters + kScanTicket);
+  // Arrival counters start at zero and every kernel that uses one resets it; the words of one-read scans lie behind them.
+  THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
   THC_CHECK(hipStreamSynchronize(st));
   // One pinned, device-mapped slot: *all reductions store their scalar there. Coherent (fine-grained),
   // so that a store by a running kernel becomes visible to the host, which polls the slot.

@@ -21,6 +21,7 @@
 // for double, wrapping 64-bit for the integer types.
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 
 #include "common.hpp"
@@ -418,34 +419,47 @@ __device__ __forceinline__ A read_lane(A v, int lane) {
 }
 
 // Accumulator values published between workgroups: every 32-bit half of the value is a 64-bit word
-// (1 << 32) | half, stored and loaded with relaxed device-scope atomics. Word 0 is "not there yet", so
-// value and flag arrive together and no fence (which would write back an XCD's L2) is needed.
+// (tag << 32) | half, stored and loaded with relaxed device-scope atomics: value and tag arrive together, so no fence
+// (which would write back an XCD's L2) is needed. A word with another tag is "not there yet". The tag is the number of
+// the scan on its stream, which the workgroups read with their tickets (draw_ticket); the words are kept for scans
+// alone and start out as zeros, so nothing has to clear them between two scans (a launch of its own before: 2^20 fp32
+// 7.8 us, 6.3 without it).
 template <typename A>
-__device__ __forceinline__ void publish_word(uint64_t* words, A v) {
+__device__ __forceinline__ void publish_word(uint64_t* words, uint32_t tag, A v) {
   constexpr int W = sizeof(A) / 4;
   uint32_t h[W];
   __builtin_memcpy(h, &v, sizeof(A));
 #pragma unroll
   for (int i = 0; i < W; ++i)
-    __hip_atomic_store(words + i, (uint64_t(1) << 32) | h[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(words + i, ((uint64_t)tag << 32) | h[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <typename A>
-__device__ __forceinline__ bool poll_word(const uint64_t* words, A& v) {
+__device__ __forceinline__ bool poll_word(const uint64_t* words, uint32_t tag, A& v) {
   constexpr int W = sizeof(A) / 4;
   uint32_t h[W];
-  uint64_t there = uint64_t(1) << 32;
+  bool there = true;
 #pragma unroll
   for (int i = 0; i < W; ++i) {
     const uint64_t w = __hip_atomic_load(words + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    there &= w;
+    there = there && (uint32_t)(w >> 32) == tag;
     h[i] = (uint32_t)w;
   }
   __builtin_memcpy(&v, h, sizeof(A));
-  return there != 0;
+  return there;
+}
+// The next chunk of a scan of `chunks` chunks and the scan's tag, in one atomic: the counter holds
+// (scans before this one << 32) | chunks drawn, and whoever draws the last chunk sets it up for the next scan (nobody
+// draws after that; the next scan of the stream starts when this one has ended). Tickets come in order, so all chunks
+// before this one belong to workgroups that are running or done. Tags are never 0 and come back after 2^32 - 1 scans.
+__device__ __forceinline__ uint32_t draw_ticket(uint64_t* counter, uint32_t chunks, uint32_t& tag) {
+  const uint64_t t = __hip_atomic_fetch_add(counter, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t scans = t >> 32;
+  if ((uint32_t)t == chunks - 1) __hip_atomic_store(counter, (scans + 1) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  tag = (uint32_t)(scans % 0xffffffffull) + 1;
+  return (uint32_t)t;
 }
 
-__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n, uint32_t* ticket) {
-  if (ticket && blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
+__global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) words[i] = 0;
 }
 
@@ -456,12 +470,8 @@ __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* word
 // in their group of 64 (a group's total is published by its last chunk), and of those of 64 x 64. Nothing
 // waits for a chain of carries: a total waits for no other total, a group's for the 63 totals before it.
 // Every wait ends: tickets are drawn in order, so all chunks before this one belong to workgroups that
-// are running or done, and each of them publishes its total before it waits for anything. The ticket is a
-// counter of its own behind the scratch buffer, zero before and after every scan, and not one of the words:
-// host threads that share a stream may put other launches between the clearing of the words and the scan, and
-// these leave anything in the buffer. Chunks then still are drawn once each, so nothing outside the
-// tensors is touched and nothing waits for a chunk that nobody draws (sums over words that were written over
-// are wrong, as the results of every call in two launches are then: a stream's scratch serves one thread at a time).
+// are running or done, and each of them publishes its total before it waits for anything. One launch, and words and
+// ticket belong to scans alone, so host threads that share a stream cannot put anything between.
 // Bound by reads and writes of HBM at the large sizes, by ticket, look-back and chunk latency below 2^22 elements.
 // fp32, before (totals of pieces, their scan, then every piece from its carry: two reads, 3 to 5 launches) and
 // now: 2^26 elements 178 -> 110 us (4.9 TB/s on 8 bytes an element), 2^24 56 -> 31, 2^22 40 -> 14, 2^17 22 -> 6.5,
@@ -476,7 +486,7 @@ __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* word
 // In place (out == in) is fine: a chunk is read only by the workgroup that then writes it.
 // words == nullptr: every row is one chunk (S == 1), nothing to look back for.
 template <typename T, typename Op, int BT>
-__global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, uint64_t* words, uint32_t* ticket,
+__global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, uint64_t* words, uint64_t* ticket,
                                                               uint32_t outer, uint64_t R, uint32_t S, uint32_t S1,
                                                               uint32_t S2, int nts) {
   using A = typename OnePassAcc<T>::type;
@@ -484,18 +494,16 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
   constexpr uint32_t kSeg = 64 * VEC;  // elements of one pack per lane of a wave
   constexpr uint32_t kChunk = kSeg * K * kWaves;
   using P = Pack<T, VEC>;
-  __shared__ uint32_t drawn;
+  __shared__ uint32_t drawn, drawnTag;
   __shared__ A waveTotal[kWaves];
   __shared__ A carryS;
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  uint32_t t = blockIdx.x;
+  uint32_t t = blockIdx.x, tag = 0;
   if (words) {
-    if (threadIdx.x == 0) {
-      drawn = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (drawn == gridDim.x - 1) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (nobody draws after it)
-    }
+    if (threadIdx.x == 0) drawn = draw_ticket(ticket, gridDim.x, drawnTag);
     __syncthreads();
     t = __builtin_amdgcn_readfirstlane(drawn);
+    tag = __builtin_amdgcn_readfirstlane(drawnTag);
     if (t >= gridDim.x) return;
   }
   const uint32_t row = t / S, c = t - row * S;
@@ -552,22 +560,22 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
       uint64_t* w0 = words + (uint64_t)row * S * W;
       uint64_t* w1 = words + ((uint64_t)outer * S + (uint64_t)row * S1) * W;
       uint64_t* w2 = words + ((uint64_t)outer * (S + S1) + (uint64_t)row * S2) * W;
-      if (lane == 0) publish_word(w0 + (uint64_t)c * W, total);
+      if (lane == 0) publish_word(w0 + (uint64_t)c * W, tag, total);
       const uint32_t g = c / 64, j = c % 64, sg = g / 64, gj = g % 64;
       // lanes below `n` wait for words[lane]; their sum, in the order of wave_scan
       auto sum_of = [&](const uint64_t* w, uint32_t n) -> A {
         A x = Op::id();
         bool have = lane >= n;
         while (!__all(have)) {
-          if (!have) have = poll_word(w + (uint64_t)lane * W, x);
+          if (!have) have = poll_word(w + (uint64_t)lane * W, tag, x);
         }
         if (lane >= n) x = Op::id();
         return read_lane(wave_scan<Op>(x), 63);
       };
       A carry = j ? sum_of(w0 + (uint64_t)(c - j) * W, j) : Op::id();
-      if (j == 63 && lane == 0) publish_word(w1 + (uint64_t)g * W, Op::op(carry, total));
+      if (j == 63 && lane == 0) publish_word(w1 + (uint64_t)g * W, tag, Op::op(carry, total));
       if (gj) carry = Op::op(sum_of(w1 + (uint64_t)(g - gj) * W, gj), carry);
-      if (j == 63 && gj == 63 && lane == 0) publish_word(w2 + (uint64_t)sg * W, Op::op(carry, total));
+      if (j == 63 && gj == 63 && lane == 0) publish_word(w2 + (uint64_t)sg * W, tag, Op::op(carry, total));
       if (sg) {
         A far = Op::id();
         for (uint32_t b = 0; b < sg; b += 64) far = Op::op(far, sum_of(w2 + (uint64_t)b * W, min(64u, sg - b)));
@@ -604,6 +612,322 @@ __global__ __launch_bounds__(BT) void scan_onepass_kernel(T* out, const T* in, u
   };
   if (full) put(std::true_type{});
   else put(std::false_type{});
+}
+
+constexpr uint32_t kMaxStripLanes = 32, kMaxStripColumns = kMaxStripLanes * 16;
+
+// What lies before chunk s of a chain of S, per column: C columns, `total[c]` in LDS holds the chunk's own totals,
+// `carry[c]` receives the sums (or products) of all chunks before it. The same tree as in scan_onepass_kernel, with
+// groups of 2^lgG chunks: the totals before the chunk in its group, of the groups before that in theirs, and of the
+// groups of groups. `w`: the chain's words, [S + S1 + S2][C] values. The threads share the words of a
+// column between them; the order in which they are added up depends on the position alone.
+template <typename Op, typename A, int BT>
+__device__ __forceinline__ void look_back(uint64_t* w, uint32_t tag, uint32_t s, uint32_t S, uint32_t S1, uint32_t lgG,
+                                          uint32_t C, uint32_t live, const A* total, A* carry, A* part) {
+  constexpr int W = sizeof(A) / 4, kBatch = 8;  // words of a column a thread asks for at once
+  const uint32_t G = 1u << lgG, j = s & (G - 1), g = s >> lgG, gj = g & (G - 1), sg = g >> lgG;
+  const bool follow = s + 1 < S;  // somebody reads this chunk's totals
+  const auto publish = [&](uint32_t slot, uint32_t c, A v) { publish_word(w + ((uint64_t)slot * C + c) * W, tag, v); };
+  if (follow)
+    for (uint32_t c = threadIdx.x; c < live; c += BT) publish(s, c, total[c]);
+  const uint32_t P = live < BT ? BT / live : 1u;  // threads per column
+  const uint32_t p = P > 1 ? threadIdx.x / live : 0u, c0 = P > 1 ? threadIdx.x - p * live : threadIdx.x;
+  // sums of `n` rows of words from row `slot` on, handed to fn(c, sum) by one thread per column
+  const auto sum_rows = [&](uint32_t slot, uint32_t n, auto&& fn) {
+    const uint32_t band = (n + P - 1) / P, kb = min(n, p * band), ke = min(n, kb + band);
+    if (p < P)
+      for (uint32_t c = c0; c < live; c += BT) {
+        A acc = Op::id();
+        const uint64_t* src = w + ((uint64_t)slot * C + c) * W;
+        for (uint32_t k = kb; k < ke; k += kBatch) {
+          A x[kBatch];
+          bool have[kBatch];
+#pragma unroll
+          for (int i = 0; i < kBatch; ++i) {
+            x[i] = Op::id();
+            have[i] = k + i >= ke;
+          }
+          bool all;
+          do {
+            all = true;
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+              if (!have[i]) {
+                A v;
+                have[i] = poll_word(src + (uint64_t)(k + i) * C * W, tag, v);
+                if (have[i]) x[i] = v;
+              }
+              all = all && have[i];
+            }
+          } while (!all);
+#pragma unroll
+          for (int i = 0; i < kBatch; ++i) acc = Op::op(acc, x[i]);
+        }
+        part[p * live + c] = acc;
+      }
+    lds_barrier();
+    for (uint32_t c = threadIdx.x; c < live; c += BT) {
+      A acc = part[c];
+      for (uint32_t q = 1; q < P; ++q) acc = Op::op(acc, part[q * live + c]);
+      fn(c, acc);
+    }
+    lds_barrier();
+  };
+  sum_rows(s - j, j, [&](uint32_t c, A near) {
+    carry[c] = near;
+    if (follow && j == G - 1) publish(S + g, c, Op::op(near, total[c]));
+  });
+  if (g) {
+    sum_rows(S + g - gj, gj, [&](uint32_t c, A mid) {
+      carry[c] = Op::op(mid, carry[c]);
+      if (follow && j == G - 1 && gj == G - 1) publish(S + S1 + sg, c, Op::op(carry[c], total[c]));
+    });
+    if (sg) sum_rows(S + S1, sg, [&](uint32_t c, A far) { carry[c] = Op::op(far, carry[c]); });
+  }
+}
+
+// Long scans along a strided dim in ONE read, rows of at least a few packs: scan_onepass_kernel's scheme with a chunk
+// of TY * 8 rows of a strip TX packs wide. Lane column tx and thread row ty hold 8 rows of a pack in registers, the
+// thread rows meet in LDS, the strips' chunks (a chain per slice and strip) look back per column. Packs sit
+// at element-aligned addresses; the last pack of a row is moved back to end with it and shares columns with its
+// neighbour of the same strip (both compute the same values). Chunks are dealt row by row of chunks over all
+// chains, so neighbouring strips run together. words: [outer * colTiles][S + S1 + S2][TX * VEC] values.
+template <typename T, typename Op, int BT>
+__global__ __launch_bounds__(BT) void scan_strips_kernel(T* out, const T* in, uint64_t* words, uint64_t* ticket, uint32_t outer,
+                                                         uint64_t R, uint32_t inner, uint32_t TX, uint32_t colTiles, uint32_t S,
+                                                         uint32_t S1, uint32_t S2, uint32_t lgG, int nts) {
+  using A = typename OnePassAcc<T>::type;
+  constexpr int VEC = 16 / sizeof(T), W = sizeof(A) / 4, K = kOnePassPacks;
+  using P = Pack<T, VEC>;
+  __shared__ uint32_t drawn, drawnTag;
+  __shared__ A tot[BT * VEC];   // thread totals, then what lies before each thread's rows
+  __shared__ A part[BT > kMaxStripColumns ? BT : kMaxStripColumns];  // partial sums, at most one a thread or one a column
+  __shared__ A total[kMaxStripColumns], carry[kMaxStripColumns];
+  const uint32_t chains = outer * colTiles;
+  uint32_t t = blockIdx.x, tag = 0;
+  if (S > 1) {
+    if (threadIdx.x == 0) drawn = draw_ticket(ticket, gridDim.x, drawnTag);
+    __syncthreads();
+    t = __builtin_amdgcn_readfirstlane(drawn);
+    tag = __builtin_amdgcn_readfirstlane(drawnTag);
+    if (t >= gridDim.x) return;
+  }
+  const uint32_t s = t / chains, chain = t - s * chains, o = chain / colTiles, ct = chain - o * colTiles;
+  const uint32_t TY = BT / TX, ty = threadIdx.x / TX, tx = threadIdx.x - ty * TX;
+  const uint32_t packs = (inner + VEC - 1) / VEC;
+  const uint32_t C = TX * VEC, live = min(TX, packs - ct * TX) * VEC;
+  const bool mine = ty < TY && tx * VEC < live;
+  const uint32_t col = min((ct * TX + tx) * VEC, inner - VEC);
+  const uint64_t r0 = ((uint64_t)s * TY + ty) * K;
+  const uint32_t rows = mine && r0 < R ? (uint32_t)min((uint64_t)K, R - r0) : 0u;
+  const uint64_t at = ((uint64_t)o * R + r0) * inner + col;
+  const T* src = in + at;
+  T* dst = out + at;
+  const T idT = scan_down<T>(Op::id());
+  P v[K];
+  if (rows == K) {
+#pragma unroll
+    for (int u = 0; u < K; ++u) v[u] = load_pack_unaligned<true, P>(src + (uint64_t)u * inner);
+  } else {
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      if ((uint32_t)u < rows) {
+        v[u] = load_pack_unaligned<true, P>(src + (uint64_t)u * inner);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[u].v[e] = idT;
+      }
+    }
+  }
+  if (mine) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      A a = scan_up<A>(v[0].v[e]);
+#pragma unroll
+      for (int u = 1; u < K; ++u) a = Op::op(a, scan_up<A>(v[u].v[e]));
+      tot[ty * C + tx * VEC + e] = a;
+    }
+  }
+  lds_barrier();
+  {
+    // thread (q, c) turns its band of column c's TY totals into what lies before each of them
+    const uint32_t Q = C < BT ? min(BT / C, TY) : 1u, q = threadIdx.x / C, cq = threadIdx.x - q * C;
+    const uint32_t band = (TY + Q - 1) / Q;
+    const uint32_t yb = min(TY, q * band), ye = min(TY, yb + band);
+    if (q < Q)
+      for (uint32_t c = cq; c < live; c += BT) {
+        A a = Op::id();
+        for (uint32_t y = yb; y < ye; ++y) a = Op::op(a, tot[y * C + c]);
+        part[q * C + c] = a;
+      }
+    lds_barrier();
+    if (q < Q)
+      for (uint32_t c = cq; c < live; c += BT) {
+        A a = Op::id();
+        for (uint32_t b = 0; b < q; ++b) a = Op::op(a, part[b * C + c]);
+        for (uint32_t y = yb; y < ye; ++y) {
+          const A x = tot[y * C + c];
+          tot[y * C + c] = a;
+          a = Op::op(a, x);
+        }
+        if (q == Q - 1) total[c] = a;
+      }
+    lds_barrier();
+  }
+  if (S > 1) {
+    look_back<Op, A, BT>(words + (uint64_t)chain * (S + S1 + S2) * C * W, tag, s, S, S1, lgG, C, live, total, carry, part);
+  }
+  if (!mine) return;
+  A base[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    base[e] = tot[ty * C + tx * VEC + e];
+    if (S > 1) base[e] = Op::op(carry[tx * VEC + e], base[e]);
+  }
+  A sum[VEC];
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    P r;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      sum[e] = u ? Op::op(sum[e], scan_up<A>(v[u].v[e])) : scan_up<A>(v[u].v[e]);
+      r.v[e] = scan_down<T>(Op::op(base[e], sum[e]));
+    }
+    if ((uint32_t)u < rows) {
+      if (nts) store_pack_unaligned<true>(dst + (uint64_t)u * inner, r);
+      else store_pack_unaligned<false>(dst + (uint64_t)u * inner, r);
+    }
+  }
+}
+
+// The same for narrow rows: a chunk is a run of whole rows (all of a slice, or chunkRows of it), staged in LDS as
+// one flat run of aligned packs whatever the rows' alignment; P threads share a column and scan a band of its rows
+// each, in place; the run goes back out as packs of the output's alignment.
+template <typename T, typename Op, int BT>
+__global__ __launch_bounds__(BT) void scan_runs_kernel(T* out, const T* in, uint64_t* words, uint64_t* ticket, uint32_t outer,
+                                                       uint64_t R, uint32_t inner, uint32_t chunkRows, uint32_t dataBytes,
+                                                       uint32_t S, uint32_t S1, uint32_t S2, uint32_t lgG) {
+  using A = typename OnePassAcc<T>::type;
+  constexpr int VEC = 16 / sizeof(T), W = sizeof(A) / 4;
+  using PK = Pack<T, VEC>;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  __shared__ uint32_t drawn, drawnTag;
+  T* lds = reinterpret_cast<T*>(lds_raw);
+  A* bands = reinterpret_cast<A*>(lds_raw + dataBytes);  // band totals, max(BT, inner)
+  const uint32_t slots = max((uint32_t)BT, inner);
+  A* part = bands + slots;
+  A* total = part + slots;  // inner each
+  A* carry = total + inner;
+  uint32_t t = blockIdx.x, tag = 0;
+  if (S > 1) {
+    if (threadIdx.x == 0) drawn = draw_ticket(ticket, gridDim.x, drawnTag);
+    __syncthreads();
+    t = __builtin_amdgcn_readfirstlane(drawn);
+    tag = __builtin_amdgcn_readfirstlane(drawnTag);
+    if (t >= gridDim.x) return;
+  }
+  const uint32_t s = t / outer, o = t - s * outer;
+  const uint64_t r0 = (uint64_t)s * chunkRows;
+  const uint32_t rows = (uint32_t)min((uint64_t)chunkRows, R - r0), count = rows * inner;
+  const uint64_t start = ((uint64_t)o * R + r0) * inner;
+  const T* first = in + start;
+  const uint32_t mis = (uint32_t)((reinterpret_cast<uintptr_t>(first) / sizeof(T)) & (uintptr_t)(VEC - 1));
+  {
+    const PK* src = reinterpret_cast<const PK*>(first - mis);
+    const uint32_t npacks = (mis + count + VEC - 1) / VEC;
+    constexpr int U = 8;
+    for (uint32_t i0 = threadIdx.x; i0 < npacks; i0 += U * BT) {
+      PK v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * BT < npacks) v[u] = load_pack<true>(src + i0 + u * BT);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * BT < npacks) reinterpret_cast<PK*>(lds)[i0 + u * BT] = v[u];
+    }
+  }
+  __syncthreads();
+  const uint32_t P = inner < BT ? min(rows, BT / inner) : 1u;
+  const uint32_t p = inner < BT ? threadIdx.x / inner : 0u, c0 = inner < BT ? threadIdx.x - p * inner : threadIdx.x;
+  const uint32_t band = (rows + P - 1) / P, rb = min(rows, p * band), re = min(rows, rb + band);
+  constexpr uint32_t B = 8;
+  if (p < P)
+    for (uint32_t c = c0; c < inner; c += BT) {
+      const T* col = lds + mis + c;
+      A acc = Op::id();
+      uint32_t r = rb;
+      for (; r + B <= re; r += B) {
+        T x[B];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) x[u] = col[(r + u) * inner];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) acc = Op::op(acc, scan_up<A>(x[u]));
+      }
+      for (; r < re; ++r) acc = Op::op(acc, scan_up<A>(col[r * inner]));
+      bands[p * inner + c] = acc;
+    }
+  __syncthreads();
+  // what lies before each band, by groups of 8 bands
+  A before = Op::id();
+  if (P > 1) {
+    if (p < P && (p & 7) == 0) {
+      A a = Op::id();
+      for (uint32_t q = p; q < min(p + 8, P); ++q) a = Op::op(a, bands[q * inner + c0]);
+      part[(p >> 3) * inner + c0] = a;
+    }
+    __syncthreads();
+    if (p < P) {
+      for (uint32_t q = 0; q < p >> 3; ++q) before = Op::op(before, part[q * inner + c0]);
+      for (uint32_t q = p & ~7u; q < p; ++q) before = Op::op(before, bands[q * inner + c0]);
+      if (p == P - 1) total[c0] = Op::op(before, bands[p * inner + c0]);
+    }
+  } else {
+    for (uint32_t c = threadIdx.x; c < inner; c += BT) total[c] = bands[c];
+  }
+  lds_barrier();
+  if (S > 1)
+    look_back<Op, A, BT>(words + (uint64_t)o * (S + S1 + S2) * inner * W, tag, s, S, S1, lgG, inner, inner, total, carry, part);
+  if (p < P)
+    for (uint32_t c = c0; c < inner; c += BT) {
+      T* col = lds + mis + c;
+      const A base = S > 1 ? Op::op(carry[c], before) : before;
+      A acc = Op::id();
+      uint32_t r = rb;
+      for (; r + B <= re; r += B) {
+        T x[B];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) x[u] = col[(r + u) * inner];
+#pragma unroll
+        for (uint32_t u = 0; u < B; ++u) {
+          acc = Op::op(acc, scan_up<A>(x[u]));
+          col[(r + u) * inner] = scan_down<T>(Op::op(base, acc));
+        }
+      }
+      for (; r < re; ++r) {
+        acc = Op::op(acc, scan_up<A>(col[r * inner]));
+        col[r * inner] = scan_down<T>(Op::op(base, acc));
+      }
+    }
+  lds_barrier();
+  {
+    T* to = out + start;
+    const T* run = lds + mis;
+    const int mo = (int)((reinterpret_cast<uintptr_t>(to) / sizeof(T)) & (uintptr_t)(VEC - 1));
+    const uint32_t npacks = ((uint32_t)mo + count + VEC - 1) / VEC;
+    for (uint32_t k = threadIdx.x; k < npacks; k += BT) {
+      const int i0 = (int)(k * VEC) - mo;  // run index of the pack's element 0
+      if (i0 >= 0 && i0 + VEC <= (int)count) {
+        PK v;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v.v[e] = run[i0 + e];
+        *reinterpret_cast<PK*>(to + i0) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (i0 + e >= 0 && i0 + e < (int)count) to[i0 + e] = run[i0 + e];
+      }
+    }
+  }
 }
 
 // Small slices of the dense [outer][R][inner] block (short rows when
@@ -990,23 +1314,26 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // totals of 32 KiB chunks of rows, their scan (this function again, on the
   // accumulator type), then every chunk scans from its carry. The input is
   // read twice, which still is 500x faster.
-  // Long rows, up to 16 per CU (a 1-D cumsum above all): a wave per row leaves the chip idle, and a wave
-  // walks its row at a microsecond per KiB or two. They are cut into chunks that scan side by side in one
-  // read; from 4096 elements (one row of 4097: 18 us with a wave, 4.4 this way; 1000 rows of 5001: 28 and
-  // 11; 4000 rows of 5001: 57 and 35, 4000 of 16384: 133 and 97). A row that fits 1024 threads x 8 packs is
+  // Long rows (a 1-D cumsum above all): a wave per row leaves the chip idle, and a wave walks its row at a microsecond
+  // per KiB or two. They are cut into chunks that scan side by side in one read (one row of 4097: 18 us with a
+  // wave, 3.9 this way; 1000 rows of 5001: 28 and 11). A row that fits 1024 threads x 8 packs is
   // one chunk and looks back for nothing (15571 elements: 4.4 us, 7.2 as two chunks). Longer rows: chunks of
   // 1024 threads where that still gives two workgroups per CU (2^24 fp32: 32 us against 38 with 512 threads
   // and 50 with 256; 2^20: 9.6 against 8.5), else of 512; 1-byte elements always 512, since their 128 elements
   // a lane take more registers than 1024 threads have (2^27 bytes: 74 us against 236).
-  // Many short rows of bytes in whole aligned packs stay a wave per row: of a chunk's 256 threads, which their 128
-  // elements a lane leave few of on a CU, they fill an eighth (4000 x 4096 bytes: 9.8 us against 21; 2000 x 6144
-  // 10.7 and 15; 1000 x 6144 9.0 and 8.1; 4000 x 8192 23.1 and 20.1; 2-byte elements win from 4096 on, 4000 x 4096
-  // halves 15.4 and 12.5).
+  // A wave per row stays where there are rows enough to fill the chip with it. Rows of whole aligned packs: from 16 per
+  // CU on; below 4096 elements, where a row fills a part of its workgroup, from 4 per CU on (fp32 2048: 1025 rows 5.6 us
+  // with a wave and 4.0, 2500 of 1024 4.8 and 5.9, of 3000 12.9 and 13.9), 1 for bytes (2048: 1000 rows 4.5 and 4.8),
+  // 16 for 8-byte elements (2500 x 1024 9.4 and 7.3); never below 1024 elements or up to 4 KiB (1000 x 1024 fp32 3.9 and 3.6, 2500 4.8 and 5.9); 1-byte elements below 8192: 4 (4000 x 4096 9.8 and 21, 1000 x 6144
+  // 9.0 and 8.1). Other rows go through a wave element by element, and the chunks win further: 16000 fp32
+  // rows of 2051 59.5 and 40.4, 30000 half rows of 1025 58.4 and 52.8, 16000 doubles of 513 36.2 and 28.9; except fp32
+  // below 2048 (3000 x 1025 9.4 and 7.4, 6000 15.5 and 17.3) and bytes below 8192 (2500 x 2049 16.2 and 15.1, 6000 24.3 and
+  // 33.5).
   // Products of floating elements keep the two reads of scan_rows_kernel's pieces below: the product of a chunk
   // that overflows turns a zero before it into NaN, and these chunks are longer than those pieces.
   constexpr bool kFloatProduct =
       std::is_same<Op, ScanMul<typename ScanAcc<T>::type>>::value && !std::is_integral<T>::value;
-  if constexpr (!kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1) && tuning("scan.onepass", 1) && outer > 0 && R >= 4096) {
+  if constexpr (!kFloatProduct) if (inner == 1 && tuning("scan.rows.split", 1) && tuning("scan.onepass", 1) && outer > 0 && R * (int64_t)sizeof(T) >= 2048) {
     using A = typename OnePassAcc<T>::type;
     using OpA = typename WithAcc<Op, A>::type;
     const int64_t cus = num_compute_units(s), unit = (int64_t)kFull * kOnePassPacks;  // elements per thread
@@ -1016,25 +1343,145 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
     for (int64_t one = most; one >= 256; one /= 2)
       if (R <= one * unit) threads = one;
     const int64_t S = chunks(threads) / outer, S1 = S / 64, S2 = S1 / 64;
-    if (!scratch) scratch = (char*)scratch_space(s, &scratchBytes);
+    const StreamScratch& sc = stream_scratch(s);
     const uint64_t nwords = (uint64_t)(outer * (S + S1 + S2)) * (sizeof(A) / 4);
-    const bool shortBytes = sizeof(T) == 1 && aligned && R % VEC == 0 && R < 8192 && outer > 4 * cus;
-    if (!shortBytes && outer <= 16 * cus && outer * S < (int64_t(1) << 31) && nwords * sizeof(uint64_t) <= scratchBytes) {
-      uint64_t* words = S > 1 ? (uint64_t*)scratch : nullptr;
-      uint32_t* ticket = words ? stream_scratch(s).counters + kScanTicket : nullptr;
-      if (words)
-        hipLaunchKernelGGL(scan_clear_words_kernel, dim3((unsigned)std::min<uint64_t>((nwords + kBlock - 1) / kBlock, 1024)),
-                           dim3(kBlock), 0, st, words, nwords, ticket);
+    const bool whole = aligned && R % VEC == 0;  // rows of whole packs
+    int64_t most_rows = 16 * cus;
+    if (!whole) {
+      if (sizeof(T) == 1 && R < 8192) most_rows = 8 * cus;
+      else if (sizeof(T) == 4 && R < 2048) most_rows = 12 * cus;
+      else most_rows = std::numeric_limits<int64_t>::max();
+    } else if (R < 1024 || (R < 4096 && R * (int64_t)sizeof(T) <= 4096)) {
+      most_rows = 0;
+    } else if (R < 4096) {
+      most_rows = (sizeof(T) == 8 ? 16 : sizeof(T) == 1 ? 1 : 4) * cus;
+    } else if (sizeof(T) == 1 && R < 8192) {
+      most_rows = 4 * cus;
+    }
+    if (outer <= most_rows && outer * S < (int64_t(1) << 31) && nwords <= sc.scanWords) {
+      uint64_t* words = S > 1 ? sc.scanWord : nullptr;
       const auto go = [&](auto tag) {
         constexpr int BT = decltype(tag)::value;
         hipLaunchKernelGGL((scan_onepass_kernel<T, OpA, BT>), dim3((unsigned)(outer * S)), dim3(BT), 0, st, out, in, words,
-                           ticket, (uint32_t)outer, (uint64_t)R, (uint32_t)S, (uint32_t)S1, (uint32_t)S2, streaming);
+                           sc.scanTicket, (uint32_t)outer, (uint64_t)R, (uint32_t)S, (uint32_t)S1, (uint32_t)S2, streaming);
       };
       if (threads == 256) go(std::integral_constant<int, 256>{});
       else if (threads == 512 || sizeof(T) == 1) go(std::integral_constant<int, 512>{});
       else go(std::integral_constant<int, sizeof(T) == 1 ? 512 : 1024>{});
       note_kernel("scan-onepass");
       return;
+    }
+  }
+  // Long scans along a strided dim, in one read: strips of columns, or runs of whole narrow rows (below). Before: totals
+  // of pieces, their scan, then every piece from its carry (three to five launches, two reads), or a
+  // workgroup per strip that walks the rows alone, element by element where rows are not whole packs. us before and now:
+  // 1 x 1526 x 866 fp32 26.4 and 10.0, 1 x 51967 x 120 25.6 and 17.5, half 29.3 and 14.3, 65536 x 1000 155 and 120, 278737 x 164
+  // 136 and 97, 5 x 40 x 1000 14.0 and 4.1, 7 x 5059 x 1258 131 and 77, half 122 and 53, 16384 x 8192 bytes 274 and 100;
+  // runs: 1893 x 2011 x 6 half 59.6 and 25.0, 6.7M x 10 fp32 146 and 132, 46 x 5014 x 8 bytes 40 and 9.
+  if constexpr (!kFloatProduct) if (inner > 1 && outer > 0 && R > 1 && inner < (int64_t(1) << 30) && tuning("scan.onepass", 1) && tuning("scan.chunked", 1) &&
+                                    tuning("scan.cols.split", 1)) {
+    using A = typename OnePassAcc<T>::type;
+    using OpA = typename WithAcc<Op, A>::type;
+    constexpr int64_t W = sizeof(A) / 4;
+    const int64_t cus = num_compute_units(s), rowBytes = inner * (int64_t)sizeof(T);
+    const StreamScratch& sc = stream_scratch(s);
+    const auto levels = [&](int64_t S, int64_t& S1, int64_t& S2) {
+      int lg = 2;
+      while (lg < 6 && (int64_t(1) << (2 * lg)) < S) ++lg;
+      S1 = S >> lg;
+      S2 = S1 >> lg;
+      return lg;
+    };
+    const long form = tuning("scan.strided", -1);
+    // Where the column kernel below stays: strips of whole packs that occupy every CU once or up to three times (64 x 4096
+    // x 512 halves 89 us against 102 here), few rows over many aligned strips, and small tensors of few rows.
+    const int64_t total = outer * R * rowBytes, packsC = inner / VECC;
+    const bool vecRows = aligned && inner % VECC == 0;
+    const auto per_cu = [&](int64_t lanes) { return (double)(outer * ((packsC + lanes - 1) / lanes)) / (double)cus; };
+    const auto fills = [&](int64_t lanes) {
+      return 4 * packsC >= 3 * lanes && per_cu(lanes) >= 0.9 && per_cu(lanes) >= 0.8 * std::ceil(per_cu(lanes));
+    };
+    const bool wellFilled =
+        vecRows && (sizeof(T) > 1 ? fills(32) || (sizeof(T) != 4 && fills(16)) || (sizeof(T) == 8 && fills(8)) ||
+                                        (R <= 256 && packsC >= 24 && per_cu(32) >= 1)
+                                  : R <= 200 && packsC >= 24 && per_cu(32) >= 0.5);
+    const bool fewRows = R <= 64 && total < (int64_t(5) << 19) && (32768 / rowBytes < 4 || R * rowBytes < 4 * 32768);
+    // Narrow rows are staged in LDS: a thread row's packs would lie too far apart.
+    const bool narrow = rowBytes < 64 || (rowBytes < 128 && total >= (int64_t(128) << 20)) ||
+                        (sizeof(T) == 1 && inner <= 350 && (R * inner <= 65536 || total >= (int64_t(32) << 20)));
+    const bool strips = form < 0 ? !narrow && !wellFilled && !fewRows && R > 32 : form == 1;
+    if (strips && inner >= kFull) {
+      const int64_t packs = (inner + kFull - 1) / kFull;
+      // Strips of 128 columns, as many words to look back over as two or more threads each share (fp32 and double: 32
+      // lanes, 512-byte segments of a row; half 16, bytes 8: 65536 x 1000 bytes 61 us, 92 with 32 lanes). Rows that fit one
+      // chunk need nobody's totals: the widest strip that holds them all. 512 threads, 1024 where a chain would
+      // have 256 chunks and more (51967 x 120 fp32 17.6 against 20.5; 8-byte sums stay at 512: 278737 x 164 189 against 210).
+      const int64_t widest = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(8, 128 / kFull), kMaxStripLanes), packs);
+      int64_t TX = tuning("scan.strips.lanes", widest), threads = tuning("scan.strips.threads", 0);
+      const auto rows_of = [&](int64_t bt, int64_t tx) { return bt / tx * kOnePassPacks; };
+      if (!threads) {
+        threads = 512;
+        bool oneChunk = false;
+        for (int64_t tx = std::min<int64_t>(kMaxStripLanes, packs); !oneChunk && (tx >= 8 || tx == packs); tx /= 2)
+          for (int64_t bt = 256; !oneChunk && bt <= 512; bt *= 2)
+            if (rows_of(bt, tx) >= R) {
+              TX = tx;
+              threads = bt;
+              oneChunk = true;
+            }
+        if (!oneChunk && sizeof(A) == 4 && sizeof(T) > 1 && R >= 256 * rows_of(512, TX)) threads = 1024;
+      }
+      int64_t colTiles = (packs + TX - 1) / TX;
+      TX = (packs + colTiles - 1) / colTiles;
+      // (a strip of one moved-back pack would share columns with the strip before it)
+      if (inner % kFull != 0)
+        while (TX < kMaxStripLanes && packs > TX && packs % TX == 1) ++TX;
+      colTiles = (packs + TX - 1) / TX;
+      const bool ownColumns = inner % kFull == 0 || packs <= TX || packs % TX != 1;
+      const auto parts = [&](int64_t bt) { return (R + rows_of(bt, TX) - 1) / rows_of(bt, TX); };
+      const int64_t S = parts(threads);
+      int64_t S1, S2;
+      const int lg = levels(S, S1, S2);
+      if (ownColumns && outer * colTiles * S < (int64_t(1) << 31) &&
+          outer * colTiles * (S + S1 + S2) * TX * kFull * W <= (int64_t)sc.scanWords) {
+        const auto go = [&](auto tag) {
+          constexpr int BT = decltype(tag)::value;
+          hipLaunchKernelGGL((scan_strips_kernel<T, OpA, BT>), dim3((unsigned)(outer * colTiles * S)), dim3(BT), 0, st, out, in,
+                             sc.scanWord, sc.scanTicket, (uint32_t)outer, (uint64_t)R, (uint32_t)inner, (uint32_t)TX,
+                             (uint32_t)colTiles, (uint32_t)S, (uint32_t)S1, (uint32_t)S2, (uint32_t)lg, streaming);
+        };
+        if (threads == 256) go(std::integral_constant<int, 256>{});
+        else if (threads == 512 || sizeof(T) == 1) go(std::integral_constant<int, 512>{});
+        else go(std::integral_constant<int, sizeof(T) == 1 ? 512 : 1024>{});
+        note_kernel("scan-cols-split");
+        return;
+      }
+    }
+    // Runs of about 8192 elements and at most 64 KiB (831303 x 5 bytes 15.1 us with 16 KiB, 20.8 with 32; fp32 26.4 and 19.7; doubles 48 and
+    // 31, 26 with 64), a slice of up to 64 KiB whole (300 x 1000 x 33 bytes 11.5 us, 19.9 in two).
+    if (form < 0 ? narrow && !fewRows : form == 2 && rowBytes <= 8192) {
+      int64_t chunk = tuning("scan.runs.bytes", 0);
+      if (!chunk) chunk = R * rowBytes <= 65536 ? 65536 : std::min<int64_t>(65536, std::max<int64_t>(std::max<int64_t>(16384, 8192 * sizeof(T)), outer * R * rowBytes / (2 * cus)));
+      const int64_t threads = chunk > 40000 ? 512 : 256;
+      int64_t chunkRows = std::min<int64_t>(R, std::max<int64_t>(1, chunk / rowBytes));
+      chunkRows = (R + (R + chunkRows - 1) / chunkRows - 1) / ((R + chunkRows - 1) / chunkRows);  // (as even as they get)
+      const int64_t S = (R + chunkRows - 1) / chunkRows;
+      int64_t S1, S2;
+      const int lg = levels(S, S1, S2);
+      const size_t data = (((size_t)(chunkRows * inner) + 2 * kFull) * sizeof(T) + 15) & ~size_t(15);
+      const size_t lds = data + (2 * (size_t)std::max<int64_t>(threads, inner) + 2 * (size_t)inner) * sizeof(A);
+      if (lds <= 96 * 1024 && outer * S < (int64_t(1) << 31) && outer * (S + S1 + S2) * inner * W <= (int64_t)sc.scanWords) {
+        const auto go = [&](auto tag) {
+          constexpr int BT = decltype(tag)::value;
+          hipLaunchKernelGGL((scan_runs_kernel<T, OpA, BT>), dim3((unsigned)(outer * S)), dim3(BT), lds, st, out, in, sc.scanWord,
+                             sc.scanTicket, (uint32_t)outer, (uint64_t)R, (uint32_t)inner, (uint32_t)chunkRows, (uint32_t)data,
+                             (uint32_t)S, (uint32_t)S1, (uint32_t)S2, (uint32_t)lg);
+        };
+        if (threads == 256) go(std::integral_constant<int, 256>{});
+        else go(std::integral_constant<int, 512>{});
+        note_kernel("scan-chunked");
+        return;
+      }
     }
   }
   // Few long rows of floating products, or of so many chunks that their words do not fit the scratch buffer (from
@@ -1169,7 +1616,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
         const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(outer * S, (int64_t)num_compute_units(s) * perCu));
         const uint64_t nwords = (uint64_t)(outer * S * inner);
         hipLaunchKernelGGL(scan_clear_words_kernel, dim3((unsigned)std::min<uint64_t>((nwords + kBlock - 1) / kBlock, 1024)),
-                           dim3(kBlock), 0, st, words, nwords, (uint32_t*)nullptr);
+                           dim3(kBlock), 0, st, words, nwords);
         hipLaunchKernelGGL((scan_lookback_kernel<T, Op>), dim3(grid), dim3(kBlock), ldsBytes, st, out, in, words,
                            (uint64_t)outer, (uint64_t)R, (uint32_t)inner, (uint64_t)S, (uint32_t)chunkRows,
                            (uint32_t)ldsData, (uint32_t)tuning("scan.lookback_spin", 4096));

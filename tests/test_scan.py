@@ -2,6 +2,7 @@
 pinned against numpy.cumsum/cumprod in float64 (and bit-exactly on
 integer-valued data); HIP path against the oracle: integer-valued data
 bit-exact, random data within 1e-5 of the running mass."""
+import ctypes
 import threading
 
 import numpy as np
@@ -450,3 +451,138 @@ def test_gpu_one_read_scans_of_two_threads_on_one_stream_stay_in_their_tensors(t
         got = out.storage_numpy()
         assert np.all(got[:guard] == 5) and np.all(got[-guard:] == 5)
         assert_bit_equal(got[guard:-guard].reshape(x.shape), np.cumsum(x, axis=1, dtype=np.int64).astype(dtype))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "int", "double", "byte", "long"])
+def test_gpu_one_read_scans_along_a_strided_dim(thc, kind):
+    """Strips of columns (1) and runs of whole narrow rows (2), each forced on shapes at their edges: rows one below, at
+    and one above a chunk and a group of chunks, more than two levels of groups, widths of one pack, one element
+    more, and of packs that leave a strip one pack; offsets off the 16-byte grid, in place; whole storages
+    are compared. Exact on small integers."""
+    dtype = {"float": np.float32, "half": np.float16, "int": np.int32, "double": np.float64, "byte": np.uint8, "long": np.int64}[kind]
+    vec = 16 // np.dtype(dtype).itemsize
+    rng = np.random.default_rng(47)
+    lanes = 128 // vec if vec < 16 else 8
+    lanes = min(max(lanes, 8), 32)
+    shapes = [(1, 512 // lanes * 8 * n + d, lanes * vec) for n in (1, 4) for d in (-1, 0, 1)]          # chunks and groups of four
+    shapes += [(2, 70, vec), (1, 4099, vec + 1), (3, 200, 33 * vec - 1), (2, 515, 97 * vec + 1), (2, 33, 1000), (7, 1, 40),
+               (1, 160000, vec), (1, 20011, 3), (40, 33, 7), (1, 300001, 2)]
+    for shape in shapes:
+        outer, n, inner = shape
+        off = int(rng.integers(0, 4))
+        every = max(24, n // 100)
+        x = ((rng.integers(0, every, outer * n * inner + off + 9) == 0) * rng.integers(0 if kind == "byte" else -2, 3, outer * n * inner + off + 9)).astype(dtype)
+        size = outer * n * inner
+        want = np.cumsum(x[off:off + size].reshape(shape).astype(np.int64), axis=1)
+        assert kind != "half" or np.abs(want).max() < 2048
+        whole = x.copy()
+        whole[off:off + size] = want.astype(dtype).reshape(-1)
+        for form, name in ((1, "scan-cols-split"), (2, "scan-chunked")):
+            if form == 1 and inner < vec or form == 2 and inner * np.dtype(dtype).itemsize > 8192:
+                continue
+            thc.set_tuning("scan.strided", form)
+            thc.set_tuning("scan.slab", 0)
+            try:
+                strides = (n * inner, inner, 1)
+                dev = thc.Tensor.from_storage(x, off, shape, strides, kind=kind)
+                out = thc.Tensor.from_storage(x, off, shape, strides, kind=kind)
+                out.cumsum(dev, 1)
+                if n > 1:
+                    assert thc.last_kernel() == name, (shape, form, thc.last_kernel())
+                dev.cumsum(dev, 1)
+            finally:
+                thc.set_tuning("scan.strided", -1)
+                thc.set_tuning("scan.slab", 1)
+            assert_bit_equal(out.storage_numpy(), whole, "%s %s form %d" % (kind, shape, form))
+            assert_bit_equal(dev.storage_numpy(), whole, "%s %s form %d in place" % (kind, shape, form))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "double"])
+def test_gpu_strided_one_read_scans_of_random_values_and_of_nans(thc, kind):
+    """Against float64 sums, with a NaN that reaches what lies behind it in its column and nothing else; the same bits on
+    every run."""
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64}[kind]
+    rng = np.random.default_rng(53)
+    for shape in ((1, 3001, 257), (3, 1000, 130), (1, 40001, 5), (2, 9001, 11)):
+        x = rng.uniform(-1, 1, shape).astype(dtype)
+        dev = thc.Tensor.from_numpy(x)
+        first = thc.Tensor(kind).cumsum(dev, 1).numpy()
+        want, mass = np.cumsum(x.astype(np.float64), axis=1), np.cumsum(np.abs(x.astype(np.float64)), axis=1)
+        # (half: one rounding of the result beside the float sums')
+        tol = {"float": 1e-5, "half": 2e-3, "double": 1e-12}[kind]
+        assert np.all(np.abs(first.astype(np.float64) - want) <= tol * np.maximum(np.abs(want), mass / 64)), shape
+        assert_bit_equal(thc.Tensor(kind).cumsum(dev, 1).numpy(), first)
+        at, col = shape[1] // 2 + 3, shape[2] - 2
+        x[0, at, col] = np.nan
+        got = thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 1).numpy()
+        assert np.all(np.isnan(got[0, at:, col]))
+        got[0, at:, col] = first[0, at:, col]
+        assert_bit_equal(got, first, "%s %s" % (kind, shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "double", "byte", "int"])
+def test_gpu_rows_below_4096_elements_in_one_chunk(thc, kind):
+    """Rows that are not whole packs from 2 KiB on, and few rows that are: a workgroup per row; row ends at and around the
+    64-pack segments and the widths of a workgroup, and row counts on both sides of where a wave per row takes over."""
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64, "byte": np.uint8, "int": np.int32}[kind]
+    item = np.dtype(dtype).itemsize
+    seg = 64 * 16 // item
+    cus = thc.lib().THCAmd_getNumComputeUnits(thc.state())
+    rng = np.random.default_rng(59)
+    for n in [m for m in (2048 // item, 2048 // item + 1, 3 * seg + 1, 2047, 2048, 2049, 3 * seg - 1, 4095) if m * item >= 2048]:
+        for rows, off in ((1, 1), (5, 0), (cus, 0), (12 * cus + 1, 0)):
+            if rows > cus and n > 2100:
+                continue
+            x = (rng.integers(0, 300, rows * n + off) == 0).astype(dtype)
+            dev = thc.Tensor.from_storage(x, off, (rows, n), (n, 1), kind=kind)
+            got = thc.Tensor(kind).cumsum(dev, 1)
+            if rows <= cus and (off or n % (16 // item)):
+                assert thc.last_kernel() == "scan-onepass", (n, rows, thc.last_kernel())
+            assert_bit_equal(got.numpy(), np.cumsum(x[off:].reshape(rows, n), axis=1, dtype=np.int64).astype(dtype), "%s %d x %d" % (kind, rows, n))
+
+
+@pytest.mark.gpu
+def test_gpu_one_read_scans_in_a_graph(thc):
+    """A captured scan is replayed with other scans and a change of its input between the replays: tickets, tags and words
+    are the device's own, so no replay meets an older one's totals."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    ptr = ctypes.c_void_p
+    rng = np.random.default_rng(61)
+    jobs = []
+    for shape in ((300001,), (3001, 257), (40001, 5)):
+        jobs.append((thc.Tensor("float").resize(shape), thc.Tensor("float").resize(shape)))
+
+    def refill():
+        values = [(rng.integers(0, 30, x.shape) == 0).astype(np.float32) for x, _ in jobs]
+        for (x, _), v in zip(jobs, values):
+            x._fn("copyFromHost")(x._st, x.h, v.ctypes.data_as(ptr))
+        return [np.cumsum(v, axis=0, dtype=np.float64).astype(np.float32) for v in values]
+
+    refill()
+    lib, st, stream, graph, ready = thc.lib(), thc.state(), ptr(), ptr(), ptr()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    lib.THCState_setCurrentStream(st, stream)
+    try:
+        for x, y in jobs:
+            y.cumsum(x, 0)                # (the stream's scratch is there before the capture)
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert hip.hipStreamBeginCapture(stream, 2) == 0
+        for x, y in jobs:
+            y.cumsum(x, 0)
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(ready), graph, None, None, ctypes.c_size_t(0)) == 0
+        for i in range(5):
+            want = refill()
+            assert hip.hipGraphLaunch(ready, stream) == 0
+            for x, y in jobs[i % 4:]:
+                thc.Tensor("float").cumsum(x, 0)
+            assert hip.hipStreamSynchronize(stream) == 0
+            for (x, y), w in zip(jobs, want):
+                assert_bit_equal(y.numpy(), w, "replay %d" % i)
+        assert hip.hipGraphExecDestroy(ready) == 0 and hip.hipGraphDestroy(graph) == 0
+    finally:
+        hip.hipStreamSynchronize(stream)
+        lib.THCState_setCurrentStream(st, None)
