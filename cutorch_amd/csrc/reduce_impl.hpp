@@ -312,10 +312,15 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
       S.divmod(vr, row, s);
       oa.offsets(row, inOff, outOff);
       const I begin = s * chunk;
-      const I end = min(R, begin + chunk);
+      const I stop = min(R, begin + chunk);
+      const I end = stop - (stop - begin) % VEC;  // whole packs
       const TIn* src = in + inOff;
       A c = (A)0;
       if constexpr (F::kCentred && FIRST) c = acc_up<A>(out[outOff]);
+      for (I t = end + lane; VEC > 1 && t < stop; t += G) {  // the elements behind the last whole pack
+        const A x = acc_up<A>(src[t]);
+        acc[0] = f.combine(acc[0], FIRST ? f.modify(x, c) : x);
+      }
       const I es = VEC == 1 ? sR : (I)1;  // element stride
       // U loads are issued back to back before any of them is consumed.
       constexpr int U = 8;
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
         P v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + (i + u * step) * es));
+          v[u] = load_pack_unaligned<true, P>(src + (i + u * step) * es);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const I at = i + u * step < end ? i + u * step : i;
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + at * es));
+          v[u] = load_pack_unaligned<true, P>(src + at * es);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -399,7 +404,8 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_index_kernel(
       oaIdx.offsets(row, unused, idxOff);
       const T* src = in + inOff;
       const I begin = sp * chunk;
-      const I end = min(R, begin + chunk);
+      const I stop = min(R, begin + chunk);
+      const I end = stop - (stop - begin) % VEC;  // whole packs
       const I es = VEC == 1 ? sR : (I)1;
       constexpr int U = 8;
       const I step = (I)G * VEC;
@@ -415,7 +421,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_index_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const I at = !PARTIAL || i + u * step < end ? i + u * step : i;
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + at * es));
+          v[u] = load_pack_unaligned<true, P>(src + at * es);
         }
         A a[U][VEC];
         A m = O::worst();
@@ -453,6 +459,13 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_index_kernel(
       I i = begin + lane * VEC;
       for (; i + (U - 1) * step < end; i += U * step) batch(i, std::false_type{});
       if (i < end) batch(i, std::true_type{});
+      for (I t = end + lane; VEC > 1 && t < stop; t += G) {  // the elements behind the last whole pack
+        const A x = acc_up<A>(src[t]);
+        if (O::better_later(x, bv)) {
+          bv = x;
+          bi = t;
+        }
+      }
     }
     for (uint32_t o = G >> 1; o > 0; o >>= 1) {
       const A ov = shfl_xor_any(bv, o);
@@ -1352,6 +1365,18 @@ __global__ __launch_bounds__(kBlock) void var_rows_lds_kernel(const T* __restric
   }
 }
 
+template <typename A>
+__device__ __forceinline__ void moments_merge(A& na, A& ma, A& sa, A nb, A mb, A sb) {
+  const A n = na + nb;
+  if (n > (A)0) {
+    const A delta = mb - ma;
+    const A w = nb / n;
+    ma += delta * w;
+    sa += sb + delta * delta * na * w;
+  }
+  na = n;
+}
+
 template <typename T, typename I>
 __global__ __launch_bounds__(kBlock) void var_slab_kernel(const T* __restrict__ in, T* __restrict__ out,
                                                           SlabArgs<I> a, typename Acc<T>::type div,
@@ -1366,37 +1391,74 @@ __global__ __launch_bounds__(kBlock) void var_slab_kernel(const T* __restrict__ 
     const uint32_t ns = (uint32_t)min((I)a.slicesPerBlock, a.O - o0);
     const uint32_t mis = stage_rows_to_lds<T, 8>(in + o0 * (I)slice, ns * slice, lds);
     __syncthreads();
-    for (uint32_t t = threadIdx.x; t < ns * C; t += kBlock) {
-      uint32_t o, c;
-      a.cdiv.divmod(t, o, c);
-      const T* col = lds + mis + o * slice + c;
-      // both sweeps read LDS in batches of 8 (past the column's end: its last element, not used)
+    // Fewer columns than threads: P threads share a column, each sweeps a band of its rows twice, and the bands' (count,
+    // mean, sum of squared deviations) meet in a fixed tree in LDS (1001 slices of 576 x 2 fp32: 51 us with a thread per column).
+    const uint32_t cols = ns * C, P = cols < kBlock ? min(R / 8, kBlock / cols) : 1u;
+    __shared__ A bands[3][kBlock];
+    // both sweeps read LDS in batches of 8 (past the band's end: its last element, not used)
+    auto sweep = [&](const T* col, uint32_t rb, uint32_t re, A& mean, A& ss) {
       A sum = (A)0;
-      for (uint32_t r = 0; r < R; r += 8) {
+      for (uint32_t r = rb; r < re; r += 8) {
         T x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, R - 1) * C];
+        for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, re - 1) * C];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-          if (r + u < R) sum += acc_up<A>(x[u]);
+          if (r + u < re) sum += acc_up<A>(x[u]);
       }
-      const A mean = sum / (A)R;
-      A ss = (A)0;
-      for (uint32_t r = 0; r < R; r += 8) {
+      mean = sum / (A)(re - rb);
+      ss = (A)0;
+      for (uint32_t r = rb; r < re; r += 8) {
         T x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, R - 1) * C];
+        for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, re - 1) * C];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          if (r + u < R) {
+          if (r + u < re) {
             const A d = acc_up<A>(x[u]) - mean;
             ss += d * d;
           }
         }
       }
+    };
+    auto put = [&](uint32_t o, uint32_t c, A ss) {
       I inOff, outOff;
       a.oa.offsets(o0 + o, inOff, outOff);
       out[outOff + (I)c * a.outInner] = acc_down<T>(wantStd ? sqrt_any(ss / div) : ss / div);
+    };
+    if (P <= 1) {
+      for (uint32_t t = threadIdx.x; t < cols; t += kBlock) {
+        uint32_t o, c;
+        a.cdiv.divmod(t, o, c);
+        A mean, ss;
+        sweep(lds + mis + o * slice + c, 0, R, mean, ss);
+        put(o, c, ss);
+      }
+    } else {
+      const uint32_t p = threadIdx.x / cols, t = threadIdx.x - p * cols;
+      uint32_t o, c;
+      a.cdiv.divmod(t, o, c);
+      if (p < P) {
+        const uint32_t rb = p * R / P, re = (p + 1) * R / P;  // (at least 8 rows)
+        A mean, ss;
+        sweep(lds + mis + o * slice + c, rb, re, mean, ss);
+        bands[0][threadIdx.x] = (A)(re - rb);
+        bands[1][threadIdx.x] = mean;
+        bands[2][threadIdx.x] = ss;
+      }
+      __syncthreads();
+      for (uint32_t h = 1; h < P; h <<= 1) {
+        if (p < P && (p & (2 * h - 1)) == 0 && p + h < P) {
+          const uint32_t i = threadIdx.x, j = i + h * cols;
+          A n = bands[0][i], mean = bands[1][i], ss = bands[2][i];
+          moments_merge(n, mean, ss, bands[0][j], bands[1][j], bands[2][j]);
+          bands[0][i] = n;
+          bands[1][i] = mean;
+          bands[2][i] = ss;
+        }
+        __syncthreads();
+      }
+      if (p == 0) put(o, c, bands[2][t]);
     }
     __syncthreads();
   }
@@ -1530,7 +1592,9 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
     a.colTiles.divmod(group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
-    const I col = (ct * TX + tx) * VEC;
+    const I at0 = (ct * TX + tx) * VEC;
+    const bool live = at0 < a.C;
+    const I col = VEC > 1 ? min(at0, a.C - VEC) : at0;  // (a row's last pack is moved back to end with it)
     A acc[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) acc[e] = f.init();
@@ -1538,7 +1602,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
     if (foldPass) {
       // second launch: one workgroup per group (S == 1 in the block index),
       // thread row ty folds planes ty, ty+TY, ...
-      if (col < a.C) {
+      if (live) {
         constexpr int UF = 8;  // planes fetched per batch
         I sp = ty;
         for (; sp + (UF - 1) * TY < a.S.d; sp += UF * TY) {
@@ -1559,7 +1623,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
           for (int e = 0; e < VEC; ++e) acc[e] = f.combine(acc[e], plane[sp * a.outElems + e]);
         }
       }
-    } else if (col < a.C) {
+    } else if (live) {
       const I begin = s * a.chunkR;
       const I end = min(a.R, begin + a.chunkR);
       const TIn* src = in + inOff + col;
@@ -1575,7 +1639,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
         P v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + (r + u * TY) * a.sR));
+          v[u] = load_pack_unaligned<true, P>(src + (r + u * TY) * a.sR);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -1584,14 +1648,14 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
         }
       }
       for (; r < end; r += TY) {
-        const P v = load_pack<true>(reinterpret_cast<const P*>(src + r * a.sR));
+        const P v = load_pack_unaligned<true, P>(src + r * a.sR);
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
           acc[e] = f.combine(acc[e], f.modify(acc_up<A>(v.v[e]), c[e]));
       }
     }
     fold_rows(acc);
-    if (ty == 0 && col < a.C) {
+    if (ty == 0 && live) {
       if (foldPass || a.S.d == 1) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
@@ -1610,29 +1674,19 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
 // reductions, workgroup partials are merged with the pairwise update of Chan,
 // Golub & LeVeque. Same geometry as reduce_cols_kernel. Partial planes hold
 // (mean, M2) per output: partial[(s * 2 + {0, 1}) * outElems + out].
-template <typename A>
-__device__ __forceinline__ void moments_merge(A& na, A& ma, A& sa, A nb, A mb, A sb) {
-  const A n = na + nb;
-  if (n > (A)0) {
-    const A delta = mb - ma;
-    const A w = nb / n;
-    ma += delta * w;
-    sa += sb + delta * delta * na * w;
-  }
-  na = n;
-}
-
-template <typename T, typename I, int VEC>
-__global__ __launch_bounds__(kBlock) void var_rows_long_kernel(const T* __restrict__ in, T* __restrict__ out,
-                                                               OuterArgs<I> oa, I numRows, I R,
-                                                               typename Acc<T>::type div, bool wantStd) {
+// BT = 0: a wave per row. BT > 0: a workgroup of BT threads per row, for rows too few to fill the chip with waves
+// (var of 328 x 15366 fp32 26.7 us in two sweeps, 9.7 in one; 44 x 14186 15.5 and 6.9, 2 x 19968 doubles 16.3 and 7.8). Packs sit at element-aligned addresses; the elements behind the last whole pack go one to a lane.
+template <typename T, typename I, int VEC, int BT>
+__global__ __launch_bounds__(BT ? BT : kBlock) void var_rows_long_kernel(const T* __restrict__ in, T* __restrict__ out,
+                                                                         OuterArgs<I> oa, I numRows, I R,
+                                                                         typename Acc<T>::type div, bool wantStd) {
   using P = Pack<T, VEC>;
   using A = typename Acc<T>::type;
-  constexpr int U = 8;
-  const uint32_t lane = threadIdx.x & 63;
-  const I wavesPerGrid = (I)gridDim.x * (kBlock / 64);
-  const I step = (I)64 * VEC;
-  for (I row = (I)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); row < numRows; row += wavesPerGrid) {
+  constexpr int U = 8, kLanes = BT ? BT : 64, kRows = (BT ? BT : kBlock) / kLanes;
+  const uint32_t lane = threadIdx.x & (kLanes - 1);
+  const I step = (I)kLanes * VEC;
+  const I packed = R - R % VEC;
+  for (I row = (I)blockIdx.x * kRows + threadIdx.x / kLanes; row < numRows; row += (I)gridDim.x * kRows) {
     I inOff, outOff;
     oa.offsets(row, inOff, outOff);
     const T* src = in + inOff;
@@ -1642,16 +1696,16 @@ __global__ __launch_bounds__(kBlock) void var_rows_long_kernel(const T* __restri
       mean[e] = (A)0;
       m2[e] = (A)0;
     }
-    for (I i = (I)lane * VEC; i < R; i += (I)U * step) {
+    for (I i = (I)lane * VEC; i < packed; i += (I)U * step) {
       P v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const I at = i + (I)u * step < R ? i + (I)u * step : i;  // (past the end: re-read, not used)
-        v[u] = load_pack<true>(reinterpret_cast<const P*>(src + at));
+        const I at = i + (I)u * step < packed ? i + (I)u * step : i;  // (past the end: re-read, not used)
+        v[u] = load_pack_unaligned<true, P>(src + at);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (i + (I)u * step < R) {
+        if (i + (I)u * step < packed) {
           cnt += (A)1;
           const A inv = (A)1 / cnt;
 #pragma unroll
@@ -1667,9 +1721,22 @@ __global__ __launch_bounds__(kBlock) void var_rows_long_kernel(const T* __restri
     A n = cnt, mu = mean[0], q = m2[0];
 #pragma unroll
     for (int e = 1; e < VEC; ++e) moments_merge(n, mu, q, cnt, mean[e], m2[e]);
+    if (packed + lane < R) moments_merge(n, mu, q, (A)1, acc_up<A>(src[packed + lane]), (A)0);
     for (uint32_t o = 32; o > 0; o >>= 1) {
       const A on = shfl_xor_any(n, o), omu = shfl_xor_any(mu, o), oq = shfl_xor_any(q, o);
       moments_merge(n, mu, q, on, omu, oq);
+    }
+    if constexpr (BT > 64) {
+      __shared__ A red[BT / 64][3];
+      if ((lane & 63) == 0) {
+        red[lane / 64][0] = n;
+        red[lane / 64][1] = mu;
+        red[lane / 64][2] = q;
+      }
+      __syncthreads();
+      if (lane == 0)
+        for (int w = 1; w < BT / 64; ++w) moments_merge(n, mu, q, red[w][0], red[w][1], red[w][2]);
+      __syncthreads();
     }
     if (lane == 0) {
       const A v = q / div;
@@ -1698,7 +1765,9 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
     a.colTiles.divmod(group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
-    const I col = (ct * TX + tx) * VEC;
+    const I at0 = (ct * TX + tx) * VEC;
+    const bool live = at0 < a.C;
+    const I col = VEC > 1 ? min(at0, a.C - VEC) : at0;
     A cnt = (A)0, mean[VEC], m2[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
@@ -1706,9 +1775,34 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
       m2[e] = (A)0;
     }
     if (foldPass) {
-      if (col < a.C) {
+      if (live) {
         const A* plane = partial + rest * a.C + col;
-        for (I sp = ty; sp < a.S.d; sp += TY) {
+        constexpr int UF = 4;  // planes fetched per batch
+        I sp = ty;
+        for (; sp + (UF - 1) * TY < a.S.d; sp += UF * TY) {
+          A vm[UF][VEC], vq[UF][VEC];
+#pragma unroll
+          for (int u = 0; u < UF; ++u) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              vm[u][e] = plane[((sp + u * TY) * 2) * a.outElems + e];
+              vq[u][e] = plane[((sp + u * TY) * 2 + 1) * a.outElems + e];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < UF; ++u) {
+            const I begin = (sp + u * TY) * a.chunkR;
+            const A nb = (A)(min(a.R, begin + a.chunkR) - begin);
+            A n = cnt;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              n = cnt;
+              moments_merge(n, mean[e], m2[e], nb, vm[u][e], vq[u][e]);
+            }
+            cnt = n;
+          }
+        }
+        for (; sp < a.S.d; sp += TY) {
           const I begin = sp * a.chunkR;
           const A nb = (A)(min(a.R, begin + a.chunkR) - begin);
           A n = cnt;
@@ -1721,7 +1815,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
           cnt = n;
         }
       }
-    } else if (col < a.C) {
+    } else if (live) {
       const I begin = s * a.chunkR;
       const I end = min(a.R, begin + a.chunkR);
       const T* src = in + inOff + col;
@@ -1731,7 +1825,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
         P v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + (r + u * TY) * a.sR));
+          v[u] = load_pack_unaligned<true, P>(src + (r + u * TY) * a.sR);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           cnt += (A)1;
@@ -1746,7 +1840,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
         }
       }
       for (; r < end; r += TY) {
-        const P v = load_pack<true>(reinterpret_cast<const P*>(src + r * a.sR));
+        const P v = load_pack_unaligned<true, P>(src + r * a.sR);
         cnt += (A)1;
         const A inv = (A)1 / cnt;
 #pragma unroll
@@ -1780,7 +1874,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
       }
       __syncthreads();
     }
-    if (ty == 0 && col < a.C) {
+    if (ty == 0 && live) {
       if (foldPass || a.S.d == 1) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
@@ -1997,7 +2091,9 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
     a.colTiles.divmod(group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
-    const I col = (ct * TX + tx) * VEC;
+    const I at0 = (ct * TX + tx) * VEC;
+    const bool live = at0 < a.C;
+    const I col = VEC > 1 ? min(at0, a.C - VEC) : at0;
     const I at = rest * a.C + col;
     A bv[VEC];
     I bi[VEC];
@@ -2007,8 +2103,32 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
       bi[e] = ~(I)0;
     }
     if (foldPass) {
-      if (col < a.C) {
-        for (I sp = ty; sp < a.S.d; sp += TY) {
+      if (live) {
+        constexpr int UF = 4;  // planes fetched per batch
+        I sp = ty;
+        for (; sp + (UF - 1) * TY < a.S.d; sp += UF * TY) {
+          A v[UF][VEC];
+          I ix[UF][VEC];
+#pragma unroll
+          for (int u = 0; u < UF; ++u) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              v[u][e] = partV[(sp + u * TY) * a.outElems + at + e];
+              ix[u][e] = partI[(sp + u * TY) * a.outElems + at + e];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < UF; ++u) {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              if (O::better(v[u][e], ix[u][e], bv[e], bi[e])) {
+                bv[e] = v[u][e];
+                bi[e] = ix[u][e];
+              }
+            }
+          }
+        }
+        for (; sp < a.S.d; sp += TY) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
             const A v = partV[sp * a.outElems + at + e];
@@ -2020,7 +2140,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
           }
         }
       }
-    } else if (col < a.C) {
+    } else if (live) {
       const I begin = s * a.chunkR;
       const I end = min(a.R, begin + a.chunkR);
       const T* src = in + inOff + col;
@@ -2030,7 +2150,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
         P v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = load_pack<true>(reinterpret_cast<const P*>(src + (r + u * TY) * a.sR));
+          v[u] = load_pack_unaligned<true, P>(src + (r + u * TY) * a.sR);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -2044,7 +2164,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
         }
       }
       for (; r < end; r += TY) {
-        const P v = load_pack<true>(reinterpret_cast<const P*>(src + r * a.sR));
+        const P v = load_pack_unaligned<true, P>(src + r * a.sR);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           const A x = acc_up<A>(v.v[e]);
@@ -2056,7 +2176,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
       }
     }
     fold_rows(bv, bi);
-    if (ty == 0 && col < a.C) {
+    if (ty == 0 && live) {
       if (foldPass || a.S.d == 1) {
         I unused, idxOff;
         oaIdx.offsets(rest, unused, idxOff);
@@ -2476,6 +2596,13 @@ bool plan_rows_lds(THCState* s, const ReduceGeom& g, bool vec, uint32_t& rowsPer
   return true;
 }
 
+// Rows off the 16-byte grid are read as packs at element-aligned addresses from 1 KiB on, the elements behind the last whole
+// pack one by one (fp32 sums of 328 x 15366 11.2 -> 6.7 us, of 44 x 14186 7.6 -> 4.8, max 11.8 -> 8.1; 1000 x 9001 12.3 -> 7.1, 16.3 -> 10.0).
+template <typename T>
+bool loose_row_packs(const ReduceGeom& g) {
+  return g.sR == 1 && g.R * (int64_t)sizeof(T) >= 1024 && tuning("reduce.rows.packs", 1);
+}
+
 // rows: a group of lanes per output. Packs when the reduced dim has unit stride
 // and everything is 16-byte aligned, scalar strided loads otherwise.
 template <typename T, typename F, typename I>
@@ -2485,6 +2612,8 @@ void run_rows(THCState* s, const ReduceGeom& g, const T* in, T* out, Epi<typenam
   const int64_t rows = g.outElems;
   bool vec = g.sR == 1 && aligned16(in) && g.R % VEC == 0;
   for (int d = 0; d < g.in.dims && vec; ++d) vec = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
+  const bool whole = vec;  // rows of whole aligned packs
+  vec = vec || loose_row_packs<T>(g);
   OuterArgs<I> oa = make_outer<I>(g.in, g.out, g.in.dims);
 
   // Few long rows: cut them so that about `target` waves have work.
@@ -2503,7 +2632,7 @@ void run_rows(THCState* s, const ReduceGeom& g, const T* in, T* out, Epi<typenam
   }
   uint32_t ldsRows = 0, ldsG = 0, quadMin = 0;
   size_t ldsBytes = 0;
-  if (S == 1 && plan_rows_lds<T>(s, g, vec, ldsRows, ldsG, ldsBytes, &quadMin)) {
+  if (S == 1 && plan_rows_lds<T>(s, g, whole, ldsRows, ldsG, ldsBytes, &quadMin)) {
     const int64_t blocks = (rows + ldsRows - 1) / ldsRows;
     const int grid = capped_grid(s, blocks, "reduce.rows.lds_blocks_per_cu", 64);
     hipLaunchKernelGGL((reduce_rows_lds_kernel<T, T, F, I>), dim3(grid), dim3(kBlock), ldsBytes,
@@ -2539,17 +2668,29 @@ struct ColsPlan {
   bool vec;
 };
 
+// Which packs a column kernel may read: only whole aligned ones, any, or any under the (value, index) kernel's rule.
+enum class ColPacks { Whole, Loose, Index };
+
 // cols: reduced dim strided, innermost joint dim has unit input stride.
 template <typename T, typename I>
 ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t partialElemBytes,
                       const char* perCuKey = "reduce.cols.blocks_per_cu", int perCuDefault = 1,
-                      const char* rowBytesKey = "reduce.cols.min_row_bytes", int rowBytesDefault = 1024) {
+                      const char* rowBytesKey = "reduce.cols.min_row_bytes", int rowBytesDefault = 1024,
+                      ColPacks packs = ColPacks::Loose) {
   constexpr int VEC = 16 / sizeof(T);
   ColsPlan<I> p{};
   const int nd = g.in.dims;
   const int64_t C = g.in.size[nd - 1];
+  // Rows off the 16-byte grid, or of no whole number of packs: packs at element-aligned addresses, the last one moved back to end
+  // with the row, from 16 MiB on; one element a lane below, where the wider strips and the more workgroups that go with it win
+  // (us one by one and in packs: 319807 x 394 along dim 0 fp32 sum 203 / 86, max 147 / 99, half sum 190 / 45; 24836 x 986 fp32 var 41 / 22;
+  // 200 x 33 x 1001 fp32 14.6 / 6.8; but 1688 x 518 max 9.2 / 12.8). 2-byte elements: few long slices or few rows (594 x
+  // 144 x 967 half 39 / 53), (value, index) only where the slices are long (8191 x 8193 42 / 48). Bytes never (sum of 24836 x 986
+  // 14 / 20: 16-byte loads at odd addresses).
   bool vec = aligned16(in) && C % VEC == 0 && g.sR % VEC == 0;
   for (int d = 0; d < nd - 1 && vec; ++d) vec = g.in.stride[d] % VEC == 0;
+  if (!vec && packs != ColPacks::Whole && C >= 64 && sizeof(T) > 1 && g.outElems * g.R * (int64_t)sizeof(T) >= tuning("reduce.cols.loose_bytes", 16 << 20))
+    vec = sizeof(T) >= 4 || g.R <= 64 || (g.outElems / C < 64 && (packs != ColPacks::Index || g.R >= 16384));
   const int pack = vec ? VEC : 1;
   const int64_t target = tuning("reduce.cols.target_blocks", (int64_t)num_compute_units(s) * tuning(perCuKey, perCuDefault));
   const int64_t outer = g.outElems / C;
@@ -2628,6 +2769,19 @@ ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t p
   p.a.TX = TX;
   p.totalBlocks = base * S;
   return p;
+}
+
+// The second launch of a split column reduction: S planes of accumulators are folded column by column, whatever packs the
+// input was read in. As many thread rows as planes up to 16 (a thread walks 8 planes a batch), so 16 columns and
+// more to a workgroup: with the first launch's geometry one workgroup folded 256 planes of 415 half columns (38 us of 49).
+template <typename I>
+ColsArgs<I> fold_geometry(const ColsArgs<I>& a, int64_t outElems, int64_t& groups) {
+  ColsArgs<I> f = a;
+  f.TX = std::max<uint32_t>(16, kBlock / (uint32_t)pow2_ceil((uint64_t)std::min<int64_t>((int64_t)a.S.d, 16)));
+  const int64_t C = (int64_t)a.C, tiles = (C + f.TX - 1) / f.TX;
+  f.colTiles.set((uint64_t)tiles);
+  groups = outElems / C * tiles;
+  return f;
 }
 
 // Small dense slices (see reduce_slab_kernel): [O][R][C] with rows of a slice
@@ -2812,22 +2966,25 @@ void run_cols(THCState* s, const ReduceGeom& g, const T* in, T* out, Epi<typenam
     }
   }
   if (run_slab_chunked<T, F, I>(s, g, in, out, epi, f)) return;
-  ColsPlan<I> p = plan_cols<T, I>(s, g, in, sizeof(A));
+  // (a functor that reads its centre from the output cannot share columns between two packs)
+  ColsPlan<I> p = plan_cols<T, I>(s, g, in, sizeof(A), "reduce.cols.blocks_per_cu", 1, "reduce.cols.min_row_bytes", 1024,
+                                  F::kCentred ? ColPacks::Whole : ColPacks::Loose);
   const bool split = p.a.S.d > 1;
   A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
   const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
-  const int64_t groups = p.totalBlocks / (int64_t)p.a.S.d;
+  int64_t groups = 0;
+    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
   hipStream_t st = current_stream(s);
   for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
     const bool fold = pass == 1;
     const int gr = fold ? (int)groups : grid;
     const I tb = fold ? (I)groups : (I)p.totalBlocks;
-    if (p.vec)
+    if (p.vec && !fold)
       hipLaunchKernelGGL((reduce_cols_kernel<T, T, F, I, VEC>), dim3(gr), dim3(kBlock), 0, st, in,
                          out, scratch, p.a, tb, epi, f, fold);
     else
       hipLaunchKernelGGL((reduce_cols_kernel<T, T, F, I, 1>), dim3(gr), dim3(kBlock), 0, st, in,
-                         out, scratch, p.a, tb, epi, f, fold);
+                         out, scratch, fold ? folds : p.a, tb, epi, f, fold);
   }
   note_kernel(split ? (p.vec ? "cols-split" : "cols-split-scalar") : (p.vec ? "cols" : "cols-scalar"));
 }
@@ -2860,6 +3017,8 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
   if (!colsShape) {
     bool vec = g.sR == 1 && aligned16(in) && g.R % VEC == 0;
     for (int d = 0; d < nd && vec; ++d) vec = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
+    const bool whole = vec;
+    vec = vec || (sizeof(T) > 1 && loose_row_packs<T>(g));  // (bytes: 8191 x 8193 24 us one by one, 38 in packs)
     const int pack = vec ? VEC : 1;
     OuterArgs<I> oa = make_outer<I>(g.in, g.out, nd);
     OuterArgs<I> oaIdx = make_outer<I>(g.in, g.idx, nd);
@@ -2867,7 +3026,7 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
     {
       uint32_t ldsRows = 0, ldsG = 0, quadMin = 0;
       size_t ldsBytes = 0;
-      if (plan_rows_lds<T>(s, g, vec, ldsRows, ldsG, ldsBytes, &quadMin, true)) {
+      if (plan_rows_lds<T>(s, g, whole, ldsRows, ldsG, ldsBytes, &quadMin, true)) {
         const int grid = capped_grid(s, (rows + ldsRows - 1) / ldsRows, "reduce.rows.lds_blocks_per_cu", 64);
         hipLaunchKernelGGL((reduce_rows_index_lds_kernel<T, I, IS_MAX>), dim3(grid), dim3(kBlock),
                            ldsBytes, st, in, outV, outI, oa, oaIdx, (I)rows, (I)g.R, ldsRows, ldsG, quadMin);
@@ -2996,7 +3155,7 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
     // the (value, index) kernel does several ALU steps per element: two workgroups
     // per CU hide them (6.5 TB/s against 4.4 with one), the plain reductions want one
     ColsPlan<I> p = plan_cols<T, I>(s, g, in, 16, "reduce.cols.index_blocks_per_cu", 2,
-                                    "reduce.cols.index_min_row_bytes", 512);
+                                    "reduce.cols.index_min_row_bytes", 512, ColPacks::Index);
     OuterArgs<I> oaIdx = make_outer<I>(g.in, g.idx, nd - 1);
     const I idxInner = (I)g.idx.stride[nd - 1];
     const bool split = p.a.S.d > 1;
@@ -3008,17 +3167,18 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
       partV = (A*)(scratch + 8 * (size_t)p.a.S.d * (size_t)g.outElems);
     }
     const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
-    const int64_t groups = p.totalBlocks / (int64_t)p.a.S.d;
+    int64_t groups = 0;
+    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
     for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
       const bool fold = pass == 1;
       const int gr = fold ? (int)groups : grid;
       const I tb = fold ? (I)groups : (I)p.totalBlocks;
-      if (p.vec)
+      if (p.vec && !fold)
         hipLaunchKernelGGL((reduce_cols_index_kernel<T, I, VEC, IS_MAX>), dim3(gr), dim3(kBlock), 0,
                            st, in, outV, outI, partV, partI, p.a, oaIdx, idxInner, tb, fold);
       else
         hipLaunchKernelGGL((reduce_cols_index_kernel<T, I, 1, IS_MAX>), dim3(gr), dim3(kBlock), 0,
-                           st, in, outV, outI, partV, partI, p.a, oaIdx, idxInner, tb, fold);
+                           st, in, outV, outI, partV, partI, fold ? folds : p.a, oaIdx, idxInner, tb, fold);
     }
     note_kernel(split ? "cols-index-split" : "cols-index");
   }
@@ -3083,22 +3243,35 @@ bool reduce_var_rows_type(THCState* s, const ReduceGeom& g, const void* in_, voi
     bool inRegisters = g.sR == 1 && aligned16(in) && g.R % VEC == 0 && g.R <= 64 * VEC * U;
     for (int d = 0; d < g.in.dims && inRegisters; ++d)
       inRegisters = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
-    bool longRows = g.sR == 1 && aligned16(in) && g.R % VEC == 0 && g.R > 64 * VEC * U && tuning("reduce.var.long_rows", 1) &&
-                    g.outElems >= (int64_t)num_compute_units(s) * 4;
-    for (int d = 0; d < g.in.dims && longRows; ++d) longRows = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
+    // Longer rows, and from 1 KiB on rows off the 16-byte grid that the LDS-staged form below does not take: one read, a wave
+    // per row, or a workgroup per row where that leaves CUs idle. Few rows beyond 64 Ki elements take two sweeps, cut into pieces.
+    uint32_t ldsRowsProbe = 0, ldsGProbe = 0;
+    size_t ldsBytesProbe = 0;
+    const int64_t cus = num_compute_units(s);
+    bool wholePacks = g.sR == 1 && aligned16(in) && g.R % VEC == 0;
+    for (int d = 0; d < g.in.dims && wholePacks; ++d) wholePacks = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
+    const bool longRows = !inRegisters && g.sR == 1 && tuning("reduce.var.long_rows", 1) &&
+                          (wholePacks ? g.R > 64 * VEC * U * (g.outElems >= cus * 4 ? 1 : 2) : loose_row_packs<T>(g) && !plan_rows_lds<T>(s, g, false, ldsRowsProbe, ldsGProbe, ldsBytesProbe)) &&
+                          (g.outElems >= cus || g.R <= 65536);
     if (longRows) {
-      const int wpb = kBlock / 64;
-      const int grid = capped_grid(s, (g.outElems + wpb - 1) / wpb, "reduce.rows.blocks_per_cu", 64);
+      // (a workgroup of 256 for rows a wave could walk in a few batches, of 1024 beyond)
+      const int bt = g.outElems >= cus * 4 ? 0 : g.R <= 256 * VEC * U ? 256 : 1024;
       hipStream_t st = current_stream(s);
-      if (g.wide) {
-        OuterArgs<uint64_t> oa = make_outer<uint64_t>(g.in, g.out, g.in.dims);
-        hipLaunchKernelGGL((var_rows_long_kernel<T, uint64_t, VEC>), dim3(grid), dim3(kBlock), 0, st, in, out, oa,
-                           (uint64_t)g.outElems, (uint64_t)g.R, (A)div, wantStd);
-      } else {
-        OuterArgs<uint32_t> oa = make_outer<uint32_t>(g.in, g.out, g.in.dims);
-        hipLaunchKernelGGL((var_rows_long_kernel<T, uint32_t, VEC>), dim3(grid), dim3(kBlock), 0, st, in, out, oa,
-                           (uint32_t)g.outElems, (uint32_t)g.R, (A)div, wantStd);
-      }
+      const auto go = [&](auto idxTag, auto btTag) {
+        using I = decltype(idxTag);
+        constexpr int BT = decltype(btTag)::value;
+        constexpr int kRows = BT ? 1 : kBlock / 64;
+        const int grid = capped_grid(s, (g.outElems + kRows - 1) / kRows, "reduce.rows.blocks_per_cu", 64);
+        hipLaunchKernelGGL((var_rows_long_kernel<T, I, VEC, BT>), dim3(grid), dim3(BT ? BT : kBlock), 0, st, in, out,
+                           make_outer<I>(g.in, g.out, g.in.dims), (I)g.outElems, (I)g.R, (A)div, wantStd);
+      };
+      const auto pick = [&](auto idxTag) {
+        if (bt == 0) go(idxTag, std::integral_constant<int, 0>{});
+        else if (bt == 256) go(idxTag, std::integral_constant<int, 256>{});
+        else go(idxTag, std::integral_constant<int, 1024>{});
+      };
+      if (g.wide) pick(uint64_t{});
+      else pick(uint32_t{});
       note_kernel("var-rows-long");
       return true;
     }
@@ -3235,18 +3408,19 @@ bool reduce_var_cols_type(THCState* s, const ReduceGeom& g, const void* in_, voi
       const bool split = p.a.S.d > 1;
       A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
       const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
-      const int64_t groups = p.totalBlocks / (int64_t)p.a.S.d;
+      int64_t groups = 0;
+    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
       hipStream_t st = current_stream(s);
       for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
         const bool fold = pass == 1;
         const int gr = fold ? (int)groups : grid;
         const I tb = fold ? (I)groups : (I)p.totalBlocks;
-        if (p.vec)
+        if (p.vec && !fold)
           hipLaunchKernelGGL((var_cols_kernel<T, I, VEC>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
                              (T*)out_, scratch, p.a, tb, (A)div, wantStd, fold);
         else
           hipLaunchKernelGGL((var_cols_kernel<T, I, 1>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
-                             (T*)out_, scratch, p.a, tb, (A)div, wantStd, fold);
+                             (T*)out_, scratch, fold ? folds : p.a, tb, (A)div, wantStd, fold);
       }
       note_kernel(split ? "var-cols-split" : "var-cols");
     };

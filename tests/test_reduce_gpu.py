@@ -857,3 +857,68 @@ def test_every_row_length_up_to_300_and_some_beyond(thc, kind):
             where = "%s %s R=%d [%s]" % (kind, which, R, thc.last_kernel())
             assert (gi == wi).all(), (where, np.flatnonzero(gi != wi)[:5])
             assert_bit_equal(gv, x[np.arange(rows), wi], where)
+
+
+@pytest.mark.parametrize("kind", ["float", "half", "double", "byte", "int"])
+def test_packs_at_element_aligned_addresses(thc, kind):
+    """Rows and columns off the 16-byte grid read as packs: row lengths one below, at and one above whole packs and lane batches, storage
+    offsets 0..3, few rows (a row cut into pieces) and many; column counts of one pack, one more and of a pack and a
+    strip more, with reduced dims that are and are not split, whose last pack of a row shares columns with the one before it.
+    Exact sums of small integers, first occurrences of ties, and a NaN that reaches its own row or column only."""
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64, "byte": np.uint8, "int": np.int32}[kind]
+    item = np.dtype(dtype).itemsize
+    vec = 16 // item
+    rng = np.random.default_rng(71)
+    floating = kind in ("float", "half", "double")
+
+    def check(shape, dim, off):
+        n = int(np.prod(shape))
+        x = rng.integers(0, 3, n + off) * (rng.integers(0, max(1, shape[dim] // 100), n + off) == 0)
+        if kind != "byte":
+            x = x - (rng.integers(0, max(2, shape[dim] // 50), n + off) == 0)
+        x = x.astype(dtype)
+        strides = tuple(int(np.prod(shape[d + 1:])) for d in range(len(shape)))
+        dev = thc.Tensor.from_storage(x, off, shape, strides, kind=kind)
+        host = x[off:].reshape(shape)
+        assert_bit_equal(thc.Tensor(kind).sum(dev, dim).numpy(), host.astype(np.int64).sum(axis=dim, keepdims=True).astype(dtype), "sum %s %d" % (shape, off))
+        for which, arg, ext in (("max", np.argmax, np.max), ("min", np.argmin, np.min)):
+            vals, idx = thc.Tensor(kind), thc.Tensor("long")
+            getattr(vals, which)(idx, dev, dim)
+            assert_bit_equal(vals.numpy(), ext(host, axis=dim, keepdims=True), "%s %s %d" % (which, shape, off))
+            assert np.array_equal(idx.numpy(), np.expand_dims(arg(host, axis=dim), dim) + 1), (which, shape, off)
+        if floating:
+            got = thc.Tensor(kind).var(dev, dim).numpy().astype(np.float64)
+            want = host.astype(np.float64).var(axis=dim, ddof=1, keepdims=True)
+            assert np.allclose(got, want, rtol={"float": 1e-5, "half": 2e-3, "double": 1e-12}[kind], atol=1e-7), (shape, off)   # (half: 2^-24 steps)
+            at = tuple(int(rng.integers(0, m)) for m in shape)
+            host = host.copy()
+            host[at] = np.nan
+            got = thc.Tensor(kind).sum(thc.Tensor.from_numpy(host), dim).numpy()
+            assert_bit_equal(got, host.astype(np.float64).sum(axis=dim, keepdims=True).astype(dtype), "NaN %s" % (shape,))
+
+    for n in (8192 // item + 1, 64 * vec * 8 - 1, 64 * vec * 8 + 1, 128 * vec * 8 + 3, 20001):
+        for rows in (1, 3, 70):
+            check((rows, n), 1, int(rng.integers(0, 4)))
+    check((1100, 8192 // item + 5), 1, 1)
+    thc.set_tuning("reduce.cols.loose_bytes", 0)
+    try:
+        for cols in (64, 65, 64 + vec - 1, 64 * vec + 1, 4 * 64 * vec + vec + 1):
+            for shape, dim in (((5, cols), 0), ((3, 40, cols), 1), ((1, 2500, cols), 1)):
+                check(shape, dim, int(rng.integers(0, 4)))
+    finally:
+        thc.set_tuning("reduce.cols.loose_bytes", 16 << 20)
+
+
+@pytest.mark.parametrize("kind", ["float", "half", "double"])
+def test_var_of_small_slices_with_few_columns(thc, kind):
+    """Threads that share a column's rows: columns one below and above what leaves several threads each, rows around the bands of 8."""
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64}[kind]
+    rng = np.random.default_rng(73)
+    for shape in ((3, 576, 2), (7, 15, 3), (1, 16, 100), (2, 17, 128), (5, 250, 4), (40, 33, 8), (9, 8, 2), (1, 700, 2)):
+        x = (rng.standard_normal(shape) * 2 + 5).astype(dtype)
+        for off in (0, 1):
+            store = np.concatenate([np.zeros(off, dtype), x.reshape(-1)])
+            dev = thc.Tensor.from_storage(store, off, shape, (shape[1] * shape[2], shape[2], 1), kind=kind)
+            got = thc.Tensor(kind).var(dev, 1).numpy().astype(np.float64)
+            want = x.astype(np.float64).var(axis=1, ddof=1, keepdims=True)
+            assert np.all(np.abs(got - want) <= {"float": 1e-5, "half": 2e-3, "double": 1e-12}[kind] * want), (shape, off)
