@@ -306,11 +306,12 @@ __global__ __launch_bounds__(kBlock) void apply_contig_kernel(TOut* out, const T
 // ------------------------------------------------------------------------
 // strided / generic: linear index -> per-operand offsets
 // ------------------------------------------------------------------------
-template <typename I>
+template <typename I, bool JOINT>
 struct IndexedArgs {
-  int dims[kMaxOps];                  // JOINT: only dims[0] is used
-  Divisor<I> size[kMaxOps][kMaxDims]; // JOINT: only size[0][*] is used
-  I stride[kMaxOps][kMaxDims];        // in elements; pre-multiplied by VEC in the packed dim
+  static constexpr int kSizes = JOINT ? 1 : kMaxOps;   // JOINT: one set of sizes for all operands
+  int dims[kSizes];
+  Divisor<I> size[kSizes][kArgDims<I>];
+  I stride[kMaxOps][kArgDims<I>];     // in elements; pre-multiplied by VEC in the packed dim
   int ntStore;                        // packs of the output go out with the streaming hint
 };
 
@@ -319,7 +320,7 @@ struct IndexedArgs {
 template <typename T, typename Op, typename I, int VEC, bool JOINT, typename TOut = T>
 __global__ __launch_bounds__(kBlock) void apply_indexed_kernel(TOut* out, const T* in0, const T* in1,
                                                                const T* in2, I total,
-                                                               IndexedArgs<I> args, Op op, I innerElems) {
+                                                               IndexedArgs<I, JOINT> args, Op op, I innerElems) {
   // (innerElems, VEC > 1: elements of the innermost dim, whose last pack may be partial)
   using P = Pack<T, VEC>;
   using PO = Pack<TOut, VEC>;
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(kBlock) void apply_indexed_kernel(TOut* out, const 
 // ------------------------------------------------------------------------
 template <typename T, typename Op, typename I, int VEC, typename TOut = T>
 __global__ __launch_bounds__(kBlock) void apply_flatmix_kernel(TOut* out, const T* in0, const T* in1,
-                                                               const T* in2, I n, IndexedArgs<I> args,
+                                                               const T* in2, I n, IndexedArgs<I, true> args,
                                                                uint32_t denseMask, Op op) {
   using P = Pack<T, VEC>;
   using PO = Pack<TOut, VEC>;
@@ -514,8 +515,8 @@ struct TiledArgs {
   Divisor<uint32_t> qsub[kMaxFuse];      // sizes of the fused dims, innermost first
   I qstride[kMaxOps][kMaxFuse];          // strides of the fused dims, innermost first
   int nbatch;                            // remaining dims
-  Divisor<uint32_t> bsize[kMaxDims];
-  I bstride[kMaxOps][kMaxDims];
+  Divisor<uint32_t> bsize[kArgDims<I>];
+  I bstride[kMaxOps][kArgDims<I>];
   Divisor<uint32_t> tilesP, tilesQ;
   uint32_t totalTiles;
   // Tiles per XCD when workgroup b (dispatched to XCD b % 8) takes tile
@@ -1269,14 +1270,15 @@ bool indexed_can_pack_unaligned(const Plan& pl) {
 template <typename T, typename Op, typename I, bool JOINT, typename TOut = T>
 void launch_indexed(THCState* s, const Plan& pl, Op op) {
   constexpr int VEC = pack_elems<T, TOut>();
-  IndexedArgs<I> args{};
+  IndexedArgs<I, JOINT> args{};
   const bool aligned = JOINT && indexed_can_pack<T, TOut>(pl);
   const bool vec = aligned || (JOINT && indexed_can_pack_unaligned<T, TOut>(pl));
   const int pack = vec ? VEC : 1;
   int64_t total = 1;
   for (int k = 0; k < pl.nops; ++k) {
     const int nd = pl.lay[k].dims;
-    args.dims[k] = nd;
+    const bool own = k < args.kSizes;
+    if (own) args.dims[k] = nd;
     for (int d = 0; d < nd; ++d) {
       int64_t sz = pl.lay[k].size[d];
       int64_t sd = pl.lay[k].stride[d];
@@ -1284,7 +1286,7 @@ void launch_indexed(THCState* s, const Plan& pl, Op op) {
         sz = (sz + pack - 1) / pack;
         sd *= pack;
       }
-      args.size[k][d].set((uint64_t)sz);
+      if (own) args.size[k][d].set((uint64_t)sz);
       args.stride[k][d] = (I)sd;
       if (k == 0) total *= sz;
     }
@@ -1613,13 +1615,11 @@ bool launch_flatmix(THCState* s, const Plan& pl, Op op) {
     ++gathered;
   }
   if (gathered == 0) return false;
-  IndexedArgs<I> args{};
-  for (int k = 0; k < pl.nops; ++k) {
-    args.dims[k] = nd;
-    for (int d = 0; d < nd; ++d) {
-      args.size[k][d].set((uint64_t)pl.lay[0].size[d]);
-      args.stride[k][d] = (I)pl.lay[k].stride[d];
-    }
+  IndexedArgs<I, true> args{};
+  args.dims[0] = nd;
+  for (int d = 0; d < nd; ++d) {
+    args.size[0][d].set((uint64_t)pl.lay[0].size[d]);
+    for (int k = 0; k < pl.nops; ++k) args.stride[k][d] = (I)pl.lay[k].stride[d];
   }
   args.ntStore = streaming_store("apply.indexed.nt_store", pl.numel * (int64_t)sizeof(TOut)) ? 1 : 0;
   const int64_t packs = pl.numel / VEC + 1;
@@ -1646,6 +1646,7 @@ bool run_plan(THCState* s, Plan& pl, bool sameShape, Op op, bool decline = false
     for (int d = 0; d < pl.lay[k].dims; ++d) wide = wide || pl.lay[k].stride[d] < 0;
   }
   if (sameShape && joint_collapse(pl.nops, pl.lay, /*reorder=*/true)) {
+    wide = wide || pl.lay[0].dims > kArgDims<uint32_t>;
     bool flat = pl.lay[0].dims == 1;
     for (int k = 0; k < pl.nops && flat; ++k) flat = pl.lay[k].stride[0] == 1;
     if (flat) {
@@ -1685,7 +1686,10 @@ bool run_plan(THCState* s, Plan& pl, bool sameShape, Op op, bool decline = false
       launch_indexed<T, Op, uint32_t, true, TOut>(s, pl, op);
     return true;
   }
-  for (int k = 0; k < pl.nops; ++k) collapse(pl.lay[k]);
+  for (int k = 0; k < pl.nops; ++k) {
+    collapse(pl.lay[k]);
+    wide = wide || pl.lay[k].dims > kArgDims<uint32_t>;
+  }
   if (wide)
     launch_indexed<T, Op, uint64_t, false, TOut>(s, pl, op);
   else

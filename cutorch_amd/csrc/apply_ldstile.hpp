@@ -41,6 +41,7 @@ __device__ __forceinline__ void static_for(Fn&& fn) {
   }
 }
 
+constexpr int kLdsTileBatchDims = 12;   // (room in the arguments, see kArgDims; layouts of more dims are declined)
 struct LdsTileArgs {
   int staged[kMaxOps];   // input k is read along p and transposed on its way into LDS
   int sameGrid[kMaxOps]; // input k is read along q and its rows share the output rows' 16-byte grid (unaligned rows)
@@ -48,8 +49,8 @@ struct LdsTileArgs {
   int64_t strideP[kMaxOps];  // elements
   int64_t strideQ[kMaxOps];
   int nbatch;            // remaining joint dims
-  Divisor<uint32_t> bsize[kMaxDims];
-  int64_t bstride[kMaxOps][kMaxDims];
+  Divisor<uint32_t> bsize[kLdsTileBatchDims];
+  int64_t bstride[kMaxOps][kLdsTileBatchDims];
   Divisor<uint32_t> tilesP, tilesQ;
   uint32_t totalTiles;
   uint32_t xcdPer;   // tiles per XCD when workgroup slot b takes tile (b % 8) * xcdPer + b / 8; 0 = identity
@@ -476,6 +477,7 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
     constexpr int LXQ = 32;
     constexpr int LXP = (sizeof(T) == 1 && VEC == 16) ? 4 : ((128 / (int)sizeof(T)) / VEC < 8 ? 8 : (128 / (int)sizeof(T)) / VEC);
     const int nd = pl.lay[0].dims;
+    if (nd - 2 > kLdsTileBatchDims) return false;
     auto elem_size = [](int k) { return k == 0 ? sizeof(TOut) : sizeof(T); };
     bool aligned = pl.lay[0].size[p] % VEC == 0 && pl.lay[0].size[q] % VEC == 0;
     for (int k = 0; k < pl.nops; ++k) {

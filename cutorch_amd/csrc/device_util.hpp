@@ -197,6 +197,13 @@ __device__ __forceinline__ D convert_value(S x) {
   }
 }
 
+// Dims that a kernel's arguments have room for. Arguments are written to device memory by the host, one write per launch that
+// the host waits for: a kernel of 16 bytes of arguments is launched in 2.4 us, of 256 bytes in 2.6, 1 KiB 3.2, 2 KiB 3.4, so the
+// 32-bit kernels carry what nearly all layouts need after their dims have been merged, and those with more dims take the
+// 64-bit kernels. (Arguments of the strided kernel 1.7 KB -> 190 bytes, of the row reductions 0.6 KB -> 170.)
+template <typename I>
+constexpr int kArgDims = sizeof(I) == 4 ? 6 : 25;
+
 // Division by a launch-invariant divisor.
 // 32-bit: round-up multiply-shift (Granlund & Montgomery, "Division by
 // invariant integers using multiplication", 1994): with s = ceil(log2 d) and

@@ -10,6 +10,7 @@
 #include <limits>
 
 #include "reduce_plan.hpp"
+#include "device_util.hpp"
 #include "stream_guard.hpp"
 
 namespace thc {
@@ -32,6 +33,7 @@ ReduceGeom make_geom(AnyTensor* in, AnyTensor* out, AnyTensor* idxT, int dim) {
   g.in = ops[0];
   g.out = ops[1];
   g.idx = ops[2];
+  g.wide = g.wide || g.in.dims > kArgDims<uint32_t>;
   g.outElems = g.in.numel();
   if (g.R == 1) g.sR = 1;
   return g;
@@ -209,7 +211,7 @@ bool reduce_all(THCState* s, DType dt, ReduceOp op, double p, AnyTensor* in, Sca
     collapse(l);
   }
   ReduceGeom g{};
-  g.wide = force_64bit_index() || !fits_32bit(l);
+  g.wide = force_64bit_index() || !fits_32bit(l) || l.dims > kArgDims<uint32_t>;
   for (int d = 0; d < l.dims; ++d) g.wide = g.wide || l.stride[d] < 0;
   g.R = l.size[l.dims - 1];
   g.sR = 1;

@@ -264,9 +264,9 @@ struct PairOrder {
 template <typename I>
 struct OuterArgs {
   int dims;
-  Divisor<I> size[kMaxDims];
-  I inStride[kMaxDims];
-  I outStride[kMaxDims];
+  Divisor<I> size[kArgDims<I>];
+  I inStride[kArgDims<I>];
+  I outStride[kArgDims<I>];
   __device__ __forceinline__ void offsets(I lin, I& inOff, I& outOff) const {
     inOff = 0;
     outOff = 0;
