@@ -50,6 +50,9 @@ def lib():
         _lib = C.CDLL(LIB_PATH)
         _declare(_lib)
         _pending = C.c_long.in_dll(_lib, "THCAmd_pendingErrors")
+        from . import _fastcall
+        _fastcall.setup(C.addressof(_pending), C.cast(_lib.THCAmd_lastError, C.c_void_p).value,
+                        C.cast(_lib.THCAmd_clearLastError, C.c_void_p).value, THCError)
         # Handlers that return: the failed entry point returns to us and the
         # message is picked up from THCAmd_lastError by _check().
         _err_cb = (C.CFUNCTYPE(None, C.c_char_p, C.c_void_p)(lambda m, d: None),
@@ -100,6 +103,37 @@ _COPY_SUFFIX = {"byte": "Byte", "char": "Char", "short": "Short", "int": "Int", 
                 "float": "Float", "double": "Double", "half": "Half"}
 _FLOAT_KINDS = ("float", "half")
 _FUNCTIONS = {kind: {} for kind in _TYPES}      # method name -> foreign function, filled as they are used
+_CODES = {C.c_float: "f", C.c_double: "d", C.c_long: "l", C.c_int: "i", C.c_short: "h", C.c_byte: "b", C.c_ubyte: "B",
+          C.c_uint16: "e", C.POINTER(_Tensor): "t", None: "v"}
+
+
+class _Calls(dict):
+    """Method name -> the entry point as a call on tensor addresses and numbers that raises the entry point's error
+    (csrc/fastcall.cpp), filled as they are used. Back-to-back calls on small tensors are bound by the host: ctypes'
+    conversions and the look-ups around them took 0.77 us of every call."""
+
+    def __init__(self, kind):
+        self.prefix = _TYPES[kind][0] + "_"
+
+    def __missing__(self, name):
+        from . import _fastcall
+        st, f = state(), getattr(lib(), self.prefix + name)
+        signature = "".join(_CODES.get(t, "?") for t in [f.restype] + list(f.argtypes[1:]))
+        call = _fastcall.bind(C.cast(f, C.c_void_p).value, signature, st)
+        if call is None:       # a signature that the fast calls do not have
+            pointers = [t is C.POINTER(_Tensor) for t in f.argtypes[1:]]
+            halves = [t is C.c_uint16 for t in f.argtypes[1:]]
+
+            def call(*args):
+                r = f(st, *[C.cast(a, C.POINTER(_Tensor)) if p else _half_bits(a) if h else a
+                            for a, p, h in zip(args, pointers, halves)])
+                _check()
+                return r
+        self[name] = call
+        return call
+
+
+_CALLS = {kind: _Calls(kind) for kind in _TYPES}
 
 
 def _declare(l):
@@ -251,8 +285,10 @@ class Tensor(object):
         self.kind = kind
         self.T, self.S, self.creal, self.np_dtype = _TYPES[kind]
         self._fns = _FUNCTIONS[kind]
+        self._calls = _CALLS[kind]
         self._st = state()
         self.h = handle if handle is not None else self._fn("new")(self._st)
+        self.a = C.cast(self.h, C.c_void_p).value     # the tensor's address, as the calls take it
 
     def _fn(self, name):
         f = self._fns.get(name)
@@ -391,139 +427,157 @@ class Tensor(object):
         return out
 
     # --------------------------------------------------------------- math --
-    def _call(self, name, *args):
-        self._fn(name)(self._st, *args)
-        _check()
+    def copy(self, src):
+        self._calls["copy"](self.a, src.a)
         return self
 
-    def copy(self, src):
-        return self._call("copy", self.h, src.h)
-
     def fill(self, v):
-        return self._call("fill", self.h, self._real(v))
+        self._calls["fill"](self.a, v)
+        return self
 
     def zero(self):
-        return self._call("zero", self.h)
+        self._calls["zero"](self.a)
+        return self
 
     def add(self, src, v):      # self = src + v
-        return self._call("add", self.h, src.h, self._real(v))
+        self._calls["add"](self.a, src.a, v)
+        return self
 
     def sub(self, src, v):
-        return self._call("sub", self.h, src.h, self._real(v))
+        self._calls["sub"](self.a, src.a, v)
+        return self
 
     def mul(self, src, v):
-        return self._call("mul", self.h, src.h, self._real(v))
+        self._calls["mul"](self.a, src.a, v)
+        return self
 
     def div(self, src, v):
-        return self._call("div", self.h, src.h, self._real(v))
+        self._calls["div"](self.a, src.a, v)
+        return self
 
     def cadd(self, src1, v, src2):  # self = src1 + v * src2
-        return self._call("cadd", self.h, src1.h, self._real(v), src2.h)
+        self._calls["cadd"](self.a, src1.a, v, src2.a)
+        return self
 
     def csub(self, src1, v, src2):
-        return self._call("csub", self.h, src1.h, self._real(v), src2.h)
+        self._calls["csub"](self.a, src1.a, v, src2.a)
+        return self
 
     def cmul(self, src1, src2):
-        return self._call("cmul", self.h, src1.h, src2.h)
+        self._calls["cmul"](self.a, src1.a, src2.a)
+        return self
 
     def cdiv(self, src1, src2):
-        return self._call("cdiv", self.h, src1.h, src2.h)
+        self._calls["cdiv"](self.a, src1.a, src2.a)
+        return self
 
     def addcmul(self, t, v, src1, src2):  # self = t + v * src1 * src2
-        return self._call("addcmul", self.h, t.h, self._real(v), src1.h, src2.h)
+        self._calls["addcmul"](self.a, t.a, v, src1.a, src2.a)
+        return self
 
     def addcdiv(self, t, v, src1, src2):
-        return self._call("addcdiv", self.h, t.h, self._real(v), src1.h, src2.h)
+        self._calls["addcdiv"](self.a, t.a, v, src1.a, src2.a)
+        return self
 
     def unary(self, name, src):          # self = name(src): exp, log, abs, ...
-        return self._call(name, self.h, src.h)
+        self._calls[name](self.a, src.a)
+        return self
 
     def clamp(self, src, lo, hi):
-        return self._call("clamp", self.h, src.h, self._real(lo), self._real(hi))
+        self._calls["clamp"](self.a, src.a, lo, hi)
+        return self
 
     def pow(self, src, v):
-        return self._call("pow", self.h, src.h, self._real(v))
+        self._calls["pow"](self.a, src.a, v)
+        return self
 
     def tpow(self, v, src):
-        return self._call("tpow", self.h, self._real(v), src.h)
+        self._calls["tpow"](self.a, v, src.a)
+        return self
 
     def scalar2(self, name, src, v):     # cmaxValue, cminValue, fmod, remainder
-        return self._call(name, self.h, src.h, self._real(v))
+        self._calls[name](self.a, src.a, v)
+        return self
 
     def binary(self, name, src1, src2):  # cpow, cmax, cmin, cfmod, cremainder, atan2
-        return self._call(name, self.h, src1.h, src2.h)
+        self._calls[name](self.a, src1.a, src2.a)
+        return self
 
     def lerp(self, a, b, w):
-        return self._call("lerp", self.h, a.h, b.h, self._real(w))
+        self._calls["lerp"](self.a, a.a, b.a, w)
+        return self
 
     def copy_from(self, src):            # type-converting copy, any kind to any kind
-        return self._call("copyCuda" + _COPY_SUFFIX[src.kind], self.h, src.h)
+        self._calls["copyCuda" + _COPY_SUFFIX[src.kind]](self.a, src.a)
+        return self
 
     def compare_value(self, cmp, src, v, same_type=False):
         """self = src (cmp) v as 0/1; self is a Byte tensor unless same_type."""
-        return getattr(lib(), "%s_%sValue%s" % (src.T, cmp, "T" if same_type else ""))(
-            self._st, self.h, src.h, src._real(v)) or _check() or self
+        src._calls[cmp + ("ValueT" if same_type else "Value")](self.a, src.a, v)
+        return self
 
     def compare_tensor(self, cmp, a, b, same_type=False):
-        return getattr(lib(), "%s_%sTensor%s" % (a.T, cmp, "T" if same_type else ""))(
-            self._st, self.h, a.h, b.h) or _check() or self
+        a._calls[cmp + ("TensorT" if same_type else "Tensor")](self.a, a.a, b.a)
+        return self
 
     def equal(self, other):
-        r = self._fn("equal")(self._st, self.h, other.h)
-        _check()
-        return bool(r)
+        return bool(self._calls["equal"](self.a, other.a))
 
     def sum(self, src, dim, keepdim=1):   # dim is 0-based, as at the C level
-        return self._call("sum", self.h, src.h, dim, keepdim)
+        self._calls["sum"](self.a, src.a, dim, keepdim)
+        return self
 
     def prod(self, src, dim, keepdim=1):
-        return self._call("prod", self.h, src.h, dim, keepdim)
+        self._calls["prod"](self.a, src.a, dim, keepdim)
+        return self
 
     def mean(self, src, dim, keepdim=1):
-        return self._call("mean", self.h, src.h, dim, keepdim)
+        self._calls["mean"](self.a, src.a, dim, keepdim)
+        return self
 
     def norm(self, src, p, dim, keepdim=1):
-        return self._call("norm", self.h, src.h, self._real(p), dim, keepdim)
+        self._calls["norm"](self.a, src.a, p, dim, keepdim)
+        return self
 
     def cumsum(self, src, dim):
-        return self._call("cumsum", self.h, src.h, dim)
+        self._calls["cumsum"](self.a, src.a, dim)
+        return self
 
     def cumprod(self, src, dim):
-        return self._call("cumprod", self.h, src.h, dim)
+        self._calls["cumprod"](self.a, src.a, dim)
+        return self
 
     def renorm(self, src, p, dim, maxnorm):
-        return self._call("renorm", self.h, src.h, self._real(p), dim, self._real(maxnorm))
+        self._calls["renorm"](self.a, src.a, p, dim, maxnorm)
+        return self
 
     def var(self, src, dim, biased=0, keepdim=1):
-        return self._call("var", self.h, src.h, dim, biased, keepdim)
+        self._calls["var"](self.a, src.a, dim, biased, keepdim)
+        return self
 
     def std(self, src, dim, biased=0, keepdim=1):
-        return self._call("std", self.h, src.h, dim, biased, keepdim)
+        self._calls["std"](self.a, src.a, dim, biased, keepdim)
+        return self
 
     def varall(self, biased=0):
-        return self._scalar("varall", biased)
+        return self._calls["varall"](self.a, biased)
 
     def stdall(self, biased=0):
-        return self._scalar("stdall", biased)
+        return self._calls["stdall"](self.a, biased)
 
     def dist(self, other, p):
-        r = self._fn("dist")(self._st, self.h, other.h, self._real(p))
-        _check()
-        return r
+        return self._calls["dist"](self.a, other.a, p)
 
     def max(self, indices, src, dim, keepdim=1):  # self = values
-        return self._call("max", self.h, indices.h, src.h, dim, keepdim)
+        self._calls["max"](self.a, indices.a, src.a, dim, keepdim)
+        return self
 
     def min(self, indices, src, dim, keepdim=1):
-        return self._call("min", self.h, indices.h, src.h, dim, keepdim)
-
-    def _scalar(self, name, *args):
-        r = self._fn(name)(self._st, self.h, *args)
-        _check()
-        return r
+        self._calls["min"](self.a, indices.a, src.a, dim, keepdim)
+        return self
 
     def sumall(self):
-        return self._scalar("sumall")
+        return self._calls["sumall"](self.a)
 
     def sumall_no_alloc(self, result):
         """Launches the sum of all elements into result[0] (a float device tensor);
@@ -533,13 +587,13 @@ class Tensor(object):
         return result
 
     def prodall(self):
-        return self._scalar("prodall")
+        return self._calls["prodall"](self.a)
 
     def meanall(self):
-        return self._scalar("meanall")
+        return self._calls["meanall"](self.a)
 
     def normall(self, p):
-        return self._scalar("normall", self._real(p))
+        return self._calls["normall"](self.a, p)
 
     def _real_out(self, r):
         if self.kind == "half":
@@ -557,10 +611,10 @@ class Tensor(object):
         return r
 
     def minall(self):
-        return self._real_out(self._scalar("minall"))
+        return self._real_out(self._calls["minall"](self.a))
 
     def maxall(self):
-        return self._real_out(self._scalar("maxall"))
+        return self._real_out(self._calls["maxall"](self.a))
 
 
 def cached_memory():

@@ -10,12 +10,14 @@ and are left on.
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libTHC.so")
+BINDING = os.path.join(HERE, "_fastcall.so")
 SOURCES = ["general.cpp", "tensor.cpp", "math.cpp", "math_wide.cpp", "caching_allocator.cpp", "apply.hip", "apply_f32_0.hip", "apply_f32_1.hip",
            "apply_f32_2.hip", "apply_f16_0.hip", "apply_f16_1.hip", "apply_f16_2.hip", "apply_raw.hip",
            "reduce.hip", "reduce_f32.hip", "reduce_f16.hip", "reduce_w_u8.hip", "reduce_w_i8.hip",
@@ -81,8 +83,21 @@ def _compile(src, force):
     return obj
 
 
+def _build_binding(force):
+    """The Python binding's calls (csrc/fastcall.cpp): host code, against the running interpreter's headers."""
+    src = os.path.join(CSRC, "fastcall.cpp")
+    if not force and not _stale(BINDING, [src]):
+        return
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-Wno-invalid-offsetof", "-I" + sysconfig.get_paths()["include"], src, "-o", BINDING]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("the binding does not build:\n" + res.stderr)
+
+
 def build(force=False, verbose=True):
     os.makedirs(BUILD, exist_ok=True)
+    _build_binding(force)
     with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
         objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
     if force or _stale(LIB, objs):

@@ -82,3 +82,51 @@ def test_a_thread_that_ends_without_reading_its_error_is_not_counted_on():
     while thc._pending.value != before and time.time() < deadline:
         time.sleep(0.01)
     assert thc._pending.value == before
+
+
+def test_fast_calls_round_halves_as_numpy_does():
+    """Scalars of half tensors: the nearest half of a double, ties to even, subnormals, overflow, signed zeros, NaN."""
+    from cutorch_amd import _fastcall
+    halves = np.arange(0x7c00, dtype=np.uint16).view(np.float16).astype(np.float64)
+    mid = (halves[:-1] + halves[1:]) / 2
+    rng = np.random.default_rng(3)
+    values = np.concatenate([halves, mid, np.nextafter(mid, 1e9), np.nextafter(mid, -1e9), [65519.9, 65520.0, 65536.0, 1e300, np.inf, 0.0],
+                             np.exp(rng.uniform(-25, 13, 20000))])
+    with np.errstate(over="ignore"):
+        for sign in (1, -1):
+            want = (sign * values).astype(np.float16).view(np.uint16)
+            got = np.array([_fastcall.half_bits(float(v)) for v in sign * values], dtype=np.uint16)
+            assert np.array_equal(got, want)
+        assert np.isnan(np.array(_fastcall.half_bits(float("nan")), dtype=np.uint16).view(np.float16))
+    assert _fastcall.half_bits(3) == np.float16(3).view(np.uint16)
+    with pytest.raises(TypeError):
+        _fastcall.half_bits("3")
+
+
+def test_every_method_has_a_fast_call():
+    """The signatures of all entry points behind the Tensor methods are served, and what ctypes refuses is refused."""
+    import ctypes
+    from cutorch_amd import _fastcall
+    lib = thc.lib()
+    names = ("copy fill zero add sub mul div cadd csub cmul cdiv addcmul addcdiv exp abs clamp pow tpow cmaxValue fmod cpow cmax lerp "
+             "copyCudaFloat copyCudaHalf ltValue ltValueT ltTensor ltTensorT equal sum prod mean norm cumsum cumprod renorm var std varall "
+             "dist max min sumall prodall meanall normall maxall minall").split()
+    served = 0
+    for kind, (T, _, _, _) in thc._TYPES.items():
+        for name in names:
+            if not hasattr(lib, T + "_" + name):
+                continue
+            f = getattr(lib, T + "_" + name)
+            if not f.argtypes:
+                continue
+            signature = "".join(thc._CODES.get(t, "?") for t in [f.restype] + list(f.argtypes[1:]))
+            call = _fastcall.bind(ctypes.cast(f, ctypes.c_void_p).value, signature, 0)
+            assert call is not None, (T, name, signature)
+            served += 1
+            with pytest.raises(TypeError):
+                call(*[1] * len(f.argtypes))                  # one too many
+            if "l" in signature[2:]:
+                with pytest.raises(TypeError):
+                    call(*[1.5] * (len(f.argtypes) - 1))      # a float for a whole number (the call itself is not reached)
+    assert served > 200
+    assert _fastcall.bind(0, "vzz", 0) is None
