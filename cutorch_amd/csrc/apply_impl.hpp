@@ -129,6 +129,21 @@ __device__ __forceinline__ float math1(int fn, float x, float v, float w) {
   }
 }
 
+// The same on an element of type T. exp and the sigmoid of a half come from the hardware's 2^x and 1/x, without the range
+// reduction and scaling that expf and the division take for all of float's 24 bits: after the rounding to half the results are
+// those of the float functions for every one of the 65536 inputs (a test compares them all). What it is for: exp of
+// 8191 x 8193 transposed halves 74.1 -> 69.5 us, and, with operands that stay in the memory-side cache, 73 -> 52.
+template <typename T>
+__device__ __forceinline__ T math1_of(int fn, T a, float v, float w) {
+  const float x = Cvt<T>::up(a);
+  if constexpr (std::is_same<T, __half>::value) {
+    constexpr float kLog2e = 1.44269504088896340736f;
+    if (fn == (int)MathFn::Exp) return Cvt<T>::down(__builtin_amdgcn_exp2f(x * kLog2e));
+    if (fn == (int)MathFn::Sigmoid) return Cvt<T>::down(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -kLog2e)));
+  }
+  return Cvt<T>::down(math1(fn, x, v, w));
+}
+
 __device__ __forceinline__ float math2(int fn, float a, float b) {
   switch (fn) {
     case (int)MathFn::CPow: return powf(a, b);
@@ -179,7 +194,7 @@ struct OpMath1Fixed {
   float v, w;
   template <typename T>
   __device__ __forceinline__ T operator()(T a, T, T) const {
-    return Cvt<T>::down(math1(FN, Cvt<T>::up(a), v, w));
+    return math1_of<T>(FN, a, v, w);
   }
 };
 struct OpMath1 {
@@ -189,7 +204,7 @@ struct OpMath1 {
   int fn;
   template <typename T>
   __device__ __forceinline__ T operator()(T a, T, T) const {
-    return Cvt<T>::down(math1(fn, Cvt<T>::up(a), v, w));
+    return math1_of<T>(fn, a, v, w);
   }
   template <typename Body>
   __device__ __forceinline__ void dispatch(Body&& body) const {

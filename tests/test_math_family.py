@@ -238,3 +238,21 @@ def test_gpu_equal_is_one_fused_reduction_on_dense_operands(thc, kind):
     assert not a.equal(thc.Tensor.from_numpy(m.reshape(30, 40)))       # shape mismatch
     assert a.t().equal(thc.Tensor.from_numpy(np.ascontiguousarray(m.T)))   # strided operand: two passes
     assert not a.t().equal(thc.Tensor.from_numpy(np.ascontiguousarray(m.T) + dt(1)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", ["exp", "sigmoid"])
+def test_gpu_half_functions_match_the_float_ones_on_every_half(thc, fn):
+    """exp and the sigmoid of a half come from the hardware's 2^x and 1/x: for all 65536 inputs the bits of the float function's
+    result rounded to half (NaNs stay NaNs), flat and through a transposed odd view."""
+    x = np.arange(65536, dtype=np.uint16).view(np.float16)
+    h = thc.Tensor.from_numpy(x)
+    f = thc.Tensor("float").resize((65536,)).copy_from(h)
+    want = thc.Tensor("half").resize((65536,)).copy_from(thc.Tensor("float").unary(fn, f)).numpy()
+    got = thc.Tensor("half").unary(fn, h).numpy()
+    y = x[:255 * 257].reshape(257, 255)
+    odd = thc.Tensor("half").unary(fn, thc.Tensor.from_numpy(y).t()).numpy()
+    for g, w in ((got, want), (odd, want[:255 * 257].reshape(257, 255).T)):
+        nan = np.isnan(w)
+        assert np.array_equal(np.isnan(g), nan)
+        assert np.array_equal(g.view(np.uint16)[~nan], np.ascontiguousarray(w).view(np.uint16)[~nan])
