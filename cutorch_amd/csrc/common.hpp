@@ -132,6 +132,9 @@ constexpr size_t kScratchTailBytes = 64 * 1024;
 constexpr size_t kScratchCounters = (kScratchTailBytes - 256) / sizeof(unsigned);
 constexpr size_t kScanTicket = 2048;  // counters kScanTicket and the one behind it: a 64-bit word that deals out the chunks of one-read scans
 constexpr size_t kScanWords = size_t(2) << 20;  // 16 MiB of words behind the tail, which only one-read scans write
+// Whole-tensor reductions: the partials that workgroups hand to the one that folds them, 32 KiB of words in the tail, and the
+// count of such launches on the stream.
+constexpr size_t kFoldWordsAt = 16 * 1024, kFoldWords = 4096, kFoldCount = kScanTicket + 2;   // (bytes into the tail; words; counter)
 struct StreamScratch {
   void* partials;
   size_t partialBytes;
@@ -142,6 +145,8 @@ struct StreamScratch {
   uint64_t* scanWord;   // what the workgroups of a one-read scan tell each other (zero at first, tagged values after that)
   size_t scanWords;     // how many
   uint64_t* scanTicket;
+  uint64_t* foldWord;   // as scanWord, for whole-tensor reductions
+  uint64_t* foldCount;
 };
 const StreamScratch& stream_scratch(THCState* state);
 void* scratch_space(THCState* state, size_t* bytes);

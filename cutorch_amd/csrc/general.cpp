@@ -138,6 +138,10 @@ const StreamScratch& stream_scratch(THCState* s) {
   sc.result = reinterpret_cast<float*>(static_cast<char*>(p) + s->scratchBytes - 256);
   sc.scanWord = reinterpret_cast<uint64_t*>(static_cast<char*>(p) + s->scratchBytes);
   sc.scanWords = kScanWords;
+  static_assert(kFoldWordsAt + kFoldWords * sizeof(uint64_t) <= kScratchTailBytes - 256 && (kFoldCount + 2) * sizeof(unsigned) <= kFoldWordsAt,
+                "the tail's parts lie behind each other");
+  sc.foldWord = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(sc.counters) + kFoldWordsAt);
+  sc.foldCount = reinterpret_cast<uint64_t*>(sc.counters + kFoldCount);
   sc.scanTicket = reinterpret_cast<uint64_t*>(sc.counters + kScanTicket);
   // Arrival counters start at zero and every kernel that uses one resets it; the words of one-read scans lie behind them.
   THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
