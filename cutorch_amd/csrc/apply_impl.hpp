@@ -980,10 +980,10 @@ constexpr int kRaggedLineBytes = 128;
 template <typename T, typename Op, typename I, int MASK, bool FUSED>
 __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, const T* in0, const T* in1,
                                                                     const T* in2, TiledArgs<I> args, Op op) {
-  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4- or 8-byte elements");
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8 || (sizeof(T) == 2 && FUSED), "4- or 8-byte elements, 2-byte ones in fused columns");
   constexpr int NOPS = Op::NIN + 1;
-  constexpr int VEC = 16 / sizeof(T), LXP = 16, LXQ = 32;
-  constexpr int TP = LXP * VEC, TQ = LXQ * VEC;  // 64 x 128 (32 x 64 for 8-byte elements)
+  constexpr int VEC = 16 / sizeof(T), LXP = sizeof(T) == 2 ? 8 : 16, LXQ = 32;
+  constexpr int TP = LXP * VEC, TQ = LXQ * VEC;  // 64 x 128 (32 x 64 for 8-byte elements, 64 x 256 for 2-byte ones)
   constexpr int LINE = kRaggedLineBytes / sizeof(T);  // elements between two cut points of a row
   constexpr int SPAN = TQ + LINE - 1;            // columns a tile may touch
   constexpr int ROWS_P = kBlock / LXP, PASSES_P = (SPAN + ROWS_P - 1) / ROWS_P;
@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
           const int have = FULL ? VEC : pn - (int)(lxp * VEC);
           if (row && have >= VEC) {
             const T* at = origin + column(cq, q);
-            v[r] = args.ntLoad ? load_loose_pack<true, P>(at) : load_loose_pack<false, P>(at);
+            v[r] = args.ntLoad ? load_pack_unaligned<true, P>(at) : load_pack_unaligned<false, P>(at);
           } else if (row) {
 #pragma unroll
             for (int e = 0; e < VEC; ++e)
@@ -1419,6 +1419,21 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
     // x:t() * y:t() on 8191 x 8193 then ran at 0.47-0.51 of peak against 0.57 with the shifted windows)
     ragged = shift && ldsR <= 48 * 1024 && nstaged <= 2 && tuning("apply.tiled.ragged", 1);
   }
+  // 2-byte elements: the same tiles where the columns of several dims fuse (below) and the shifted windows of q alone, 248
+  // columns wide, would stay emptier than 70 %. us a copy with
+  // the windows and with these: 393 x 392 x 47 26.7 and 11.3, 366 x 677 x 269 137.5 and 65.3, 116 x 540 x 60 14.4 and 7.0,
+  // 1001 x 1003 x 129 214 and 159; few tiles gain nothing (429 x 15 x 79 7.6 and 8.1): 2^17 elements at least.
+  if constexpr (kSameType && sizeof(T) == 2 && Op::NIN <= 2) {
+    const int d = q - 1;
+    const int64_t Q = pl.lay[0].size[q], wide = tqV - VEC;
+    if (shift && nstaged == 1 && d >= 0 && d != p && pl.numel >= tuning("apply.tiled.fuse_half_min", 1 << 17) &&
+        tuning("apply.tiled.ragged", 1) && tuning("apply.tiled.fuse_q", 1)) {
+      ldsR = (size_t)(tqV + kRaggedSlack) * (tpV + 1) * sizeof(T);
+      ragged = Q * pl.lay[0].size[d] < kIndex32Limit && Q * 100 < (Q + wide - 1) / wide * wide * 70;
+      for (int k = 0; k < pl.nops && ragged; ++k)
+        if (!staged[k]) ragged = pl.lay[k].stride[d] == Q;
+    }
+  }
   if (!vec && !shift && ldsS > 64 * 1024) return false;
   const int64_t tileP = vec || ragged ? tpV : (shift ? tpV - VEC : tS);
   const int64_t tileQ = vec || ragged ? tqV : (shift ? tqV - VEC : tS);
@@ -1451,7 +1466,7 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   };
   const int64_t fuseKnob = tuning("apply.tiled.fuse_q", 1);   // 2: wherever the layout allows it
   bool fuse = (vec || ragged) && fuseKnob != 0;
-  if (fuse && ragged && fuseKnob == 1 && pl.lay[0].size[p] > tpV && pl.lay[0].size[p] <= 2 * tpV) {
+  if (fuse && ragged && sizeof(T) > 2 && fuseKnob == 1 && pl.lay[0].size[p] > tpV && pl.lay[0].size[p] <= 2 * tpV) {
     int64_t run = sizeQ;
     for (int d = q - 1, n = 1; d >= 0 && d != p && n < kMaxFuse && continues(d, run); --d, ++n) run *= pl.lay[0].size[d];
     const int64_t columns = (sizeQ + kRaggedSlack + tqV - 1) / tqV * tqV;   // of a row's tiles, unfused
@@ -1546,6 +1561,11 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
                              dim3(kBlock), ldsR, st, out, i0, i1, i2, args, op);                  \
         else if (ragged)                                                                          \
           hipLaunchKernelGGL((apply_tiled_ragged_kernel<T, Op, I, MM, false>), dim3(grid),        \
+                             dim3(kBlock), ldsR, st, out, i0, i1, i2, args, op);                  \
+      }                                                                                           \
+      if constexpr (kSameType && sizeof(T) == 2 && Op::NIN <= 2 && (MM & (MM - 1)) == 0) {        \
+        if (ragged)                                                                               \
+          hipLaunchKernelGGL((apply_tiled_ragged_kernel<T, Op, I, MM, true>), dim3(grid),         \
                              dim3(kBlock), ldsR, st, out, i0, i1, i2, args, op);                  \
       }                                                                                           \
       if constexpr (kSameType) {                                                                  \

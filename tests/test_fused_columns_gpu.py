@@ -105,3 +105,26 @@ def test_a_gap_behind_the_rows_keeps_the_dims_apart(thc):
     want = c.reshape(x, y, z + 2).copy()
     want[:, :, :z] = a.reshape(z, y, x).transpose(2, 1, 0) + b.reshape(x, y, z)
     assert_bit_equal(tc.storage_numpy(), want.reshape(-1))
+
+
+@pytest.mark.parametrize("forced64", [False, True])
+def test_halves_fuse_their_columns_where_one_dim_leaves_tiles_empty(thc, forced64):
+    """Halves take the line-cut tiles (64 x 256, whose columns start up to 63 early) over fused columns only: sizes around those
+    extents, one staged operand in either place and copies, offsets off the grid, and larger tensors without the knob."""
+    thc.force_64bit_index(forced64)
+    thc.set_tuning("apply.tiled.fuse_half_min", 0)
+    try:
+        for seed, sizes in enumerate(((65, 3, 43), (63, 129, 9), (9, 7, 8), (127, 5, 51), (33, 65, 17), (130, 31, 11), (16, 257, 101))):
+            for off in (0, 1, 3):
+                for a_order, b_order in (((2, 1, 0), (0, 1, 2)), ((0, 1, 2), (2, 1, 0))):
+                    _check(thc, "half", np.float16, sizes, a_order, b_order, off, "tiled-ragged-fused", seed)
+    finally:
+        thc.set_tuning("apply.tiled.fuse_half_min", 1 << 17)
+        thc.force_64bit_index(False)
+    _check(thc, "half", np.float16, (301, 67, 47), (2, 1, 0), (0, 1, 2), 1, "tiled-ragged-fused", 77)
+    _check(thc, "half", np.float16, (301, 17, 241), (2, 1, 0), (0, 1, 2), 1, "tiled-shift", 78)      # (rows that fill their tiles)
+    x = np.random.default_rng(5).integers(0, 9, 201 * 33 * 47).astype(np.float16)
+    src = thc.Tensor.from_numpy(x).view_as_strided(0, (201, 33, 47), (1, 201, 201 * 33))
+    got = thc.Tensor("half").resize((201, 33, 47)).copy(src)
+    assert thc.last_kernel() == "tiled-ragged-fused"
+    assert_bit_equal(got.numpy(), np.ascontiguousarray(x.reshape(47, 33, 201).transpose(2, 1, 0)))
