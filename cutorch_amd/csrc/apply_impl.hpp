@@ -544,7 +544,6 @@ struct TiledArgs {
   // share cache lines run back to back; 1 = q fastest throughout.
   uint32_t groupP;
   uint32_t ntStore;  // shifted-window variant: whole packs of the output go out with the streaming hint
-  uint32_t ntLoad;   // shifted-window variant: inputs are read with the streaming hint
 };
 
 // A tile spans TP = LXP*VEC elements of dim p and TQ = LXQ*VEC of dim q.
@@ -821,18 +820,6 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
       slot[k] = staged[k] ? s++ : -1;
     }
   }
-  uint32_t vo[kMaxOps];     // lane's row offset (elements) inside a tile
-  size_t rowStep[kMaxOps];  // uniform distance between two passes
-#pragma unroll
-  for (int k = 0; k < NOPS; ++k) {
-    if (staged[k]) {
-      vo[k] = lyp * (uint32_t)args.strideQ[k];
-      rowStep[k] = (size_t)ROWS_P * (size_t)args.strideQ[k];
-    } else {
-      vo[k] = lyq * (uint32_t)args.strideP[k];
-      rowStep[k] = (size_t)ROWS_Q * (size_t)args.strideP[k];
-    }
-  }
 
   const uint32_t slots = args.xcdPer ? args.xcdPer * 8 : args.totalTiles;
   for (uint32_t b = blockIdx.x; b < slots; b += gridDim.x) {
@@ -876,17 +863,17 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
       int first[PASSES_P];  // tile coordinate (along p) of the pack's element 0
 #pragma unroll
       for (int r = 0; r < PASSES_P; ++r) {
-        const int qi = (int)lyp + r * ROWS_P;
-        const T* row = tbase[k] + r * rowStep[k] + vo[k];
-        first[r] = (int)(lxp * VEC) - misalignment(row);
-        if (qi < qn && first[r] < pn)
-          v[r] = args.ntLoad ? load_pack<true>(reinterpret_cast<const P*>(row + first[r]))
-                             : load_pack<false>(reinterpret_cast<const P*>(row + first[r]));
+        // (no load carries a predicate: lanes past the tile's edges re-read its last row, their row's last pack)
+        const int qi = min((int)lyp + r * ROWS_P, qn - 1);
+        const T* row = tbase[k] + (size_t)qi * (size_t)args.strideQ[k];
+        const int m = misalignment(row);
+        first[r] = min((int)lxp, (pn - 1 + m) / VEC) * VEC - m;
+        v[r] = load_pack<true>(reinterpret_cast<const P*>(row + first[r]));
       }
 #pragma unroll
       for (int r = 0; r < PASSES_P; ++r) {
         const int qi = (int)lyp + r * ROWS_P;
-        if (qi < qn && first[r] < pn) {
+        if (qi < qn) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
             const int pi = first[r] + e;
@@ -900,22 +887,16 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
     // phase 2: compute with lanes along q
     P din[3][PASSES_Q];
     int first[PASSES_Q];  // tile coordinate (along q) of the pack's element 0
+    // row pi of operand k, the last one for lanes past the tile's edge
+    auto row_of = [&](int k, int r) { return tbase[k] + (size_t)min((int)lyq + r * ROWS_Q, pn - 1) * (size_t)args.strideP[k]; };
 #pragma unroll
     for (int r = 0; r < PASSES_Q; ++r) {
-      const int pi = (int)lyq + r * ROWS_Q;
-      first[r] = (int)(lxq * VEC) - misalignment(tbase[0] + r * rowStep[0] + vo[0]);
-      if (!(pi < pn && first[r] < qn)) first[r] = qn;  // marks an idle pass
-    }
+      const int pi = (int)lyq + r * ROWS_Q, m = misalignment(row_of(0, r)), last = (qn - 1 + m) / VEC;
+      first[r] = min((int)lxq, last) * VEC - m;
 #pragma unroll
-    for (int k = 1; k < NOPS; ++k) {
-      if (staged[k]) continue;
-#pragma unroll
-      for (int r = 0; r < PASSES_Q; ++r) {
-        if (first[r] < qn) {
-          const P* src = reinterpret_cast<const P*>(tbase[k] + r * rowStep[k] + vo[k] + first[r]);
-          din[k - 1][r] = args.ntLoad ? load_pack<true>(src) : load_pack<false>(src);
-        }
-      }
+      for (int k = 1; k < NOPS; ++k)
+        if (!staged[k]) din[k - 1][r] = load_pack<true>(reinterpret_cast<const P*>(row_of(k, r) + first[r]));
+      if (pi >= pn || (int)lxq > last) first[r] = qn;  // marks an idle pass
     }
 #pragma unroll
     for (int r = 0; r < PASSES_Q; ++r) {
@@ -938,7 +919,7 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_shift_kernel(T* out, const
         P res;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) res.v[e] = op(in[0].v[e], in[1].v[e], in[2].v[e]);
-        T* orow = const_cast<T*>(tbase[0]) + r * rowStep[0] + vo[0];
+        T* orow = const_cast<T*>(row_of(0, r));
         if (first[r] >= 0 && first[r] + VEC <= qn) {
           if (args.ntStore) store_pack<true>(reinterpret_cast<P*>(orow + first[r]), res);
           else store_pack<false>(reinterpret_cast<P*>(orow + first[r]), res);
@@ -1058,7 +1039,13 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
       for (int k = 1; k < NOPS; ++k) {
         if (!staged[k]) continue;
         T* slab = lds + slot[k] * (SPAN * PITCH);
-        const T* origin = ptr[k] + (base[k] + (I)p0 * args.strideP[k]) + lxp * VEC;  // unit stride along p
+        // (no load carries a predicate, which would put it into a branch and its memory latency into a chain with the others:
+        // us of x + y:t() on floats with predicates and without: 208 x 21 8.1 and 5.6, 1001 x 1003 8.7 and 5.9, 4097 x 1025 17.9
+        // and 11.4, 301 x 20001 21.4 and 17.4, 8191 x 8193 153.5 and 145.2; of permuted 751 x 189 x 266 116 and 84, 301 x 301 x
+        // 301 59 and 52. Columns outside the tensor re-read its nearest one, and the packs behind the tile's last row piece are
+        // moved back to end with it)
+        const int po = FULL ? (int)(lxp * VEC) : min((int)(lxp * VEC), pn - VEC);
+        const T* origin = ptr[k] + (base[k] + (I)p0 * args.strideP[k]) + po;  // unit stride along p
         P v[PASSES_P];
         auto column = [&](int cq, int q) -> I {
           if constexpr (FUSED) return columnOff[slot[k] & 1][cq];
@@ -1066,24 +1053,17 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
         };
 #pragma unroll
         for (int r = 0; r < PASSES_P; ++r) {
-          const int cq = (int)lyp + r * ROWS_P, q = qL + cq;
-          const bool row = cq < SPAN && (FULL || (q >= 0 && q < sizeQ));
-          const int have = FULL ? VEC : pn - (int)(lxp * VEC);
-          if (row && have >= VEC) {
-            const T* at = origin + column(cq, q);
-            v[r] = args.ntLoad ? load_pack_unaligned<true, P>(at) : load_pack_unaligned<false, P>(at);
-          } else if (row) {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-              if (e < have) v[r].v[e] = origin[column(cq, q) + e];
-          }
+          const int cq = min((int)lyp + r * ROWS_P, SPAN - 1);
+          const int q = FULL ? qL + cq : min(max(qL + cq, 0), sizeQ - 1);
+          v[r] = load_pack_unaligned<false, P>(origin + column(cq, q));
         }
 #pragma unroll
         for (int r = 0; r < PASSES_P; ++r) {
           const int cq = (int)lyp + r * ROWS_P;
           if (cq < SPAN) {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) slab[cq * PITCH + lxp * VEC + e] = v[r].v[e];
+            for (int e = 0; e < VEC; ++e)
+              if (FULL || po + e >= 0) slab[cq * PITCH + po + e] = v[r].v[e];
           }
         }
       }
@@ -1108,15 +1088,11 @@ __global__ __launch_bounds__(kBlock) void apply_tiled_ragged_kernel(T* out, cons
         if (staged[k]) continue;
 #pragma unroll
         for (int r = 0; r < PASSES_Q; ++r) {
-          const int pi = (int)lyq + r * ROWS_Q;
+          // (a pack at a row's end is loaded whole: it holds at least one element of the row; lanes without one read the row's first)
+          const int pi = FULL ? (int)lyq + r * ROWS_Q : min((int)lyq + r * ROWS_Q, pn - 1);
           const T* row = ptr[k] + (base[k] + (I)(p0 + pi) * args.strideP[k]);
-          if (whole[r]) {
-            din[k - 1][r] = load_pack<true>(reinterpret_cast<const P*>(row + q1[r]));
-          } else if (any[r]) {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e)
-              if (q1[r] + e >= 0 && q1[r] + e < sizeQ) din[k - 1][r].v[e] = row[q1[r] + e];
-          }
+          const int at = any[r] ? q1[r] : -(int)((reinterpret_cast<uintptr_t>(row) / sizeof(T)) & (uintptr_t)(VEC - 1));
+          din[k - 1][r] = load_pack<true>(reinterpret_cast<const P*>(row + at));
         }
       }
 #pragma unroll
@@ -1510,7 +1486,6 @@ bool launch_tiled(THCState* s, const Plan& pl, Op op, bool vecOnly = false) {
   const bool nts = ntKnob >= 0 ? ntKnob != 0
                                : (outSpan >= (int64_t(32) << 20) || pl.numel * (int64_t)sizeof(TOut) >= (int64_t(64) << 20));
   args.ntStore = nts ? 1u : 0u;
-  args.ntLoad = tuning("apply.tiled.shift_nt_load", 1) ? 1u : 0u;
   bool lineAligned = true;  // every row of every operand starts on a 128-byte line
   for (int k = 0; k < pl.nops; ++k) {
     lineAligned = lineAligned && reinterpret_cast<uintptr_t>(pl.ptr[k]) % 128 == 0;
