@@ -1326,9 +1326,9 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // with a wave and 4.0, 2500 of 1024 4.8 and 5.9, of 3000 12.9 and 13.9), 1 for bytes (2048: 1000 rows 4.5 and 4.8),
   // 16 for 8-byte elements (2500 x 1024 9.4 and 7.3); never below 1024 elements or up to 4 KiB (1000 x 1024 fp32 3.9 and 3.6, 2500 4.8 and 5.9); 1-byte elements below 8192: 4 (4000 x 4096 9.8 and 21, 1000 x 6144
   // 9.0 and 8.1). Other rows go through a wave element by element, and the chunks win further: 16000 fp32
-  // rows of 2051 59.5 and 40.4, 30000 half rows of 1025 58.4 and 52.8, 16000 doubles of 513 36.2 and 28.9; except fp32
-  // below 2048 (3000 x 1025 9.4 and 7.4, 6000 15.5 and 17.3) and bytes below 8192 (2500 x 2049 16.2 and 15.1, 6000 24.3 and
-  // 33.5).
+  // rows of 2051 59.5 and 40.4, 30000 half rows of 1025 58.4 and 52.8, 16000 doubles of 1025 58.7 and 40.4; except below 1024
+  // elements (19798 x 491 doubles 34.2 and 38.4), fp32 below 2048 (3000 x 1025 9.4 and 7.4, 6000 15.5 and 17.3) and bytes
+  // below 8192 (2500 x 2049 16.2 and 15.1, 6000 24.3 and 33.5).
   // Products of floating elements keep the two reads of scan_rows_kernel's pieces below: the product of a chunk
   // that overflows turns a zero before it into NaN, and these chunks are longer than those pieces.
   constexpr bool kFloatProduct =
@@ -1349,7 +1349,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
     int64_t most_rows = 16 * cus;
     if (!whole) {
       if (sizeof(T) == 1 && R < 8192) most_rows = 8 * cus;
-      else if (sizeof(T) == 4 && R < 2048) most_rows = 12 * cus;
+      else if ((sizeof(T) == 4 && R < 2048) || R < 1024) most_rows = 12 * cus;
       else most_rows = std::numeric_limits<int64_t>::max();
     } else if (R < 1024 || (R < 4096 && R * (int64_t)sizeof(T) <= 4096)) {
       most_rows = 0;
