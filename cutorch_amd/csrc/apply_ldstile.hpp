@@ -471,11 +471,17 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
     if (!tuning("apply.ldstile.enable", 1) || !tile_plan(pl, p, q, staged)) return false;
     constexpr int W = sizeof(T) > sizeof(TOut) ? sizeof(T) : sizeof(TOut);
     constexpr int VEC = 16 / W;
-    // 512-byte rows (of the wider type) along q (256 on unaligned rows with one input of narrow elements, LXQU below);
-    // along p 128 bytes of the input type at least (64 bytes for 1-byte elements, whose 128 x 512 tile would take 66 KiB
-    // of LDS per input)
+    // The base shape: 512-byte rows (of the wider type) along q; along p 128 bytes of the input type at least (64 bytes for
+    // 1-byte elements, whose 128 x 512 tile would take 66 KiB of LDS per input). Smaller tiles where input and output are of
+    // one width and they measured better (us of a transposed operand, base shape first): bytes, cmax 8192 x 8192 74 and 53, 352 x 256 8.9 and 5.7, char abs
+    // 55 and 26, 6.6 and 4.8; halves, cmax 75.8 and 73.4, 5.7 and 4.4, exp 50.2 and 45.3, 6.5 and 4.3; one 4-byte input, int abs
+    // 95.6 and 89.1, 4.6 and 3.7. (cmax of two 4-byte inputs 8192 x 8192 154 and, 16 packs along q, 177: as it was.)
+    constexpr bool kOneWidth = sizeof(T) == sizeof(TOut);
     constexpr int LXQ = 32;
     constexpr int LXP = (sizeof(T) == 1 && VEC == 16) ? 4 : ((128 / (int)sizeof(T)) / VEC < 8 ? 8 : (128 / (int)sizeof(T)) / VEC);
+    constexpr bool kWords = kOneWidth && W == 4 && Op::NIN == 1;
+    constexpr int LXPA = kOneWidth && W == 1 ? 8 : kWords ? 16 : LXP;
+    constexpr int LXQA = kOneWidth && W == 1 ? 8 : (kOneWidth && W == 2) || kWords ? 16 : LXQ;
     const int nd = pl.lay[0].dims;
     if (nd - 2 > kLdsTileBatchDims) return false;
     auto elem_size = [](int k) { return k == 0 ? sizeof(TOut) : sizeof(T); };
@@ -517,15 +523,22 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
       ++args.nbatch;
       batch *= pl.lay[0].size[d];
     }
-    using SA = LdsTileShape<T, TOut, LXP, LXQ, true>;
-    // Unaligned rows of narrow elements with one input: half as wide along q. Twice the tiles fill the chip where there are few
-    // and hide the compute phases of each other (full and half width: int8 abs on a transposed 349 x 255 8.7 and 6.2 us, 127 x 8193
-    // 8.1 and 6.1, 20001 x 301 10.5 and 8.9, 8191 x 8193 33.6 and 32.6; int16 abs 5.8 and 4.5, 6.2 and 5.1, 9.1 and 7.8, 50.7 and
-    // 50.8; half exp 7.7 and 5.6, 8.0 and 5.8, 13.5 and 11.9, 71.6 and 65.9). With a second input, whose row pieces would halve
-    // as well, it loses (half cmax on 8191 x 8193 112 -> 124 us).
-    constexpr int LXQU = Op::NIN == 1 && VEC >= 8 ? 16 : LXQ;
-    using SU = LdsTileShape<T, TOut, LXP, LXQU, false>;
-    const int64_t tileP = aligned ? SA::TP : SU::TP, tileQ = aligned ? SA::TQ : SU::TQ;
+    using SA = LdsTileShape<T, TOut, LXPA, LXQA, true>;
+    // Unaligned rows of narrow elements: a half or a quarter as wide along q. More tiles fill the chip where there are few
+    // and hide the compute phases of each other (int16 abs on a transposed 349 x 255 5.8 and 4.5 us, 127 x 8193 6.2 and 5.1,
+    // 20001 x 301 9.1 and 7.8, 8191 x 8193 50.7 and 50.8; half exp 7.7 and 5.6, 8.0 and 5.8, 13.5 and 11.9, 71.6 and 65.9;
+    // byte cmax 349 x 255 10.1 and 5.2, 3001 x 2999 15.1 and 11.4). On large tensors bytes with one input are as well
+    // off with tiles of 256 columns (char abs 7001 x 6999 23.1, narrow 24.2), several inputs with 128 x 128 tiles (byte cmax 8191 x
+    // 8193 65 with the base shape, 61, narrow 70), and 2-byte elements with several inputs, whose row pieces would halve
+    // as well, with the base shape (half cmax 7001 x 6999 72.8, narrow 75.7; 5001 x 5003 40.4 and 38.4).
+    constexpr bool kNarrow = kOneWidth && (W == 1 || (W == 2 && Op::NIN > 1));
+    constexpr int LXPU = kOneWidth && W == 1 && Op::NIN > 1 ? 8 : LXP;
+    constexpr int LXQU = kOneWidth && W == 1 && Op::NIN > 1 ? 8 : Op::NIN == 1 && VEC >= 8 ? 16 : LXQ;
+    constexpr int LXPN = kNarrow ? (W == 1 ? 4 : 8) : LXPU, LXQN = kNarrow ? (W == 1 ? 8 : 16) : LXQU;
+    const bool narrow = kNarrow && pl.numel < tuning("apply.ldstile.narrow_max", 32 << 20);
+    using SU = LdsTileShape<T, TOut, LXPU, LXQU, false>;
+    using SN = LdsTileShape<T, TOut, LXPN, LXQN, false>;
+    const int64_t tileP = aligned ? SA::TP : narrow ? SN::TP : SU::TP, tileQ = aligned ? SA::TQ : narrow ? SN::TQ : SU::TQ;
     // (an unaligned row's first run starts up to VEC - 1 columns before the row does)
     const int64_t tp = (args.sizeP + tileP - 1) / tileP, tq = (args.sizeQ + (aligned ? 0 : VEC - 1) + tileQ - 1) / tileQ;
     args.tilesP.set((uint64_t)tp);
@@ -543,7 +556,7 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
     if ((int64_t)args.groupP * 2 > tp) args.groupP = 1;
     if (!aligned && tuning("apply.ldstile.xcd_swizzle", 1) && total >= 64 && total < (int64_t(1) << 28))
       args.xcdPer = (uint32_t)((total + 7) / 8);
-    const size_t ldsBytes = aligned ? SA::lds_bytes(Op::NIN) : SU::lds_bytes(Op::NIN);
+    const size_t ldsBytes = aligned ? SA::lds_bytes(Op::NIN) : narrow ? SN::lds_bytes(Op::NIN) : SU::lds_bytes(Op::NIN);
     if (ldsBytes > 160 * 1024) return false;
     // persistent grid: as many workgroups as the LDS admits per CU (160 KiB), capped by registers at 8
     const int64_t perCu = std::max<int64_t>(1, std::min<int64_t>(tuning("apply.ldstile.max_per_cu", 8),
@@ -565,19 +578,23 @@ bool launch_ldstile(THCState* s, const Plan& pl, Op op) {
       const int64_t knob = tuning("apply.ldstile.nt_load", -1);
       ntl = knob >= 0 ? knob != 0 : !(sizeof(T) == sizeof(TOut) && sizeof(T) < 4);
     }
-    auto go = [&](auto alignedTag, auto ntlTag) {
-      constexpr bool kAl = decltype(alignedTag)::value;
-      hipLaunchKernelGGL((apply_ldstile_kernel<T, TOut, Op, LXP, kAl ? LXQ : LXQU, kAl, decltype(ntlTag)::value>),
+    auto go = [&](auto shapeTag, auto ntlTag) {   // shape: 0 aligned, 1 unaligned, 2 unaligned and narrow
+      constexpr int kS = decltype(shapeTag)::value;
+      constexpr int kP = kS == 0 ? LXPA : kS == 1 ? LXPU : LXPN, kQ = kS == 0 ? LXQA : kS == 1 ? LXQU : LXQN;
+      hipLaunchKernelGGL((apply_ldstile_kernel<T, TOut, Op, kP, kQ, kS == 0, decltype(ntlTag)::value>),
                          dim3(grid), dim3(kBlock), ldsBytes, st, o, i0, i1, i2, args, op);
     };
+    using std::integral_constant;
     if constexpr (Op::NIN == 1) {
-      if (aligned && ntl) go(std::true_type{}, std::true_type{});
-      else if (aligned) go(std::true_type{}, std::false_type{});
-      else if (ntl) go(std::false_type{}, std::true_type{});
-      else go(std::false_type{}, std::false_type{});
+      if (aligned && ntl) go(integral_constant<int, 0>{}, std::true_type{});
+      else if (aligned) go(integral_constant<int, 0>{}, std::false_type{});
+      else if (kNarrow && narrow) go(integral_constant<int, kNarrow ? 2 : 1>{}, std::false_type{});   // (ntl: the knob's alone)
+      else if (ntl) go(integral_constant<int, 1>{}, std::true_type{});
+      else go(integral_constant<int, 1>{}, std::false_type{});
     } else {
-      if (aligned) go(std::true_type{}, std::true_type{});
-      else go(std::false_type{}, std::true_type{});
+      if (aligned) go(integral_constant<int, 0>{}, std::true_type{});
+      else if (kNarrow && narrow) go(integral_constant<int, kNarrow ? 2 : 1>{}, std::true_type{});
+      else go(integral_constant<int, 1>{}, std::true_type{});
     }
     note_kernel(aligned ? "lds-tile" : "lds-tile-shift");
     return true;

@@ -401,3 +401,34 @@ def test_tiles_of_few_rows(thc, kind, p):
                 run(tc)
                 c[off:off + n] = want.astype(tdt).reshape(-1)
                 assert_bit_equal(tc.storage_numpy(), c, "%s -> %s %d x %d +%d %s" % (kind, to, p, q, off, thc.last_kernel()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("narrow_max", [0, 1 << 40])
+@pytest.mark.parametrize("kind", ["byte", "char", "short", "half"])
+def test_tile_widths_of_narrow_types_give_the_same_bits(thc, oracle, kind, narrow_max):
+    """Odd rows of 1- and 2-byte elements have a tile shape for small and one for large tensors; the knob forces either
+    onto sizes around the edges of both (tiles of 61, 64 and 125 rows, of 112, 120 and 248 columns)."""
+    rng = np.random.default_rng(310)
+    ref = oracle.pointwise if kind == "half" else oracle.typed_pointwise
+    thc.set_tuning("apply.ldstile.narrow_max", narrow_max)
+    try:
+        for shape in ((9, 8), (61, 113), (62, 112), (65, 121), (125, 249), (126, 257), (251, 225)):
+            for transposed in ((1,), (2,), (0,), (1, 2)):
+                go, ga, gb, gc = operand_geoms(rng, shape, False, transposed)
+                da, ra = pair(thc, oracle, storage_of(rng, oracle, kind, ga[0]), ga, kind)
+                db, rb = pair(thc, oracle, storage_of(rng, oracle, kind, gb[0]), gb, kind)
+                dc, rc = pair(thc, oracle, storage_of(rng, oracle, kind, gc[0], nonzero=True), gc, kind)
+                do, ro = pair(thc, oracle, storage_of(rng, oracle, kind, go[0]), go, kind)
+                do.binary("cmax", da, db)
+                assert thc.last_kernel() == "lds-tile-shift", thc.last_kernel()
+                ref("fn:cmax", ro, ra, rb)
+                assert_bit_equal(do.storage_numpy(), ro.storage, "%s cmax %s t=%s" % (kind, shape, transposed))
+                do.mul(da, 3)
+                ref("mulc", ro, ra, value=3)
+                assert_bit_equal(do.storage_numpy(), ro.storage, "%s mulc %s t=%s" % (kind, shape, transposed))
+                do.addcdiv(da, 2, db, dc)
+                ref("addcdiv", ro, ra, rb, rc, value=2)
+                assert_bit_equal(do.storage_numpy(), ro.storage, "%s addcdiv %s t=%s" % (kind, shape, transposed))
+    finally:
+        thc.set_tuning("apply.ldstile.narrow_max", 32 << 20)
