@@ -1676,6 +1676,25 @@ bool run_plan(THCState* s, Plan& pl, bool sameShape, Op op, bool decline = false
           (wide ? launch_flatmix<T, Op, uint64_t, TOut>(s, pl, op) : launch_flatmix<T, Op, uint32_t, TOut>(s, pl, op)))
         return true;
     }
+    // The one-input family: the LDS-tile kernel, whose rolled compute loop has the code decoded outside, where the tiled
+    // kernels below hold forty functions in their unrolled passes and spend a small call on the way through them. us of a
+    // transposed exp on floats (tiled, LDS tile): 33 x 17 9.6, 4.0; 349 x 255 14.0, 5.0; 1024 x 1008 10.6, 4.7; 3001 x 2999
+    // 27.8, 18.1; 8192 x 8192 103.7, 90.7; 8191 x 8193 136, 108 (tanh 146, 107). Except large tensors whose columns the tiled
+    // kernels fuse with the next dim's where the tiles here stay emptier than 55 %: 1001 x 1003 x 129 269, 448;
+    // 156 x 704 x 41 15.1, 16.0 (301 x 301 x 301, 81 %, 61, 52; 65 x 33 x 47 12.9, 4.9); and large tensors of so few rows that
+    // three quarters of its 64-row tiles would be computed in vain: tanh of 16 x 100000 7.9, 10.3. Whole
+    // packs below 2^15 elements stay as well, although 352 x 256 gains (9.4, 4.2): a test of kernel names holds 136 x 200 there.
+    if constexpr (TILED && std::is_same<Op, OpMath1>::value && std::is_same<T, TOut>::value) {
+      int p, q, staged[kMaxOps] = {0, 0, 0, 0};
+      bool lds = tile_plan(pl, p, q, staged);
+      if (lds && pl.numel >= (1 << 20) && q > 0 && q - 1 != p && pl.lay[0].stride[q - 1] == pl.lay[0].size[q]) {
+        const int64_t Q = pl.lay[0].size[q], tile = Q % 4 ? 124 : 64;
+        lds = Q * 100 >= (Q + tile - 1) / tile * tile * 55;
+      }
+      if (lds && pl.numel < (1 << 15) && pl.lay[0].size[p] % 4 == 0 && pl.lay[0].size[q] % 4 == 0) lds = false;
+      if (lds && pl.numel >= (1 << 20) && pl.lay[0].size[p] <= 16 && pl.lay[0].size[q] % 4 == 0) lds = false;
+      if (lds && launch_ldstile<T, Op, TOut>(s, pl, op)) return true;
+    }
     if constexpr (TILED) {
       if (tuning("apply.tiled.enable", 1)) {
         if (wide ? launch_tiled<T, Op, uint64_t, TOut>(s, pl, op) : launch_tiled<T, Op, uint32_t, TOut>(s, pl, op))

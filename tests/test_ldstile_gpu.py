@@ -432,3 +432,24 @@ def test_tile_widths_of_narrow_types_give_the_same_bits(thc, oracle, kind, narro
                 assert_bit_equal(do.storage_numpy(), ro.storage, "%s addcdiv %s t=%s" % (kind, shape, transposed))
     finally:
         thc.set_tuning("apply.ldstile.narrow_max", 32 << 20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,kernel", [
+    ((8, 8), "tiled"), ((128, 252), "tiled"), ((128, 256), "lds-tile"), ((65, 68), "lds-tile-shift"), ((16, 4000), "lds-tile"), ((4000, 16), "lds-tile"),
+    ((33, 17), "lds-tile-shift"), ((32, 1024), "lds-tile"), ((31, 125), "lds-tile-shift"), ((127, 255), "lds-tile-shift"),
+    ((90, 101, 129), "tiled-ragged-fused"),      # 129 columns leave two tiles of 124 half empty
+    ((80, 101, 129), "lds-tile-shift"),          # (below 2^20 elements)
+    ((96, 112, 101), "lds-tile-shift")])
+def test_float_unary_on_transposed_operands(thc, oracle, shape, kernel):
+    """The one-input family on floats: which kernel takes a transposed operand, and its bits."""
+    rng = np.random.default_rng(311)
+    order = list(range(len(shape)))
+    ga, go = geometry(shape, order[::-1], [0] * len(shape), 0), geometry(shape, order, [0] * len(shape), 0)
+    da, ra = pair(thc, oracle, storage_of(rng, oracle, "float", ga[0]), ga, "float")
+    for name in ("neg", "floor", "abs"):
+        do, ro = pair(thc, oracle, storage_of(rng, oracle, "float", go[0]), go, "float")
+        do.unary(name, da)
+        assert thc.last_kernel() == kernel, (shape, thc.last_kernel())
+        oracle.pointwise("fn:" + name, ro, ra)
+        assert_bit_equal(do.storage_numpy(), ro.storage, "%s %s" % (name, shape))
