@@ -414,15 +414,15 @@ def build_configs(thc, hip, which, only=None, stagger=0):
                 "N-sum-tall": ("sum over dim 0 of 6710886x10 fp32 (tall, 40-byte rows)", 4 * n10, n10,
                                lambda i: otall.sum(v10, 0)),
                 "N-var-tall": ("var over dim 0 of 6710886x10 fp32 (one read)", 4 * n10, n10, lambda i: otall.var(v10, 0)),
-                "N-cumsum-wide": ("cumsum over dim 0 of 65536x1000 fp32 (rows cut into parts, input read twice, "
-                                  "counted once)", 8 * 65536 * 1000, 65536 * 1000,
+                "N-cumsum-wide": ("cumsum over dim 0 of 65536x1000 fp32 (strips of columns, one read)",
+                                  8 * 65536 * 1000, 65536 * 1000,
                                   lambda i: swide.cumsum(vwide, 0)),
                 "N-cumsum-1d": ("cumsum of a 2^26-element fp32 vector (chunks of one read)",
                                 8 * nr, nr, lambda i: s1d.cumsum(flat, 0)),
                 "N-argmax-tall": ("max+argmax over dim 0 of 6710886x10 fp32", 4 * n10, n10, lambda i: omaxt.max(imaxt, v10, 0)),
                 "N-argmax-1d": ("max+argmax of a 2^26-element fp32 vector", 4 * nr, nr, lambda i: omax1.max(imax1, flat, 0)),
                 "N-cumsum-rows10": ("cumsum over last dim of 6710886x10 fp32", 8 * n10, n10, lambda i: s10.cumsum(v10, 1)),
-                "N-cumsum-tall": ("cumsum over dim 0 of 6710886x10 fp32 (input read twice, counted once)", 8 * n10, n10,
+                "N-cumsum-tall": ("cumsum over dim 0 of 6710886x10 fp32 (chunks of one read)", 8 * n10, n10,
                                   lambda i: s10.cumsum(v10, 0)),
                 "N-add-t-odd": ("c = a:t() + b, 8191x8193 fp32 (no 16-byte aligned rows)", 12 * nodd, nodd,
                                 lambda i: oddO.cadd(oddT, 1.0, oddB)),
