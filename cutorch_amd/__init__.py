@@ -13,6 +13,11 @@ import struct
 
 import numpy as np
 
+try:
+    from . import _fastcall      # csrc/fastcall.cpp, built for the running interpreter
+except ImportError:              # another interpreter, or one without headers: the same calls go through ctypes
+    _fastcall = None
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libTHC.so")
 
@@ -50,9 +55,9 @@ def lib():
         _lib = C.CDLL(LIB_PATH)
         _declare(_lib)
         _pending = C.c_long.in_dll(_lib, "THCAmd_pendingErrors")
-        from . import _fastcall
-        _fastcall.setup(C.addressof(_pending), C.cast(_lib.THCAmd_lastError, C.c_void_p).value,
-                        C.cast(_lib.THCAmd_clearLastError, C.c_void_p).value, THCError)
+        if _fastcall is not None:
+            _fastcall.setup(C.addressof(_pending), C.cast(_lib.THCAmd_lastError, C.c_void_p).value,
+                            C.cast(_lib.THCAmd_clearLastError, C.c_void_p).value, THCError)
         # Handlers that return: the failed entry point returns to us and the
         # message is picked up from THCAmd_lastError by _check().
         _err_cb = (C.CFUNCTYPE(None, C.c_char_p, C.c_void_p)(lambda m, d: None),
@@ -116,11 +121,12 @@ class _Calls(dict):
         self.prefix = _TYPES[kind][0] + "_"
 
     def __missing__(self, name):
-        from . import _fastcall
         st, f = state(), getattr(lib(), self.prefix + name)
-        signature = "".join(_CODES.get(t, "?") for t in [f.restype] + list(f.argtypes[1:]))
-        call = _fastcall.bind(C.cast(f, C.c_void_p).value, signature, st)
-        if call is None:       # a signature that the fast calls do not have
+        call = None
+        if _fastcall is not None:
+            signature = "".join(_CODES.get(t, "?") for t in [f.restype] + list(f.argtypes[1:]))
+            call = _fastcall.bind(C.cast(f, C.c_void_p).value, signature, st)
+        if call is None:       # no fast calls for this interpreter, or a signature that they do not have
             pointers = [t is C.POINTER(_Tensor) for t in f.argtypes[1:]]
             halves = [t is C.c_uint16 for t in f.argtypes[1:]]
 

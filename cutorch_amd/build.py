@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libTHC.so")
-BINDING = os.path.join(HERE, "_fastcall.so")
+BINDING = os.path.join(HERE, "_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))   # (one per interpreter: its name holds the ABI)
 SOURCES = ["general.cpp", "tensor.cpp", "math.cpp", "math_wide.cpp", "caching_allocator.cpp", "apply.hip", "apply_f32_0.hip", "apply_f32_1.hip",
            "apply_f32_2.hip", "apply_f16_0.hip", "apply_f16_1.hip", "apply_f16_2.hip", "apply_raw.hip",
            "reduce.hip", "reduce_f32.hip", "reduce_f16.hip", "reduce_w_u8.hip", "reduce_w_i8.hip",
@@ -84,8 +84,12 @@ def _compile(src, force):
 
 
 def _build_binding(force):
-    """The Python binding's calls (csrc/fastcall.cpp): host code, against the running interpreter's headers."""
+    """The Python binding's calls (csrc/fastcall.cpp): host code, against the running interpreter's headers. Without those the
+    binding calls the library through ctypes, as it does for any interpreter that this was not built for."""
     src = os.path.join(CSRC, "fastcall.cpp")
+    if not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        sys.stderr.write("no headers of this Python: the binding calls libTHC.so through ctypes\n")
+        return
     if not force and not _stale(BINDING, [src]):
         return
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",

@@ -1,7 +1,11 @@
 """The binding's host-side short cuts: half scalars and the pending-error count."""
 import ctypes as C
+import os
 import random
 import struct
+import subprocess
+import sys
+import sysconfig
 import threading
 import time
 
@@ -130,3 +134,34 @@ def test_every_method_has_a_fast_call():
                     call(*[1.5] * (len(f.argtypes) - 1))      # a float for a whole number (the call itself is not reached)
     assert served > 200
     assert _fastcall.bind(0, "vzz", 0) is None
+
+
+def test_the_binding_works_without_its_native_module():
+    """An interpreter that csrc/fastcall.cpp was not built for calls the same entry points through ctypes."""
+    code = """if True:
+        import sys
+        sys.modules["cutorch_amd._fastcall"] = None          # (an import of it raises ImportError)
+        import cutorch_amd as thc
+        thc._state = thc.lib().THCState_alloc()
+        for kind in ("float", "half", "long"):
+            t = thc.Tensor(kind)
+            assert t.fill(3) is t and t.mul(t, 2) is t and t.cmul(t, t) is t and t.compare_value("lt", t, 1, True) is t
+        f = thc.Tensor("float")
+        for bad in (lambda: f.var(f, 2), lambda: f.max(thc.Tensor("long"), f, 3)):
+            try:
+                bad()
+                raise SystemExit("no error")
+            except thc.THCError as e:
+                assert "out of range" in str(e), e
+        print("ok", thc._fastcall)
+    """
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert done.stdout.strip() == "ok None", done.stdout + done.stderr
+
+
+def test_the_native_module_is_named_for_its_interpreter():
+    """Its name holds the ABI that it was built for, so no other interpreter loads it."""
+    from cutorch_amd import build
+    assert build.BINDING.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and len(sysconfig.get_config_var("EXT_SUFFIX")) > len(".so")
+    assert thc._fastcall is None or os.path.realpath(thc._fastcall.__file__) == os.path.realpath(build.BINDING)
