@@ -1530,14 +1530,133 @@ __global__ __launch_bounds__(kBlock) void var_rows_kernel(const T* __restrict__ 
   }
 }
 
-// var / std along a unit-stride dim of rows too long for the registers (layer statistics over 4096 or
+// var / std along a unit-stride dim, a workgroup of BT threads per row: rows too few to fill the chip with waves, and rows off the
+// 16-byte grid. Two sweeps (the mean, then the squared deviations from it) in one launch: the first sweep leaves a
+// thread's first 8 packs in registers, and what a row has beyond BT * 8 packs (of at most 131072 elements in all) the second one finds
+// in the caches. Packs sit at element-aligned addresses; the elements behind the last whole pack go one to a lane.
+// A running mean in one sweep would round the mean at every element, relative to the mean and not to the deviation: relative error of
+// the variance of 15366 fp32 elements 1000 deviations away from zero 8e-7 that way, 4e-8 in two sweeps; 10000 away 1e-5 and 2e-7.
+template <typename T, typename I, int VEC, int BT>
+__global__ __launch_bounds__(BT) void var_rows_block_kernel(const T* __restrict__ in, T* __restrict__ out, OuterArgs<I> oa, I numRows,
+                                                            I R, typename Acc<T>::type div, bool wantStd) {
+  using P = Pack<T, VEC>;
+  using A = typename Acc<T>::type;
+  constexpr int U = 8, kWaves = BT / 64;
+  __shared__ A red[2][kWaves];  // (a sweep's sums are read before the next barrier, which the other sweep's lie behind)
+  const I step = (I)BT * VEC, packed = R - R % VEC, mine = (I)threadIdx.x * VEC;
+  const auto block_sum = [&](A x, A* sums) {
+    for (uint32_t o = 32; o > 0; o >>= 1) x += shfl_xor_any(x, o);
+    if constexpr (kWaves == 1) return x;
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = x;
+    __syncthreads();
+    A t = sums[0];
+    for (int w = 1; w < kWaves; ++w) t += sums[w];
+    return t;
+  };
+  for (I row = blockIdx.x; row < numRows; row += gridDim.x) {
+    I inOff, outOff;
+    oa.offsets(row, inOff, outOff);
+    const T* src = in + inOff;
+    P v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const I at = mine + (I)u * step;
+      v[u] = load_pack_unaligned<false, P>(src + (at < packed ? at : 0));  // (past the end: the first pack, not used)
+    }
+    const auto sweep = [&](auto&& term) {
+      A acc[VEC];
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) acc[e] = (A)0;
+      const auto take = [&](const P& x) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[e] += term(acc_up<A>(x.v[e]));
+      };
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (mine + (I)u * step < packed) take(v[u]);
+      for (I i = mine + (I)U * step; i < packed; i += 4 * step) {
+        P w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = load_pack_unaligned<false, P>(src + (i + (I)u * step < packed ? i + (I)u * step : i));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (i + (I)u * step < packed) take(w[u]);
+      }
+      if (packed + threadIdx.x < R) acc[0] += term(acc_up<A>(src[packed + threadIdx.x]));
+      A t = acc[0];
+#pragma unroll
+      for (int e = 1; e < VEC; ++e) t += acc[e];
+      return t;
+    };
+    const A mean = block_sum(sweep([](A x) { return x; }), red[0]) / (A)R;
+    const A ss = block_sum(sweep([mean](A x) {
+                             const A d = x - mean;
+                             return d * d;
+                           }),
+                           red[1]);
+    if (threadIdx.x == 0) out[outOff] = acc_down<T>(wantStd ? sqrt_any(ss / div) : ss / div);
+  }
+}
+
+// var / std along a unit-stride dim of many rows too long for the registers, in whole packs (layer statistics over 4096 or
 // 8192 features): a wave per row in ONE read, every lane running (count, mean, M2) per pack slot over
 // its packs, 8 requested at a time, then the slots and the lanes merged pairwise (the two-sweep
 // form read such rows twice: 0.40 of peak on 8192 x 8192).
 template <typename T, typename I, int VEC>
 __global__ __launch_bounds__(kBlock) void var_rows_long_kernel(const T* __restrict__ in, T* __restrict__ out,
                                                                OuterArgs<I> oa, I numRows, I R,
-                                                               typename Acc<T>::type div, bool wantStd);
+                                                               typename Acc<T>::type div, bool wantStd) {
+  using P = Pack<T, VEC>;
+  using A = typename Acc<T>::type;
+  constexpr int U = 8;
+  const uint32_t lane = threadIdx.x & 63;
+  const I wavesPerGrid = (I)gridDim.x * (kBlock / 64);
+  const I step = (I)64 * VEC;
+  for (I row = (I)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); row < numRows; row += wavesPerGrid) {
+    I inOff, outOff;
+    oa.offsets(row, inOff, outOff);
+    const T* src = in + inOff;
+    A cnt = (A)0, mean[VEC], m2[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      mean[e] = (A)0;
+      m2[e] = (A)0;
+    }
+    for (I i = (I)lane * VEC; i < R; i += (I)U * step) {
+      P v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const I at = i + (I)u * step < R ? i + (I)u * step : i;  // (past the end: re-read, not used)
+        v[u] = load_pack<true>(reinterpret_cast<const P*>(src + at));
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (i + (I)u * step < R) {
+          cnt += (A)1;
+          const A inv = (A)1 / cnt;
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            const A x = acc_up<A>(v[u].v[e]);
+            const A delta = x - mean[e];
+            mean[e] += delta * inv;
+            m2[e] += delta * (x - mean[e]);
+          }
+        }
+      }
+    }
+    A n = cnt, mu = mean[0], q = m2[0];
+#pragma unroll
+    for (int e = 1; e < VEC; ++e) moments_merge(n, mu, q, cnt, mean[e], m2[e]);
+    for (uint32_t o = 32; o > 0; o >>= 1) {
+      const A on = shfl_xor_any(n, o), omu = shfl_xor_any(mu, o), oq = shfl_xor_any(q, o);
+      moments_merge(n, mu, q, on, omu, oq);
+    }
+    if (lane == 0) {
+      const A v = q / div;
+      out[outOff] = acc_down<T>(wantStd ? sqrt_any(v) : v);
+    }
+  }
+}
 
 // ------------------------------------------------------------------ cols --
 template <typename I>
@@ -1674,77 +1793,6 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
 // reductions, workgroup partials are merged with the pairwise update of Chan,
 // Golub & LeVeque. Same geometry as reduce_cols_kernel. Partial planes hold
 // (mean, M2) per output: partial[(s * 2 + {0, 1}) * outElems + out].
-// BT = 0: a wave per row. BT > 0: a workgroup of BT threads per row, for rows too few to fill the chip with waves
-// (var of 328 x 15366 fp32 26.7 us in two sweeps, 9.7 in one; 44 x 14186 15.5 and 6.9, 2 x 19968 doubles 16.3 and 7.8). Packs sit at element-aligned addresses; the elements behind the last whole pack go one to a lane.
-template <typename T, typename I, int VEC, int BT>
-__global__ __launch_bounds__(BT ? BT : kBlock) void var_rows_long_kernel(const T* __restrict__ in, T* __restrict__ out,
-                                                                         OuterArgs<I> oa, I numRows, I R,
-                                                                         typename Acc<T>::type div, bool wantStd) {
-  using P = Pack<T, VEC>;
-  using A = typename Acc<T>::type;
-  constexpr int U = 8, kLanes = BT ? BT : 64, kRows = (BT ? BT : kBlock) / kLanes;
-  const uint32_t lane = threadIdx.x & (kLanes - 1);
-  const I step = (I)kLanes * VEC;
-  const I packed = R - R % VEC;
-  for (I row = (I)blockIdx.x * kRows + threadIdx.x / kLanes; row < numRows; row += (I)gridDim.x * kRows) {
-    I inOff, outOff;
-    oa.offsets(row, inOff, outOff);
-    const T* src = in + inOff;
-    A cnt = (A)0, mean[VEC], m2[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      mean[e] = (A)0;
-      m2[e] = (A)0;
-    }
-    for (I i = (I)lane * VEC; i < packed; i += (I)U * step) {
-      P v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const I at = i + (I)u * step < packed ? i + (I)u * step : i;  // (past the end: re-read, not used)
-        v[u] = load_pack_unaligned<true, P>(src + at);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (i + (I)u * step < packed) {
-          cnt += (A)1;
-          const A inv = (A)1 / cnt;
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) {
-            const A x = acc_up<A>(v[u].v[e]);
-            const A delta = x - mean[e];
-            mean[e] += delta * inv;
-            m2[e] += delta * (x - mean[e]);
-          }
-        }
-      }
-    }
-    A n = cnt, mu = mean[0], q = m2[0];
-#pragma unroll
-    for (int e = 1; e < VEC; ++e) moments_merge(n, mu, q, cnt, mean[e], m2[e]);
-    if (packed + lane < R) moments_merge(n, mu, q, (A)1, acc_up<A>(src[packed + lane]), (A)0);
-    for (uint32_t o = 32; o > 0; o >>= 1) {
-      const A on = shfl_xor_any(n, o), omu = shfl_xor_any(mu, o), oq = shfl_xor_any(q, o);
-      moments_merge(n, mu, q, on, omu, oq);
-    }
-    if constexpr (BT > 64) {
-      __shared__ A red[BT / 64][3];
-      if ((lane & 63) == 0) {
-        red[lane / 64][0] = n;
-        red[lane / 64][1] = mu;
-        red[lane / 64][2] = q;
-      }
-      __syncthreads();
-      if (lane == 0)
-        for (int w = 1; w < BT / 64; ++w) moments_merge(n, mu, q, red[w][0], red[w][1], red[w][2]);
-      __syncthreads();
-    }
-    if (lane == 0) {
-      const A v = q / div;
-      out[outOff] = acc_down<T>(wantStd ? sqrt_any(v) : v);
-    }
-  }
-}
-
 template <typename T, typename I, int VEC>
 __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ in,
                                                           T* __restrict__ out,
@@ -3252,36 +3300,54 @@ bool reduce_var_rows_type(THCState* s, const ReduceGeom& g, const void* in_, voi
     bool inRegisters = g.sR == 1 && aligned16(in) && g.R % VEC == 0 && g.R <= 64 * VEC * U;
     for (int d = 0; d < g.in.dims && inRegisters; ++d)
       inRegisters = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
-    // Longer rows, and from 1 KiB on rows off the 16-byte grid that the LDS-staged form below does not take: one read, a wave
-    // per row, or a workgroup per row where that leaves CUs idle. Few rows beyond 64 Ki elements take two sweeps, cut into pieces.
+    // Longer rows of whole packs, a wave each where that fills the chip. Else, and from 1 KiB on for rows off the 16-byte grid that
+    // the LDS-staged form below does not take, a workgroup per row of up to 65536 elements, which the caches
+    // hold between its sweeps; longer ones take the two launches.
     uint32_t ldsRowsProbe = 0, ldsGProbe = 0;
     size_t ldsBytesProbe = 0;
     const int64_t cus = num_compute_units(s);
     bool wholePacks = g.sR == 1 && aligned16(in) && g.R % VEC == 0;
     for (int d = 0; d < g.in.dims && wholePacks; ++d) wholePacks = g.in.stride[d] % VEC == 0 || g.in.size[d] == 1;
-    const bool longRows = !inRegisters && g.sR == 1 && tuning("reduce.var.long_rows", 1) &&
-                          (wholePacks ? g.R > 64 * VEC * U * (g.outElems >= cus * 4 ? 1 : 2) : loose_row_packs<T>(g) && !plan_rows_lds<T>(s, g, false, ldsRowsProbe, ldsGProbe, ldsBytesProbe)) &&
-                          (g.outElems >= cus || g.R <= 65536);
-    if (longRows) {
-      // (a workgroup of 256 for rows a wave could walk in a few batches, of 1024 beyond)
-      const int bt = g.outElems >= cus * 4 ? 0 : g.R <= 256 * VEC * U ? 256 : 1024;
+    const bool manyRows = g.outElems >= cus * 4, longTuning = !inRegisters && g.sR == 1 && tuning("reduce.var.long_rows", 1);
+    if (longTuning && wholePacks && manyRows) {
+      const int wpb = kBlock / 64;
+      const int grid = capped_grid(s, (g.outElems + wpb - 1) / wpb, "reduce.rows.blocks_per_cu", 64);
+      hipStream_t st = current_stream(s);
+      const auto go = [&](auto idxTag) {
+        using I = decltype(idxTag);
+        hipLaunchKernelGGL((var_rows_long_kernel<T, I, VEC>), dim3(grid), dim3(kBlock), 0, st, in, out,
+                           make_outer<I>(g.in, g.out, g.in.dims), (I)g.outElems, (I)g.R, (A)div, wantStd);
+      };
+      if (g.wide) go(uint64_t{});
+      else go(uint32_t{});
+      note_kernel("var-rows-long");
+      return true;
+    }
+    if (longTuning && g.R <= 131072 &&
+        (wholePacks ? g.R > 2 * 64 * VEC * U : loose_row_packs<T>(g) && !plan_rows_lds<T>(s, g, false, ldsRowsProbe, ldsGProbe, ldsBytesProbe))) {
+      // The fewest threads that hold two thirds of the row in registers, up to 1024; 64 for many rows only. us with 64, 256, 512
+      // and 1024 threads and in two launches, fp32: 8000 x 2103 13.7, 17.3, 30.7, 74.4, 27.0; 300 x 4097 4.8, 4.4, 4.7, 6.7, 12.0; 5000 x
+      // 9001 46.8, 29.3, 29.6, 55.5, 58.6; 328 x 15366 12.5, 5.7, 4.9, 6.9, 21.1; 300 x 25001 22.6, 8.3, 6.4, 7.4, 20.5; 300 x 60001 -,
+      // 25.8, 20.9, 18.7, 37.8; 300 x 100003 -, 41.6, 34.0, 33.1, 48.0; 300 x 250001 -, -, 92.2, 97.4, 101.5.
+      const int64_t held = g.R * 2 / (3 * VEC * U);   // threads
+      const int bt = manyRows && held <= 64 ? 64 : held <= 256 ? 256 : held <= 512 ? 512 : 1024;
+      const int grid = capped_grid(s, g.outElems, "reduce.rows.blocks_per_cu", 64);
       hipStream_t st = current_stream(s);
       const auto go = [&](auto idxTag, auto btTag) {
         using I = decltype(idxTag);
         constexpr int BT = decltype(btTag)::value;
-        constexpr int kRows = BT ? 1 : kBlock / 64;
-        const int grid = capped_grid(s, (g.outElems + kRows - 1) / kRows, "reduce.rows.blocks_per_cu", 64);
-        hipLaunchKernelGGL((var_rows_long_kernel<T, I, VEC, BT>), dim3(grid), dim3(BT ? BT : kBlock), 0, st, in, out,
+        hipLaunchKernelGGL((var_rows_block_kernel<T, I, VEC, BT>), dim3(grid), dim3(BT), 0, st, in, out,
                            make_outer<I>(g.in, g.out, g.in.dims), (I)g.outElems, (I)g.R, (A)div, wantStd);
       };
       const auto pick = [&](auto idxTag) {
-        if (bt == 0) go(idxTag, std::integral_constant<int, 0>{});
+        if (bt == 64) go(idxTag, std::integral_constant<int, 64>{});
         else if (bt == 256) go(idxTag, std::integral_constant<int, 256>{});
+        else if (bt == 512) go(idxTag, std::integral_constant<int, 512>{});
         else go(idxTag, std::integral_constant<int, 1024>{});
       };
       if (g.wide) pick(uint64_t{});
       else pick(uint32_t{});
-      note_kernel("var-rows-long");
+      note_kernel("var-rows-block");
       return true;
     }
     if (!inRegisters) {

@@ -277,3 +277,46 @@ def test_gpu_var_of_short_rows_and_small_slices_is_one_read(thc, kind):
                     want = fn(ref, axis=dim, ddof=0 if biased else 1, keepdims=True)
                     np.testing.assert_allclose(out.numpy().astype(np.float64), want, rtol=tol, atol=atol,
                                                err_msg="%s %s %s off %d" % (kind, name, shape, off))
+
+
+def _variance_bound(kind, n, offset):
+    """Relative error that two sweeps may show on n values of deviation 1 around `offset`. The mean of at most 128 Ki values is off by
+    a few roundings of the offset (sums of 32 to 128 terms a lane, then a tree: 4 are allowed for), which adds its square; squares and their sum
+    are off by a few more; a result of 2 bytes is rounded once (a step of 2^-10 at most)."""
+    eps = {"float": 2.0 ** -24, "half": 2.0 ** -24, "double": 2.0 ** -53}[kind]
+    return (4 * eps * offset) ** 2 + 8 * eps + (2.0 ** -11 if kind == "half" else 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "double"])
+def test_gpu_var_of_few_and_of_odd_rows_keeps_two_sweeps(thc, kind):
+    """Rows that a workgroup takes: few of whole packs, and rows off the 16-byte grid, at offsets of up to 10000 deviations
+    from zero, where a running mean loses two digits. Row lengths around those that 64, 256, 512 and 1024 threads
+    take, within and beyond their registers, and the longest; storage offsets 0..3; strided rows."""
+    rng = np.random.default_rng(89)
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64}[kind]
+    item = np.dtype(dtype).itemsize
+    unit = 16 // item * 8                                # elements a thread holds
+    cus = thc.lib().THCAmd_getNumComputeUnits(thc.state())
+    cases = [(rows, n, n) for n in (15366, 9001, 256 * unit, 384 * unit + 1, 386 * unit + 1, 768 * unit - 1, 770 * unit + 1, 1024 * unit + 3, 131071,
+                                    131072) for rows in (1, 5) if n * item > 8192]
+    cases += [(4 * cus + 1, n, n + 3) for n in (1024 // item + 1, 64 * unit + 1, 96 * unit + 1, 98 * unit + 1)]
+    cases += [(4 * cus, 3 * 64 * unit + 5, 3 * 64 * unit + 5)]
+    for offset in (0, 16, 128) if kind == "half" else (0, 1000, 10000):
+        for rows, n, pitch in cases:
+            off = int(rng.integers(0, 4))
+            store = (rng.standard_normal(rows * pitch + off) + offset).astype(dtype)
+            dev = thc.Tensor.from_storage(store, off, (rows, n), (pitch, 1), kind=kind)
+            ref = store[off:].reshape(rows, pitch)[:, :n].astype(np.float64)
+            for name, fn in (("var", np.var), ("std", np.std)):
+                got = getattr(thc.Tensor(kind), name)(dev, 1).numpy().astype(np.float64)
+                if n > 2 * 64 * unit or n % (unit // 8) or off % (unit // 8):
+                    assert thc.last_kernel() == "var-rows-block", (rows, n, off, thc.last_kernel())
+                want = fn(ref, axis=1, ddof=1, keepdims=True)
+                err = np.max(np.abs(got - want) / want)
+                assert err <= _variance_bound(kind, n, offset), (name, rows, n, offset, err)
+    x = rng.standard_normal((3, 9001)).astype(dtype)
+    x[1, 8999] = np.nan
+    x[2, 4] = np.inf
+    got = thc.Tensor(kind).var(thc.Tensor.from_numpy(x), 1).numpy()
+    assert np.isfinite(got[0, 0]) and np.isnan(got[1, 0]) and np.isnan(got[2, 0])
