@@ -1391,12 +1391,14 @@ __global__ __launch_bounds__(kBlock) void var_slab_kernel(const T* __restrict__ 
     const uint32_t ns = (uint32_t)min((I)a.slicesPerBlock, a.O - o0);
     const uint32_t mis = stage_rows_to_lds<T, 8>(in + o0 * (I)slice, ns * slice, lds);
     __syncthreads();
-    // Fewer columns than threads: P threads share a column, each sweeps a band of its rows twice, and the bands' (count,
-    // mean, sum of squared deviations) meet in a fixed tree in LDS (1001 slices of 576 x 2 fp32: 51 us with a thread per column).
+    // Fewer columns than threads: P threads share a column, each sweeps a band of its rows, and the bands' sums meet in
+    // a fixed tree in LDS, first for the column's mean, then for the squared deviations from it (1001 slices of 576 x 2 fp32: 51 us
+    // with a thread per column, 6.4 now). Bands with means of their own, merged, would round those relative to the mean: relative error of
+    // 576 fp32 rows 1000 deviations away from zero 4e-6 that way, 5e-8 with one mean.
     const uint32_t cols = ns * C, P = cols < kBlock ? min(R / 8, kBlock / cols) : 1u;
-    __shared__ A bands[3][kBlock];
-    // both sweeps read LDS in batches of 8 (past the band's end: its last element, not used)
-    auto sweep = [&](const T* col, uint32_t rb, uint32_t re, A& mean, A& ss) {
+    __shared__ A bands[kBlock];
+    // a sweep reads LDS in batches of 8 (past the band's end: its last element, not used)
+    auto sweep = [&](const T* col, uint32_t rb, uint32_t re, auto&& term) {
       A sum = (A)0;
       for (uint32_t r = rb; r < re; r += 8) {
         T x[8];
@@ -1404,22 +1406,16 @@ __global__ __launch_bounds__(kBlock) void var_slab_kernel(const T* __restrict__ 
         for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, re - 1) * C];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-          if (r + u < re) sum += acc_up<A>(x[u]);
+          if (r + u < re) sum += term(acc_up<A>(x[u]));
       }
-      mean = sum / (A)(re - rb);
-      ss = (A)0;
-      for (uint32_t r = rb; r < re; r += 8) {
-        T x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = col[min(r + u, re - 1) * C];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          if (r + u < re) {
-            const A d = acc_up<A>(x[u]) - mean;
-            ss += d * d;
-          }
-        }
-      }
+      return sum;
+    };
+    const auto value = [](A x) { return x; };
+    const auto deviation = [](A mean) {
+      return [mean](A x) {
+        const A d = x - mean;
+        return d * d;
+      };
     };
     auto put = [&](uint32_t o, uint32_t c, A ss) {
       I inOff, outOff;
@@ -1430,35 +1426,30 @@ __global__ __launch_bounds__(kBlock) void var_slab_kernel(const T* __restrict__ 
       for (uint32_t t = threadIdx.x; t < cols; t += kBlock) {
         uint32_t o, c;
         a.cdiv.divmod(t, o, c);
-        A mean, ss;
-        sweep(lds + mis + o * slice + c, 0, R, mean, ss);
-        put(o, c, ss);
+        const T* col = lds + mis + o * slice + c;
+        const A mean = sweep(col, 0, R, value) / (A)R;
+        put(o, c, sweep(col, 0, R, deviation(mean)));
       }
     } else {
       const uint32_t p = threadIdx.x / cols, t = threadIdx.x - p * cols;
       uint32_t o, c;
       a.cdiv.divmod(t, o, c);
-      if (p < P) {
-        const uint32_t rb = p * R / P, re = (p + 1) * R / P;  // (at least 8 rows)
-        A mean, ss;
-        sweep(lds + mis + o * slice + c, rb, re, mean, ss);
-        bands[0][threadIdx.x] = (A)(re - rb);
-        bands[1][threadIdx.x] = mean;
-        bands[2][threadIdx.x] = ss;
-      }
-      __syncthreads();
-      for (uint32_t h = 1; h < P; h <<= 1) {
-        if (p < P && (p & (2 * h - 1)) == 0 && p + h < P) {
-          const uint32_t i = threadIdx.x, j = i + h * cols;
-          A n = bands[0][i], mean = bands[1][i], ss = bands[2][i];
-          moments_merge(n, mean, ss, bands[0][j], bands[1][j], bands[2][j]);
-          bands[0][i] = n;
-          bands[1][i] = mean;
-          bands[2][i] = ss;
-        }
+      const T* col = lds + mis + o * slice + c;
+      const uint32_t rb = p * R / P, re = (p + 1) * R / P;  // (at least 8 rows)
+      auto meet = [&](A v) {  // v summed over the bands of the thread's column
+        bands[threadIdx.x] = v;
         __syncthreads();
-      }
-      if (p == 0) put(o, c, bands[2][t]);
+        for (uint32_t h = 1; h < P; h <<= 1) {
+          if (p < P && (p & (2 * h - 1)) == 0 && p + h < P) bands[threadIdx.x] += bands[threadIdx.x + h * cols];
+          __syncthreads();
+        }
+        return bands[t];
+      };
+      const A mean = meet(p < P ? sweep(col, rb, re, value) : (A)0) / (A)R;
+      const A ss = p < P ? sweep(col, rb, re, deviation(mean)) : (A)0;
+      __syncthreads();  // (everybody has read the mean)
+      const A all = meet(ss);
+      if (p == 0) put(o, c, all);
     }
     __syncthreads();
   }

@@ -320,3 +320,23 @@ def test_gpu_var_of_few_and_of_odd_rows_keeps_two_sweeps(thc, kind):
     x[2, 4] = np.inf
     got = thc.Tensor(kind).var(thc.Tensor.from_numpy(x), 1).numpy()
     assert np.isfinite(got[0, 0]) and np.isnan(got[1, 0]) and np.isnan(got[2, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "half", "double"])
+def test_gpu_var_of_small_slices_far_from_zero(thc, kind):
+    """Threads that share a column of a small slice take one mean for all of its rows: at offsets of up to 10000 deviations, with
+    bands of 8 rows and more, one band, and a thread per column."""
+    rng = np.random.default_rng(91)
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64}[kind]
+    for offset in (0, 16, 128) if kind == "half" else (0, 1000, 10000):
+        for shape in ((50, 576, 2), (9, 33, 4), (1, 16, 100), (3, 700, 2), (70, 64, 8), (2, 17, 100), (300, 15, 7), (5, 250, 4)):
+            x = (rng.standard_normal(shape) + offset).astype(dtype)
+            want = x.astype(np.float64).var(axis=1, ddof=1, keepdims=True)
+            got = thc.Tensor(kind).var(thc.Tensor.from_numpy(x), 1).numpy().astype(np.float64)
+            assert thc.last_kernel() == "var-slab", (shape, thc.last_kernel())
+            # A thread sums up to 96 rows one by one here. Roundings add up like a random walk, four deviations of which are allowed
+            # for: of the mean, t roundings of partial sums of k offsets (k = 1..t) over t: eps offset sqrt(t) / 3; of the sum of squares eps sqrt(t).
+            t, eps = 96, 2.0 ** (-53 if kind == "double" else -24)
+            bound = (4 * eps * offset * t ** 0.5 / 3) ** 2 + 4 * eps * t ** 0.5 + (2.0 ** -11 if kind == "half" else 0)
+            assert np.max(np.abs(got - want) / want) <= bound, (shape, offset, np.max(np.abs(got - want) / want))
