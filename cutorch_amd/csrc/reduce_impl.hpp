@@ -1540,8 +1540,8 @@ __global__ __launch_bounds__(BT) void var_rows_block_kernel(const T* __restrict_
     if constexpr (kWaves == 1) return x;
     if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = x;
     __syncthreads();
-    A t = sums[0];
-    for (int w = 1; w < kWaves; ++w) t += sums[w];
+    A t = sums[threadIdx.x & (kWaves - 1)];
+    for (uint32_t o = kWaves / 2; o > 0; o >>= 1) t += shfl_xor_any(t, o);  // (a tree: one by one, 16 waves cost half a digit)
     return t;
   };
   for (I row = blockIdx.x; row < numRows; row += gridDim.x) {
