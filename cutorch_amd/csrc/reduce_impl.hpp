@@ -3702,7 +3702,7 @@ void reduce_all_moments_type(THCState* s, int64_t n, const void* src, Scalar* re
     const int64_t batch = (int64_t)kBlock * V * 8;
     int64_t blocks = std::min<int64_t>((int64_t)num_compute_units(s) * tuning("reduce.all.blocks_per_cu", 2),
                                        (n + batch - 1) / batch);
-    blocks = std::max<int64_t>(1, std::min<int64_t>(blocks, (int64_t)(sc.partialBytes / (3 * sizeof(A)))));
+    blocks = std::max<int64_t>(1, std::min<int64_t>(blocks, (int64_t)(kFoldWords / (3 * (sizeof(A) / 4)))));  // (three values a workgroup)
     int64_t chunk = (n + blocks - 1) / blocks;
     chunk = (chunk + batch - 1) / batch * batch;
     blocks = (n + chunk - 1) / chunk;

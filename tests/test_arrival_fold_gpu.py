@@ -43,3 +43,24 @@ def test_var_of_tall_matrices_folds_in_one_workgroup_per_column_tile(thc, rows, 
     assert thc.last_kernel() == "var-tall", thc.last_kernel()
     want = x.astype(np.float64).var(axis=0, ddof=1)
     assert np.all(np.abs(got - want) <= 64 * np.finfo(np.float32).eps * want)
+
+
+@pytest.mark.parametrize("kind,dtype", [("float", np.float32), ("double", np.float64)])
+def test_more_workgroups_than_the_handed_over_values_have_room_for(thc, kind, dtype):
+    """Variances publish three values a workgroup, of two words each for doubles: their workgroups are held to the room there is,
+    behind which the words of one-read scans lie (a scan afterwards meets none of theirs)."""
+    cus = thc.lib().THCAmd_getNumComputeUnits(thc.state())
+    n = 9 * cus * 256 * 8 * (16 // np.dtype(dtype).itemsize) + 5
+    x = (np.arange(n) % 3 == 0).astype(dtype)
+    t = thc.Tensor.from_numpy(x)
+    want, sums = x.astype(np.float64).var(ddof=1), np.cumsum(x, dtype=np.float64)
+    for per_cu in (2, 3, 4, 5, 8):
+        thc.set_tuning("reduce.all.blocks_per_cu", per_cu)
+        try:
+            for _ in range(2):
+                assert abs(t.varall() - want) <= 64 * np.finfo(dtype).eps * want, per_cu
+                assert t.sumall() == x.sum(dtype=np.float64), per_cu
+                if sums[-1] < 2 ** 24 or kind == "double":
+                    assert np.array_equal(thc.Tensor(kind).cumsum(t, 0).numpy(), sums.astype(dtype)), per_cu
+        finally:
+            thc.set_tuning("reduce.all.blocks_per_cu", 2)
