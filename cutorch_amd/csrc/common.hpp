@@ -132,9 +132,8 @@ constexpr size_t kScratchTailBytes = 64 * 1024;
 constexpr size_t kScratchCounters = (kScratchTailBytes - 256) / sizeof(unsigned);
 constexpr size_t kScanTicket = 2048;  // counters kScanTicket and the one behind it: a 64-bit word that deals out the chunks of one-read scans
 constexpr size_t kScanWords = size_t(2) << 20;  // 16 MiB of words behind the tail, which only one-read scans write
-// Whole-tensor reductions: the partials that workgroups hand to the one that folds them, 32 KiB of words in the tail, and the
-// count of such launches on the stream.
-constexpr size_t kFoldWordsAt = 16 * 1024, kFoldWords = 4096, kFoldCount = kScanTicket + 2;   // (bytes into the tail; words; counter)
+// Whole-tensor reductions: the partials that workgroups hand to the one that folds them, 32 KiB of words in the tail.
+constexpr size_t kFoldWordsAt = 16 * 1024, kFoldWords = 4096;   // (bytes into the tail; words)
 struct StreamScratch {
   void* partials;
   size_t partialBytes;
@@ -146,9 +145,12 @@ struct StreamScratch {
   size_t scanWords;     // how many
   uint64_t* scanTicket;
   uint64_t* foldWord;   // as scanWord, for whole-tensor reductions
-  uint64_t* foldCount;
 };
 const StreamScratch& stream_scratch(THCState* state);
+// A number for a launch that hands partials over in foldWord: never 0, another for every launch on any stream until
+// 2^32 - 1 have been given. It comes from the host, since these calls return a number and so are never captured: read from device
+// memory and advanced there it cost every total 0.3-0.8 us, also those of one workgroup.
+uint32_t next_fold_tag(THCState* state);
 void* scratch_space(THCState* state, size_t* bytes);
 void check_same_gpu(THCState* state, int n, const AnyTensor* const* ts);
 void note_kernel(const char* name);  // for THCAmd_lastKernel

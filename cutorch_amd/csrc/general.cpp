@@ -24,6 +24,7 @@ struct THCState {
   std::mutex mu;
   std::map<hipStream_t, thc::StreamScratch> scratch;  // per stream, lazily allocated
   size_t scratchBytes = 0;
+  std::atomic<uint32_t> foldTag{0};
 };
 
 // Threads whose THCAmd_lastError holds a message; a binding reads it instead of asking after every call.
@@ -138,10 +139,9 @@ const StreamScratch& stream_scratch(THCState* s) {
   sc.result = reinterpret_cast<float*>(static_cast<char*>(p) + s->scratchBytes - 256);
   sc.scanWord = reinterpret_cast<uint64_t*>(static_cast<char*>(p) + s->scratchBytes);
   sc.scanWords = kScanWords;
-  static_assert(kFoldWordsAt + kFoldWords * sizeof(uint64_t) <= kScratchTailBytes - 256 && (kFoldCount + 2) * sizeof(unsigned) <= kFoldWordsAt,
+  static_assert(kFoldWordsAt + kFoldWords * sizeof(uint64_t) <= kScratchTailBytes - 256 && (kScanTicket + 2) * sizeof(unsigned) <= kFoldWordsAt,
                 "the tail's parts lie behind each other");
   sc.foldWord = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(sc.counters) + kFoldWordsAt);
-  sc.foldCount = reinterpret_cast<uint64_t*>(sc.counters + kFoldCount);
   sc.scanTicket = reinterpret_cast<uint64_t*>(sc.counters + kScanTicket);
   // Arrival counters start at zero and every kernel that uses one resets it; the words of one-read scans lie behind them.
   THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
@@ -153,6 +153,13 @@ const StreamScratch& stream_scratch(THCState* s) {
   THC_CHECK(hipHostGetDevicePointer(&dv, sc.hostResult, 0));
   sc.hostResultDev = static_cast<float*>(dv);
   return s->scratch[st] = sc;
+}
+
+uint32_t next_fold_tag(THCState* s) {
+  uint32_t t;
+  do t = s->foldTag.fetch_add(1, std::memory_order_relaxed) + 1;
+  while (t == 0);
+  return t;
 }
 
 void* scratch_space(THCState* s, size_t* bytes) {

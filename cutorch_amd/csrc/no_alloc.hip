@@ -95,13 +95,13 @@ void sumall_no_alloc(THCState* s, AnyTensor* self, float* result) {
     using I = decltype(idxTag);
     if (aligned16(src))
       hipLaunchKernelGGL((reduce_all_kernel<float, F, I, V, true>), dim3((int)blocks), dim3(kBlock), 0, st, src,
-                         (I)n, (I)chunk, part, result, result, none, f, FoldWords{nullptr, nullptr});
+                         (I)n, (I)chunk, part, result, result, none, f, FoldWords{nullptr, 0});
     else
       hipLaunchKernelGGL((reduce_all_kernel<float, F, I, 1, true>), dim3((int)blocks), dim3(kBlock), 0, st, src,
-                         (I)n, (I)chunk, part, result, result, none, f, FoldWords{nullptr, nullptr});
+                         (I)n, (I)chunk, part, result, result, none, f, FoldWords{nullptr, 0});
     if (blocks > 1)
       hipLaunchKernelGGL((reduce_all_kernel<float, F, I, 1, false>), dim3(1), dim3(kBlock), 0, st,
-                         (const float*)part, (I)blocks, (I)blocks, part, result, result, none, f, FoldWords{nullptr, nullptr});
+                         (const float*)part, (I)blocks, (I)blocks, part, result, result, none, f, FoldWords{nullptr, 0});
   };
   if (force_64bit_index() || n >= kIndex32Limit) go(uint64_t{});
   else go(uint32_t{});

@@ -2257,22 +2257,17 @@ __device__ __forceinline__ typename F::A block_fold(typename F::A r, typename F:
 
 // Partials of a launch that folds them itself: the launch's last workgroup waits for those of the others. A 32-bit half
 // of a value travels as the 64-bit word (tag << 32) | half, by relaxed device-scope accesses, which the XCDs' L2s
-// pass through; the tag is the launch's number on its stream, which every workgroup reads as it starts and the last one advances when
-// it has all partials (so everybody has read it). Value and tag arrive together: no fence (a release fence writes back an
-// L2), no counter to be counted in at, and no wait for a store's acknowledgement before that. One
-// workgroup waits, whatever the grid; the others depend on nobody. us a call with a second launch for the fold, with
-// counters of arrivals whose last one folds (16 groups of them), and this way: sum of 30 000 floats 12.4, 9.8, 9.1; of 50 000
-// -, 10.0, 9.6; of 1M -, 10.1, 9.6; of 5M -, 12.2, 11.6; var of 30 000 -, 11.7, 11.1; of 1369 12.1 with a second launch.
+// pass through; the tag is the launch's number (next_fold_tag), so nothing clears the words. Value and tag arrive together: no
+// fence (a release fence writes back an L2), no counter to be counted in at, and no wait for a store's acknowledgement before that. One
+// workgroup waits, whatever the grid; the others depend on nobody. A launch of one workgroup hands nothing over.
+// Numbers come back after 2^32 - 1 launches: a word that nobody has written since the launch that many before would be taken for a new one.
+// us a call with a second launch for the fold, with counters of arrivals whose last one folds, with the number read from
+// device memory, and this way: sum of 30 000 floats 12.4, 9.9, 9.1, 8.6; of 1M -, 10.2, 9.6, 9.0; of 5M -, 13.0, 11.8, 11.1; of 256 -, 7.4,
+// 7.4, 7.0; var of 30 000 -, 11.7, 11.0, 10.5; of 1000 -, 8.4, 8.2, 7.8.
 struct FoldWords {
-  uint64_t* words;   // nullptr: partials go to memory, another launch folds them
-  uint64_t* count;
+  uint64_t* words;   // nullptr: one workgroup, or partials go to memory and another launch folds them
+  uint32_t tag;
 };
-__device__ __forceinline__ uint32_t fold_tag(const FoldWords& f) {
-  return (uint32_t)(__hip_atomic_load(f.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) % 0xffffffffull) + 1;
-}
-__device__ __forceinline__ void fold_done(const FoldWords& f) {
-  __hip_atomic_store(f.count, __hip_atomic_load(f.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 template <typename A>
 __device__ __forceinline__ void publish_partial(uint64_t* p, uint32_t tag, A v) {
   constexpr int W = sizeof(A) / 4;
@@ -2309,7 +2304,6 @@ __global__ __launch_bounds__(kBlock) void reduce_all_kernel(const TIn* __restric
   using P = Pack<TIn, VEC>;
   using A = typename F::A;
   __shared__ A red[kBlock / 64];
-  const uint32_t tag = fold.words ? fold_tag(fold) : 0u;
   A acc[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) acc[e] = f.init();
@@ -2355,27 +2349,26 @@ __global__ __launch_bounds__(kBlock) void reduce_all_kernel(const TIn* __restric
       return;
     }
     if (blockIdx.x != gridDim.x - 1) {
-      if (threadIdx.x == 0) publish_partial(fold.words + blockIdx.x * W, tag, r);
+      if (threadIdx.x == 0) publish_partial(fold.words + blockIdx.x * W, fold.tag, r);
       return;
     }
     const A own = r;
     r = f.init();
     for (unsigned b = threadIdx.x; b < gridDim.x; b += kBlock)
-      r = f.combine(r, b == blockIdx.x ? own : await_partial<A>(fold.words + b * W, tag));
+      r = f.combine(r, b == blockIdx.x ? own : await_partial<A>(fold.words + b * W, fold.tag));
     r = block_fold(r, red, f);
   }
   if (threadIdx.x == 0) {
     const A fin = epi.template finish<A>(r);
     *hostResult = fin;
     *result = fin;
-    if (fold.words) fold_done(fold);
   }
 }
 
 // Sum of squared deviations from the mean of a dense run in ONE read (varall /
 // stdall): every lane runs Welford's update per pack slot over its share, and
 // (count, mean, M2) triples merge pairwise (Chan et al.) across slots, lanes,
-// waves and, in the workgroup that arrives last, workgroups. partial[3 * b + {0, 1, 2}].
+// waves and, in the launch's last workgroup, workgroups. Words: (count, mean, M2) of workgroup b from 3 * b values on.
 template <typename A>
 __device__ __forceinline__ void moments_wave_merge(A& n, A& mean, A& m2) {
   for (uint32_t o = 32; o > 0; o >>= 1) {
@@ -2401,13 +2394,11 @@ __device__ __forceinline__ void moments_block_merge(A& n, A& mean, A& m2, A (*re
 
 template <typename TIn, typename I, int VEC>
 __global__ __launch_bounds__(kBlock) void moments_all_kernel(const TIn* __restrict__ in, I n, I chunk,
-                                                             typename Acc<TIn>::type* partial,
                                                              typename Acc<TIn>::type* result,
                                                              typename Acc<TIn>::type* hostResult, FoldWords fold) {
   using P = Pack<TIn, VEC>;
   using A = typename Acc<TIn>::type;
   __shared__ A red[kBlock / 64][3];
-  const uint32_t tag = fold_tag(fold);
   A cnt = (A)0, mean[VEC], m2[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
@@ -2449,7 +2440,7 @@ __global__ __launch_bounds__(kBlock) void moments_all_kernel(const TIn* __restri
   if (gridDim.x > 1) {
     constexpr int W = sizeof(A) / 4;
     if (blockIdx.x != gridDim.x - 1) {
-      if (threadIdx.x < 3) publish_partial(fold.words + (3 * blockIdx.x + threadIdx.x) * W, tag, threadIdx.x == 0 ? nn : threadIdx.x == 1 ? mm : ss);
+      if (threadIdx.x < 3) publish_partial(fold.words + (3 * blockIdx.x + threadIdx.x) * W, fold.tag, threadIdx.x == 0 ? nn : threadIdx.x == 1 ? mm : ss);
       return;
     }
     const A on = nn, om = mm, os = ss;
@@ -2458,14 +2449,13 @@ __global__ __launch_bounds__(kBlock) void moments_all_kernel(const TIn* __restri
     for (unsigned b = threadIdx.x; b < gridDim.x; b += kBlock) {
       const uint64_t* w = fold.words + 3 * b * W;
       if (b == blockIdx.x) moments_merge(nn, mm, ss, on, om, os);
-      else moments_merge(nn, mm, ss, await_partial<A>(w, tag), await_partial<A>(w + W, tag), await_partial<A>(w + 2 * W, tag));
+      else moments_merge(nn, mm, ss, await_partial<A>(w, fold.tag), await_partial<A>(w + W, fold.tag), await_partial<A>(w + 2 * W, fold.tag));
     }
     moments_block_merge(nn, mm, ss, red);
   }
   if (threadIdx.x == 0) {
     *hostResult = ss;
     *result = ss;
-    fold_done(fold);
   }
 }
 
@@ -3618,15 +3608,16 @@ void reduce_all_with(THCState* s, ReduceGeom g, const void* src, const void* src
       if (blocks > 1)
         hipLaunchKernelGGL((reduce_all_kernel<A, FSum<A>, I, 1, false>), dim3(1), dim3(kBlock), 0,
                            st, (const A*)part, (I)blocks, (I)blocks, part, devOut, hostDev, none,
-                           FSum<A>{(A)0}, FoldWords{nullptr, nullptr});
+                           FSum<A>{(A)0}, FoldWords{nullptr, 0});
       return;
     }
+    const FoldWords fold = blocks > 1 ? FoldWords{sc.foldWord, next_fold_tag(s)} : FoldWords{nullptr, 0};
     if (aligned16(src))
       hipLaunchKernelGGL((reduce_all_kernel<TI, F2, I, V, true>), dim3((int)blocks), dim3(kBlock), 0,
-                         st, (const TI*)src, (I)g.R, (I)chunk, part, devOut, hostDev, none, f, FoldWords{sc.foldWord, sc.foldCount});
+                         st, (const TI*)src, (I)g.R, (I)chunk, part, devOut, hostDev, none, f, fold);
     else
       hipLaunchKernelGGL((reduce_all_kernel<TI, F2, I, 1, true>), dim3((int)blocks), dim3(kBlock), 0,
-                         st, (const TI*)src, (I)g.R, (I)chunk, part, devOut, hostDev, none, f, FoldWords{sc.foldWord, sc.foldCount});
+                         st, (const TI*)src, (I)g.R, (I)chunk, part, devOut, hostDev, none, f, fold);
   };
   auto pick_index = [&](auto srcTag, auto f) {
     if (g.wide) stage2(srcTag, f, uint64_t{});
@@ -3707,16 +3698,16 @@ void reduce_all_moments_type(THCState* s, int64_t n, const void* src, Scalar* re
     chunk = (chunk + batch - 1) / batch * batch;
     blocks = (n + chunk - 1) / chunk;
     hipStream_t st = current_stream(s);
-    A* part = (A*)sc.partials;
+    const FoldWords fold = blocks > 1 ? FoldWords{sc.foldWord, next_fold_tag(s)} : FoldWords{nullptr, 0};
     arm_host_slot(sc);
     auto go = [&](auto idxTag) {
       using I = decltype(idxTag);
       if (aligned16(src))
         hipLaunchKernelGGL((moments_all_kernel<T, I, V>), dim3((int)blocks), dim3(kBlock), 0, st, (const T*)src,
-                           (I)n, (I)chunk, part, devOut, hostDev, FoldWords{sc.foldWord, sc.foldCount});
+                           (I)n, (I)chunk, devOut, hostDev, fold);
       else
         hipLaunchKernelGGL((moments_all_kernel<T, I, 1>), dim3((int)blocks), dim3(kBlock), 0, st, (const T*)src,
-                           (I)n, (I)chunk, part, devOut, hostDev, FoldWords{sc.foldWord, sc.foldCount});
+                           (I)n, (I)chunk, devOut, hostDev, fold);
     };
     if (force_64bit_index() || n >= kIndex32Limit) go(uint64_t{});
     else go(uint32_t{});

@@ -1,6 +1,6 @@
-"""Whole-tensor reductions whose last workgroup folds the partials of the others: sizes around the
-workgroup counts at which the arrival counters change shape (1, 2, 16, 17 and 512 workgroups), every
-accumulator width, repeated so that counters left unset would show."""
+"""Whole-tensor reductions whose last workgroup folds the partials of the others: one workgroup, which hands nothing
+over, two, as many as there are, and some between; every accumulator width, repeated so that an
+older launch's partials would show."""
 import numpy as np
 import pytest
 
