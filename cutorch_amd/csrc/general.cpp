@@ -12,6 +12,7 @@
 #include <string>
 
 #include "common.hpp"
+#include "scan_ticket.hpp"
 #include "stream_guard.hpp"
 
 struct THCState {
@@ -145,6 +146,9 @@ const StreamScratch& stream_scratch(THCState* s) {
   sc.scanTicket = reinterpret_cast<uint64_t*>(sc.counters + kScanTicket);
   // Arrival counters start at zero and every kernel that uses one resets it; the words of one-read scans lie behind them.
   THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
+  const uint32_t firstTag = (uint32_t)tuning("scan.first_tag", 1);
+  const uint64_t firstScan = scan_counter(firstTag ? firstTag : 1);
+  THC_CHECK(hipMemcpyAsync(sc.scanTicket, &firstScan, sizeof(firstScan), hipMemcpyHostToDevice, st));
   THC_CHECK(hipStreamSynchronize(st));
   // One pinned, device-mapped slot: *all reductions store their scalar there. Coherent (fine-grained),
   // so that a store by a running kernel becomes visible to the host, which polls the slot.

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "scan_ticket.hpp"
 #include "stream_guard.hpp"
 #include "device_util.hpp"
 
@@ -420,8 +421,8 @@ __device__ __forceinline__ A read_lane(A v, int lane) {
 
 // Accumulator values published between workgroups: every 32-bit half of the value is a 64-bit word
 // (tag << 32) | half, stored and loaded with relaxed device-scope atomics: value and tag arrive together, so no fence
-// (which would write back an XCD's L2) is needed. A word with another tag is "not there yet". The tag is the number of
-// the scan on its stream, which the workgroups read with their tickets (draw_ticket); the words are kept for scans
+// (which would write back an XCD's L2) is needed. A word with another tag is "not there yet". The tag is the scan's,
+// which the workgroups read with their tickets (draw_ticket); the words are kept for scans
 // alone and start out as zeros, so nothing has to clear them between two scans (a launch of its own before: 2^20 fp32
 // 7.8 us, 6.3 without it).
 template <typename A>
@@ -447,16 +448,14 @@ __device__ __forceinline__ bool poll_word(const uint64_t* words, uint32_t tag, A
   __builtin_memcpy(&v, h, sizeof(A));
   return there;
 }
-// The next chunk of a scan of `chunks` chunks and the scan's tag, in one atomic: the counter holds
-// (scans before this one << 32) | chunks drawn, and whoever draws the last chunk sets it up for the next scan (nobody
-// draws after that; the next scan of the stream starts when this one has ended). Tickets come in order, so all chunks
-// before this one belong to workgroups that are running or done. Tags are never 0 and come back after 2^32 - 1 scans.
+// The next chunk of a scan of `chunks` chunks and the scan's tag, in one atomic (scan_ticket.hpp). Whoever draws the last chunk
+// sets the counter up for the next scan: nobody draws after that, and the next scan of the stream starts when this one has ended.
+// Tickets come in order, so all chunks before this one belong to workgroups that are running or done.
 __device__ __forceinline__ uint32_t draw_ticket(uint64_t* counter, uint32_t chunks, uint32_t& tag) {
   const uint64_t t = __hip_atomic_fetch_add(counter, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint64_t scans = t >> 32;
-  if ((uint32_t)t == chunks - 1) __hip_atomic_store(counter, (scans + 1) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  tag = (uint32_t)(scans % 0xffffffffull) + 1;
-  return (uint32_t)t;
+  if (scan_chunk(t) == chunks - 1) __hip_atomic_store(counter, next_scan(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  tag = scan_tag(t);
+  return scan_chunk(t);
 }
 
 __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* words, uint64_t n) {

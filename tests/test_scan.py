@@ -3,6 +3,8 @@ pinned against numpy.cumsum/cumprod in float64 (and bit-exactly on
 integer-valued data); HIP path against the oracle: integer-valued data
 bit-exact, random data within 1e-5 of the running mass."""
 import ctypes
+import os
+import subprocess
 import threading
 
 import numpy as np
@@ -586,3 +588,37 @@ def test_gpu_one_read_scans_in_a_graph(thc):
     finally:
         hip.hipStreamSynchronize(stream)
         lib.THCState_setCurrentStream(st, None)
+
+
+def test_the_counter_of_one_read_scans_starts_its_tags_again(tmp_path):
+    """On the host (tests/scan_ticket_test.cpp): no scan accepts what the scan before it published, also where the tags start again."""
+    root, exe = os.path.dirname(os.path.dirname(os.path.abspath(__file__))), str(tmp_path / "scan_ticket_test")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(root, "cutorch_amd", "csrc"),
+                    os.path.join(root, "tests", "scan_ticket_test.cpp"), "-o", exe], check=True)
+    res = subprocess.run([exe], capture_output=True, text=True)
+    assert res.returncode == 0 and res.stdout.strip() == "ok", res.stdout + res.stderr
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [1, 0xfffffffd])
+def test_gpu_one_read_scans_where_the_tags_start_again(thc, first):
+    """Scans of several chunks on a new stream whose counter starts a few tags before the last one: rows, strips and runs."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(67)
+    inputs = [(rng.integers(0, 30, shape) == 0).astype(np.float32) for shape in ((300001,), (3001, 257), (40001, 5))]
+    dev = [thc.Tensor.from_numpy(x) for x in inputs]
+    want = [np.cumsum(x, axis=0, dtype=np.float64).astype(np.float32) for x in inputs]
+    stream = ctypes.c_void_p()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    thc.set_tuning("scan.first_tag", first)
+    thc.lib().THCState_setCurrentStream(thc.state(), stream)
+    try:
+        for i in range(6):
+            for k in range(3):
+                got = thc.Tensor("float").cumsum(dev[k], 0)
+                assert hip.hipStreamSynchronize(stream) == 0
+                assert_bit_equal(got.numpy(), want[k], "scan %d of input %d" % (i, k))
+    finally:
+        thc.set_tuning("scan.first_tag", 1)
+        hip.hipStreamSynchronize(stream)
+        thc.lib().THCState_setCurrentStream(thc.state(), None)
