@@ -1357,7 +1357,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
     } else if (sizeof(T) == 1 && R < 8192) {
       most_rows = 4 * cus;
     }
-    if (outer <= most_rows && outer * S < (int64_t(1) << 31) && nwords <= sc.scanWords) {
+    if (outer <= most_rows && outer * S < (int64_t(1) << 31) && (S == 1 || nwords <= sc.scanWords)) {
       uint64_t* words = S > 1 ? sc.scanWord : nullptr;
       const auto go = [&](auto tag) {
         constexpr int BT = decltype(tag)::value;
@@ -1442,7 +1442,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       int64_t S1, S2;
       const int lg = levels(S, S1, S2);
       if (ownColumns && outer * colTiles * S < (int64_t(1) << 31) &&
-          outer * colTiles * (S + S1 + S2) * TX * kFull * W <= (int64_t)sc.scanWords) {
+          (S == 1 || outer * colTiles * (S + S1 + S2) * TX * kFull * W <= (int64_t)sc.scanWords)) {   // (one chunk publishes nothing)
         const auto go = [&](auto tag) {
           constexpr int BT = decltype(tag)::value;
           hipLaunchKernelGGL((scan_strips_kernel<T, OpA, BT>), dim3((unsigned)(outer * colTiles * S)), dim3(BT), 0, st, out, in,
@@ -1469,7 +1469,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       const int lg = levels(S, S1, S2);
       const size_t data = (((size_t)(chunkRows * inner) + 2 * kFull) * sizeof(T) + 15) & ~size_t(15);
       const size_t lds = data + (2 * (size_t)std::max<int64_t>(threads, inner) + 2 * (size_t)inner) * sizeof(A);
-      if (lds <= 96 * 1024 && outer * S < (int64_t(1) << 31) && outer * (S + S1 + S2) * inner * W <= (int64_t)sc.scanWords) {
+      if (lds <= 96 * 1024 && outer * S < (int64_t(1) << 31) && (S == 1 || outer * (S + S1 + S2) * inner * W <= (int64_t)sc.scanWords)) {
         const auto go = [&](auto tag) {
           constexpr int BT = decltype(tag)::value;
           hipLaunchKernelGGL((scan_runs_kernel<T, OpA, BT>), dim3((unsigned)(outer * S)), dim3(BT), lds, st, out, in, sc.scanWord,

@@ -622,3 +622,20 @@ def test_gpu_one_read_scans_where_the_tags_start_again(thc, first):
         thc.set_tuning("scan.first_tag", 1)
         hip.hipStreamSynchronize(stream)
         thc.lib().THCState_setCurrentStream(thc.state(), None)
+
+
+@pytest.mark.gpu
+def test_gpu_scans_of_many_slices_of_one_chunk_each_need_no_words(thc):
+    """Slices that fit one chunk publish nothing, so their number is not held to the room for published totals: on both sides of that
+    room, strips and runs (the element-wise column kernel, which they went to, walks such rows alone)."""
+    rng = np.random.default_rng(79)
+    for shape, name in (((1010, 33, 1025), "scan-cols-split"), ((1030, 33, 1025), "scan-cols-split"),
+                        ((60000, 5, 15), "scan-chunked"), ((139000, 5, 15), "scan-chunked")):
+        x = rng.integers(-9, 10, shape).astype(np.float64)      # (two words a total)
+        thc.set_tuning("scan.slab", 0)
+        try:
+            got = thc.Tensor("double").cumsum(thc.Tensor.from_numpy(x), 1)
+            assert thc.last_kernel() == name, (shape, thc.last_kernel())
+        finally:
+            thc.set_tuning("scan.slab", 1)
+        assert_bit_equal(got.numpy(), np.cumsum(x, axis=1), "%s" % (shape,))
