@@ -630,7 +630,7 @@ def test_gpu_scans_of_many_slices_of_one_chunk_each_need_no_words(thc):
     room, strips and runs (the element-wise column kernel, which they went to, walks such rows alone)."""
     rng = np.random.default_rng(79)
     for shape, name in (((1010, 33, 1025), "scan-cols-split"), ((1030, 33, 1025), "scan-cols-split"),
-                        ((60000, 5, 15), "scan-chunked"), ((139000, 5, 15), "scan-chunked")):
+                        ((140000, 5, 7), "scan-chunked"), ((155000, 5, 7), "scan-chunked")):
         x = rng.integers(-9, 10, shape).astype(np.float64)      # (two words a total)
         thc.set_tuning("scan.slab", 0)
         try:
