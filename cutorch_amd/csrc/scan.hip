@@ -1416,7 +1416,11 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       // chunk need nobody's totals: the widest strip that holds them all. 512 threads, 1024 where a chain would
       // have 256 chunks and more (51967 x 120 fp32 17.6 against 20.5; 8-byte sums stay at 512: 278737 x 164 189 against 210).
       const int64_t widest = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(8, 128 / kFull), kMaxStripLanes), packs);
-      int64_t TX = tuning("scan.strips.lanes", widest), threads = tuning("scan.strips.threads", 0);
+      // (both knobs are held to what the kernel has room for and is built for; 0: as the rules say)
+      const int64_t lanes = tuning("scan.strips.lanes", 0);
+      int64_t TX = lanes > 0 ? std::min<int64_t>(lanes, std::min<int64_t>(kMaxStripLanes, packs)) : widest;
+      int64_t threads = tuning("scan.strips.threads", 0);
+      if (threads) threads = threads <= 256 ? 256 : threads <= 512 || sizeof(T) == 1 ? 512 : 1024;
       const auto rows_of = [&](int64_t bt, int64_t tx) { return bt / tx * kOnePassPacks; };
       if (!threads) {
         threads = 512;
@@ -1433,10 +1437,10 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       int64_t colTiles = (packs + TX - 1) / TX;
       TX = (packs + colTiles - 1) / colTiles;
       // (a strip of one moved-back pack would share columns with the strip before it)
-      if (inner % kFull != 0)
-        while (TX < kMaxStripLanes && packs > TX && packs % TX == 1) ++TX;
+      const auto lone_pack = [&]() { return inner % kFull != 0 && packs > TX && (packs - 1) % TX == 0; };
+      while (TX < kMaxStripLanes && lone_pack()) ++TX;
       colTiles = (packs + TX - 1) / TX;
-      const bool ownColumns = inner % kFull == 0 || packs <= TX || packs % TX != 1;
+      const bool ownColumns = !lone_pack();
       const auto parts = [&](int64_t bt) { return (R + rows_of(bt, TX) - 1) / rows_of(bt, TX); };
       const int64_t S = parts(threads);
       int64_t S1, S2;
@@ -1450,7 +1454,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
                              (uint32_t)colTiles, (uint32_t)S, (uint32_t)S1, (uint32_t)S2, (uint32_t)lg, streaming);
         };
         if (threads == 256) go(std::integral_constant<int, 256>{});
-        else if (threads == 512 || sizeof(T) == 1) go(std::integral_constant<int, 512>{});
+        else if (threads == 512) go(std::integral_constant<int, 512>{});
         else go(std::integral_constant<int, sizeof(T) == 1 ? 512 : 1024>{});
         note_kernel("scan-cols-split");
         return;

@@ -639,3 +639,34 @@ def test_gpu_scans_of_many_slices_of_one_chunk_each_need_no_words(thc):
         finally:
             thc.set_tuning("scan.slab", 1)
         assert_bit_equal(got.numpy(), np.cumsum(x, axis=1), "%s" % (shape,))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "byte", "double"])
+def test_gpu_strips_of_any_knob_value(thc, kind):
+    """Widths and threads of the strips that the kernel has no room for or is not built for are held to those that it is: every
+    row is written, in place as well, and nothing else."""
+    dtype = {"float": np.float32, "byte": np.uint8, "double": np.float64}[kind]
+    vec = 16 // np.dtype(dtype).itemsize
+    rng = np.random.default_rng(83)
+    thc.set_tuning("scan.strided", 1)
+    thc.set_tuning("scan.slab", 0)
+    try:
+        for inner in (vec, 3 * vec + 1, 40 * vec, 65 * vec - 1):
+            shape = (2, 1200, inner)
+            x = ((rng.integers(0, 60, 2 * 1200 * inner + 3) == 0) * 1).astype(dtype)
+            size = x.size - 3
+            want = x.copy()
+            want[1:1 + size] = np.cumsum(x[1:1 + size].reshape(shape), axis=1, dtype=np.int64).astype(dtype).reshape(-1)
+            for lanes in (-3, 0, 1, 2, 7, 32, 33, 1000):
+                for threads in (1, 256, 300, 512, 1024, 5000):
+                    thc.set_tuning("scan.strips.lanes", lanes)
+                    thc.set_tuning("scan.strips.threads", threads)
+                    dev = thc.Tensor.from_storage(x, 1, shape, (1200 * inner, inner, 1), kind=kind)
+                    dev.cumsum(dev, 1)
+                    assert_bit_equal(dev.storage_numpy(), want, "%s %d lanes %d threads %d" % (kind, inner, lanes, threads))
+    finally:
+        thc.set_tuning("scan.strided", -1)
+        thc.set_tuning("scan.slab", 1)
+        thc.set_tuning("scan.strips.lanes", 0)
+        thc.set_tuning("scan.strips.threads", 0)
