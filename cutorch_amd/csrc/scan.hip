@@ -480,7 +480,7 @@ __global__ __launch_bounds__(kBlock) void scan_clear_words_kernel(uint64_t* word
 // infinite behind it although its prefixes may be finite (the pieces had this over shorter spans).
 // A chunk costs about 13 ns at its row's ticket and look-back words wherever it runs, so chunks have to be large:
 // 16 KiB chunks took 525 us on 2^26 elements, 64 KiB 116, 128 KiB 110, 256 KiB 115 (too few in flight).
-// words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, all zeroed, W words per value;
+// words: [outer][S] chunk totals, [outer][S1] totals of 64 chunks, [outer][S2] of 4096, W words per value, under the scan's tag;
 // the grid is one workgroup per chunk.
 // In place (out == in) is fine: a chunk is read only by the workgroup that then writes it.
 // words == nullptr: every row is one chunk (S == 1), nothing to look back for.
@@ -691,6 +691,9 @@ __device__ __forceinline__ void look_back(uint64_t* w, uint32_t tag, uint32_t s,
 // at element-aligned addresses; the last pack of a row is moved back to end with it and shares columns with its
 // neighbour of the same strip (both compute the same values). Chunks are dealt row by row of chunks over all
 // chains, so neighbouring strips run together. words: [outer * colTiles][S + S1 + S2][TX * VEC] values.
+// A column's totals of a chunk, of a group of chunks and of a group of groups (up to 64 x 64 chunks) are formed on their own, here and in
+// scan_runs_kernel: where one of them overflows, the column is infinite behind it although its prefixes may be finite. The
+// two-read forms have this too, over the totals of their chunks or parts.
 template <typename T, typename Op, int BT>
 __global__ __launch_bounds__(BT) void scan_strips_kernel(T* out, const T* in, uint64_t* words, uint64_t* ticket, uint32_t outer,
                                                          uint64_t R, uint32_t inner, uint32_t TX, uint32_t colTiles, uint32_t S,
@@ -1529,6 +1532,8 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       }
     }
   }
+  // (0: strided dims never take the two-read forms below, which report the names of the one-read ones above; for tests of those)
+  const bool twoReads = inner <= 1 || tuning("scan.strided_two_reads", 1);
   // The column kernel with the rows cut into parts that scan side by side (totals of the parts, their
   // scan by this function on the accumulator type, then every part from its carry): for long scans over
   // rows of whole packs of at least `scan.cols.split_min_row_bytes`, whose lanes the column tiling keeps
@@ -1538,7 +1543,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
   // 0.09 of peak -> 0.41; 524288 x 100 doubles 0.02 -> 0.31). The input is read twice here too.
   auto split_cols = [&]() -> bool {
     using A = typename ScanAcc<T>::type;
-    if (inner <= 1 || !tuning("scan.cols.split", 1)) return false;
+    if (inner <= 1 || !tuning("scan.cols.split", 1) || !twoReads) return false;
     const bool vec = aligned && inner % VECC == 0;
     const int64_t pack = vec ? VECC : 1;
     const int64_t packs = (inner + pack - 1) / pack;
@@ -1598,7 +1603,7 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
     const size_t need = (((size_t)(outer * S * inner) * sizeof(A)) + 255) & ~size_t(255);
     // (chunks of at least 4 rows: with one row per chunk the totals are the input again, and the levels
     // below would repeat this one until the scratch buffer is used up)
-    const bool longScan = tuning("scan.chunked", 1) && rowBytes <= 32768 && S >= 4 && chunkRows >= 4 &&
+    const bool longScan = twoReads && tuning("scan.chunked", 1) && rowBytes <= 32768 && S >= 4 && chunkRows >= 4 &&
                           plainBlocks < (int64_t)num_compute_units(s);
     if constexpr (sizeof(A) == 4) {
       // (a chunk and its neighbours' elements in its first and last pack must fit RunPrefetch: 32 KiB)

@@ -108,7 +108,9 @@ def test_gpu_long_scans_with_few_columns_run_in_chunks(thc, oracle, kind):
     rows, every = (150000, 1000) if kind == "double" else (40000, 2000)
     ones = np.ones((rows, 2), dtype)
     ones[::every] = 2
+    thc.set_tuning("scan.strided", 0)        # (products of integers would be read once)
     got = thc.Tensor(kind).cumprod(thc.Tensor.from_numpy(ones), 0)
+    thc.set_tuning("scan.strided", -1)
     assert thc.last_kernel() == "scan-chunked"
     want = np.cumprod(ones, axis=0, dtype=np.int64 if kind == "int" else np.float64)
     if kind == "half":
@@ -246,13 +248,17 @@ def test_gpu_long_scans_over_wide_rows_split_the_rows(thc, oracle, kind):
         ones = np.ones((9000, 320), dtype)
         ones[::700] = 2
         ones[1::1300, ::7] = -1
+        thc.set_tuning("scan.strided", 0)    # (products of integers would be read once)
         got = thc.Tensor(kind).cumprod(thc.Tensor.from_numpy(ones), 0)
+        thc.set_tuning("scan.strided", -1)
         assert thc.last_kernel() == "scan-cols-split"
         assert_bit_equal(got.numpy(), np.cumprod(ones.astype(np.float64), axis=0).astype(dtype))
     if kind in ("float", "double"):
         x = rng.standard_normal((50000, 520)).astype(dtype)
         dev, ref = thc.Tensor.from_numpy(x), oracle.View.of(x)
+        thc.set_tuning("scan.strided", 0)
         got = thc.Tensor(kind).cumsum(dev, 0).numpy().astype(np.float64)
+        thc.set_tuning("scan.strided", -1)
         assert thc.last_kernel() == "scan-cols-split"
         want = oracle.scan_dim(ref, 0).numpy().astype(np.float64) if kind == "float" else np.cumsum(x, axis=0)
         mass = np.cumsum(np.abs(x.astype(np.float64)), axis=0)
@@ -422,9 +428,8 @@ def test_gpu_rows_that_end_early_in_a_chunk(thc, kind):
 
 @pytest.mark.gpu
 def test_gpu_one_read_scans_of_two_threads_on_one_stream_stay_in_their_tensors(thc):
-    """Two host threads on the default stream: their launches interleave in the stream's scratch buffer (a scan's
-    words are cleared by one launch and used by the next). Sums are the caller's business then, but every chunk is
-    still drawn once: both threads' calls end, nothing outside the outputs is written, and the next scans are right."""
+    """Two host threads on the default stream: their launches interleave, and each scan is one launch whose words and ticket belong
+    to scans alone. Both threads' calls end, nothing outside the outputs is written, and the next scans are right."""
     rng = np.random.default_rng(37)
     guard, jobs = 64, []
     for kind, dtype, rows, n in (("float", np.float32, 3, 70001), ("long", np.int64, 2, 40003), ("byte", np.uint8, 1, 900001),
@@ -484,6 +489,7 @@ def test_gpu_one_read_scans_along_a_strided_dim(thc, kind):
             if form == 1 and inner < vec or form == 2 and inner * np.dtype(dtype).itemsize > 8192:
                 continue
             thc.set_tuning("scan.strided", form)
+            thc.set_tuning("scan.strided_two_reads", 0)      # (the forms of two reads have the same names)
             thc.set_tuning("scan.slab", 0)
             try:
                 strides = (n * inner, inner, 1)
@@ -495,6 +501,7 @@ def test_gpu_one_read_scans_along_a_strided_dim(thc, kind):
                 dev.cumsum(dev, 1)
             finally:
                 thc.set_tuning("scan.strided", -1)
+                thc.set_tuning("scan.strided_two_reads", 1)
                 thc.set_tuning("scan.slab", 1)
             assert_bit_equal(out.storage_numpy(), whole, "%s %s form %d" % (kind, shape, form))
             assert_bit_equal(dev.storage_numpy(), whole, "%s %s form %d in place" % (kind, shape, form))
@@ -633,11 +640,13 @@ def test_gpu_scans_of_many_slices_of_one_chunk_each_need_no_words(thc):
                         ((140000, 5, 7), "scan-chunked"), ((155000, 5, 7), "scan-chunked")):
         x = rng.integers(-9, 10, shape).astype(np.float64)      # (two words a total)
         thc.set_tuning("scan.slab", 0)
+        thc.set_tuning("scan.strided_two_reads", 0)
         try:
             got = thc.Tensor("double").cumsum(thc.Tensor.from_numpy(x), 1)
             assert thc.last_kernel() == name, (shape, thc.last_kernel())
         finally:
             thc.set_tuning("scan.slab", 1)
+            thc.set_tuning("scan.strided_two_reads", 1)
         assert_bit_equal(got.numpy(), np.cumsum(x, axis=1), "%s" % (shape,))
 
 
@@ -650,6 +659,7 @@ def test_gpu_strips_of_any_knob_value(thc, kind):
     vec = 16 // np.dtype(dtype).itemsize
     rng = np.random.default_rng(83)
     thc.set_tuning("scan.strided", 1)
+    thc.set_tuning("scan.strided_two_reads", 0)
     thc.set_tuning("scan.slab", 0)
     try:
         for inner in (vec, 3 * vec + 1, 40 * vec, 65 * vec - 1):
@@ -664,9 +674,11 @@ def test_gpu_strips_of_any_knob_value(thc, kind):
                     thc.set_tuning("scan.strips.threads", threads)
                     dev = thc.Tensor.from_storage(x, 1, shape, (1200 * inner, inner, 1), kind=kind)
                     dev.cumsum(dev, 1)
+                    assert thc.last_kernel() == "scan-cols-split", (inner, lanes, threads)
                     assert_bit_equal(dev.storage_numpy(), want, "%s %d lanes %d threads %d" % (kind, inner, lanes, threads))
     finally:
         thc.set_tuning("scan.strided", -1)
+        thc.set_tuning("scan.strided_two_reads", 1)
         thc.set_tuning("scan.slab", 1)
         thc.set_tuning("scan.strips.lanes", 0)
         thc.set_tuning("scan.strips.threads", 0)
