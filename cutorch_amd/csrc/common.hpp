@@ -124,27 +124,22 @@ hipStream_t current_stream(THCState* state);
 THCDeviceAllocator* state_allocator(THCState* state);  // THCGeneral.h.in:98-100
 int state_device(THCState* state);
 int num_compute_units(THCState* state);
-// Per-stream device scratch for partial results (THCGeneral.c:677-712):
-// `partials` for split reductions, a tail of zero-initialised arrival
-// counters (each kernel resets the ones it used), and a pinned host slot that
-// kernels can write the scalar result of an *all reduction into.
+// Per-stream device scratch (THCGeneral.c:677-712): `partials` for split reductions and chunked scans; a tail with the words by which
+// workgroups of one launch hand each other values (tagged, see FoldWords and scan_ticket.hpp: zero at first and never cleared after
+// that) and a scalar result; and a pinned host slot that kernels write the scalar result of an *all reduction into.
 constexpr size_t kScratchTailBytes = 64 * 1024;
-constexpr size_t kScratchCounters = (kScratchTailBytes - 256) / sizeof(unsigned);
-constexpr size_t kScanTicket = 2048;  // counters kScanTicket and the one behind it: a 64-bit word that deals out the chunks of one-read scans
+constexpr size_t kFoldWords = 4096;   // whole-tensor reductions: 32 KiB of words at the start of the tail, the ticket of one-read scans behind them
 constexpr size_t kScanWords = size_t(2) << 20;  // 16 MiB of words behind the tail, which only one-read scans write
-// Whole-tensor reductions: the partials that workgroups hand to the one that folds them, 32 KiB of words in the tail.
-constexpr size_t kFoldWordsAt = 16 * 1024, kFoldWords = 4096;   // (bytes into the tail; words)
 struct StreamScratch {
   void* partials;
   size_t partialBytes;
-  unsigned* counters;   // kScratchCounters arrival counters
   float* result;        // device slot for a scalar result (last 256 bytes of the tail)
   float* hostResult;    // pinned host memory ...
   float* hostResultDev; // ... and its device-side address
-  uint64_t* scanWord;   // what the workgroups of a one-read scan tell each other (zero at first, tagged values after that)
-  size_t scanWords;     // how many
+  uint64_t* foldWord;   // kFoldWords
   uint64_t* scanTicket;
-  uint64_t* foldWord;   // as scanWord, for whole-tensor reductions
+  uint64_t* scanWord;
+  size_t scanWords;     // how many
 };
 const StreamScratch& stream_scratch(THCState* state);
 // A number for a launch that hands partials over in foldWord: never 0, another for every launch on any stream until

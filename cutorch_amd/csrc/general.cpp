@@ -136,16 +136,14 @@ const StreamScratch& stream_scratch(THCState* s) {
                                             (hipStream_t_)st));  // scratch stays with hipMalloc
   sc.partials = p;
   sc.partialBytes = s->scratchBytes - kScratchTailBytes;
-  sc.counters = reinterpret_cast<unsigned*>(static_cast<char*>(p) + sc.partialBytes);
+  char* tail = static_cast<char*>(p) + sc.partialBytes;
+  static_assert(kFoldWords * sizeof(uint64_t) + 256 <= kScratchTailBytes - 256, "the tail's parts lie behind each other");
+  sc.foldWord = reinterpret_cast<uint64_t*>(tail);
+  sc.scanTicket = sc.foldWord + kFoldWords;
   sc.result = reinterpret_cast<float*>(static_cast<char*>(p) + s->scratchBytes - 256);
   sc.scanWord = reinterpret_cast<uint64_t*>(static_cast<char*>(p) + s->scratchBytes);
   sc.scanWords = kScanWords;
-  static_assert(kFoldWordsAt + kFoldWords * sizeof(uint64_t) <= kScratchTailBytes - 256 && (kScanTicket + 2) * sizeof(unsigned) <= kFoldWordsAt,
-                "the tail's parts lie behind each other");
-  sc.foldWord = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(sc.counters) + kFoldWordsAt);
-  sc.scanTicket = reinterpret_cast<uint64_t*>(sc.counters + kScanTicket);
-  // Arrival counters start at zero and every kernel that uses one resets it; the words of one-read scans lie behind them.
-  THC_CHECK(hipMemsetAsync(sc.counters, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
+  THC_CHECK(hipMemsetAsync(tail, 0, kScratchTailBytes + kScanWords * sizeof(uint64_t), st));
   const uint32_t firstTag = (uint32_t)tuning("scan.first_tag", 1);
   const uint64_t firstScan = scan_counter(firstTag ? firstTag : 1);
   THC_CHECK(hipMemcpyAsync(sc.scanTicket, &firstScan, sizeof(firstScan), hipMemcpyHostToDevice, st));
