@@ -2709,6 +2709,30 @@ struct ColsPlan {
 // Which packs a column kernel may read: only whole aligned ones, any, or any under the (value, index) kernel's rule.
 enum class ColPacks { Whole, Loose, Index };
 
+// Where packs at element-aligned addresses are faster than one element a lane: `outer` slices of R rows of C >= 64 columns.
+// A row of packs takes a half to an eighth of the lanes, so the other lanes become further thread rows, which a slice
+// of few rows leaves without a batch of 8 rows, or idle. us along the middle dim of a window, one by one and in packs:
+// * 4- and 8-byte elements: from 8 rows a thread row on (fp32 sum of 2048 x 200 x 64 20.9 / 20.1, 3971 x 33 x 200 20.7 / 18.9; fewer: 102400
+//   x 4 x 64 105 / 147, max 138 / 333; 25013 x 8 x 131 32 / 44; double 8192 x 8 x 200 24.6 / 34.0), and where a row of single
+//   elements takes more than a workgroup's lanes (50803 x 2 x 258 128 / 68).
+// * 4-byte elements in slices so few that one by one their rows are split over two launches: from 2.7 rows a thread on (sum of
+//   1092 x 24 x 200 14.8 / 8.6). 8-byte ones of 129 to 256 columns: below 8 rows, which fill no batch one by one
+//   either (var of 20103 x 4 x 163 70 / 54).
+// * 2-byte elements, whose packs leave the most thread rows: wide rows (R < 8: sum of 25450 x 4 x 515 128 / 108, but 65536 x 4 x 200
+//   112 / 272; R <= 16: 2906 x 12 x 1503 44 / 32), slices that would be split (819 x 64 x 200 21.5 / 11.2) and few long ones, which (value,
+//   index) takes only where they are very long (8191 x 8193 42 / 48; 594 x 144 x 967 39 / 53).
+inline bool loose_col_packs(size_t elem, int64_t outer, int64_t R, int64_t C, int64_t cus, bool index) {
+  const int64_t vec = 16 / (int64_t)elem, packs = (C + vec - 1) / vec;
+  const bool split = outer * ((C + kBlock - 1) / kBlock) < 8 * cus && R * packs >= 680;   // (2.7 rows of packs a thread)
+  if (elem == 2) {
+    if (R > 64) return outer < 64 && (!index || R >= 16384);
+    return (R < 8 && C > 512) || (R <= 16 && C > 1024) || (R > 24 && split);
+  }
+  const int64_t threadRows = std::max<int64_t>(1, kBlock / (int64_t)pow2_ceil((uint64_t)packs));
+  if (C > kBlock || R >= 8 * threadRows) return true;
+  return elem == 4 ? split && packs > 16 : R < 8 && C > kBlock / 2;
+}
+
 // cols: reduced dim strided, innermost joint dim has unit input stride.
 template <typename T, typename I>
 ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t partialElemBytes,
@@ -2720,15 +2744,15 @@ ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t p
   const int nd = g.in.dims;
   const int64_t C = g.in.size[nd - 1];
   // Rows off the 16-byte grid, or of no whole number of packs: packs at element-aligned addresses, the last one moved back to end
-  // with the row, from 16 MiB on; one element a lane below, where the wider strips and the more workgroups that go with it win
-  // (us one by one and in packs: 319807 x 394 along dim 0 fp32 sum 203 / 86, max 147 / 99, half sum 190 / 45; 24836 x 986 fp32 var 41 / 22;
-  // 200 x 33 x 1001 fp32 14.6 / 6.8; but 1688 x 518 max 9.2 / 12.8). 2-byte elements: few long slices or few rows (594 x
-  // 144 x 967 half 39 / 53), (value, index) only where the slices are long (8191 x 8193 42 / 48). Bytes never (sum of 24836 x 986
-  // 14 / 20: 16-byte loads at odd addresses).
+  // with the row, from 16 MiB on and where loose_col_packs below has them ahead; one element a lane else, where the wider strips
+  // and the more workgroups that go with it win (us one by one and in packs: 319807 x 394 along dim 0 fp32 sum 203 / 86, max 147 / 99,
+  // half sum 190 / 45; 24836 x 986 fp32 var 41 / 22; 200 x 33 x 1001 fp32 14.6 / 6.8; but 1688 x 518 max 9.2 / 12.8). Bytes never (sum
+  // of 24836 x 986 14 / 20: 16-byte loads at odd addresses).
   bool vec = aligned16(in) && C % VEC == 0 && g.sR % VEC == 0;
   for (int d = 0; d < nd - 1 && vec; ++d) vec = g.in.stride[d] % VEC == 0;
-  if (!vec && packs != ColPacks::Whole && C >= 64 && sizeof(T) > 1 && g.outElems * g.R * (int64_t)sizeof(T) >= tuning("reduce.cols.loose_bytes", 16 << 20))
-    vec = sizeof(T) >= 4 || g.R <= 64 || (g.outElems / C < 64 && (packs != ColPacks::Index || g.R >= 16384));
+  const int64_t looseFrom = tuning("reduce.cols.loose_bytes", 16 << 20);   // (0: wherever the kernels can read them)
+  if (!vec && packs != ColPacks::Whole && C >= 64 && sizeof(T) > 1 && g.outElems * g.R * (int64_t)sizeof(T) >= looseFrom)
+    vec = looseFrom == 0 || loose_col_packs(sizeof(T), g.outElems / C, g.R, C, num_compute_units(s), packs == ColPacks::Index);
   const int pack = vec ? VEC : 1;
   const int64_t target = tuning("reduce.cols.target_blocks", (int64_t)num_compute_units(s) * tuning(perCuKey, perCuDefault));
   const int64_t outer = g.outElems / C;

@@ -909,6 +909,37 @@ def test_packs_at_element_aligned_addresses(thc, kind):
         thc.set_tuning("reduce.cols.loose_bytes", 16 << 20)
 
 
+@pytest.mark.parametrize("kind,shape,packs", [
+    # a slice's rows fill a batch of 8 in every thread row, or not
+    ("float", (22000, 3, 64), False), ("float", (400, 200, 67), True), ("float", (3500, 12, 101), False), ("float", (2100, 31, 131), False),
+    ("float", (1100, 24, 200), True), ("float", (2600, 24, 200), False), ("float", (8200, 2, 258), True),
+    ("int", (10300, 8, 64), False), ("int", (2500, 31, 70), False),
+    ("double", (6500, 5, 65), False), ("double", (1600, 8, 200), False), ("double", (3200, 4, 200), True), ("double", (1100, 16, 131), True),
+    ("half", (33000, 4, 64), False), ("half", (10500, 4, 200), False), ("half", (4100, 4, 515), True), ("half", (520, 16, 1030), True),
+    ("half", (820, 64, 200), True), ("half", (4200, 32, 67), False)])
+def test_slices_of_few_rows_are_not_read_as_packs(thc, kind, shape, packs):
+    """Windows off the 16-byte grid, reduced along the middle dim: packs take a part of the lanes that single elements take, and the
+    thread rows that the other lanes become have nothing to do in slices of few rows (102400 x 8 x 64 halves took 4 times as long)."""
+    outer, n, cols = shape
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64, "int": np.int32}[kind]
+    rng = np.random.default_rng(97)
+    x = rng.integers(-3, 4, (outer, n, cols + 3)).astype(dtype)
+    dev = thc.Tensor.from_numpy(x).narrow(2, 1, cols)
+    host = x[:, :, 1:1 + cols]
+    got = thc.Tensor(kind).sum(dev, 1)
+    name = thc.last_kernel()
+    assert ("scalar" not in name) == packs, (shape, name)
+    assert_bit_equal(got.numpy(), host.sum(axis=1, keepdims=True, dtype=np.int64).astype(dtype), "sum %s" % (shape,))
+    vals, idx = thc.Tensor(kind), thc.Tensor("long")
+    vals.max(idx, dev, 1)
+    assert_bit_equal(vals.numpy(), host.max(axis=1, keepdims=True), "max %s" % (shape,))
+    assert np.array_equal(idx.numpy(), np.expand_dims(host.argmax(axis=1), 1) + 1), shape
+    if kind != "int":
+        var = thc.Tensor(kind).var(dev, 1).numpy().astype(np.float64)
+        want = host.astype(np.float64).var(axis=1, ddof=1, keepdims=True)
+        assert np.allclose(var, want, rtol={"float": 1e-5, "half": 2e-3, "double": 1e-12}[kind], atol=1e-7), shape   # (half: 2^-24 steps)
+
+
 @pytest.mark.parametrize("kind", ["float", "half", "double"])
 def test_var_of_small_slices_with_few_columns(thc, kind):
     """Threads that share a column's rows: columns one below and above what leaves several threads each, rows around the bands of 8."""
