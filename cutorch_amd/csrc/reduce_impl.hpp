@@ -1784,13 +1784,14 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
 // reductions, workgroup partials are merged with the pairwise update of Chan,
 // Golub & LeVeque. Same geometry as reduce_cols_kernel. Partial planes hold
 // (mean, M2) per output: partial[(s * 2 + {0, 1}) * outElems + out].
-template <typename T, typename I, int VEC>
+// FOLD: the second launch, which folds the planes. A kernel of its own: with its batches in the same one, chosen at run time, their
+// registers cost the first launch a fifth (614400 x 2 x 64 fp32 899 us, 744 without them).
+template <typename T, typename I, int VEC, bool FOLD>
 __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ in,
                                                           T* __restrict__ out,
                                                           typename Acc<T>::type* __restrict__ partial,
                                                           ColsArgs<I> a, I totalBlocks,
-                                                          typename Acc<T>::type div, bool wantStd,
-                                                          bool foldPass) {
+                                                          typename Acc<T>::type div, bool wantStd) {
   using P = Pack<T, VEC>;
   using A = typename Acc<T>::type;
   __shared__ A smean[kBlock * VEC];
@@ -1800,7 +1801,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
   const uint32_t tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   for (I b = blockIdx.x; b < totalBlocks; b += gridDim.x) {
     I group = b, s = 0, rest, ct;
-    if (!foldPass) a.S.divmod(b, group, s);
+    if (!FOLD) a.S.divmod(b, group, s);
     a.colTiles.divmod(group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
@@ -1813,7 +1814,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
       mean[e] = (A)0;
       m2[e] = (A)0;
     }
-    if (foldPass) {
+    if constexpr (FOLD) {
       if (live) {
         const A* plane = partial + rest * a.C + col;
         constexpr int UF = 4;  // planes fetched per batch
@@ -1914,7 +1915,7 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
       __syncthreads();
     }
     if (ty == 0 && live) {
-      if (foldPass || a.S.d == 1) {
+      if (FOLD || a.S.d == 1) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           const A v = sm2[tx * VEC + e] / div;
@@ -3035,7 +3036,7 @@ void run_cols(THCState* s, const ReduceGeom& g, const T* in, T* out, Epi<typenam
   A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
   const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
   int64_t groups = 0;
-    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
+  const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
   hipStream_t st = current_stream(s);
   for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
     const bool fold = pass == 1;
@@ -3489,18 +3490,21 @@ bool reduce_var_cols_type(THCState* s, const ReduceGeom& g, const void* in_, voi
       A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
       const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
       int64_t groups = 0;
-    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
+      const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
       hipStream_t st = current_stream(s);
       for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
         const bool fold = pass == 1;
         const int gr = fold ? (int)groups : grid;
         const I tb = fold ? (I)groups : (I)p.totalBlocks;
-        if (p.vec && !fold)
-          hipLaunchKernelGGL((var_cols_kernel<T, I, VEC>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
-                             (T*)out_, scratch, p.a, tb, (A)div, wantStd, fold);
+        if (fold)
+          hipLaunchKernelGGL((var_cols_kernel<T, I, 1, true>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
+                             (T*)out_, scratch, folds, tb, (A)div, wantStd);
+        else if (p.vec)
+          hipLaunchKernelGGL((var_cols_kernel<T, I, VEC, false>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
+                             (T*)out_, scratch, p.a, tb, (A)div, wantStd);
         else
-          hipLaunchKernelGGL((var_cols_kernel<T, I, 1>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
-                             (T*)out_, scratch, fold ? folds : p.a, tb, (A)div, wantStd, fold);
+          hipLaunchKernelGGL((var_cols_kernel<T, I, 1, false>), dim3(gr), dim3(kBlock), 0, st, (const T*)in_,
+                             (T*)out_, scratch, p.a, tb, (A)div, wantStd);
       }
       note_kernel(split ? "var-cols-split" : "var-cols");
     };
