@@ -2835,15 +2835,18 @@ ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t p
 }
 
 // The second launch of a split column reduction: S planes of accumulators are folded column by column, whatever packs the
-// input was read in. As many thread rows as planes up to 16 (a thread walks 8 planes a batch), so 16 columns and
-// more to a workgroup: with the first launch's geometry one workgroup folded 256 planes of 415 half columns (38 us of 49).
+// input was read in. A thread per column (it walks 8 planes a batch) while that fills the chip; for fewer outputs more
+// thread rows, down to 16 columns a workgroup: with the first launch's geometry one workgroup folded 256 planes of 415 half
+// columns (38 us of 49), with 16 columns for any number of outputs 3 planes of 209600 took 5 us more.
 template <typename I>
-ColsArgs<I> fold_geometry(const ColsArgs<I>& a, int64_t outElems, int64_t& groups) {
+ColsArgs<I> fold_geometry(const ColsArgs<I>& a, int64_t outElems, int64_t cus, int64_t& groups) {
   ColsArgs<I> f = a;
-  f.TX = std::max<uint32_t>(16, kBlock / (uint32_t)pow2_ceil((uint64_t)std::min<int64_t>((int64_t)a.S.d, 16)));
-  const int64_t C = (int64_t)a.C, tiles = (C + f.TX - 1) / f.TX;
-  f.colTiles.set((uint64_t)tiles);
-  groups = outElems / C * tiles;
+  const int64_t C = (int64_t)a.C, outer = outElems / C, planes = (int64_t)a.S.d;
+  const auto tiles = [&]() { return (C + f.TX - 1) / f.TX; };
+  f.TX = std::min<uint32_t>(kBlock, std::max<uint32_t>(16, pow2_ceil((uint64_t)C)));
+  while (f.TX > 16 && kBlock / f.TX < planes && outer * tiles() < 2 * cus) f.TX >>= 1;
+  f.colTiles.set((uint64_t)tiles());
+  groups = outer * tiles();
   return f;
 }
 
@@ -3036,7 +3039,7 @@ void run_cols(THCState* s, const ReduceGeom& g, const T* in, T* out, Epi<typenam
   A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
   const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
   int64_t groups = 0;
-  const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
+  const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, num_compute_units(s), groups);
   hipStream_t st = current_stream(s);
   for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
     const bool fold = pass == 1;
@@ -3231,7 +3234,7 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
     }
     const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
     int64_t groups = 0;
-    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
+    const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, num_compute_units(s), groups);
     for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
       const bool fold = pass == 1;
       const int gr = fold ? (int)groups : grid;
@@ -3490,7 +3493,7 @@ bool reduce_var_cols_type(THCState* s, const ReduceGeom& g, const void* in_, voi
       A* scratch = split ? (A*)scratch_space(s, nullptr) : nullptr;
       const int grid = (int)std::min<int64_t>(p.totalBlocks, 1 << 30);
       int64_t groups = 0;
-      const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, groups);
+      const ColsArgs<I> folds = fold_geometry(p.a, g.outElems, num_compute_units(s), groups);
       hipStream_t st = current_stream(s);
       for (int pass = 0; pass < (split ? 2 : 1); ++pass) {
         const bool fold = pass == 1;
