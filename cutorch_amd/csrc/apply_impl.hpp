@@ -328,6 +328,41 @@ struct IndexedArgs {
   Divisor<I> size[kSizes][kArgDims<I>];
   I stride[kMaxOps][kArgDims<I>];     // in elements; pre-multiplied by VEC in the packed dim
   int ntStore;                        // packs of the output go out with the streaming hint
+  int narrow;                         // I of 64 bits: the divisors are 32-bit ones, and so are all offsets
+  // Offsets of N operands from k + FIRST on, and the index along the innermost dim, at linear index `lin` by the sizes of set k.
+  template <int FIRST, int N, typename U, int M>
+  __device__ __forceinline__ void chain(int k, U lin, U (&off)[M], U& inner) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) off[i] = 0;
+    const int last = dims[k] - 1;
+    inner = 0;
+    for (int d = last; d > 0; --d) {
+      U q, r;
+      size[k][d].divmod(lin, q, r);
+      lin = q;
+      if (d == last) inner = r;
+#pragma unroll
+      for (int i = 0; i < N; ++i) off[i] += r * (U)stride[FIRST + k + i][d];
+    }
+    if (last == 0) inner = lin;
+#pragma unroll
+    for (int i = 0; i < N; ++i) off[i] += lin * (U)stride[FIRST + k + i][0];
+  }
+  template <int FIRST, int N, int M>
+  __device__ __forceinline__ void offsets(int k, I lin, I (&off)[M], I& inner) const {
+    if constexpr (sizeof(I) == 8) {
+      // us in the 64-bit chain and this way: REPLACE_ME
+      if (narrow) {
+        uint32_t o[M], c;
+        chain<FIRST, N>(k, (uint32_t)lin, o, c);
+#pragma unroll
+        for (int i = 0; i < N; ++i) off[i] = o[i];
+        inner = c;
+        return;
+      }
+    }
+    chain<FIRST, N>(k, lin, off, inner);
+  }
 };
 
 // JOINT = all operands share sizes (one division chain); VEC packs along the
@@ -342,33 +377,15 @@ __global__ __launch_bounds__(kBlock) void apply_indexed_kernel(TOut* out, const 
   constexpr int NOPS = Op::NIN + 1;
   const I step = (I)gridDim.x * kBlock;
   for (I lin = (I)blockIdx.x * kBlock + threadIdx.x; lin < total; lin += step) {
-    I off[kMaxOps] = {0, 0, 0, 0};
-    I inner = 0;  // JOINT: this pack's index along the innermost dim
-    if (JOINT) {
-      I rest = lin;
-      const int last = args.dims[0] - 1;
-      for (int d = last; d > 0; --d) {
-        I q, r;
-        args.size[0][d].divmod(rest, q, r);
-        rest = q;
-        if (VEC > 1 && d == last) inner = r;
-#pragma unroll
-        for (int k = 0; k < NOPS; ++k) off[k] += r * args.stride[k][d];
-      }
-      if (VEC > 1 && last == 0) inner = rest;
-#pragma unroll
-      for (int k = 0; k < NOPS; ++k) off[k] += rest * args.stride[k][0];
+    I off[kMaxOps] = {0, 0, 0, 0}, inner = 0;  // inner, JOINT: this pack's index along the innermost dim
+    if constexpr (JOINT) {
+      args.template offsets<0, NOPS>(0, lin, off, inner);
     } else {
 #pragma unroll
       for (int k = 0; k < NOPS; ++k) {
-        I rest = lin;
-        for (int d = args.dims[k] - 1; d > 0; --d) {
-          I q, r;
-          args.size[k][d].divmod(rest, q, r);
-          rest = q;
-          off[k] += r * args.stride[k][d];
-        }
-        off[k] += rest * args.stride[k][0];
+        I own[1];
+        args.template offsets<0, 1>(k, lin, own, inner);
+        off[k] = own[0];
       }
     }
     if constexpr (VEC == 1) {
@@ -440,23 +457,7 @@ __global__ __launch_bounds__(kBlock) void apply_flatmix_kernel(TOut* out, const 
   const I step = (I)gridDim.x * kBlock;
   const I lastSize = args.size[0][nd - 1].d;
   // offsets of the gathered inputs at flat index `lin`; c = innermost coordinate
-  auto locate = [&](I lin, I (&off)[3], I& c) {
-#pragma unroll
-    for (int k = 0; k < NIN; ++k) off[k] = 0;
-    I rest = lin;
-    c = 0;
-    for (int d = nd - 1; d > 0; --d) {
-      I q, r;
-      args.size[0][d].divmod(rest, q, r);
-      rest = q;
-      if (d == nd - 1) c = r;
-#pragma unroll
-      for (int k = 0; k < NIN; ++k) off[k] += r * args.stride[k + 1][d];
-    }
-    if (nd == 1) c = rest;
-#pragma unroll
-    for (int k = 0; k < NIN; ++k) off[k] += rest * args.stride[k + 1][0];
-  };
+  auto locate = [&](I lin, I (&off)[3], I& c) { args.template offsets<1, NIN>(0, lin, off, c); };
   with_fixed_code(op, [&](auto f) {
     // pack index `packs` stands for the n % VEC elements after the last whole pack
     for (I pk = (I)blockIdx.x * kBlock + threadIdx.x; pk <= packs; pk += step) {
@@ -1262,6 +1263,8 @@ template <typename T, typename Op, typename I, bool JOINT, typename TOut = T>
 void launch_indexed(THCState* s, const Plan& pl, Op op) {
   constexpr int VEC = pack_elems<T, TOut>();
   IndexedArgs<I, JOINT> args{};
+  args.narrow = sizeof(I) == 8;
+  for (int k = 0; k < pl.nops && args.narrow; ++k) args.narrow = narrow_chain(pl.lay[k]);
   const bool aligned = JOINT && indexed_can_pack<T, TOut>(pl);
   const bool vec = aligned || (JOINT && indexed_can_pack_unaligned<T, TOut>(pl));
   const int pack = vec ? VEC : 1;
@@ -1277,7 +1280,7 @@ void launch_indexed(THCState* s, const Plan& pl, Op op) {
         sz = (sz + pack - 1) / pack;
         sd *= pack;
       }
-      if (own) args.size[k][d].set((uint64_t)sz);
+      if (own) set_divisor(args.size[k][d], args.narrow, sz);
       args.stride[k][d] = (I)sd;
       if (k == 0) total *= sz;
     }
@@ -1626,9 +1629,11 @@ bool launch_flatmix(THCState* s, const Plan& pl, Op op) {
   }
   if (gathered == 0) return false;
   IndexedArgs<I, true> args{};
+  args.narrow = sizeof(I) == 8;
+  for (int k = 0; k < pl.nops && args.narrow; ++k) args.narrow = narrow_chain(pl.lay[k]);
   args.dims[0] = nd;
   for (int d = 0; d < nd; ++d) {
-    args.size[0][d].set((uint64_t)pl.lay[0].size[d]);
+    set_divisor(args.size[0][d], args.narrow, pl.lay[0].size[d]);
     for (int k = 0; k < pl.nops; ++k) args.stride[k][d] = (I)pl.lay[k].stride[d];
   }
   args.ntStore = streaming_store("apply.indexed.nt_store", pl.numel * (int64_t)sizeof(TOut)) ? 1 : 0;
@@ -1682,8 +1687,9 @@ bool run_plan(THCState* s, Plan& pl, bool sameShape, Op op, bool decline = false
     // 27.8, 18.1; 8192 x 8192 103.7, 90.7; 8191 x 8193 136, 108 (tanh 146, 107). Except large tensors whose columns the tiled
     // kernels fuse with the next dim's where the tiles here stay emptier than 55 %: 1001 x 1003 x 129 269, 448;
     // 156 x 704 x 41 15.1, 16.0 (301 x 301 x 301, 81 %, 61, 52; 65 x 33 x 47 12.9, 4.9); and large tensors of so few rows that
-    // three quarters of its 64-row tiles would be computed in vain: tanh of 16 x 100000 7.9, 10.3. Whole
-    // packs below 2^15 elements stay as well, although 352 x 256 gains (9.4, 4.2): a test of kernel names holds 136 x 200 there.
+    // three quarters of its 64-row tiles would be computed in vain: tanh of 16 x 100000 7.9, 10.3. Floats
+    // in whole packs below 2^15 elements stay as well, for no gain: 8 x 8 4.2, 4.0; 64 x 64 8.8, 4.5; 136 x 200 8.9, 4.8; 128 x 252 9.1, 4.7
+    // (352 x 256, above the line, 9.4, 4.2). Tests of kernel names hold such shapes there.
     if constexpr (TILED && std::is_same<Op, OpMath1>::value && std::is_same<T, TOut>::value) {
       int p, q, staged[kMaxOps] = {0, 0, 0, 0};
       bool lds = tile_plan(pl, p, q, staged);

@@ -168,6 +168,14 @@ inline bool streaming_store(const char* knob, int64_t bytes) {
   return k >= 0 ? k != 0 : bytes >= (int64_t(64) << 20);
 }
 bool force_64bit_index();
+// All offsets of the layout fit 32 bits. Kernels with 64-bit offsets get such layouts too: those of more dims than the 32-bit kernels'
+// arguments have room for.
+inline bool narrow_chain(const Layout& l) {
+  if (force_64bit_index() || !fits_32bit(l)) return false;
+  for (int d = 0; d < l.dims; ++d)
+    if (l.stride[d] < 0) return false;
+  return true;
+}
 
 // --------------------------------------------------------- storage/tensor --
 AnyStorage* storage_new(THCState* s, DType dt, ptrdiff_t size);

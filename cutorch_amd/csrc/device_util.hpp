@@ -187,7 +187,10 @@ __device__ __forceinline__ D convert_value(S x) {
 // Dims that a kernel's arguments have room for. Arguments are written to device memory by the host, one write per launch that
 // the host waits for: a kernel of 16 bytes of arguments is launched in 2.4 us, of 256 bytes in 2.6, 1 KiB 3.2, 2 KiB 3.4, so the
 // 32-bit kernels carry what nearly all layouts need after their dims have been merged, and those with more dims take the
-// 64-bit kernels. (Arguments of the strided kernel 1.7 KB -> 190 bytes, of the row reductions 0.6 KB -> 170.)
+// 64-bit kernels, which go through their dims in 32 bits where the offsets fit. (Arguments of the strided kernel 1.7 KB -> 190 bytes,
+// of the row reductions 0.6 KB -> 170.) us on fp32 windows whose dims do not merge, with 32-bit kernels that have room for them, with
+// 64-bit chains, and with 32-bit chains in the 64-bit kernels: copy of 13 dims 10.7, 19.8, 11.8; sum over the middle one of 9 dims 29, 65,
+// 37, of 8 dims 55, 135, 73; over the last one of 10 8.4, 12.1, 10.2; exp of 7 reversed dims 28.1, 37.7, 29.7.
 template <typename I>
 constexpr int kArgDims = sizeof(I) == 4 ? 6 : 25;
 
@@ -260,7 +263,45 @@ struct Divisor<uint64_t> {
     q = one ? n : (((n - t) >> 1) + t) >> s;
     r = n - q * d;
   }
+  // The same fields as the 32-bit divisor's, for n < 2^31: a chain of these in a kernel with 64-bit offsets.
+  __host__ void set_narrow(uint64_t div) {
+    Divisor<uint32_t> n;
+    n.set(div);
+    d = n.d;
+    m = n.m;
+    s = n.s;
+    one = 0;
+  }
+  __device__ __forceinline__ void divmod(uint32_t n, uint32_t& q, uint32_t& r) const {
+    q = (__umulhi(n, (uint32_t)m) + n) >> s;
+    r = n - q * (uint32_t)d;
+  }
 };
+
+// By a divisor that was set in 32 bits if `narrow` (I of 64 bits only).
+template <typename I>
+__device__ __forceinline__ void divide(const Divisor<I>& by, bool narrow, I n, I& q, I& r) {
+  if constexpr (sizeof(I) == 8) {
+    if (narrow) {
+      uint32_t q32, r32;
+      by.divmod((uint32_t)n, q32, r32);
+      q = q32;
+      r = r32;
+      return;
+    }
+  }
+  by.divmod(n, q, r);
+}
+template <typename I>
+__host__ inline void set_divisor(Divisor<I>& by, bool narrow, int64_t n) {
+  if constexpr (sizeof(I) == 8) {
+    if (narrow) {
+      by.set_narrow((uint64_t)n);
+      return;
+    }
+  }
+  by.set((uint64_t)n);
+}
 
 // Streams `count` elements starting at `first` (any alignment) into LDS as
 // aligned 16-byte packs, U loads in flight per lane: the first pack starts at

@@ -264,20 +264,34 @@ struct PairOrder {
 template <typename I>
 struct OuterArgs {
   int dims;
+  int narrow;   // I of 64 bits: the divisors, those of the workgroups' and rows' numbers too, are 32-bit ones, and so are all offsets
   Divisor<I> size[kArgDims<I>];
   I inStride[kArgDims<I>];
   I outStride[kArgDims<I>];
-  __device__ __forceinline__ void offsets(I lin, I& inOff, I& outOff) const {
+  template <typename N>
+  __device__ __forceinline__ void chain(N lin, N& inOff, N& outOff) const {
     inOff = 0;
     outOff = 0;
     for (int d = dims - 1; d > 0; --d) {
-      I r;
+      N r;
       size[d].divmod(lin, lin, r);
-      inOff += r * inStride[d];
-      outOff += r * outStride[d];
+      inOff += r * (N)inStride[d];
+      outOff += r * (N)outStride[d];
     }
-    inOff += lin * inStride[0];
-    outOff += lin * outStride[0];
+    inOff += lin * (N)inStride[0];
+    outOff += lin * (N)outStride[0];
+  }
+  __device__ __forceinline__ void offsets(I lin, I& inOff, I& outOff) const {
+    if constexpr (sizeof(I) == 8) {
+      if (narrow) {
+        uint32_t i, o;
+        chain((uint32_t)lin, i, o);
+        inOff = i;
+        outOff = o;
+        return;
+      }
+    }
+    chain(lin, inOff, outOff);
   }
 };
 
@@ -309,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
     I outOff = 0;
     if (active) {
       I row, s, inOff;
-      S.divmod(vr, row, s);
+      divide(S, oa.narrow, vr, row, s);
       oa.offsets(row, inOff, outOff);
       const I begin = s * chunk;
       const I stop = min(R, begin + chunk);
@@ -399,7 +413,7 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_index_kernel(
     I outOff = 0, idxOff = 0;
     if (active) {
       I row, sp, inOff, unused;
-      S.divmod(vr, row, sp);
+      divide(S, oa.narrow, vr, row, sp);
       oa.offsets(row, inOff, outOff);
       oaIdx.offsets(row, unused, idxOff);
       const T* src = in + inOff;
@@ -1698,8 +1712,8 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
   };
   for (I b = blockIdx.x; b < totalBlocks; b += gridDim.x) {
     I group = b, s = 0, rest, ct;
-    if (!foldPass) a.S.divmod(b, group, s);
-    a.colTiles.divmod(group, rest, ct);
+    if (!foldPass) divide(a.S, a.oa.narrow, b, group, s);
+    divide(a.colTiles, a.oa.narrow, group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
     const I at0 = (ct * TX + tx) * VEC;
@@ -1785,7 +1799,7 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_kernel(const TIn* __restri
 // Golub & LeVeque. Same geometry as reduce_cols_kernel. Partial planes hold
 // (mean, M2) per output: partial[(s * 2 + {0, 1}) * outElems + out].
 // FOLD: the second launch, which folds the planes. A kernel of its own: with its batches in the same one, chosen at run time, their
-// registers cost the first launch a fifth (614400 x 2 x 64 fp32 899 us, 744 without them).
+// registers cost the first launch a fifth (614400 x 2 x 64 fp32 899 us, 609 without them).
 template <typename T, typename I, int VEC, bool FOLD>
 __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ in,
                                                           T* __restrict__ out,
@@ -1801,8 +1815,8 @@ __global__ __launch_bounds__(kBlock) void var_cols_kernel(const T* __restrict__ 
   const uint32_t tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   for (I b = blockIdx.x; b < totalBlocks; b += gridDim.x) {
     I group = b, s = 0, rest, ct;
-    if (!FOLD) a.S.divmod(b, group, s);
-    a.colTiles.divmod(group, rest, ct);
+    if (!FOLD) divide(a.S, a.oa.narrow, b, group, s);
+    divide(a.colTiles, a.oa.narrow, group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
     const I at0 = (ct * TX + tx) * VEC;
@@ -2127,8 +2141,8 @@ __global__ __launch_bounds__(kBlock) void reduce_cols_index_kernel(
   };
   for (I b = blockIdx.x; b < totalBlocks; b += gridDim.x) {
     I group = b, s = 0, rest, ct;
-    if (!foldPass) a.S.divmod(b, group, s);
-    a.colTiles.divmod(group, rest, ct);
+    if (!foldPass) divide(a.S, a.oa.narrow, b, group, s);
+    divide(a.colTiles, a.oa.narrow, group, rest, ct);
     I inOff, outOff;
     a.oa.offsets(rest, inOff, outOff);
     const I at0 = (ct * TX + tx) * VEC;
@@ -2537,8 +2551,9 @@ OuterArgs<I> make_outer(const Layout& in, const Layout& out, int dims) {
     oa.outStride[0] = 0;
     return oa;
   }
+  if constexpr (sizeof(I) == 8) oa.narrow = narrow_chain(in) && narrow_chain(out) ? 1 : 0;
   for (int d = 0; d < dims; ++d) {
-    oa.size[d].set((uint64_t)in.size[d]);
+    set_divisor(oa.size[d], oa.narrow, in.size[d]);
     oa.inStride[d] = (I)in.stride[d];
     oa.outStride[d] = (I)out.stride[d];
   }
@@ -2564,7 +2579,7 @@ void launch_rows_pass(THCState* s, const TIn* in, TOut* out, typename F::A* part
   const int64_t blocks = (numRows * S + groups - 1) / groups;
   const int grid = capped_grid(s, blocks, "reduce.rows.blocks_per_cu", 64);
   Divisor<I> Sd;
-  Sd.set((uint64_t)S);
+  set_divisor(Sd, oa.narrow, S);
   hipStream_t st = current_stream(s);
   if (vec)
     hipLaunchKernelGGL((reduce_rows_kernel<TIn, TOut, F, I, VEC, FIRST>), dim3(grid), dim3(kBlock),
@@ -2826,8 +2841,8 @@ ColsPlan<I> plan_cols(THCState* s, const ReduceGeom& g, const void* in, size_t p
   p.a.sR = (I)g.sR;
   p.a.outInner = (I)g.out.stride[nd - 1];
   p.a.chunkR = (I)chunk;
-  p.a.S.set((uint64_t)S);
-  p.a.colTiles.set((uint64_t)colTiles);
+  set_divisor(p.a.S, p.a.oa.narrow, S);
+  set_divisor(p.a.colTiles, p.a.oa.narrow, colTiles);
   p.a.outElems = (I)g.outElems;
   p.a.TX = TX;
   p.totalBlocks = base * S;
@@ -2845,7 +2860,7 @@ ColsArgs<I> fold_geometry(const ColsArgs<I>& a, int64_t outElems, int64_t cus, i
   const auto tiles = [&]() { return (C + f.TX - 1) / f.TX; };
   f.TX = std::min<uint32_t>(kBlock, std::max<uint32_t>(16, pow2_ceil((uint64_t)C)));
   while (f.TX > 16 && kBlock / f.TX < planes && outer * tiles() < 2 * cus) f.TX >>= 1;
-  f.colTiles.set((uint64_t)tiles());
+  set_divisor(f.colTiles, f.oa.narrow, tiles());
   groups = outer * tiles();
   return f;
 }
@@ -3128,7 +3143,7 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
     const int64_t groups = kBlock / G;
     const int grid = capped_grid(s, (rows * S + groups - 1) / groups, "reduce.rows.blocks_per_cu", 64);
     Divisor<I> Sd;
-    Sd.set((uint64_t)S);
+    set_divisor(Sd, oa.narrow, S);
     if (vec)
       hipLaunchKernelGGL((reduce_rows_index_kernel<T, I, VEC, IS_MAX>), dim3(grid), dim3(kBlock), 0,
                          st, in, outV, outI, partV, partI, oa, oaIdx, (I)rows, (I)g.R, (I)1, Sd,
