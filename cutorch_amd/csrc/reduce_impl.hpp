@@ -331,10 +331,9 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
       const TIn* src = in + inOff;
       A c = (A)0;
       if constexpr (F::kCentred && FIRST) c = acc_up<A>(out[outOff]);
-      for (I t = end + lane; VEC > 1 && t < stop; t += G) {  // the elements behind the last whole pack
-        const A x = acc_up<A>(src[t]);
-        acc[0] = f.combine(acc[0], FIRST ? f.modify(x, c) : x);
-      }
+      // the elements behind the last whole pack: a lane's first one is requested ahead of the packs and used behind them
+      A rest = (A)0;
+      if (VEC > 1 && end + lane < stop) rest = acc_up<A>(src[end + lane]);
       const I es = VEC == 1 ? sR : (I)1;  // element stride
       // U loads are issued back to back before any of them is consumed.
       constexpr int U = 8;
@@ -373,6 +372,10 @@ __global__ __launch_bounds__(kBlock) void reduce_rows_kernel(const TIn* __restri
             }
           }
         }
+      }
+      for (I t = end + lane; VEC > 1 && t < stop; t += G) {
+        const A x = t == end + lane ? rest : acc_up<A>(src[t]);
+        acc[0] = f.combine(acc[0], FIRST ? f.modify(x, c) : x);
       }
     }
     A r = acc[0];
@@ -2573,7 +2576,7 @@ void launch_rows_pass(THCState* s, const TIn* in, TOut* out, typename F::A* part
   const int pack = vec ? VEC : 1;
   const int64_t span = std::min(R, chunk);
   const int64_t perLane = tuning("reduce.rows.packs_per_lane", 8);
-  uint32_t G = pow2_ceil((uint64_t)((span + pack * perLane - 1) / (pack * perLane)));
+  uint32_t G = pow2_ceil((uint64_t)((span / pack + perLane - 1) / perLane));   // (whole packs: 1025 elements take the lanes of 1024)
   G = std::min<uint32_t>(64, std::max<uint32_t>(1, G));
   const int64_t groups = kBlock / G;
   const int64_t blocks = (numRows * S + groups - 1) / groups;
@@ -2652,6 +2655,9 @@ bool plan_rows_lds(THCState* s, const ReduceGeom& g, bool vec, uint32_t& rowsPer
 
 // Rows off the 16-byte grid are read as packs at element-aligned addresses from 1 KiB on, the elements behind the last whole
 // pack one by one (fp32 sums of 328 x 15366 11.2 -> 6.7 us, of 44 x 14186 7.6 -> 4.8, max 11.8 -> 8.1; 1000 x 9001 12.3 -> 7.1, 16.3 -> 10.0).
+// Lanes are counted by whole packs, and a row's last elements requested ahead of them: with the lanes of 2048 for 1025 elements, each
+// for half a batch, and a wait for the last ones first, many such rows were slower than one by one (sums, one by one, so and now:
+// 20000 x 1025 fp32 16.4, 18.5, 14.5 us, half 12.9, 17.5, 12.1; max of 20000 x 2050 half 22.3, 31.5, 20.1).
 template <typename T>
 bool loose_row_packs(const ReduceGeom& g) {
   return g.sR == 1 && g.R * (int64_t)sizeof(T) >= 1024 && tuning("reduce.rows.packs", 1);
@@ -3138,7 +3144,7 @@ void run_index_typed(THCState* s, const ReduceGeom& g, const T* in, T* outV, lon
     }
     const int64_t span = std::min(g.R, chunk);
     const int64_t perLane = tuning("reduce.rows.packs_per_lane", 8);
-    uint32_t G = pow2_ceil((uint64_t)((span + pack * perLane - 1) / (pack * perLane)));
+    uint32_t G = pow2_ceil((uint64_t)((span / pack + perLane - 1) / perLane));   // (whole packs: 1025 elements take the lanes of 1024)
     G = std::min<uint32_t>(64, std::max<uint32_t>(1, G));
     const int64_t groups = kBlock / G;
     const int grid = capped_grid(s, (rows * S + groups - 1) / groups, "reduce.rows.blocks_per_cu", 64);

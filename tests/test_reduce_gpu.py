@@ -940,6 +940,36 @@ def test_slices_of_few_rows_are_not_read_as_packs(thc, kind, shape, packs):
         assert np.allclose(var, want, rtol={"float": 1e-5, "half": 2e-3, "double": 1e-12}[kind], atol=1e-7), shape   # (half: 2^-24 steps)
 
 
+@pytest.mark.parametrize("kind", ["float", "half", "double", "byte", "int"])
+def test_elements_behind_the_last_whole_pack_of_a_row(thc, kind):
+    """Every number of them, in rows whose lanes are fewer than those elements (8 lanes of bytes for up to 15), around full batches of 8
+    packs a lane, and in rows cut into pieces; the largest value, the first of two, and a NaN among them."""
+    dtype = {"float": np.float32, "half": np.float16, "double": np.float64, "byte": np.uint8, "int": np.int32}[kind]
+    vec = 16 // np.dtype(dtype).itemsize
+    rng = np.random.default_rng(103)
+    for packs, rows in ((64, 50), (127, 9), (128, 1100), (256, 7), (512, 5), (513, 3), (6000, 2)):
+        for rest in range(vec):
+            n = packs * vec + rest
+            x = rng.integers(0, 3, (rows, n + 3)).astype(dtype)
+            x[:, 1 + n - 1 - min(rest, 1)] = 5                 # behind the last pack, or in it
+            x[0, n] = 5
+            x[:, -2:] = 77                                       # (past the window)
+            dev, host = thc.Tensor.from_numpy(x).narrow(1, 1, n), x[:, 1:1 + n]
+            if kind == "half":
+                assert host.sum(dtype=np.float64, axis=1).max() < 65504
+            assert_bit_equal(thc.Tensor(kind).sum(dev, 1).numpy(), host.astype(np.int64).sum(axis=1, keepdims=True).astype(dtype), "sum %d x %d" % (rows, n))
+            vals, idx = thc.Tensor(kind), thc.Tensor("long")
+            vals.max(idx, dev, 1)
+            assert_bit_equal(vals.numpy(), host.max(axis=1, keepdims=True), "max %d x %d" % (rows, n))
+            assert np.array_equal(idx.numpy(), host.argmax(axis=1)[:, None] + 1), (rows, n)
+            if kind in ("float", "half", "double") and rest:
+                host = host.copy()
+                host[rows - 1, n - 1] = np.nan
+                x[rows - 1, n] = np.nan
+                got = thc.Tensor(kind).sum(thc.Tensor.from_numpy(x).narrow(1, 1, n), 1).numpy()
+                assert_bit_equal(got, host.astype(np.float64).sum(axis=1, keepdims=True).astype(dtype), "NaN %d x %d" % (rows, n))
+
+
 @pytest.mark.parametrize("kind", ["float", "half", "double"])
 def test_var_of_small_slices_with_few_columns(thc, kind):
     """Threads that share a column's rows: columns one below and above what leaves several threads each, rows around the bands of 8."""
