@@ -1407,7 +1407,12 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
         vecRows && (sizeof(T) > 1 ? fills(32) || (sizeof(T) != 4 && fills(16)) || (sizeof(T) == 8 && fills(8)) ||
                                         (R <= 256 && packsC >= 24 && per_cu(32) >= 1)
                                   : R <= 200 && packsC >= 24 && per_cu(32) >= 0.5);
-    const bool fewRows = R <= 64 && total < (int64_t(5) << 19) && (32768 / rowBytes < 4 || R * rowBytes < 4 * 32768);
+    // Bytes, whose 128 elements a lane and 64-bit totals make a strip's chunk slow to scan, up to 512 rows (small tensors that the
+    // chunks below would not take either; us there and here: 1 x 200 x 257 6.8 and 13.1, 6 x 128 x 515 6.7 and 11.2, 1 x 65 x 1001 6.6, 8.8).
+    const int64_t rowsAChunk = std::max<int64_t>(1, 32768 / rowBytes);
+    const bool fewRows = total < (int64_t(5) << 19) &&
+                         (sizeof(T) == 1 && R > 64 ? R <= 512 && (rowsAChunk < 4 || (R + rowsAChunk - 1) / rowsAChunk < 4)
+                                                   : R <= 64 && (rowsAChunk < 4 || R * rowBytes < 4 * 32768));
     // Narrow rows are staged in LDS: a thread row's packs would lie too far apart.
     const bool narrow = rowBytes < 64 || (rowBytes < 128 && total >= (int64_t(128) << 20)) ||
                         (sizeof(T) == 1 && inner <= 350 && (R * inner <= 65536 || total >= (int64_t(32) << 20)));
@@ -1416,7 +1421,9 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       const int64_t packs = (inner + kFull - 1) / kFull;
       // Strips of 128 columns, as many words to look back over as two or more threads each share (fp32 and double: 32
       // lanes, 512-byte segments of a row; half 16, bytes 8: 65536 x 1000 bytes 61 us, 92 with 32 lanes). Rows that fit one
-      // chunk need nobody's totals: the widest strip that holds them all. 512 threads, 1024 where a chain would
+      // chunk need nobody's totals: the widest strip that holds them all, except large tensors of 4- and 8-byte elements, whose
+      // row pieces would be 128 bytes then (8 lanes and 32, R in 257..512, us: 40 x 300 x 1001 fp32 39.0 and 31.1, double 63.9 and 50.2, 1 x 300 x
+      // 100003 double 143.7 and 103.4; 6 x 257 x 1001, 12 MB, 10.7 and 13.5). 512 threads, 1024 where a chain would
       // have 256 chunks and more (51967 x 120 fp32 17.6 against 20.5; 8-byte sums stay at 512: 278737 x 164 189 against 210).
       const int64_t widest = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(8, 128 / kFull), kMaxStripLanes), packs);
       // (both knobs are held to what the kernel has room for and is built for; 0: as the rules say)
@@ -1428,7 +1435,8 @@ void launch_scan(THCState* s, T* out, const T* in, int64_t outer, int64_t R, int
       if (!threads) {
         threads = 512;
         bool oneChunk = false;
-        for (int64_t tx = std::min<int64_t>(kMaxStripLanes, packs); !oneChunk && (tx >= 8 || tx == packs); tx /= 2)
+        const int64_t least = sizeof(T) >= 4 && total >= (int64_t(20) << 20) ? 16 : 8;
+        for (int64_t tx = std::min<int64_t>(kMaxStripLanes, packs); !oneChunk && (tx >= least || tx == packs); tx /= 2)
           for (int64_t bt = 256; !oneChunk && bt <= 512; bt *= 2)
             if (rows_of(bt, tx) >= R) {
               TX = tx;

@@ -682,3 +682,28 @@ def test_gpu_strips_of_any_knob_value(thc, kind):
         thc.set_tuning("scan.slab", 1)
         thc.set_tuning("scan.strips.lanes", 0)
         thc.set_tuning("scan.strips.threads", 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,name", [((1, 200, 257), "scan-cols"), ((39, 128, 515), "scan-cols"), ((40, 128, 515), "scan-cols-split"), ((1, 65, 1001), "scan-cols"), ((6, 400, 131), "scan-cols"),
+                                        ((1, 600, 257), "scan-cols-split"), ((1, 300, 515), "scan-cols-split"), ((6, 65, 9001), "scan-cols-split")])
+def test_gpu_small_scans_of_bytes_along_a_strided_dim_are_not_chunked(thc, shape, name):
+    """Tensors of a few hundred rows of bytes stay with the column kernel, which is the faster one there."""
+    x = np.random.default_rng(101).integers(0, 9, shape).astype(np.uint8)
+    got = thc.Tensor("byte").cumsum(thc.Tensor.from_numpy(x), 1)
+    assert thc.last_kernel() == name, thc.last_kernel()
+    assert_bit_equal(got.numpy(), np.cumsum(x, axis=1, dtype=np.int64).astype(np.uint8), "%s" % (shape,))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["float", "double"])
+@pytest.mark.parametrize("rows", [256, 257, 300, 512, 513])
+def test_gpu_strips_of_a_few_hundred_rows(thc, kind, rows):
+    """On both sides of 20 MiB, from which on strips of 4- and 8-byte elements are cut along the rows instead of being made 128 bytes wide."""
+    dtype = {"float": np.float32, "double": np.float64}[kind]
+    for mb in (19.5, 20.5):
+        inner = int(mb * 2 ** 20 / (6 * rows * np.dtype(dtype).itemsize)) | 1
+        x = np.random.default_rng(rows).integers(-9, 10, (6, rows, inner)).astype(dtype)
+        got = thc.Tensor(kind).cumsum(thc.Tensor.from_numpy(x), 1)
+        assert thc.last_kernel() == "scan-cols-split", (inner, thc.last_kernel())
+        assert_bit_equal(got.numpy(), np.cumsum(x, axis=1, dtype=np.float64).astype(dtype), "%s %d x %d" % (kind, rows, inner))
