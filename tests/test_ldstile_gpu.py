@@ -453,3 +453,17 @@ def test_float_unary_on_transposed_operands(thc, oracle, shape, kernel):
         assert thc.last_kernel() == kernel, (shape, thc.last_kernel())
         oracle.pointwise("fn:" + name, ro, ra)
         assert_bit_equal(do.storage_numpy(), ro.storage, "%s %s" % (name, shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [8, 9, 24, 31, 32, 33, 123, 124, 125, 248, 249, 372])
+def test_shifted_windows_of_few_columns(thc, cols):
+    """Tiles of 248 columns leave out the passes of 32 columns that a narrow tensor, or the rest of a row, does not have."""
+    rng = np.random.default_rng(cols)
+    for rows, off in ((57, 1), (120, 3)):
+        x = rng.integers(-9, 10, 3 * rows * cols + off).astype(np.float16)
+        a = thc.Tensor.from_storage(x, off, (3, rows, cols), (rows * cols, 1, rows), kind="half")
+        host = x[off:].reshape(3, cols, rows).transpose(0, 2, 1)
+        out = thc.Tensor("half").resize((3, rows, cols)).mul(a, 3)
+        assert thc.last_kernel() == "tiled-shift", thc.last_kernel()
+        assert_bit_equal(out.numpy(), (host * np.float16(3)), "%d x %d" % (rows, cols))
